@@ -216,21 +216,20 @@ void fill_common(StageArgs& a, const ncn_shape* sh, const Plan& p, int stage, fl
     fill_step_table(a.tab, sh->n_cache, alpha, m, activation);
 }
 
-// With context lengths, after the main launch: the rows past the lengths pass through.  The register kernels run
-// the group a length cuts themselves (masked steps); the generic kernel leaves it to a second launch of its own,
-// one tile per batch entry.  `a` is the stage's argument block as the main launch used it.
+// With context lengths, after the main launch of the generic kernel: the group a length cuts (a second launch, one tile
+// per batch entry), then the rows past the lengths, which pass through.  The register kernels do both themselves.  `a`
+// is the stage's argument block as the main launch used it.
 hipError_t launch_ragged_rest(Pass pass, StageArgs a, const ncn_shape* sh, int path, int partial_rows_used,
                               hipStream_t s) {
-    if (path != 2) {
-        StageArgs e = a;
-        e.edge = 1;
-        e.total_tiles = (uint32_t)sh->batch;
-        e.tiles_per_inst = 1;
-        if (pass == kBackward) e.dw_partials = a.dw_partials + (int64_t)partial_rows_used * 2 * sh->E;
-        const int grid = (int)(sh->batch < kEdgeGridX ? sh->batch : kEdgeGridX);
-        hipError_t err = launch_generic(pass, e, sh->n_head, grid, s);
-        if (err != hipSuccess) return err;
-    }
+    if (path == 2) return hipSuccess;
+    StageArgs e = a;
+    e.edge = 1;
+    e.total_tiles = (uint32_t)sh->batch;
+    e.tiles_per_inst = 1;
+    if (pass == kBackward) e.dw_partials = a.dw_partials + (int64_t)partial_rows_used * 2 * sh->E;
+    const int grid = (int)(sh->batch < kEdgeGridX ? sh->batch : kEdgeGridX);
+    hipError_t err = launch_generic(pass, e, sh->n_head, grid, s);
+    if (err != hipSuccess) return err;
     return launch_pass_through(pass, a, sh->batch, s);
 }
 int edge_rows(const ncn_shape* sh) { return (int)(sh->batch < kEdgeGridX ? sh->batch : kEdgeGridX); }

@@ -222,8 +222,18 @@ __device__ __forceinline__ void headwise_backward_core(float (&Y)[R][F], float (
 
 #define NCN_HW_ROW_LIVE(rr) ((int)(((lane / T::LF) % T::LR) * R + (rr)) < live)
 
+// rows past a context length pass through, stored as they were loaded
+#define NCN_HW_PASS_DEAD(base0, base1, dtype, p, q)                                             \
+    if (INDEXED && __any(live >= 0 && live < NC)) {                                             \
+        _Pragma("unroll") for (int rr = 0; rr < R; ++rr) {                                      \
+            const bool dead = live >= 0 && !NCN_HW_ROW_LIVE(rr);                                \
+            store_frag<F>(base0, dtype, off[rr], dead, p[rr], A.plane);                         \
+            store_frag<F>(base1, dtype, off[rr], dead, q[rr], A.plane);                         \
+        }                                                                                       \
+    }
+
 // rows past a context length, and the lanes of a wave tile past the last group: loaded from rows that exist, zeroed
-// here, not stored
+// here, not stored with the results
 #define NCN_HW_ZERO_DEAD(p, q)                                                                  \
     if (__any(live != NC)) {                                                                    \
         _Pragma("unroll") for (int rr = 0; rr < R; ++rr) {                                      \
@@ -247,6 +257,8 @@ __global__ void __launch_bounds__(kBlockThreads) headwise_forward_kernel(const S
         issue_tile<R, F>(A.in1, A.in_dtype, off, a, A.plane);
         finish_tile<R, F>(A.in_dtype, x);
         finish_tile<R, F>(A.in_dtype, a);
+        NCN_HW_PASS_DEAD(A.out0, A.out1, A.out_dtype, x, a)
+        if (!INVERSE && A.aux0) { NCN_HW_PASS_DEAD(A.aux0, A.aux1, NCN_F32, x, a) }
         NCN_HW_ZERO_DEAD(x, a)
         if constexpr (INVERSE) {
             scale_tile<R, F>(x, a, A.tab.kappa, A.tab.b_scale);
@@ -298,6 +310,8 @@ __global__ void __launch_bounds__(kBlockThreads, (TANH_ONLY && !INDEXED && R * F
         finish_tile<R, F>(A.in_dtype, B);
         finish_tile<R, F>(A.g_dtype, G);
         if (A.g1) finish_tile<R, F>(A.g_dtype, H);
+        NCN_HW_PASS_DEAD(A.out0, A.out1, A.out_dtype, G, H)
+        if (A.aux0) { NCN_HW_PASS_DEAD(A.aux0, A.aux1, NCN_F32, Y, B) }
         NCN_HW_ZERO_DEAD(Y, B)
         NCN_HW_ZERO_DEAD(G, H)
         // as if the NC - live skipped steps of a cut group had been done: G, P carry m^-t
@@ -356,5 +370,6 @@ __global__ void __launch_bounds__(kBlockThreads, (TANH_ONLY && !INDEXED && R * F
 #undef NCN_HW_PROLOGUE
 #undef NCN_HW_ROW_LIVE
 #undef NCN_HW_ZERO_DEAD
+#undef NCN_HW_PASS_DEAD
 
 }  // namespace ncn
