@@ -1,0 +1,420 @@
+// Register-tile stage kernels for group sizes and head widths that are no powers of two.
+//
+// Same decomposition and step arithmetic as ncn_stage_kernels.h (see there for the formulas and their reference
+// citations), with a geometry that is chosen per launch instead of compiled in: a lane holds an R x F tile (R = 2..5
+// rows, F = 3..5 features), a row is spread over LF = 2^lf_log2 lanes and a group over
+// LR = 2^lr_log2 row lanes, so that R * LR covers n_cache rows and F * LF the head's features with little padding
+// (any_tile() in ncn_launch.h; 5 rows of 40 features: R = F = 5, LF = 8, LR = 1, nothing wasted).  What does not exist
+// is zero: padded features have zero weights and stay zero; padded rows have zero gradients, which stay zero, and never
+// are a pivot.  The feature of a lane's register f is f * LF + (lane % LF): a load instruction reads LF consecutive
+// elements of a row, at any alignment, where F consecutive ones per lane would touch every line F times over.
+//
+// What bounds it: vector issue, as for the shapes of powers of two; the levels of the cross-lane sums are taken under
+// wave-uniform branches because LF and LR are not known at compile time.  One lane per row with the state in LDS (the
+// generic kernels, which still take what fits no tile and scalars outside the scaled state) leaves three quarters of
+// the time to LDS traffic and its barriers.
+// 16 x 1005 x 160 float32, groups of 5 rows, heads of 40: forward 113 -> 17.6 us, backward 519 -> 31.7 us per stage.
+#pragma once
+#include <type_traits>
+
+#include "ncn_stage_kernels.h"
+
+namespace ncn {
+
+// sums over the lanes {lane ^ k * 2^LO : k} for the levels LO <= level < HI, LO = 0 or (FROM0 = false) `lo`
+template <int N>
+__device__ __forceinline__ void any_sum_rows(float (&v)[N], int hi) {   // over the 2^hi lanes of a row
+#define NCN_LEVEL(S)                                                    \
+    _Pragma("unroll") for (int k = 0; k < N; ++k) v[k] += lane_xor<S, true>(v[k]);
+    if (hi > 0) {
+        NCN_LEVEL(1)
+        if (hi > 1) {
+            NCN_LEVEL(2)
+            if (hi > 2) {
+                NCN_LEVEL(4)
+                if (hi > 3) {
+                    NCN_LEVEL(8)
+                    if (hi > 4) { NCN_LEVEL(16) }
+                }
+            }
+        }
+    }
+}
+template <int N>
+__device__ __forceinline__ void any_sum_span(float (&v)[N], int lo, int hi) {   // over lane bits lo .. hi-1
+    if (lo >= hi) return;
+    if (lo <= 0) { NCN_LEVEL(1) }
+    if (lo <= 1 && hi > 1) { NCN_LEVEL(2) }
+    if (lo <= 2 && hi > 2) { NCN_LEVEL(4) }
+    if (lo <= 3 && hi > 3) { NCN_LEVEL(8) }
+    if (lo <= 4 && hi > 4) { NCN_LEVEL(16) }
+    if (lo <= 5 && hi > 5) { NCN_LEVEL(32) }
+#undef NCN_LEVEL
+}
+
+// One wave tile of a launch: where this lane's rows and features are.
+template <int R, int F, bool LENGTHS>
+struct AnyLane {
+    int lfl, lrl, fl, rl, gw;   // log2 of lanes per row and row lanes per group; this lane's place
+    int feat[F];                // feature of register f, clamped into the head
+    bool has[F];                // that feature exists
+    int64_t entry;              // element offset of the tile's batch entry (wave-uniform)
+    uint32_t row[R];            // elements from there to the row's head slice: 32-bit offsets from a scalar base
+    int live;                   // live rows of the lane's group, -1 past the last group
+    __device__ __forceinline__ void place(const StageArgs& A, int lane) {
+        lfl = (A.any_tile >> 16) & 0xff;
+        lrl = A.any_tile >> 24;
+        fl = lane & ((1 << lfl) - 1);
+        rl = (lane >> lfl) & ((1 << lrl) - 1);
+        gw = lane >> (lfl + lrl);
+#pragma unroll
+        for (int f = 0; f < F; ++f) {
+            const int k = (f << lfl) + fl;
+            has[f] = k < A.head_dim;
+            feat[f] = min(k, A.head_dim - 1);
+        }
+    }
+    __device__ __forceinline__ void rows(const StageArgs& A, uint32_t t, int head) {
+        const uint32_t b = t / A.tiles_per_inst;
+        const uint32_t group = (t - b * A.tiles_per_inst) * (64u >> (lfl + lrl)) + gw;
+        const bool valid = group < A.groups;
+        live = !valid ? -1 : LENGTHS ? live_rows(A, b, group) : A.n_cache;
+        entry = (int64_t)b * A.N * A.E;
+#pragma unroll
+        for (int rr = 0; rr < R; ++rr) {
+            const uint32_t slot = min(rl * R + rr, A.n_cache - 1);
+            row[rr] = (uint32_t)slot_position(A, valid ? group : 0u, slot) * (uint32_t)A.E + head * A.head_dim;
+        }
+    }
+    // Between the loads and the stores of a tile: the compiler would otherwise keep the R x F element offsets it made for
+    // the loads in registers across the steps instead of making them again.
+    __device__ __forceinline__ void forget_offsets() {
+#pragma unroll
+        for (int rr = 0; rr < R; ++rr) asm volatile("" : "+v"(row[rr]));
+    }
+    // the row is one of the group's: it takes part in the steps (run) or lies past a context length (pass)
+    __device__ __forceinline__ bool run(int rr) const { return rl * R + rr < live; }
+    __device__ __forceinline__ bool pass(const StageArgs& A, int rr) const {
+        return live >= 0 && rl * R + rr >= live && rl * R + rr < A.n_cache;
+    }
+};
+
+template <typename T>
+__device__ __forceinline__ T* any_at(T* entry, uint32_t elem) {
+    return reinterpret_cast<T*>(reinterpret_cast<uintptr_t>(entry) + (uint32_t)(elem * sizeof(T)));
+}
+
+// The loads of a tile, as raw words (converted by any_finish), so that those of all arrays of a tile are under way together.
+template <int R, int F, bool LENGTHS>
+__device__ __forceinline__ void any_issue(const void* base, int dtype, const AnyLane<R, F, LENGTHS>& L, float (&v)[R][F]) {
+    if (dtype == NCN_F32) {
+#pragma unroll
+        for (int rr = 0; rr < R; ++rr)
+#pragma unroll
+            for (int f = 0; f < F; ++f) v[rr][f] = *any_at(static_cast<const float*>(base) + L.entry, L.row[rr] + L.feat[f]);
+    } else {
+#pragma unroll
+        for (int rr = 0; rr < R; ++rr)
+#pragma unroll
+            for (int f = 0; f < F; ++f)
+                v[rr][f] = __uint_as_float(*any_at(static_cast<const uint16_t*>(base) + L.entry, L.row[rr] + L.feat[f]));
+    }
+}
+template <int R, int F>
+__device__ __forceinline__ void any_finish(int dtype, float (&v)[R][F]) {
+    if (dtype == NCN_F32) return;
+#pragma unroll
+    for (int rr = 0; rr < R; ++rr)
+#pragma unroll
+        for (int f = 0; f < F; ++f) v[rr][f] = __uint_as_float(__float_as_uint(v[rr][f]) << 16);
+}
+template <int R, int F, bool LENGTHS>
+__device__ __forceinline__ void any_zero_padding(const AnyLane<R, F, LENGTHS>& L, float (&v)[R][F]) {
+#pragma unroll
+    for (int rr = 0; rr < R; ++rr)
+#pragma unroll
+        for (int f = 0; f < F; ++f) v[rr][f] = L.run(rr) && L.has[f] ? v[rr][f] : 0.f;
+}
+// both arrays of a pair, the rows that take part in the steps (DEAD = false) or those that pass through
+template <bool DEAD, int R, int F, bool LENGTHS>
+__device__ __forceinline__ void any_store(const StageArgs& A, const AnyLane<R, F, LENGTHS>& L, void* base0, void* base1, int dtype,
+                                          const float (&p)[R][F], const float (&q)[R][F]) {
+#pragma unroll
+    for (int rr = 0; rr < R; ++rr)
+        if (DEAD ? L.pass(A, rr) : L.run(rr)) {
+#pragma unroll
+            for (int f = 0; f < F; ++f)
+                if (L.has[f]) {
+                    const uint32_t at = L.row[rr] + L.feat[f];
+                    if (dtype == NCN_F32) {
+                        *any_at(static_cast<float*>(base0) + L.entry, at) = p[rr][f];
+                        *any_at(static_cast<float*>(base1) + L.entry, at) = q[rr][f];
+                    } else {
+                        const uint32_t pq = pack_bf16x2(p[rr][f], q[rr][f]);
+                        *any_at(static_cast<uint16_t*>(base0) + L.entry, at) = (uint16_t)pq;
+                        *any_at(static_cast<uint16_t*>(base1) + L.entry, at) = (uint16_t)(pq >> 16);
+                    }
+                }
+        }
+}
+
+// The pivot row's fragment for every lane of its group (row lane jo holds it), through wave-private LDS slots; a wave's
+// LDS operations complete in order, so no barrier.
+template <int F>
+__device__ __forceinline__ void any_broadcast(const float (&v)[F], float (&out)[F], bool many, int src, int lane, float* slots) {
+    if (!many) {
+#pragma unroll
+        for (int f = 0; f < F; ++f) out[f] = v[f];
+        return;
+    }
+#pragma unroll
+    for (int f = 0; f < F; ++f) slots[f * 64 + lane] = v[f];
+#pragma unroll
+    for (int f = 0; f < F; ++f) out[f] = slots[f * 64 + src];
+}
+
+template <int R, int F>
+__device__ __forceinline__ void any_row_sums(const float (&x)[R][F], const float (&wi)[F], float e, int lfl, float (&c)[R]) {
+#pragma unroll
+    for (int rr = 0; rr < R; ++rr) {
+        c[rr] = e;
+#pragma unroll
+        for (int f = 0; f < F; ++f) c[rr] = fmaf(x[rr][f], wi[f], c[rr]);
+    }
+    any_sum_rows<R>(c, lfl);
+}
+
+// f(0), f(1), .., f(N-1) with the index a compile-time constant.  (An unrolled loop over the pivot rows is not enough: with
+// a step that may be skipped the compiler gives the tile a place in scratch memory before it unrolls.)
+template <int N, int I = 0, typename Fn>
+__device__ __forceinline__ void for_each_row(const Fn& f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        for_each_row<N, I + 1>(f);
+    }
+}
+
+#define NCN_ANY_PROLOGUE                                                                        \
+    const int lane = threadIdx.x & 63;                                                          \
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);                          \
+    const uint32_t gwave = blockIdx.x * kWavesPerBlock + wave;                                  \
+    const int head = gwave % A.n_head;                                                          \
+    const uint32_t tile_step = gridDim.x * kWavesPerBlock / A.n_head;                           \
+    __shared__ float bcast_lds[kWavesPerBlock * F * 64];                                        \
+    float* slots = bcast_lds + wave * F * 64;                                                   \
+    AnyLane<R, F, LENGTHS> L;                                                                            \
+    L.place(A, lane);                                                                           \
+    const int lr = 1 << L.lrl;                                                                  \
+    const StepTable& S = A.tab;                                                                 \
+    float wi[F], wj[F];                                                                         \
+    _Pragma("unroll") for (int f = 0; f < F; ++f) {                                             \
+        const float* w = A.W + (int64_t)head * A.head_dim + L.feat[f];                          \
+        wi[f] = L.has[f] ? S.gamma * w[0] : 0.f;                                                \
+        wj[f] = L.has[f] ? S.gamma * w[A.E] : 0.f;                                              \
+    }
+
+// INVERSE = false: x, xa -> y, ya (optional float32 copies);  true: y, ya -> x, xa
+template <int R, int F, bool TANH_ONLY, bool INVERSE, bool LENGTHS>
+__global__ void __launch_bounds__(kBlockThreads, R * F <= 16 ? 4 : R * F <= 20 ? 3 : 2) any_forward_kernel(const StageArgs A) {
+    NCN_ANY_PROLOGUE
+    for (uint32_t t = gwave / A.n_head; t < A.total_tiles; t += tile_step) {
+        L.rows(A, t, head);
+        float x[R][F], a[R][F];
+        any_issue(A.in0, A.in_dtype, L, x);
+        any_issue(A.in1, A.in_dtype, L, a);
+        any_finish(A.in_dtype, x);
+        any_finish(A.in_dtype, a);
+        if (LENGTHS) {   // rows past a context length pass through
+            any_store<true>(A, L, A.out0, A.out1, A.out_dtype, x, a);
+            if (!INVERSE && A.aux0) any_store<true>(A, L, A.aux0, A.aux1, NCN_F32, x, a);
+        }
+        any_zero_padding(L, x);
+        any_zero_padding(L, a);
+        scale_tile<R, F>(x, a, S.kappa, INVERSE ? S.b_scale : S.a_scale);
+#pragma unroll 1
+        for (int k = 0; k < lr; ++k) {
+            const int jo = INVERSE ? lr - 1 - k : k;
+            const int src = (lane & ~((lr - 1) << L.lfl)) | (jo << L.lfl);
+            for_each_row<R>([&](auto q) __attribute__((always_inline)) {
+                constexpr int jr = INVERSE ? R - 1 - q.value : q.value;
+                if (jo * R + jr >= (LENGTHS ? L.live : A.n_cache)) return;   // LENGTHS: the lanes of a group agree
+                if constexpr (INVERSE) {
+#pragma unroll
+                    for (int rr = 0; rr < R; ++rr)
+#pragma unroll
+                        for (int f = 0; f < F; ++f) x[rr][f] = fmaf(S.im, x[rr][f], -a[rr][f]);
+                }
+                float xj[F], c[R];
+                any_broadcast<F>(x[jr], xj, lr > 1, src, lane, slots);
+                any_row_sums<R, F>(x, wi, dot_chain<F>(xj, wj), L.lfl, c);
+#pragma unroll
+                for (int rr = 0; rr < R; ++rr)
+#pragma unroll
+                    for (int f = 0; f < F; ++f) {
+                        const float z = fmaf(c[rr], xj[f], x[rr][f]);
+                        const float keep = INVERSE ? S.im : S.m;
+                        if constexpr (TANH_ONLY) {
+                            const float r = __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(z) + 1.0f);
+                            a[rr][f] = fmaf(INVERSE ? S.bk1 : S.m2k2, r, fmaf(keep, a[rr][f], INVERSE ? S.bk0 : S.k2));
+                        } else {
+                            float Fv, w;
+                            act_Fw(z, S.activation, Fv, w);
+                            a[rr][f] = fmaf(INVERSE ? S.bk0 : S.k2, Fv, keep * a[rr][f]);
+                        }
+                        if constexpr (!INVERSE) x[rr][f] = fmaf(S.m, x[rr][f], a[rr][f]);
+                    }
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        }
+        L.forget_offsets();
+        scale_tile<R, F>(x, a, S.inv_kappa, INVERSE ? S.inv_b_scale : S.inv_a_scale);
+        any_store<false>(A, L, A.out0, A.out1, A.out_dtype, x, a);
+        if (!INVERSE && A.aux0) any_store<false>(A, L, A.aux0, A.aux1, NCN_F32, x, a);
+    }
+}
+
+template <int R, int F, bool TANH_ONLY, bool LENGTHS>
+__global__ void __launch_bounds__(kBlockThreads, R * F <= 10 ? 4 : R * F <= 16 ? 3 : 2) any_backward_kernel(const StageArgs A) {
+    NCN_ANY_PROLOGUE
+    float dwi[F], dwj[F], wiku[F];
+#pragma unroll
+    for (int f = 0; f < F; ++f) {
+        dwi[f] = dwj[f] = 0.f;
+        wiku[f] = S.ku * wi[f];
+    }
+    for (uint32_t t = gwave / A.n_head; t < A.total_tiles; t += tile_step) {
+        L.rows(A, t, head);
+        float Y[R][F], B[R][F], G[R][F], P[R][F];
+        any_issue(A.in0, A.in_dtype, L, Y);
+        any_issue(A.in1, A.in_dtype, L, B);
+        any_issue(A.g0, A.g_dtype, L, G);
+        if (A.g1) {
+            any_issue(A.g1, A.g_dtype, L, P);
+        } else {
+#pragma unroll
+            for (int rr = 0; rr < R; ++rr)
+#pragma unroll
+                for (int f = 0; f < F; ++f) P[rr][f] = 0.f;
+        }
+        any_finish(A.in_dtype, Y);
+        any_finish(A.in_dtype, B);
+        any_finish(A.g_dtype, G);
+        if (A.g1) any_finish(A.g_dtype, P);
+        if (LENGTHS) {
+            any_store<true>(A, L, A.out0, A.out1, A.out_dtype, G, P);
+            if (A.aux0) any_store<true>(A, L, A.aux0, A.aux1, NCN_F32, Y, B);
+        }
+        any_zero_padding(L, Y);
+        any_zero_padding(L, B);
+        any_zero_padding(L, G);
+        any_zero_padding(L, P);
+        // as if the steps that a group cut by a context length skips had been done: G, P carry m^-t
+        const float isc = LENGTHS && L.live < A.n_cache ? pow_steps(S.im, A.n_cache - L.live) : 1.0f;
+#pragma unroll
+        for (int rr = 0; rr < R; ++rr)
+#pragma unroll
+            for (int f = 0; f < F; ++f) {
+                Y[rr][f] *= S.kappa;
+                B[rr][f] *= S.b_scale;
+                P[rr][f] = isc * fmaf(S.om, G[rr][f], P[rr][f]);   // h -> p
+                G[rr][f] *= isc;
+            }
+#pragma unroll 1
+        for (int jo = lr - 1; jo >= 0; --jo) {
+            const float selku = L.rl == jo ? S.ku : 0.f;   // this lane holds the pivot row
+            const int src = (lane & ~((lr - 1) << L.lfl)) | (jo << L.lfl);
+            for_each_row<R>([&](auto q) __attribute__((always_inline)) {
+                constexpr int jr = R - 1 - q.value;
+                const int j = jo * R + jr;
+                if (j >= (LENGTHS ? L.live : A.n_cache)) return;
+                const float krho = S.krho[A.n_cache - 1 - j];
+#pragma unroll
+                for (int rr = 0; rr < R; ++rr)
+#pragma unroll
+                    for (int f = 0; f < F; ++f) Y[rr][f] = fmaf(S.im, Y[rr][f], -B[rr][f]);
+                float xj[F], c[R], rh[R], v[F];
+                any_broadcast<F>(Y[jr], xj, lr > 1, src, lane, slots);
+                any_row_sums<R, F>(Y, wi, dot_chain<F>(xj, wj), L.lfl, c);
+#pragma unroll
+                for (int f = 0; f < F; ++f) v[f] = 0.f;
+#pragma unroll
+                for (int rr = 0; rr < R; ++rr) {
+                    rh[rr] = 0.f;
+#pragma unroll
+                    for (int f = 0; f < F; ++f) {
+                        const float z = fmaf(c[rr], xj[f], Y[rr][f]);
+                        float w;
+                        if constexpr (TANH_ONLY) {
+                            const float r = __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(z) + 1.0f);
+                            B[rr][f] = fmaf(S.bk1, r, fmaf(S.im, B[rr][f], S.bk0));
+                            w = fmaf(-r, r, r);
+                        } else {
+                            float Fv;
+                            act_Fw(z, S.activation, Fv, w);
+                            B[rr][f] = fmaf(S.bk0, Fv, S.im * B[rr][f]);
+                        }
+                        const float U = P[rr][f] * w;
+                        rh[rr] = fmaf(U, xj[f], rh[rr]);
+                        v[f] = fmaf(c[rr], U, v[f]);
+                        G[rr][f] = fmaf(S.ku, U, G[rr][f]);
+                    }
+                }
+                any_sum_rows<R>(rh, L.lfl);
+                float rhosum = 0.f;
+#pragma unroll
+                for (int rr = 0; rr < R; ++rr) {
+                    const float rho_w = krho * rh[rr];
+                    rhosum += rh[rr];
+#pragma unroll
+                    for (int f = 0; f < F; ++f) {
+                        dwi[f] = fmaf(rho_w, Y[rr][f], dwi[f]);
+                        G[rr][f] = fmaf(rh[rr], wiku[f], G[rr][f]);
+                        if (rr != jr) P[rr][f] = fmaf(S.om, G[rr][f], P[rr][f]);
+                    }
+                }
+                const float rhosum_w = krho * rhosum;
+                float s[F];
+#pragma unroll
+                for (int f = 0; f < F; ++f) {
+                    dwj[f] = fmaf(rhosum_w, xj[f], dwj[f]);
+                    s[f] = fmaf(rhosum, wj[f], v[f]);
+                }
+                any_sum_span<F>(s, L.lfl, L.lfl + L.lrl);   // over the group's row lanes
+#pragma unroll
+                for (int f = 0; f < F; ++f) {
+                    G[jr][f] = fmaf(selku, s[f], G[jr][f]);
+                    P[jr][f] = fmaf(S.om, G[jr][f], P[jr][f]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        }
+#pragma unroll
+        for (int rr = 0; rr < R; ++rr)
+#pragma unroll
+            for (int f = 0; f < F; ++f) {
+                G[rr][f] *= S.m_pow_n;
+                P[rr][f] = fmaf(P[rr][f], S.m_pow_n, -S.om * G[rr][f]);   // back to h = p - (1-m) g
+            }
+        L.forget_offsets();
+        any_store<false>(A, L, A.out0, A.out1, A.out_dtype, G, P);
+        if (A.aux0) {
+            scale_tile<R, F>(Y, B, S.inv_kappa, S.inv_b_scale);
+            any_store<false>(A, L, A.aux0, A.aux1, NCN_F32, Y, B);
+        }
+    }
+    // dW: lanes holding the same features -> one value; this wave owns slot (gwave / n_head, head)
+    any_sum_span<F>(dwi, L.lfl, 6);
+    any_sum_span<F>(dwj, L.lfl, 6);
+    if (lane < (1 << L.lfl)) {
+        float* out = A.dw_partials + (int64_t)(gwave / A.n_head) * (2 * A.E) + (int64_t)head * A.head_dim;
+#pragma unroll
+        for (int f = 0; f < F; ++f)
+            if (L.has[f]) {
+                out[L.feat[f]] = dwi[f];
+                out[A.E + L.feat[f]] = dwj[f];
+            }
+    }
+}
+#undef NCN_ANY_PROLOGUE
+
+}  // namespace ncn

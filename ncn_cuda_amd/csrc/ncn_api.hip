@@ -49,6 +49,13 @@ int kernel_path_for(const ncn_shape* sh, int activation, float alpha, float m) {
     return (sh->E / sh->n_head <= kGenericMaxHeadDim) ? 1 : 0;
 }
 
+// The register tile that runs a path-1 call: any group that fits a wave, with scalars that fit the scaled state.  Offsets
+// inside a batch entry are 32-bit byte counts there.
+AnyTile any_tile_for(const ncn_shape* sh, int path, float alpha, float m) {
+    if (path != 1 || !scalars_fit_scaled_state(alpha, m) || sh->N * sh->E >= (int64_t)1 << 29) return AnyTile{0, 0, 0, 0};
+    return any_tile(sh->n_cache, (int)(sh->E / sh->n_head));
+}
+
 int check_shape(const ncn_shape* sh, int first_stage, int n_stages, int activation) {
     if (!sh) return NCN_ERR_NULL;
     if (sh->batch <= 0 || sh->N <= 0 || sh->E <= 0 || sh->n_head <= 0 || sh->n_cache <= 0) return NCN_ERR_SHAPE;
@@ -76,6 +83,7 @@ uint32_t stage_stride(int stage, uint32_t groups) {
 
 struct Plan {
     int path;
+    AnyTile any;       // path 1 on the register tiles of ncn_anyshape_kernels.h (any.r != 0), else the generic kernels
     int groups_per_tile;
     uint32_t groups, tiles_per_inst, total_tiles;
     int grid_x;        // backward launch
@@ -85,16 +93,18 @@ struct Plan {
 
 // reserve_rows: rows of the dW partial buffer kept free for another launch of the same stage
 // row_cap: rows of the dW partial buffer the caller has (kMaxGridX in a workspace of ncn_workspace_bytes)
-Plan make_plan(const ncn_shape* sh, int path, int reserve_rows = 0, int row_cap = kMaxGridX) {
+Plan make_plan(const ncn_shape* sh, int path, const AnyTile& any, int reserve_rows = 0, int row_cap = kMaxGridX) {
     Plan p;
     const int max_rows = row_cap - reserve_rows;
     p.path = path;
+    p.any = any;
     const int ec = (int)(sh->E / sh->n_head);
-    p.groups_per_tile = (p.path == 2) ? fast_groups_per_tile(sh->n_cache, ec) : generic_groups_per_tile(sh->n_cache);
+    p.groups_per_tile = any.r ? 64 >> (any.lf_log2 + any.lr_log2)
+                              : (p.path == 2) ? fast_groups_per_tile(sh->n_cache, ec) : generic_groups_per_tile(sh->n_cache);
     p.groups = (uint32_t)(sh->N / sh->n_cache);
     p.tiles_per_inst = (p.groups + p.groups_per_tile - 1) / p.groups_per_tile;
     p.total_tiles = (uint32_t)(sh->batch * p.tiles_per_inst);
-    if (p.path == 2) {
+    if (p.path == 2 || any.r) {
         // 4 waves per block, wave w works on head w % n_head: the grid holds a multiple of n_head waves and at
         // most kMaxGridX partial rows (one per n_head consecutive waves)
         const int C = sh->n_head;
@@ -209,6 +219,7 @@ void fill_common(StageArgs& a, const ncn_shape* sh, const Plan& p, int stage, fl
     a.groups = p.groups;
     a.stride = stage_stride(stage, p.groups);
     a.groups_pow2 = (p.groups & (p.groups - 1)) == 0 ? 1u : 0u;
+    a.any_tile = (uint32_t)(p.any.r | p.any.f << 8 | p.any.lf_log2 << 16 | p.any.lr_log2 << 24);
     a.n_cache = sh->n_cache;
     a.head_dim = (int)(sh->E / sh->n_head);
     a.n_head = sh->n_head;
@@ -217,11 +228,11 @@ void fill_common(StageArgs& a, const ncn_shape* sh, const Plan& p, int stage, fl
 }
 
 // With context lengths, after the main launch of the generic kernel: the group a length cuts (a second launch, one tile
-// per batch entry), then the rows past the lengths, which pass through.  The register kernels do both themselves.  `a`
+// per batch entry), then the rows past the lengths, which pass through.  The register-tile kernels do both themselves.  `a`
 // is the stage's argument block as the main launch used it.
-hipError_t launch_ragged_rest(Pass pass, StageArgs a, const ncn_shape* sh, int path, int partial_rows_used,
+hipError_t launch_ragged_rest(Pass pass, StageArgs a, const ncn_shape* sh, const Plan& p, int partial_rows_used,
                               hipStream_t s) {
-    if (path == 2) return hipSuccess;
+    if (p.path == 2 || p.any.r) return hipSuccess;
     StageArgs e = a;
     e.edge = 1;
     e.total_tiles = (uint32_t)sh->batch;
@@ -249,16 +260,21 @@ const ncn_shape* planning_shape(const ncn_shape* sh, ncn_shape* as_wide) {
     return headwise_call(sh, 2, as_wide) ? as_wide : sh;
 }
 
-// one stage on the register kernels: the plain builds know the stride permutation only, the others read the
-// launch's table, radix level and context lengths
-hipError_t run_forward_kernel(Pass pass, const StageArgs& a, bool plain, bool headwise, int n_head, int grid,
-                              hipStream_t s) {
-    if (headwise) return plain ? launch_headwise_forward(pass, a, grid, s) : launch_headwise_forward_indexed(pass, a, grid, s);
-    return plain ? launch_fast_forward(pass, a, n_head, grid, s) : launch_fast_forward_indexed(pass, a, n_head, grid, s);
+// One stage.  Register kernels: the plain builds know the stride permutation only, the others read the launch's table,
+// radix level and context lengths.
+hipError_t run_forward_kernel(Pass pass, const StageArgs& a, const Plan& p, bool plain, bool headwise, hipStream_t s) {
+    if (p.any.r) return launch_any_forward(pass, a, p.grid_fwd, s);
+    if (p.path != 2) return launch_generic(pass, a, a.n_head, p.grid_fwd, s);
+    if (headwise)
+        return plain ? launch_headwise_forward(pass, a, p.grid_fwd, s) : launch_headwise_forward_indexed(pass, a, p.grid_fwd, s);
+    return plain ? launch_fast_forward(pass, a, a.n_head, p.grid_fwd, s)
+                 : launch_fast_forward_indexed(pass, a, a.n_head, p.grid_fwd, s);
 }
-hipError_t run_backward_kernel(const StageArgs& a, bool plain, bool headwise, int n_head, int grid, hipStream_t s) {
-    if (headwise) return plain ? launch_headwise_backward(a, grid, s) : launch_headwise_backward_indexed(a, grid, s);
-    return plain ? launch_fast_backward(a, n_head, grid, s) : launch_fast_backward_indexed(a, n_head, grid, s);
+hipError_t run_backward_kernel(const StageArgs& a, const Plan& p, bool plain, bool headwise, hipStream_t s) {
+    if (p.any.r) return launch_any_backward(a, p.grid_x, s);
+    if (p.path != 2) return launch_generic(kBackward, a, a.n_head, p.grid_x, s);
+    if (headwise) return plain ? launch_headwise_backward(a, p.grid_x, s) : launch_headwise_backward_indexed(a, p.grid_x, s);
+    return plain ? launch_fast_backward(a, a.n_head, p.grid_x, s) : launch_fast_backward_indexed(a, a.n_head, p.grid_x, s);
 }
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
@@ -485,7 +501,7 @@ static int forward_impl(const void* x, const void* xa, int in_dtype, void* y, vo
     if (!aligned16(x) || !aligned16(xa) || !aligned16(y) || !aligned16(ya) || !aligned16(W) || !aligned16(y32) ||
         !aligned16(ya32) || !aligned16(workspace))
         return NCN_ERR_ALIGN;
-    const Plan p = make_plan(shape, path);
+    const Plan p = make_plan(shape, path, any_tile_for(shape, path, alpha, m));
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int64_t wstride = 2 * shape->E;
 
@@ -502,8 +518,8 @@ static int forward_impl(const void* x, const void* xa, int in_dtype, void* y, vo
         a.out0 = o0; a.out1 = o1; a.out_dtype = o_dtype;
         a.aux0 = with_copies ? y32 : nullptr; a.aux1 = with_copies ? ya32 : nullptr;
         a.W = W + k * wstride;
-        hipError_t err = run_forward_kernel(kForward, a, grouping.plain(), headwise, shape->n_head, p.grid_fwd, s);
-        if (err == hipSuccess && grouping.ctx_len) err = launch_ragged_rest(kForward, a, shape, p.path, 0, s);
+        hipError_t err = run_forward_kernel(kForward, a, p, grouping.plain(), headwise, s);
+        if (err == hipSuccess && grouping.ctx_len) err = launch_ragged_rest(kForward, a, shape, p, 0, s);
         return err;
     };
     bool fused_ok = np > 0 && (np < 2 || out_dtype == NCN_F32);
@@ -585,9 +601,8 @@ static int forward_impl(const void* x, const void* xa, int in_dtype, void* y, vo
         a.aux0 = last ? y32 : nullptr;
         a.aux1 = last ? ya32 : nullptr;
         a.W = W + k * wstride;
-        hipError_t err = (p.path != 2) ? launch_generic(kForward, a, shape->n_head, p.grid_fwd, s)
-                                       : run_forward_kernel(kForward, a, grouping.plain(), headwise, shape->n_head, p.grid_fwd, s);
-        if (err == hipSuccess && grouping.ctx_len) err = launch_ragged_rest(kForward, a, shape, p.path, 0, s);
+        hipError_t err = run_forward_kernel(kForward, a, p, grouping.plain(), headwise, s);
+        if (err == hipSuccess && grouping.ctx_len) err = launch_ragged_rest(kForward, a, shape, p, 0, s);
         if (err != hipSuccess) return (int)err;
     }
     return NCN_OK;
@@ -609,7 +624,7 @@ static int inverse_impl(const void* y, const void* ya, int in_dtype, void* x, vo
     if (!known_dtype_or_x2(in_dtype, n_stages, path) || !known_dtype(out_dtype)) return NCN_ERR_DTYPE;
     if (!aligned16(x) || !aligned16(xa) || !aligned16(y) || !aligned16(ya) || !aligned16(W) || !aligned16(workspace))
         return NCN_ERR_ALIGN;
-    const Plan p = make_plan(shape, path);
+    const Plan p = make_plan(shape, path, any_tile_for(shape, path, alpha, m));
     hipStream_t s = static_cast<hipStream_t>(stream);
 
     // several stages: LDS-resident passes, last pass of the range first.  Without scratch to ping-pong with, the
@@ -624,8 +639,8 @@ static int inverse_impl(const void* y, const void* ya, int in_dtype, void* x, vo
         a.in0 = i0; a.in1 = i1; a.in_dtype = i_dtype;
         a.out0 = o0; a.out1 = o1; a.out_dtype = o_dtype;
         a.W = W + (int64_t)k * 2 * shape->E;
-        hipError_t err = run_forward_kernel(kInverse, a, grouping.plain(), headwise, shape->n_head, p.grid_fwd, s);
-        if (err == hipSuccess && grouping.ctx_len) err = launch_ragged_rest(kInverse, a, shape, p.path, 0, s);
+        hipError_t err = run_forward_kernel(kInverse, a, p, grouping.plain(), headwise, s);
+        if (err == hipSuccess && grouping.ctx_len) err = launch_ragged_rest(kInverse, a, shape, p, 0, s);
         return err;
     };
     // With scratch every pass reads one pair of buffers and writes another (scratch and x, xa in turns, so that the
@@ -703,9 +718,8 @@ static int inverse_impl(const void* y, const void* ya, int in_dtype, void* x, vo
         a.out1 = xa;
         a.out_dtype = out_dtype;
         a.W = W + (int64_t)k * 2 * shape->E;
-        hipError_t err = (p.path != 2) ? launch_generic(kInverse, a, shape->n_head, p.grid_fwd, s)
-                                       : run_forward_kernel(kInverse, a, grouping.plain(), headwise, shape->n_head, p.grid_fwd, s);
-        if (err == hipSuccess && grouping.ctx_len) err = launch_ragged_rest(kInverse, a, shape, p.path, 0, s);
+        hipError_t err = run_forward_kernel(kInverse, a, p, grouping.plain(), headwise, s);
+        if (err == hipSuccess && grouping.ctx_len) err = launch_ragged_rest(kInverse, a, shape, p, 0, s);
         if (err != hipSuccess) return (int)err;
     }
     return NCN_OK;
@@ -739,8 +753,9 @@ static int backward_impl(const void* y, const void* ya, int y_dtype, const void*
         !aligned16(x_rec) || !aligned16(xa_rec) || !aligned16(W) || !aligned16(dW) || !aligned16(workspace))
         return NCN_ERR_ALIGN;
     // partial rows of the generic kernel's second launch
-    const int extra_rows = (grouping.ctx_len && path != 2) ? edge_rows(shape) : 0;
-    const Plan p = make_plan(shape, path, extra_rows, row_cap);
+    const AnyTile any = any_tile_for(shape, path, alpha, m);
+    const int extra_rows = (grouping.ctx_len && path != 2 && !any.r) ? edge_rows(shape) : 0;
+    const Plan p = make_plan(shape, path, any, extra_rows, row_cap);
     hipStream_t s = static_cast<hipStream_t>(stream);
     float* partials = static_cast<float*>(workspace);
     float* level1 = partials + (int64_t)row_cap * 2 * shape->E;
@@ -800,9 +815,9 @@ static int backward_impl(const void* y, const void* ya, int y_dtype, const void*
                 a.aux0 = dxr; a.aux1 = dxar;
                 a.W = W + ps.first * wstride;
                 a.dw_partials = region;
-                err = run_backward_kernel(a, grouping.plain(), headwise, shape->n_head, p.grid_x, s);
+                err = run_backward_kernel(a, p, grouping.plain(), headwise, s);
                 if (err == hipSuccess && grouping.ctx_len)
-                    err = launch_ragged_rest(kBackward, a, shape, p.path, p.partial_rows, s);
+                    err = launch_ragged_rest(kBackward, a, shape, p, p.partial_rows, s);
             } else {
                 FusedArgs a{};
                 a.in0 = cy; a.in1 = cya; a.in_dtype = cy_dtype;
@@ -850,9 +865,8 @@ static int backward_impl(const void* y, const void* ya, int y_dtype, const void*
         a.aux1 = (no_rec && k == 0) ? nullptr : xa_rec;
         a.W = W + (int64_t)k * 2 * shape->E;
         a.dw_partials = region;
-        err = (p.path != 2) ? launch_generic(kBackward, a, shape->n_head, p.grid_x, s)
-                            : run_backward_kernel(a, grouping.plain(), headwise, shape->n_head, p.grid_x, s);
-        if (err == hipSuccess && grouping.ctx_len) err = launch_ragged_rest(kBackward, a, shape, p.path, p.partial_rows, s);
+        err = run_backward_kernel(a, p, grouping.plain(), headwise, s);
+        if (err == hipSuccess && grouping.ctx_len) err = launch_ragged_rest(kBackward, a, shape, p, p.partial_rows, s);
         if (err != hipSuccess) return (int)err;
         reducer.add(region, p.partial_rows + extra_rows, 1, dW + k * wstride);
     }
@@ -949,7 +963,7 @@ int ncn_forward_radix(const void* x, const void* xa, int in_dtype, void* y, void
     ncn_shape as_wide;
     const bool headwise = headwise_call(shape, path, &as_wide);
     if (headwise) shape = &as_wide;
-    const Plan p = make_plan(shape, path);
+    const Plan p = make_plan(shape, path, any_tile_for(shape, path, alpha, m));
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int64_t wstride = 2 * shape->E;
     const std::vector<RadixPass> passes = plan_radix(shape, first_level, n_levels, false, path == 2);
@@ -967,8 +981,7 @@ int ncn_forward_radix(const void* x, const void* xa, int in_dtype, void* y, void
             a.out0 = y; a.out1 = ya; a.out_dtype = out_dtype;
             a.aux0 = last ? y32 : nullptr; a.aux1 = last ? ya32 : nullptr;
             a.W = W + ps.first * wstride;
-            err = (p.path != 2) ? launch_generic(kForward, a, shape->n_head, p.grid_fwd, s)
-                                : run_forward_kernel(kForward, a, false, headwise, shape->n_head, p.grid_fwd, s);
+            err = run_forward_kernel(kForward, a, p, false, headwise, s);
         } else {
             FusedArgs a{};
             a.in0 = first ? x : y; a.in1 = first ? xa : ya; a.in_dtype = first ? in_dtype : out_dtype;
@@ -1014,7 +1027,7 @@ int ncn_backward_radix(const void* y, const void* ya, int y_dtype, const void* d
     ncn_shape as_wide;
     const bool headwise = headwise_call(shape, path, &as_wide);
     if (headwise) shape = &as_wide;
-    const Plan p = make_plan(shape, path);
+    const Plan p = make_plan(shape, path, any_tile_for(shape, path, alpha, m));
     hipStream_t s = static_cast<hipStream_t>(stream);
     float* partials = static_cast<float*>(workspace);
     float* level1 = partials + (int64_t)kMaxGridX * 2 * shape->E;
@@ -1040,8 +1053,7 @@ int ncn_backward_radix(const void* y, const void* ya, int y_dtype, const void* d
             a.aux0 = drop_rec ? nullptr : x_rec; a.aux1 = drop_rec ? nullptr : xa_rec;
             a.W = W + ps.first * wstride;
             a.dw_partials = region;
-            err = (p.path != 2) ? launch_generic(kBackward, a, shape->n_head, p.grid_x, s)
-                                : run_backward_kernel(a, false, headwise, shape->n_head, p.grid_x, s);
+            err = run_backward_kernel(a, p, false, headwise, s);
         } else {
             FusedArgs a{};
             a.in0 = top ? y : x_rec; a.in1 = top ? ya : xa_rec; a.in_dtype = top ? y_dtype : NCN_F32;
@@ -1074,7 +1086,7 @@ int ncn_inverse_radix(const void* y, const void* ya, int in_dtype, void* x, void
     ncn_shape as_wide;
     const bool headwise = headwise_call(shape, path, &as_wide);
     if (headwise) shape = &as_wide;
-    const Plan p = make_plan(shape, path);
+    const Plan p = make_plan(shape, path, any_tile_for(shape, path, alpha, m));
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int64_t wstride = 2 * shape->E;
     const std::vector<RadixPass> passes = plan_radix(shape, first_level, n_levels, false, path == 2);
@@ -1089,8 +1101,7 @@ int ncn_inverse_radix(const void* y, const void* ya, int in_dtype, void* x, void
             a.in0 = top ? y : x; a.in1 = top ? ya : xa; a.in_dtype = top ? in_dtype : out_dtype;
             a.out0 = x; a.out1 = xa; a.out_dtype = out_dtype;
             a.W = W + ps.first * wstride;
-            err = (p.path != 2) ? launch_generic(kInverse, a, shape->n_head, p.grid_fwd, s)
-                                : run_forward_kernel(kInverse, a, false, headwise, shape->n_head, p.grid_fwd, s);
+            err = run_forward_kernel(kInverse, a, p, false, headwise, s);
         } else {
             FusedArgs a{};
             a.in0 = top ? y : x; a.in1 = top ? ya : xa; a.in_dtype = top ? in_dtype : out_dtype;

@@ -72,7 +72,7 @@ struct StageArgs {
     int32_t activation;
     int32_t edge;
     uint32_t radix_stride;   // n_cache^level: groups are the radix-n digit groups of that level (0: not used)
-    uint32_t reserved;
+    uint32_t any_tile;       // ncn_anyshape_kernels.h: R | F << 8 | log2(lanes per row) << 16 | log2(row lanes) << 24
     StepTable tab;
 };
 

@@ -88,6 +88,37 @@ hipError_t launch_headwise_forward(Pass pass, const StageArgs& a, int grid_x, hi
 hipError_t launch_headwise_forward_indexed(Pass pass, const StageArgs& a, int grid_x, hipStream_t s);
 hipError_t launch_headwise_backward(const StageArgs& a, int grid_x, hipStream_t s);
 hipError_t launch_headwise_backward_indexed(const StageArgs& a, int grid_x, hipStream_t s);
+// Shapes that are no powers of two (ncn_anyshape_kernels.h): a.any_tile says which tile.
+struct AnyTile {
+    int r, f;               // rows and features per lane; r == 0: no tile holds the group in one wave
+    int lf_log2, lr_log2;   // log2 of the lanes per row and of the row lanes per group
+};
+// The tile whose wave issues the least for a group: padded elements times what one costs (some 20 instructions), plus
+// the sums across lanes (2 R over the lanes of a row, F over the row lanes) and the pivot row's own terms, per lane.  Tiles
+// of more than 16 elements (two waves per SIMD, spills) only where the group fits no smaller one.
+inline AnyTile any_tile(int nc, int ec) {
+    AnyTile best{0, 0, 0, 0};
+    int best_cost = 0;
+    for (int r = 2; r <= 5; ++r)
+        for (int f = 3; f <= 5; ++f) {
+            int lf = 0, lr = 0;
+            while ((f << lf) < ec) ++lf;
+            while ((r << lr) < nc) ++lr;
+            if (lf + lr > 6 || lf > 5) continue;
+            int cost = (20 * r * f + 4 * r * lf + 2 * f * lr + 10 * f) << (lf + lr);
+            if (r * f > 16) cost *= 4;
+            if (best.r == 0 || cost < best_cost) {
+                best = AnyTile{r, f, lf, lr};
+                best_cost = cost;
+            }
+        }
+    return best;
+}
+hipError_t launch_any_forward(Pass pass, const StageArgs& a, int grid_x, hipStream_t s);
+hipError_t launch_any_backward(const StageArgs& a, int grid_x, hipStream_t s);
+// the builds with context lengths (a.ctx_len set); the two above go there by themselves
+hipError_t launch_any_forward_lengths(Pass pass, const StageArgs& a, int grid_x, hipStream_t s);
+hipError_t launch_any_backward_lengths(const StageArgs& a, int grid_x, hipStream_t s);
 hipError_t launch_generic(Pass pass, const StageArgs& a, int n_head, int grid_x, hipStream_t s);
 // Rows past the context length of their batch entry: copied through (a.ctx_len must be set).
 hipError_t launch_pass_through(Pass pass, const StageArgs& a, int64_t batch, hipStream_t s);

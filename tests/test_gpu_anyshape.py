@@ -1,0 +1,103 @@
+"""Register-tile kernels for group sizes and head widths that are no powers of two (csrc/ncn_anyshape_kernels.h) against
+the float64 oracle: every tile of theirs, heads that fill a tile and heads that end inside it, one and several row
+lanes, group counts that leave the last wave tile partly empty."""
+import pytest
+import torch
+
+from oracle import ncn_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+# (n_cache, head width, heads, groups, batch): tile R x F, lanes per row x row lanes
+CASES = [
+    (3, 3, 3, 7, 3),     # 3x3, 1x1, a wave tile of 64 groups, three heads
+    (1, 5, 2, 70, 2),    # 2x5, 1x1, one row of two that exist
+    (5, 1, 5, 1, 2),     # 5x3, 1x1, one feature of three; one group
+    (6, 10, 1, 5, 4),    # 3x5, 2x2, one head
+    (7, 40, 4, 3, 2),    # 2x5, 8x4, seven rows of eight
+    (4, 20, 2, 9, 2),    # power-of-two rows, 4x3 or 4x4 with padded features
+    (8, 12, 4, 4, 2),    # 4x3, 4x2
+    (9, 7, 2, 3, 2),     # 5x4 does not fit better: padded both ways
+    (10, 56, 2, 3, 2),   # 16 lanes per row
+    (13, 16, 2, 3, 2),   # power-of-two width, 13 rows
+    (16, 24, 3, 2, 2),   # three heads (a wave of the block works on the next tile)
+    (20, 56, 1, 2, 2),   # 5x4, 16x4: only a tile of 20 elements holds the group
+    (20, 64, 1, 2, 1),   # 5x4, 16x4 exactly
+    (48, 12, 1, 2, 1),   # 3x3, 4x16: every lane of the wave in one group
+    (24, 64, 1, 2, 1),   # 4x.. no tile: generic kernels
+]
+TOL = 1e-5
+
+
+def _tolerance(n):
+    """1e-5 up to 16 rows; beyond, the inversion amplifies float32 rounding by (1/m)^n: 1.2e-6 per unit, as measured for
+    32 rows and used by the random-shape sweep (gradients)."""
+    return max(TOL, 1.2e-6 * 0.9 ** -n)
+
+
+@pytest.fixture(scope="module")
+def M():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from ncn_cuda_amd import ncn_cuda_module
+    return ncn_cuda_module
+
+
+def _inputs(case, L=1):
+    n, ec, C, groups, batch = case
+    return O.make_inputs(batch, n * groups, ec * C, L, n, seed=sum(case), xa_zero=False)
+
+
+@pytest.mark.parametrize("act", [0, 2])
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "n%d_e%d_C%d_g%d_b%d" % c)
+def test_stage(M, case, act):
+    n, ec, C, groups, batch = case
+    x, xa, Ws, dy, dya = _inputs(case)
+    d = torch.float64
+    for stage in (0, 2):
+        ref = O.net_autograd(x.to(d), xa.to(d), [Ws[0].to(d)], dy.to(d), dya.to(d), 0.9, n, C, activation=act, first_stage=stage)
+        W = Ws[0].cuda()
+        y, ya = M.forward_stages(x.cuda(), xa.cuda(), W, 0.9, act, n, C, stage, 1)
+        assert O.rel_err(y, ref[0]) < TOL and O.rel_err(ya, ref[1]) < TOL
+        xr, xar, dx, dxa, dW = M.backward_stages(y, ya, dy.cuda(), dya.cuda(), W, 0.9, act, n, C, stage, 1)
+        tol = _tolerance(n)
+        assert O.rel_err(dx, ref[2]) < tol and O.rel_err(dxa, ref[3]) < tol and O.rel_err(dW[0], ref[4][0]) < tol
+        ix, ixa = M.inverse_stages(y, ya, W, 0.9, act, n, C, stage, 1)
+        # the float32 outputs are undone: their rounding, amplified by (1/m)^n (6e-6 per unit, the sweep's bound)
+        rtol = max(3e-5, 6e-6 * 0.9 ** -n)
+        for a, b in ((xr, x), (xar, xa), (ix, x), (ixa, xa)):
+            assert O.rel_err(a, b) < rtol
+
+
+@pytest.mark.parametrize("case", [CASES[0], CASES[4], CASES[11]], ids=lambda c: "n%d_e%d_C%d_g%d_b%d" % c)
+def test_table_and_lengths(M, case):
+    """A random table, lengths that cut a group, end between groups, are zero and the whole of N."""
+    n, ec, C, groups, batch = case
+    batch, N = 4, n * groups
+    x, xa, Ws, dy, dya = O.make_inputs(batch, N, ec * C, 1, n, seed=7, xa_zero=False)
+    table = torch.randperm(N, generator=torch.Generator().manual_seed(3))
+    lens = [0, N, n * (groups // 2), N - 1]
+    d = torch.float64
+    ref = O.net_autograd_indexed(x.to(d), xa.to(d), [Ws[0].to(d)], dy.to(d), dya.to(d), 0.9, n, C, [table], lens)
+    gt, gl = table.to(torch.int32).cuda(), torch.tensor(lens, dtype=torch.int32).cuda()
+    W = Ws[0].cuda()
+    y, ya = M.forward_stages(x.cuda(), xa.cuda(), W, 0.9, 0, n, C, 0, 1, group_index=gt, ctx_len=gl)
+    assert O.rel_err(y, ref[0]) < TOL and O.rel_err(ya, ref[1]) < TOL
+    assert torch.equal(y[0].cpu(), x[0]) and torch.equal(ya[0].cpu(), xa[0])
+    xr, xar, dx, dxa, dW = M.backward_stages(y, ya, dy.cuda(), dya.cuda(), W, 0.9, 0, n, C, 0, 1, group_index=gt, ctx_len=gl)
+    tol = _tolerance(n)
+    assert O.rel_err(dx, ref[2]) < tol and O.rel_err(dxa, ref[3]) < tol and O.rel_err(dW[0], ref[4][0]) < tol
+    assert torch.equal(dx[0].cpu(), dy[0]) and torch.equal(xr[0].cpu(), x[0])
+
+
+@pytest.mark.parametrize("case", [CASES[3], CASES[4]], ids=lambda c: "n%d_e%d_C%d_g%d_b%d" % c)
+def test_bfloat16(M, case):
+    n, ec, C, groups, batch = case
+    x, xa, Ws, dy, dya = (t.bfloat16() if isinstance(t, torch.Tensor) else t for t in _inputs(case))
+    d = torch.float64
+    ref = O.net_autograd(x.to(d), xa.to(d), [Ws[0].to(d)], dy.to(d), dya.to(d), 0.9, n, C)
+    W = Ws[0].cuda()
+    y, ya, sy, sya = M.forward_stages_saving(x.cuda(), xa.cuda(), W, 0.9, 0, n, C, 0)
+    _, _, dx, dxa, dW = M.backward_stages(sy, sya, dy.cuda(), dya.cuda(), W, 0.9, 0, n, C, 0, 1, want_inputs=False)
+    for got, want in ((y, ref[0]), (ya, ref[1]), (dx, ref[2]), (dxa, ref[3]), (dW[0], ref[4][0])):
+        assert O.rel_err(got, want) < 2e-2
