@@ -190,7 +190,41 @@ __global__ void __launch_bounds__(64) generic_backward_kernel(const StageArgs A)
     }
 }
 
-// dW partial rows are summed in two launches so that the first has enough loads in flight to run at memory speed:
+// dW partial rows, one launch: block (x, y) sums 8 columns of segment y.  A lane takes every 128th row of one column, then
+// its wave and the block's 16 waves are summed, all in a fixed order.  Bound by the latency of its few rounds of loads.
+// Workgroups go round the XCDs in turn, so the four blocks that share the 128-byte lines of 32 columns are numbered
+// eight apart: their lines are fetched into one L2 instead of four (16384 x 256: 10 against 34 us).
+// Against the two launches below, back to back: 2.4 : 4.8 us up to 1024 rows, 4.1 : 5.0 at 4096 x 256, 5.1 : 5.4 at
+// 6144 x 256, 6.2 : 7.5 at 4096 x 1792 and 12.2 : 11.1 at 6144 x 1792, 10 : 7.7 at 16384 x 256 -- hence up to
+// kReduceOneLaunchRows.
+constexpr int kReduceColumns = 8, kReduceOneLaunchRows = 4096;
+__device__ __forceinline__ uint32_t reduce_column_block(uint32_t x, uint32_t n) {
+    const uint32_t base = x & ~31u;
+    return base + 32u <= n ? base + (x & 7u) * 4u + (x >> 3 & 3u) : x;
+}
+__global__ void __launch_bounds__(1024) reduce_rows_kernel(const ReduceJob J) {
+    const ReduceSegment& g = J.seg[blockIdx.y];
+    const int64_t col0 = (int64_t)reduce_column_block(blockIdx.x, gridDim.x) * kReduceColumns;
+    const int64_t col = col0 + threadIdx.x % kReduceColumns;
+    float sum[1] = {0.f};
+    if (col < g.cols) {
+#pragma unroll 8
+        for (int r = threadIdx.x / kReduceColumns; r < g.rows; r += 1024 / kReduceColumns) sum[0] += g.in[(int64_t)r * g.cols + col];
+    }
+    lane_sum_n<kReduceColumns, 64, false, 1>(sum);
+    __shared__ float red[16][kReduceColumns];
+    if ((threadIdx.x & 63) < kReduceColumns) red[threadIdx.x >> 6][threadIdx.x & 63] = sum[0];
+    __syncthreads();
+    if (threadIdx.x < kReduceColumns && col0 + threadIdx.x < g.cols) {
+        float total = 0.f;
+#pragma unroll
+        for (int w = 0; w < 16; w += 4)
+            total += (red[w][threadIdx.x] + red[w + 1][threadIdx.x]) + (red[w + 2][threadIdx.x] + red[w + 3][threadIdx.x]);
+        g.out[col0 + threadIdx.x] = total;
+    }
+}
+
+// More rows than that: two launches, so that the first has enough loads in flight to run at memory speed:
 // level 1 sums chunks of kReduceRowsPerBlock rows (block y = one chunk of one segment of the job), level 2 the chunk
 // sums of each segment (block y = segment).  A block is 256 / RL columns x RL row lanes (level 2 has few rows of
 // blocks, so it takes narrow blocks with many row lanes); the order of additions is fixed.
@@ -307,6 +341,13 @@ hipError_t launch_reduce_job(const ReduceJob& job, float* level1, hipStream_t s)
     if (job.n == 0) return hipSuccess;
     int64_t max_cols = 0;
     for (int k = 0; k < job.n; ++k) max_cols = job.seg[k].cols > max_cols ? job.seg[k].cols : max_cols;
+    int max_rows = 0;
+    for (int k = 0; k < job.n; ++k) max_rows = job.seg[k].rows > max_rows ? job.seg[k].rows : max_rows;
+    if (max_rows <= kReduceOneLaunchRows) {
+        hipLaunchKernelGGL(reduce_rows_kernel, dim3((unsigned)((max_cols + kReduceColumns - 1) / kReduceColumns), job.n),
+                           dim3(1024), 0, s, job);
+        return hipGetLastError();
+    }
     const ReduceSegment& last = job.seg[job.n - 1];
     const int chunks = last.chunk0 + (last.rows + kReduceRowsPerBlock - 1) / kReduceRowsPerBlock;
     constexpr int cw1 = 256 / kReduceLevel1Lanes, cw2 = 256 / kReduceLevel2Lanes;
