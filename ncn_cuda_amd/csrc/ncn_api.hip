@@ -267,14 +267,13 @@ hipError_t run_forward_kernel(Pass pass, const StageArgs& a, const Plan& p, bool
     if (p.path != 2) return launch_generic(pass, a, a.n_head, p.grid_fwd, s);
     if (headwise)
         return plain ? launch_headwise_forward(pass, a, p.grid_fwd, s) : launch_headwise_forward_indexed(pass, a, p.grid_fwd, s);
-    return plain ? launch_fast_forward(pass, a, a.n_head, p.grid_fwd, s)
-                 : launch_fast_forward_indexed(pass, a, a.n_head, p.grid_fwd, s);
+    return plain ? launch_stage_forward<false>(pass, a, p.grid_fwd, s) : launch_stage_forward<true>(pass, a, p.grid_fwd, s);
 }
 hipError_t run_backward_kernel(const StageArgs& a, const Plan& p, bool plain, bool headwise, hipStream_t s) {
     if (p.any.r) return launch_any_backward(a, p.grid_x, s);
     if (p.path != 2) return launch_generic(kBackward, a, a.n_head, p.grid_x, s);
     if (headwise) return plain ? launch_headwise_backward(a, p.grid_x, s) : launch_headwise_backward_indexed(a, p.grid_x, s);
-    return plain ? launch_fast_backward(a, a.n_head, p.grid_x, s) : launch_fast_backward_indexed(a, a.n_head, p.grid_x, s);
+    return plain ? launch_stage_backward<false>(a, p.grid_x, s) : launch_stage_backward<true>(a, p.grid_x, s);
 }
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }

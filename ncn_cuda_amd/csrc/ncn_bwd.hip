@@ -1,8 +1,9 @@
 // Instantiations and dispatch of the register-resident reversible backward stage kernel.
-// Compiled four times: as it stands for the stride permutation; through ncn_bwd_indexed.hip (NCN_INDEXED_BUILD = 1)
-// for launches that carry a grouping table or context lengths; and each of the two once more (ncn_bwd_once.hip,
-// ncn_bwd_indexed_once.hip: NCN_ONCE_BUILD = 1) in the form without a loop over tiles, which the launchers pick by
-// themselves when the grid has a wave for every tile.
+// Compiled six times: as it stands for the stride permutation, and through ncn_bwd_indexed.hip (NCN_INDEXED_BUILD = 1)
+// for launches that carry a grouping table or context lengths; each of the two takes every element type and activation,
+// with a loop over tiles, and hands tanh launches of one storage type whose grid has a wave for every tile on to its
+// builds for that type, which have no loop (ncn_bwd_f32.hip, ncn_bwd_bf16.hip, ncn_bwd_indexed_f32.hip,
+// ncn_bwd_indexed_bf16.hip: NCN_TYPES_BUILD).
 #include "ncn_configs.h"
 #include "ncn_launch.h"
 #include "ncn_stage_kernels.h"
@@ -10,38 +11,37 @@
 #ifndef NCN_INDEXED_BUILD
 #define NCN_INDEXED_BUILD 0
 #endif
-#ifndef NCN_ONCE_BUILD
-#define NCN_ONCE_BUILD 0
+#ifndef NCN_TYPES_BUILD
+#define NCN_TYPES_BUILD kAnyTypes
 #endif
 
 namespace ncn {
 
-#if NCN_INDEXED_BUILD && NCN_ONCE_BUILD
-hipError_t launch_fast_backward_indexed_once(const StageArgs& a, int /*n_head*/, int grid_x, hipStream_t s) {
-#elif NCN_INDEXED_BUILD
-hipError_t launch_fast_backward_indexed(const StageArgs& a, int n_head, int grid_x, hipStream_t s) {
-    if ((uint64_t)a.total_tiles * (uint64_t)a.n_head <= (uint64_t)grid_x * kWavesPerBlock)
-        return launch_fast_backward_indexed_once(a, n_head, grid_x, s);   // a wave for every tile
-#elif NCN_ONCE_BUILD
-hipError_t launch_fast_backward_once(const StageArgs& a, int /*n_head*/, int grid_x, hipStream_t s) {
-#else
-hipError_t launch_fast_backward(const StageArgs& a, int n_head, int grid_x, hipStream_t s) {
-    if ((uint64_t)a.total_tiles * (uint64_t)a.n_head <= (uint64_t)grid_x * kWavesPerBlock)
-        return launch_fast_backward_once(a, n_head, grid_x, s);   // a wave for every tile
-#endif
+template <>
+hipError_t launch_stage_backward<NCN_INDEXED_BUILD != 0, NCN_TYPES_BUILD>(const StageArgs& a, int grid_x, hipStream_t s) {
     constexpr bool kIndexed = NCN_INDEXED_BUILD != 0;
-    constexpr bool kLoop = NCN_ONCE_BUILD == 0;
+    constexpr int kTypes = NCN_TYPES_BUILD;
+    constexpr bool kLoop = kTypes == kAnyTypes;
     const dim3 grid(grid_x), block(kBlockThreads);
     const bool tanh_only = a.activation == NCN_ACT_TANH;
-#define NCN_CASE(NC, EC, R, F)                                                                  \
-    static_assert(fast_tile(NC, EC).r == R && fast_tile(NC, EC).f == F, "duplicate config entry");          \
-    if (a.n_cache == NC && a.head_dim == EC) {                                                 \
-        if (tanh_only) hipLaunchKernelGGL((stage_backward_kernel<NC, EC, R, F, true, kIndexed, kLoop>), grid, block, 0, s, a); \
-        else hipLaunchKernelGGL((stage_backward_kernel<NC, EC, R, F, false, kIndexed, kLoop>), grid, block, 0, s, a);          \
-        return hipGetLastError();                                                              \
+    if constexpr (kTypes == kAnyTypes) {
+        if ((uint64_t)a.total_tiles * (uint64_t)a.n_head <= (uint64_t)grid_x * kWavesPerBlock) {   // a wave for every tile
+            const int types = stage_types(kBackward, a);
+            if (types == kF32Types) return launch_stage_backward<kIndexed, kF32Types>(a, grid_x, s);
+            if (types == kBf16Types) return launch_stage_backward<kIndexed, kBf16Types>(a, grid_x, s);
+        }
+    }
+#define NCN_LAUNCH(KERNEL) hipLaunchKernelGGL(KERNEL, grid, block, 0, s, a)
+#define NCN_CASE(NC, EC, R, F)                                                                        \
+    static_assert(fast_tile(NC, EC).r == R && fast_tile(NC, EC).f == F, "duplicate config entry");    \
+    if (a.n_cache == NC && a.head_dim == EC) {                                                        \
+        if (tanh_only) NCN_LAUNCH((stage_backward_kernel<NC, EC, R, F, true, kIndexed, kLoop, kTypes>));     \
+        else if constexpr (kTypes == kAnyTypes) NCN_LAUNCH((stage_backward_kernel<NC, EC, R, F, false, kIndexed, kLoop>)); \
+        return hipGetLastError();                                                                     \
     }
     NCN_FOR_EACH_FAST_CONFIG(NCN_CASE)
 #undef NCN_CASE
+#undef NCN_LAUNCH
     return hipErrorInvalidConfiguration;
 }
 

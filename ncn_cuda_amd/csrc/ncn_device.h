@@ -90,7 +90,6 @@ __device__ __forceinline__ uint32_t f32_to_bf16(float f) {
 // two floats -> packed bf16 pair (lo in bits 0..15): one v_cvt_pk_bf16_f32 on gfx950, round to nearest even
 typedef __bf16 ncn_bf16x2 __attribute__((ext_vector_type(2)));
 typedef float ncn_floatx2 __attribute__((ext_vector_type(2)));
-typedef uint32_t ncn_u32x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
     const ncn_floatx2 v = {lo, hi};
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, ncn_bf16x2));
@@ -143,19 +142,19 @@ __device__ __forceinline__ void store_frag(void* base, int dtype, int64_t off, b
 #pragma unroll
         for (int k = 0; k < FPL / 4; ++k) p[k] = make_float4(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]);
     } else {
-        ncn_u32x2* p = reinterpret_cast<ncn_u32x2*>(static_cast<uint16_t*>(base) + off);
-        uint32_t w[FPL / 2];
+        uint2* p = reinterpret_cast<uint2*>(static_cast<uint16_t*>(base) + off);
 #pragma unroll
-        for (int k = 0; k < FPL / 2; ++k) w[k] = pack_bf16x2(v[2 * k], v[2 * k + 1]);
-#pragma unroll
-        for (int k = 0; k < FPL / 4; ++k) p[k] = ncn_u32x2{w[2 * k], w[2 * k + 1]};
-        if (dtype == NCN_BF16X2) {   // second plane: what the rounding took away (the difference is exact in float32)
-            ncn_u32x2* q = reinterpret_cast<ncn_u32x2*>(static_cast<uint16_t*>(base) + off + plane);
-#pragma unroll
-            for (int k = 0; k < FPL / 2; ++k)
-                w[k] = pack_bf16x2(v[2 * k] - bf16_to_f32(w[k] & 0xffffu), v[2 * k + 1] - bf16_to_f32(w[k] >> 16));
-#pragma unroll
-            for (int k = 0; k < FPL / 4; ++k) q[k] = ncn_u32x2{w[2 * k], w[2 * k + 1]};
+        for (int k = 0; k < FPL / 4; ++k) {
+            uint2 t;
+            t.x = pack_bf16x2(v[4 * k + 0], v[4 * k + 1]);
+            t.y = pack_bf16x2(v[4 * k + 2], v[4 * k + 3]);
+            p[k] = t;
+            if (dtype == NCN_BF16X2) {   // second plane: what the rounding took away (the difference is exact in float32)
+                uint2 u;
+                u.x = pack_bf16x2(v[4 * k + 0] - bf16_to_f32(t.x & 0xffffu), v[4 * k + 1] - bf16_to_f32(t.x >> 16));
+                u.y = pack_bf16x2(v[4 * k + 2] - bf16_to_f32(t.y & 0xffffu), v[4 * k + 3] - bf16_to_f32(t.y >> 16));
+                reinterpret_cast<uint2*>(static_cast<uint16_t*>(base) + off + plane)[k] = u;
+            }
         }
     }
 }
@@ -187,8 +186,11 @@ __device__ __forceinline__ void issue_tile(const void* base, int dtype, const in
             for (int k = 0; k < FPL / 4; ++k) {
                 const float2 t = reinterpret_cast<const float2*>(static_cast<const uint16_t*>(base) + off[rr])[k];
                 v[rr][4 * k] = t.x; v[rr][4 * k + 1] = t.y;
-                // not read; but a branch that leaves part of the tile alone makes the compiler keep it in scratch memory
-                v[rr][4 * k + 2] = __builtin_nondeterministic_value(t.x); v[rr][4 * k + 3] = __builtin_nondeterministic_value(t.x);
+                if constexpr (FPL > 4) {
+                    // not read; but a branch that leaves part of a wide tile alone makes the compiler keep it in scratch memory
+                    v[rr][4 * k + 2] = __builtin_nondeterministic_value(t.x);
+                    v[rr][4 * k + 3] = __builtin_nondeterministic_value(t.x);
+                }
             }
     } else {
 #pragma unroll
@@ -209,15 +211,15 @@ __device__ __forceinline__ void finish_tile(int dtype, float (&v)[R][FPL]) {
     for (int rr = 0; rr < R; ++rr)
 #pragma unroll
         for (int k = 0; k < FPL / 4; ++k) {
-            const uint32_t w0 = __float_as_uint(v[rr][4 * k]), w1 = __float_as_uint(v[rr][4 * k + 1]);
-            const uint32_t r0 = __float_as_uint(v[rr][4 * k + 2]), r1 = __float_as_uint(v[rr][4 * k + 3]);
-            float o0 = __uint_as_float(w0 << 16), o1 = __uint_as_float(w0 & 0xffff0000u);
-            float o2 = __uint_as_float(w1 << 16), o3 = __uint_as_float(w1 & 0xffff0000u);
+            float* o = &v[rr][4 * k];
+            const uint32_t w0 = __float_as_uint(o[0]), w1 = __float_as_uint(o[1]);
+            const uint32_t r0 = __float_as_uint(o[2]), r1 = __float_as_uint(o[3]);
+            o[0] = __uint_as_float(w0 << 16); o[1] = __uint_as_float(w0 & 0xffff0000u);
+            o[2] = __uint_as_float(w1 << 16); o[3] = __uint_as_float(w1 & 0xffff0000u);
             if (dtype == NCN_BF16X2) {
-                o0 += __uint_as_float(r0 << 16); o1 += __uint_as_float(r0 & 0xffff0000u);
-                o2 += __uint_as_float(r1 << 16); o3 += __uint_as_float(r1 & 0xffff0000u);
+                o[0] += __uint_as_float(r0 << 16); o[1] += __uint_as_float(r0 & 0xffff0000u);
+                o[2] += __uint_as_float(r1 << 16); o[3] += __uint_as_float(r1 & 0xffff0000u);
             }
-            v[rr][4 * k] = o0; v[rr][4 * k + 1] = o1; v[rr][4 * k + 2] = o2; v[rr][4 * k + 3] = o3;
         }
 }
 

@@ -1,0 +1,5 @@
+// The forward and inverse stage kernels for bfloat16 launches that carry a grouping table or context lengths (see
+// ncn_fwd.hip).
+#define NCN_INDEXED_BUILD 1
+#define NCN_TYPES_BUILD kBf16Types
+#include "ncn_fwd.hip"

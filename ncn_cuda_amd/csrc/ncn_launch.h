@@ -66,14 +66,34 @@ hipError_t launch_reduce_job(const ReduceJob& job, float* level1, hipStream_t s)
 // far (the limit is kept per device and kernel for the life of the process: one driver call instead of one per launch).
 hipError_t ensure_dynamic_lds(const void* kernel, size_t bytes);
 
-hipError_t launch_fast_forward(Pass pass, const StageArgs& a, int n_head, int grid_x, hipStream_t s);
-hipError_t launch_fast_backward(const StageArgs& a, int n_head, int grid_x, hipStream_t s);
-// the same for a grid that has a wave for every tile (ncn_bwd_once.hip); launch_fast_backward goes there by itself
-hipError_t launch_fast_backward_once(const StageArgs& a, int n_head, int grid_x, hipStream_t s);
-// the same kernels built to honour a.table and a.ctx_len (the plain builds ignore both)
-hipError_t launch_fast_forward_indexed(Pass pass, const StageArgs& a, int n_head, int grid_x, hipStream_t s);
-hipError_t launch_fast_backward_indexed(const StageArgs& a, int n_head, int grid_x, hipStream_t s);
-hipError_t launch_fast_backward_indexed_once(const StageArgs& a, int n_head, int grid_x, hipStream_t s);
+// Element types of a launch, where a kernel is built for one combination (tanh builds): with the branch on the type gone
+// the loads of a tile go straight into its registers and nothing is copied where the branches meet.
+//   kAnyTypes: read from the arguments
+//   kF32Types: float32 everywhere
+//   kBf16Types: bfloat16 storage -- forward and inverse read bfloat16, the backward reads saved outputs in two planes and
+//   bfloat16 gradients, everything is written as bfloat16 (forward: one plane or two)
+enum { kAnyTypes = -1, kF32Types = 0, kBf16Types = 1 };
+// which of them a launch of the stage kernels is
+inline int stage_types(Pass pass, const StageArgs& a) {
+    if (a.activation != NCN_ACT_TANH) return kAnyTypes;
+    if (a.in_dtype == NCN_F32 && a.out_dtype == NCN_F32 && (pass != kBackward || a.g_dtype == NCN_F32)) return kF32Types;
+    const bool bf16 = pass == kForward    ? a.in_dtype == NCN_BF16 && a.out_dtype != NCN_F32
+                      : pass == kInverse ? a.in_dtype == NCN_BF16 && a.out_dtype == NCN_BF16
+                                         : a.in_dtype == NCN_BF16X2 && a.g_dtype == NCN_BF16 && a.out_dtype == NCN_BF16;
+    return bf16 ? kBf16Types : kAnyTypes;
+}
+// One stage on the register kernels (ncn_fwd*.hip, ncn_bwd*.hip).  INDEXED: the builds that honour a.table,
+// a.radix_stride and a.ctx_len.  Callers take TYPES = kAnyTypes, which goes to the builds for one type by itself.
+template <bool INDEXED, int TYPES = kAnyTypes>
+hipError_t launch_stage_forward(Pass pass, const StageArgs& a, int grid_x, hipStream_t s);
+template <bool INDEXED, int TYPES = kAnyTypes>
+hipError_t launch_stage_backward(const StageArgs& a, int grid_x, hipStream_t s);
+#define NCN_DECLARE(INDEXED, TYPES)                                                                             \
+    template <> hipError_t launch_stage_forward<INDEXED, TYPES>(Pass, const StageArgs&, int, hipStream_t);      \
+    template <> hipError_t launch_stage_backward<INDEXED, TYPES>(const StageArgs&, int, hipStream_t);
+NCN_DECLARE(false, kAnyTypes) NCN_DECLARE(false, kF32Types) NCN_DECLARE(false, kBf16Types)
+NCN_DECLARE(true, kAnyTypes) NCN_DECLARE(true, kF32Types) NCN_DECLARE(true, kBf16Types)
+#undef NCN_DECLARE
 // Heads of one feature (ncn_headwise_kernels.h): `a` carries the geometry of E / w heads of w features, w =
 // headwise_width(E), for which the grid was planned as well; the second form honours a.table, a.radix_stride and
 // a.ctx_len.

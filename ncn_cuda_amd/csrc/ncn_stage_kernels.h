@@ -26,6 +26,7 @@
 // per stage.
 #pragma once
 #include "ncn_device.h"
+#include "ncn_launch.h"
 
 namespace ncn {
 
@@ -477,6 +478,12 @@ __device__ __forceinline__ void backward_steps(float (&Y)[R][F], float (&B)[R][F
         }                                                                                       \
     }
 
+// the element type of an array in a build for TYPES: as the arguments say, or as the build does
+template <int TYPES>
+__device__ __forceinline__ int dtype_of(int from_args, int when_bf16) {
+    return TYPES == kF32Types ? NCN_F32 : TYPES == kBf16Types ? when_bf16 : from_args;
+}
+
 // Rows past a context length take no part in the stage: they pass through, stored as they were loaded.  (A launch of
 // its own for them, one element per lane, cost 38 us per stage and direction on 32 x 4096 x 128 bfloat16 with a quarter
 // of the rows past their lengths, 0.22 of the 0.89 ms of a three-stage training step.)
@@ -489,19 +496,21 @@ __device__ __forceinline__ void backward_steps(float (&Y)[R][F], float (&B)[R][F
         }                                                                                       \
     }
 
-template <int NC, int EC, int R, int F, bool TANH_ONLY = true, bool INDEXED = false>
+template <int NC, int EC, int R, int F, bool TANH_ONLY = true, bool INDEXED = false, int TYPES = kAnyTypes>
 __global__ void __launch_bounds__(kBlockThreads, (TANH_ONLY && !INDEXED && R == 4 && F == 4) ? 5 : 1) stage_forward_kernel(const StageArgs A) {
     NCN_WAVE_PROLOGUE
+    const int in_dtype = dtype_of<TYPES>(A.in_dtype, NCN_BF16);
+    const int out_dtype = TYPES == kBf16Types && A.out_dtype != NCN_BF16X2 ? NCN_BF16 : dtype_of<TYPES>(A.out_dtype, NCN_BF16X2);
     for (uint32_t t = gwave / A.n_head; t < A.total_tiles; t += tile_step) {
         int64_t off[R];
         const int live = tile_offsets<NC, EC, R, F, INDEXED>(A, t, lane, head, off);
         float x[R][F], a[R][F];
-        issue_tile<R, F>(A.in0, A.in_dtype, off, x);
-        issue_tile<R, F>(A.in1, A.in_dtype, off, a);
+        issue_tile<R, F>(A.in0, in_dtype, off, x);
+        issue_tile<R, F>(A.in1, in_dtype, off, a);
         NCN_SCALE_W_ONCE
-        finish_tile<R, F>(A.in_dtype, x);
-        finish_tile<R, F>(A.in_dtype, a);
-        NCN_PASS_DEAD_ROWS(A.out0, A.out1, A.out_dtype, x, a)
+        finish_tile<R, F>(in_dtype, x);
+        finish_tile<R, F>(in_dtype, a);
+        NCN_PASS_DEAD_ROWS(A.out0, A.out1, out_dtype, x, a)
         if (A.aux0) { NCN_PASS_DEAD_ROWS(A.aux0, A.aux1, NCN_F32, x, a) }
         NCN_ZERO_DEAD_ROWS(x, a, true)
         scale_tile<R, F>(x, a, A.tab.kappa, A.tab.a_scale);
@@ -510,8 +519,8 @@ __global__ void __launch_bounds__(kBlockThreads, (TANH_ONLY && !INDEXED && R == 
 #pragma unroll
         for (int rr = 0; rr < R; ++rr) {
             const bool valid = INDEXED ? NCN_ROW_LIVE(rr) : live != 0;
-            store_frag<F>(A.out0, A.out_dtype, off[rr], valid, x[rr], A.plane);
-            store_frag<F>(A.out1, A.out_dtype, off[rr], valid, a[rr], A.plane);
+            store_frag<F>(A.out0, out_dtype, off[rr], valid, x[rr], A.plane);
+            store_frag<F>(A.out1, out_dtype, off[rr], valid, a[rr], A.plane);
             if (A.aux0) {
                 store_frag<F>(A.aux0, NCN_F32, off[rr], valid, x[rr]);
                 store_frag<F>(A.aux1, NCN_F32, off[rr], valid, a[rr]);
@@ -520,19 +529,20 @@ __global__ void __launch_bounds__(kBlockThreads, (TANH_ONLY && !INDEXED && R == 
     }
 }
 
-template <int NC, int EC, int R, int F, bool TANH_ONLY = true, bool INDEXED = false>
+template <int NC, int EC, int R, int F, bool TANH_ONLY = true, bool INDEXED = false, int TYPES = kAnyTypes>
 __global__ void __launch_bounds__(kBlockThreads) stage_inverse_kernel(const StageArgs A) {
     NCN_WAVE_PROLOGUE
+    const int in_dtype = dtype_of<TYPES>(A.in_dtype, NCN_BF16), out_dtype = dtype_of<TYPES>(A.out_dtype, NCN_BF16);
     for (uint32_t t = gwave / A.n_head; t < A.total_tiles; t += tile_step) {
         int64_t off[R];
         const int live = tile_offsets<NC, EC, R, F, INDEXED>(A, t, lane, head, off);
         float y[R][F], b[R][F];
-        issue_tile<R, F>(A.in0, A.in_dtype, off, y, A.plane);
-        issue_tile<R, F>(A.in1, A.in_dtype, off, b, A.plane);
+        issue_tile<R, F>(A.in0, in_dtype, off, y, A.plane);
+        issue_tile<R, F>(A.in1, in_dtype, off, b, A.plane);
         NCN_SCALE_W_ONCE
-        finish_tile<R, F>(A.in_dtype, y);
-        finish_tile<R, F>(A.in_dtype, b);
-        NCN_PASS_DEAD_ROWS(A.out0, A.out1, A.out_dtype, y, b)
+        finish_tile<R, F>(in_dtype, y);
+        finish_tile<R, F>(in_dtype, b);
+        NCN_PASS_DEAD_ROWS(A.out0, A.out1, out_dtype, y, b)
         NCN_ZERO_DEAD_ROWS(y, b, true)
         scale_tile<R, F>(y, b, A.tab.kappa, A.tab.b_scale);
         inverse_core<NC, EC, R, F, TANH_ONLY, INDEXED>(y, b, wi, wj, A.tab, lane, slots, live);
@@ -540,8 +550,8 @@ __global__ void __launch_bounds__(kBlockThreads) stage_inverse_kernel(const Stag
 #pragma unroll
         for (int rr = 0; rr < R; ++rr) {
             const bool valid = INDEXED ? NCN_ROW_LIVE(rr) : live != 0;
-            store_frag<F>(A.out0, A.out_dtype, off[rr], valid, y[rr]);
-            store_frag<F>(A.out1, A.out_dtype, off[rr], valid, b[rr]);
+            store_frag<F>(A.out0, out_dtype, off[rr], valid, y[rr]);
+            store_frag<F>(A.out1, out_dtype, off[rr], valid, b[rr]);
         }
     }
 }
@@ -551,9 +561,11 @@ __global__ void __launch_bounds__(kBlockThreads) stage_inverse_kernel(const Stag
 // LOOP = false is for launches with a wave for every tile: without the loop around them the tile's addresses and
 // offsets are not carried in registers across it (the loop build spills 6 of them per lane at R x F = 16, which a
 // launch bound by its traffic pays for), and the steps come out in an order that issues better.
-template <int NC, int EC, int R, int F, bool TANH_ONLY = true, bool INDEXED = false, bool LOOP = true>
-__global__ void __launch_bounds__(kBlockThreads, (TANH_ONLY && R * F <= 16 && F == 4) ? 4 : 1) stage_backward_kernel(const StageArgs A) {
+template <int NC, int EC, int R, int F, bool TANH_ONLY = true, bool INDEXED = false, bool LOOP = true, int TYPES = kAnyTypes>
+__global__ void __launch_bounds__(kBlockThreads, (TANH_ONLY && R * F <= 16 && F == 4) ? 4 : (TYPES != kAnyTypes && R * F == 32) ? 2 : 1) stage_backward_kernel(const StageArgs A) {
     NCN_WAVE_PROLOGUE
+    const int in_dtype = dtype_of<TYPES>(A.in_dtype, NCN_BF16X2), g_dtype = dtype_of<TYPES>(A.g_dtype, NCN_BF16);
+    const int out_dtype = dtype_of<TYPES>(A.out_dtype, NCN_BF16);
     float dwi[F], dwj[F];
 #pragma unroll
     for (int f = 0; f < F; ++f) dwi[f] = dwj[f] = 0.f;
@@ -563,11 +575,11 @@ __global__ void __launch_bounds__(kBlockThreads, (TANH_ONLY && R * F <= 16 && F 
         int64_t off[R];
         const int live = tile_offsets<NC, EC, R, F, INDEXED>(A, t, lane, head, off);
         float Y[R][F], B[R][F], G[R][F], H[R][F];
-        issue_tile<R, F>(A.in0, A.in_dtype, off, Y, A.plane);
-        issue_tile<R, F>(A.in1, A.in_dtype, off, B, A.plane);
-        issue_tile<R, F>(A.g0, A.g_dtype, off, G);
+        issue_tile<R, F>(A.in0, in_dtype, off, Y, A.plane);
+        issue_tile<R, F>(A.in1, in_dtype, off, B, A.plane);
+        issue_tile<R, F>(A.g0, g_dtype, off, G);
         if (A.g1) {
-            issue_tile<R, F>(A.g1, A.g_dtype, off, H);
+            issue_tile<R, F>(A.g1, g_dtype, off, H);
         } else {
 #pragma unroll
             for (int rr = 0; rr < R; ++rr)
@@ -575,11 +587,11 @@ __global__ void __launch_bounds__(kBlockThreads, (TANH_ONLY && R * F <= 16 && F 
                 for (int f = 0; f < F; ++f) H[rr][f] = 0.f;
         }
         NCN_SCALE_W_ONCE
-        finish_tile<R, F>(A.in_dtype, Y);
-        finish_tile<R, F>(A.in_dtype, B);
-        finish_tile<R, F>(A.g_dtype, G);
-        if (A.g1) finish_tile<R, F>(A.g_dtype, H);
-        NCN_PASS_DEAD_ROWS(A.out0, A.out1, A.out_dtype, G, H)
+        finish_tile<R, F>(in_dtype, Y);
+        finish_tile<R, F>(in_dtype, B);
+        finish_tile<R, F>(g_dtype, G);
+        if (A.g1) finish_tile<R, F>(g_dtype, H);
+        NCN_PASS_DEAD_ROWS(A.out0, A.out1, out_dtype, G, H)
         if (A.aux0) { NCN_PASS_DEAD_ROWS(A.aux0, A.aux1, NCN_F32, Y, B) }
         NCN_ZERO_DEAD_ROWS(Y, B, false)
         NCN_ZERO_DEAD_ROWS(G, H, false)
@@ -588,8 +600,8 @@ __global__ void __launch_bounds__(kBlockThreads, (TANH_ONLY && R * F <= 16 && F 
 #pragma unroll
         for (int rr = 0; rr < R; ++rr) {
             const bool valid = INDEXED ? NCN_ROW_LIVE(rr) : live != 0;
-            store_frag<F>(A.out0, A.out_dtype, off[rr], valid, G[rr]);
-            store_frag<F>(A.out1, A.out_dtype, off[rr], valid, H[rr]);
+            store_frag<F>(A.out0, out_dtype, off[rr], valid, G[rr]);
+            store_frag<F>(A.out1, out_dtype, off[rr], valid, H[rr]);
             if (A.aux0) {
 #pragma unroll
                 for (int f = 0; f < F; ++f) {
