@@ -49,6 +49,13 @@ extern "C" {
  * (ncn_kernel_path() == 2); NCN_ERR_DTYPE elsewhere. */
 #define NCN_BF16X2 2
 
+/* Flags that may be or'ed into the first element type of a call (in_dtype of the forwards and inverses, y_dtype of the
+ * backwards).  NCN_W_BF16: W is bfloat16, and so is the dW that a backward writes (summed in float32, rounded once).
+ * NCN_W_ARRAYS: W is a host array of n_stages device pointers, each to the [2E] weights of one stage and 16-byte
+ * aligned (read during the call only); dW stays one array [n_stages, 2E]. */
+#define NCN_W_BF16 0x100
+#define NCN_W_ARRAYS 0x200
+
 /* activation codes: those of the reference's CUDA surface (ncn_pytorch_wrapper_v2.py:111,
  * ncn_fwd_cuda_kernel.cu:86-95): 0 tanh, 1 relu, 2 sigmoid, anything else the reference treats as
  * linear; here only -1 is accepted for linear.  Code 3 is the leaky relu of the reference's Triton kernels
@@ -92,7 +99,7 @@ typedef struct ncn_shape {
  *                  run in place on y, ya.
  * y32, ya32   out  optional (NULL to skip) float32 copies of the final y, ya: what a bf16 caller saves
  *                  for the reversible backward.
- * W           in   [n_stages, 2E] float32
+ * W           in   [n_stages, 2E] float32 (or as NCN_W_BF16, NCN_W_ARRAYS say)
  * workspace        optional scratch (NULL, 0 to skip).  With n_stages > 1 and small groups the library keeps
  *                  tiles of rows in LDS across several stages instead of launching stage by stage; when that
  *                  takes more than one pass it needs ncn_workspace_bytes_stages(.., backward = 0) bytes here
@@ -123,8 +130,8 @@ int ncn_forward(const void* x, const void* xa, int in_dtype,
  *                  two arrays of the workspace do (ncn_workspace_bytes_stages(.., backward = 2) bytes) and the
  *                  last stage to run writes no reconstructed inputs at all (NCN_ERR_ALIAS if the workspace is
  *                  smaller).
- * W           in   [n_stages, 2E] float32
- * dW          out  [n_stages, 2E] float32, overwritten (summed over batch, groups and rows)
+ * W           in   [n_stages, 2E] float32 (or as NCN_W_BF16, NCN_W_ARRAYS say)
+ * dW          out  [n_stages, 2E] float32 (NCN_W_BF16: bfloat16), overwritten (summed over batch, groups and rows)
  * workspace        scratch of at least ncn_workspace_bytes(shape) bytes; with n_stages > 1,
  *                  ncn_workspace_bytes_stages(.., backward = 1) bytes let the library use its multi-stage
  *                  LDS-resident passes (it falls back to one launch per stage with less)

@@ -10,6 +10,7 @@ PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(PKG_DIR, "libncn_hip.so")
 
 NCN_F32, NCN_BF16, NCN_BF16X2 = 0, 1, 2
+NCN_W_BF16, NCN_W_ARRAYS = 0x100, 0x200   # flags on the first element type of a call
 ACT_TANH, ACT_RELU, ACT_SIGMOID, ACT_LEAKY_RELU, ACT_LINEAR = 0, 1, 2, 3, -1
 
 EXPORTS = ("ncn_forward", "ncn_backward", "ncn_inverse", "ncn_forward_indexed", "ncn_backward_indexed",

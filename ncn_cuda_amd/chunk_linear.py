@@ -84,8 +84,8 @@ class FusedLinearChunkNCNFunction(torch.autograd.Function):
         _, _, dx, dxa, dW = ncn_cuda_module.backward_stages(
             yi, ya, dyi.contiguous(), dya.contiguous() if dya is not None else None, W, alpha, code, cache, heads, 0, 1,
             grad_dtype=ctx.io_dtype, want_inputs=False, group_index=ctx.group_tensor, ctx_len=ctx.ctxlen_tensor,
-            check_tables=False)
-        return dx, dxa, dW.reshape(W.shape).to(W.dtype), None, None, None, None, None, None, None
+            check_tables=False, dw_dtype=W.dtype)
+        return dx, dxa, dW.reshape(W.shape), None, None, None, None, None, None, None
 
 
 def fused_chunk_linear_ncn(x, xa, W, group_tensor, ctxlen_tensor, ALPHA, ACTIVATION, NHEAD, CACHE, l):

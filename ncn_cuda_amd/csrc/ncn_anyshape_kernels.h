@@ -208,9 +208,10 @@ __device__ __forceinline__ void for_each_row(const Fn& f) {
     const StepTable& S = A.tab;                                                                 \
     float wi[F], wj[F];                                                                         \
     _Pragma("unroll") for (int f = 0; f < F; ++f) {                                             \
-        const float* w = A.W + (int64_t)head * A.head_dim + L.feat[f];                          \
-        wi[f] = L.has[f] ? S.gamma * w[0] : 0.f;                                                \
-        wj[f] = L.has[f] ? S.gamma * w[A.E] : 0.f;                                              \
+        const int64_t at = (int64_t)head * A.head_dim + L.feat[f];                              \
+        const int w_dtype = A.w_bf16 ? NCN_BF16 : NCN_F32;                                      \
+        wi[f] = L.has[f] ? S.gamma * load_elem(A.W, w_dtype, at) : 0.f;                         \
+        wj[f] = L.has[f] ? S.gamma * load_elem(A.W, w_dtype, at + A.E) : 0.f;                   \
     }
 
 // INVERSE = false: x, xa -> y, ya (optional float32 copies);  true: y, ya -> x, xa

@@ -12,6 +12,46 @@ namespace {
 
 using namespace ncn;
 
+// The weights of a call: [n_stages][2E] of one array, or one array per stage (NCN_W_ARRAYS), float32 or bfloat16
+// (NCN_W_BF16); dW, always one array, has the same type.  The two flags come with the call's first element type.
+struct Weights {
+    const void* base;
+    int64_t two_e;
+    bool bf16, arrays;
+    // takes the flags out of dtype
+    Weights(const void* W, int& dtype, const ncn_shape* sh) : base(W), two_e(2 * sh->E) {
+        bf16 = (dtype & NCN_W_BF16) != 0;
+        arrays = (dtype & NCN_W_ARRAYS) != 0;
+        dtype &= ~(NCN_W_BF16 | NCN_W_ARRAYS);
+    }
+    size_t size() const { return bf16 ? 2 : 4; }
+    const void* at(int stage) const {
+        if (arrays) return static_cast<const void* const*>(base)[stage];
+        return static_cast<const char*>(base) + (size_t)stage * two_e * size();
+    }
+    void* out_at(void* dW, int stage) const { return static_cast<char*>(dW) + (size_t)stage * two_e * size(); }
+    bool aligned(int n_stages) const {
+        if (!arrays) return (reinterpret_cast<uintptr_t>(base) & 15u) == 0;
+        for (int k = 0; k < n_stages; ++k)
+            if (reinterpret_cast<uintptr_t>(at(k)) & 15u) return false;
+        return true;
+    }
+    bool null(int n_stages) const {
+        if (!base) return true;
+        for (int k = 0; arrays && k < n_stages; ++k)
+            if (!at(k)) return true;
+        return false;
+    }
+    void set(StageArgs& a, int stage) const {
+        a.W = at(stage);
+        a.w_bf16 = bf16;
+    }
+    void set(FusedArgs& a, int first, int count) const {
+        for (int k = 0; k < kFusedMaxStages; ++k) a.W[k] = k < count ? at(first + k) : nullptr;
+        a.w_bf16 = bf16;
+    }
+};
+
 bool known_activation(int a) {
     return a == NCN_ACT_TANH || a == NCN_ACT_RELU || a == NCN_ACT_SIGMOID || a == NCN_ACT_LEAKY_RELU || a == NCN_ACT_LINEAR;
 }
@@ -321,8 +361,11 @@ size_t temp_bytes(const ncn_shape* sh, bool backward) {
 // and the job (kReduceMaxSegments launches, kReduceMaxStages stages) hold them.
 class DwReducer {
   public:
-    DwReducer(float* partials, float* level1, int64_t two_e, hipStream_t s, int row_cap = kMaxGridX)
-        : partials_(partials), level1_(level1), two_e_(two_e), stream_(s), row_cap_(row_cap) { job_.n = 0; }
+    DwReducer(float* partials, float* level1, int64_t two_e, bool out_bf16, hipStream_t s, int row_cap = kMaxGridX)
+        : partials_(partials), level1_(level1), two_e_(two_e), stream_(s), row_cap_(row_cap) {
+        job_.n = 0;
+        job_.out_dtype = out_bf16 ? NCN_BF16 : NCN_F32;
+    }
     // Where a launch of `rows` partial rows of `stages` stages each may write; earlier launches are summed first
     // if it would not fit behind them.
     hipError_t reserve(int rows, int stages, float** region) {
@@ -334,7 +377,7 @@ class DwReducer {
         return err;
     }
     // The launch that got `region` from reserve() has been enqueued: its column sums go to dW_out[stages * 2E].
-    void add(const float* region, int rows, int stages, float* dW_out) {
+    void add(const float* region, int rows, int stages, void* dW_out) {
         ReduceSegment& g = job_.seg[job_.n];
         g.in = region;
         g.out = dW_out;
@@ -489,7 +532,8 @@ static int forward_impl(const void* x, const void* xa, int in_dtype, void* y, vo
     if (rc != NCN_OK) return rc;
     rc = check_grouping(grouping, shape);
     if (rc != NCN_OK) return rc;
-    if (!x || !xa || !y || !ya || !W) return NCN_ERR_NULL;
+    const Weights w(W, in_dtype, shape);
+    if (!x || !xa || !y || !ya || w.null(n_stages)) return NCN_ERR_NULL;
     if ((y32 == nullptr) != (ya32 == nullptr)) return NCN_ERR_NULL;
     const int path = kernel_path_for(shape, activation, alpha, m);
     if (path == 0) return NCN_ERR_UNSUPPORTED;
@@ -497,12 +541,11 @@ static int forward_impl(const void* x, const void* xa, int in_dtype, void* y, vo
     const bool headwise = headwise_call(shape, path, &as_wide);
     if (headwise) shape = &as_wide;
     if (!known_dtype(in_dtype) || !known_dtype_or_x2(out_dtype, n_stages, path)) return NCN_ERR_DTYPE;
-    if (!aligned16(x) || !aligned16(xa) || !aligned16(y) || !aligned16(ya) || !aligned16(W) || !aligned16(y32) ||
+    if (!aligned16(x) || !aligned16(xa) || !aligned16(y) || !aligned16(ya) || !w.aligned(n_stages) || !aligned16(y32) ||
         !aligned16(ya32) || !aligned16(workspace))
         return NCN_ERR_ALIGN;
     const Plan p = make_plan(shape, path, any_tile_for(shape, path, alpha, m));
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const int64_t wstride = 2 * shape->E;
 
     // several stages: LDS-resident passes when the shape allows and the buffers permit the ping-pong
     std::vector<FusedPass> passes;
@@ -516,7 +559,7 @@ static int forward_impl(const void* x, const void* xa, int in_dtype, void* y, vo
         a.in0 = i0; a.in1 = i1; a.in_dtype = i_dtype;
         a.out0 = o0; a.out1 = o1; a.out_dtype = o_dtype;
         a.aux0 = with_copies ? y32 : nullptr; a.aux1 = with_copies ? ya32 : nullptr;
-        a.W = W + k * wstride;
+        w.set(a, k);
         hipError_t err = run_forward_kernel(kForward, a, p, grouping.plain(), headwise, s);
         if (err == hipSuccess && grouping.ctx_len) err = launch_ragged_rest(kForward, a, shape, p, 0, s);
         return err;
@@ -545,7 +588,7 @@ static int forward_impl(const void* x, const void* xa, int in_dtype, void* y, vo
                 a.in0 = k == 0 ? x : y; a.in1 = k == 0 ? xa : ya; a.in_dtype = k == 0 ? in_dtype : out_dtype;
                 a.out0 = y; a.out1 = ya; a.out_dtype = out_dtype;
                 a.aux0 = last ? y32 : nullptr; a.aux1 = last ? ya32 : nullptr;
-                a.W = W + ps.first * wstride;
+                w.set(a, ps.first, ps.count);
                 a.ctx_len = grouping.ctx_len;
                 fill_step_table(a.tab, shape->n_cache, alpha, m, activation);
                 err = launch_fused(kForward, a, shape, ps, s, kMaxGridX, headwise);
@@ -576,7 +619,7 @@ static int forward_impl(const void* x, const void* xa, int in_dtype, void* y, vo
                 a.in0 = cur0; a.in1 = cur1; a.in_dtype = cur_dtype;
                 a.out0 = d0; a.out1 = d1; a.out_dtype = d_dtype;
                 a.aux0 = last ? y32 : nullptr; a.aux1 = last ? ya32 : nullptr;
-                a.W = W + ps.first * wstride;
+                w.set(a, ps.first, ps.count);
                 a.ctx_len = grouping.ctx_len;
                 fill_step_table(a.tab, shape->n_cache, alpha, m, activation);
                 err = launch_fused(kForward, a, shape, ps, s, kMaxGridX, headwise);
@@ -599,7 +642,7 @@ static int forward_impl(const void* x, const void* xa, int in_dtype, void* y, vo
         const bool last = (k == n_stages - 1);
         a.aux0 = last ? y32 : nullptr;
         a.aux1 = last ? ya32 : nullptr;
-        a.W = W + k * wstride;
+        w.set(a, k);
         hipError_t err = run_forward_kernel(kForward, a, p, grouping.plain(), headwise, s);
         if (err == hipSuccess && grouping.ctx_len) err = launch_ragged_rest(kForward, a, shape, p, 0, s);
         if (err != hipSuccess) return (int)err;
@@ -614,14 +657,15 @@ static int inverse_impl(const void* y, const void* ya, int in_dtype, void* x, vo
     if (rc != NCN_OK) return rc;
     rc = check_grouping(grouping, shape);
     if (rc != NCN_OK) return rc;
-    if (!x || !xa || !y || !ya || !W) return NCN_ERR_NULL;
+    const Weights w(W, in_dtype, shape);
+    if (!x || !xa || !y || !ya || w.null(n_stages)) return NCN_ERR_NULL;
     const int path = kernel_path_for(shape, activation, alpha, m);
     if (path == 0) return NCN_ERR_UNSUPPORTED;
     ncn_shape as_wide;
     const bool headwise = headwise_call(shape, path, &as_wide);
     if (headwise) shape = &as_wide;
     if (!known_dtype_or_x2(in_dtype, n_stages, path) || !known_dtype(out_dtype)) return NCN_ERR_DTYPE;
-    if (!aligned16(x) || !aligned16(xa) || !aligned16(y) || !aligned16(ya) || !aligned16(W) || !aligned16(workspace))
+    if (!aligned16(x) || !aligned16(xa) || !aligned16(y) || !aligned16(ya) || !w.aligned(n_stages) || !aligned16(workspace))
         return NCN_ERR_ALIGN;
     const Plan p = make_plan(shape, path, any_tile_for(shape, path, alpha, m));
     hipStream_t s = static_cast<hipStream_t>(stream);
@@ -637,7 +681,7 @@ static int inverse_impl(const void* y, const void* ya, int in_dtype, void* x, vo
         fill_common(a, shape, p, first_stage + k, alpha, m, activation, grouping, k);
         a.in0 = i0; a.in1 = i1; a.in_dtype = i_dtype;
         a.out0 = o0; a.out1 = o1; a.out_dtype = o_dtype;
-        a.W = W + (int64_t)k * 2 * shape->E;
+        w.set(a, k);
         hipError_t err = run_forward_kernel(kInverse, a, p, grouping.plain(), headwise, s);
         if (err == hipSuccess && grouping.ctx_len) err = launch_ragged_rest(kInverse, a, shape, p, 0, s);
         return err;
@@ -648,7 +692,6 @@ static int inverse_impl(const void* y, const void* ya, int in_dtype, void* x, vo
                            workspace_bytes >= temp_bytes(shape, false) &&
                            !((x == y || xa == ya) && ((passes.size() - 1) % 2) == 0);   // never straight from y into y
     if (ping_pong) {
-        const int64_t wstride = 2 * shape->E;
         const size_t np = passes.size();
         const size_t one = temp_bytes(shape, false) / 2;
         void* t0 = workspace;
@@ -668,7 +711,7 @@ static int inverse_impl(const void* y, const void* ya, int in_dtype, void* x, vo
                 FusedArgs a{};
                 a.in0 = cur0; a.in1 = cur1; a.in_dtype = cur_dtype;
                 a.out0 = d0; a.out1 = d1; a.out_dtype = NCN_F32;
-                a.W = W + ps.first * wstride;
+                w.set(a, ps.first, ps.count);
                 a.ctx_len = grouping.ctx_len;
                 fill_step_table(a.tab, shape->n_cache, alpha, m, activation);
                 err = launch_fused(kInverse, a, shape, ps, s, kMaxGridX, headwise);
@@ -679,7 +722,6 @@ static int inverse_impl(const void* y, const void* ya, int in_dtype, void* x, vo
         return NCN_OK;
     }
     if (!passes.empty()) {
-        const int64_t wstride = 2 * shape->E;
         const size_t np = passes.size();
         for (size_t e = 0; e < np; ++e) {
             const FusedPass& ps = passes[np - 1 - e];
@@ -696,7 +738,7 @@ static int inverse_impl(const void* y, const void* ya, int in_dtype, void* x, vo
                 FusedArgs a{};
                 a.in0 = top ? y : x; a.in1 = top ? ya : xa; a.in_dtype = top ? in_dtype : out_dtype;
                 a.out0 = x; a.out1 = xa; a.out_dtype = out_dtype;
-                a.W = W + ps.first * wstride;
+                w.set(a, ps.first, ps.count);
                 a.ctx_len = grouping.ctx_len;
                 fill_step_table(a.tab, shape->n_cache, alpha, m, activation);
                 hipError_t err = launch_fused(kInverse, a, shape, ps, s, kMaxGridX, headwise);
@@ -716,7 +758,7 @@ static int inverse_impl(const void* y, const void* ya, int in_dtype, void* x, vo
         a.out0 = x;
         a.out1 = xa;
         a.out_dtype = out_dtype;
-        a.W = W + (int64_t)k * 2 * shape->E;
+        w.set(a, k);
         hipError_t err = run_forward_kernel(kInverse, a, p, grouping.plain(), headwise, s);
         if (err == hipSuccess && grouping.ctx_len) err = launch_ragged_rest(kInverse, a, shape, p, 0, s);
         if (err != hipSuccess) return (int)err;
@@ -733,7 +775,8 @@ static int backward_impl(const void* y, const void* ya, int y_dtype, const void*
     if (rc != NCN_OK) return rc;
     rc = check_grouping(grouping, shape);
     if (rc != NCN_OK) return rc;
-    if (!y || !ya || !dy || !dx || !dxa || !W || !dW) return NCN_ERR_NULL;
+    const Weights w(W, y_dtype, shape);
+    if (!y || !ya || !dy || !dx || !dxa || w.null(n_stages) || !dW) return NCN_ERR_NULL;
     if ((x_rec == nullptr) != (xa_rec == nullptr)) return NCN_ERR_NULL;
     const int path = kernel_path_for(shape, activation, alpha, m);
     if (path == 0) return NCN_ERR_UNSUPPORTED;
@@ -749,7 +792,7 @@ static int backward_impl(const void* y, const void* ya, int y_dtype, const void*
     const bool no_rec = n_stages > 1 && !x_rec;
     const size_t plane_bytes = temp_bytes(shape, true) / 4;
     if (!aligned16(y) || !aligned16(ya) || !aligned16(dy) || !aligned16(dya) || !aligned16(dx) || !aligned16(dxa) ||
-        !aligned16(x_rec) || !aligned16(xa_rec) || !aligned16(W) || !aligned16(dW) || !aligned16(workspace))
+        !aligned16(x_rec) || !aligned16(xa_rec) || !w.aligned(n_stages) || !aligned16(dW) || !aligned16(workspace))
         return NCN_ERR_ALIGN;
     // partial rows of the generic kernel's second launch
     const AnyTile any = any_tile_for(shape, path, alpha, m);
@@ -790,7 +833,7 @@ static int backward_impl(const void* y, const void* ya, int y_dtype, const void*
         float* reca = no_rec ? (np >= 2 ? reinterpret_cast<float*>(tb + 5 * one) : nullptr) : xa_rec;
         const void* cy = y; const void* cya = ya; int cy_dtype = y_dtype;
         const void* cg = dy; const void* cga = dya; int cg_dtype = dy_dtype;
-        DwReducer reducer(partials, partials + (int64_t)fused_cap * wstride, wstride, s, fused_cap);
+        DwReducer reducer(partials, partials + (int64_t)fused_cap * wstride, wstride, w.bf16, s, fused_cap);
         for (size_t e = 0; e < np; ++e) {
             const FusedPass& ps = passes[np - 1 - e];
             const bool to_out = ((np - 1 - e) % 2) == 0;
@@ -812,7 +855,7 @@ static int backward_impl(const void* y, const void* ya, int y_dtype, const void*
                 a.g0 = cg; a.g1 = cga; a.g_dtype = cg_dtype;
                 a.out0 = ddx; a.out1 = ddxa; a.out_dtype = d_dtype;
                 a.aux0 = dxr; a.aux1 = dxar;
-                a.W = W + ps.first * wstride;
+                w.set(a, ps.first);
                 a.dw_partials = region;
                 err = run_backward_kernel(a, p, grouping.plain(), headwise, s);
                 if (err == hipSuccess && grouping.ctx_len)
@@ -823,14 +866,14 @@ static int backward_impl(const void* y, const void* ya, int y_dtype, const void*
                 a.g0 = cg; a.g1 = cga; a.g_dtype = cg_dtype;
                 a.out0 = ddx; a.out1 = ddxa; a.out_dtype = d_dtype;
                 a.aux0 = dxr; a.aux1 = dxar;
-                a.W = W + ps.first * wstride;
+                w.set(a, ps.first, ps.count);
                 a.dw_partials = region;
                 a.ctx_len = grouping.ctx_len;
                 fill_step_table(a.tab, shape->n_cache, alpha, m, activation);
                 err = launch_fused(kBackward, a, shape, ps, s, fused_cap, headwise);
             }
             if (err != hipSuccess) return (int)err;
-            reducer.add(region, rows, ps.count, dW + ps.first * wstride);
+            reducer.add(region, rows, ps.count, w.out_at(dW, ps.first));
             cy = dxr; cya = dxar; cy_dtype = NCN_F32;
             cg = ddx; cga = ddxa; cg_dtype = d_dtype;
         }
@@ -843,7 +886,7 @@ static int backward_impl(const void* y, const void* ya, int y_dtype, const void*
         x_rec = reinterpret_cast<float*>(cb);
         xa_rec = reinterpret_cast<float*>(cb + plane_bytes);
     }
-    DwReducer reducer(partials, level1, wstride, s, row_cap);
+    DwReducer reducer(partials, level1, wstride, w.bf16, s, row_cap);
     for (int k = n_stages - 1; k >= 0; --k) {
         float* region;
         hipError_t err = reducer.reserve(p.partial_rows + extra_rows, 1, &region);
@@ -862,12 +905,12 @@ static int backward_impl(const void* y, const void* ya, int y_dtype, const void*
         a.out_dtype = dx_dtype;
         a.aux0 = (no_rec && k == 0) ? nullptr : x_rec;   // the last stage to run hands nothing on
         a.aux1 = (no_rec && k == 0) ? nullptr : xa_rec;
-        a.W = W + (int64_t)k * 2 * shape->E;
+        w.set(a, k);
         a.dw_partials = region;
         err = run_backward_kernel(a, p, grouping.plain(), headwise, s);
         if (err == hipSuccess && grouping.ctx_len) err = launch_ragged_rest(kBackward, a, shape, p, p.partial_rows, s);
         if (err != hipSuccess) return (int)err;
-        reducer.add(region, p.partial_rows + extra_rows, 1, dW + k * wstride);
+        reducer.add(region, p.partial_rows + extra_rows, 1, w.out_at(dW, k));
     }
     return (int)reducer.flush();
 }
@@ -951,10 +994,11 @@ int ncn_forward_radix(const void* x, const void* xa, int in_dtype, void* y, void
     if (rc != NCN_OK) return rc;
     rc = check_radix(shape, first_level, n_levels);
     if (rc != NCN_OK) return rc;
-    if (!x || !xa || !y || !ya || !W) return NCN_ERR_NULL;
+    const Weights w(W, in_dtype, shape);
+    if (!x || !xa || !y || !ya || w.null(n_levels)) return NCN_ERR_NULL;
     if ((y32 == nullptr) != (ya32 == nullptr)) return NCN_ERR_NULL;
     if (!known_dtype(in_dtype) || !known_dtype(out_dtype)) return NCN_ERR_DTYPE;
-    if (!aligned16(x) || !aligned16(xa) || !aligned16(y) || !aligned16(ya) || !aligned16(W) || !aligned16(y32) ||
+    if (!aligned16(x) || !aligned16(xa) || !aligned16(y) || !aligned16(ya) || !w.aligned(n_levels) || !aligned16(y32) ||
         !aligned16(ya32))
         return NCN_ERR_ALIGN;
     const int path = kernel_path_for(shape, activation, alpha, m);
@@ -964,7 +1008,6 @@ int ncn_forward_radix(const void* x, const void* xa, int in_dtype, void* y, void
     if (headwise) shape = &as_wide;
     const Plan p = make_plan(shape, path, any_tile_for(shape, path, alpha, m));
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const int64_t wstride = 2 * shape->E;
     const std::vector<RadixPass> passes = plan_radix(shape, first_level, n_levels, false, path == 2);
     // every pass is closed: the first reads x, xa and the later ones run in place on y, ya; passes of several levels
     // keep their state in float32 LDS and convert on the way out
@@ -979,14 +1022,14 @@ int ncn_forward_radix(const void* x, const void* xa, int in_dtype, void* y, void
             a.in0 = first ? x : y; a.in1 = first ? xa : ya; a.in_dtype = first ? in_dtype : out_dtype;
             a.out0 = y; a.out1 = ya; a.out_dtype = out_dtype;
             a.aux0 = last ? y32 : nullptr; a.aux1 = last ? ya32 : nullptr;
-            a.W = W + ps.first * wstride;
+            w.set(a, ps.first);
             err = run_forward_kernel(kForward, a, p, false, headwise, s);
         } else {
             FusedArgs a{};
             a.in0 = first ? x : y; a.in1 = first ? xa : ya; a.in_dtype = first ? in_dtype : out_dtype;
             a.out0 = y; a.out1 = ya; a.out_dtype = out_dtype;
             a.aux0 = last ? y32 : nullptr; a.aux1 = last ? ya32 : nullptr;
-            a.W = W + ps.first * wstride;
+            w.set(a, ps.first, ps.count);
             fill_step_table(a.tab, shape->n_cache, alpha, m, activation);
             err = launch_fused_radix(kForward, a, shape, ps, s, headwise);
         }
@@ -1003,7 +1046,8 @@ int ncn_backward_radix(const void* y, const void* ya, int y_dtype, const void* d
     if (rc != NCN_OK) return rc;
     rc = check_radix(shape, first_level, n_levels);
     if (rc != NCN_OK) return rc;
-    if (!y || !ya || !dy || !dx || !dxa || !W || !dW) return NCN_ERR_NULL;
+    const Weights w(W, y_dtype, shape);
+    if (!y || !ya || !dy || !dx || !dxa || w.null(n_levels) || !dW) return NCN_ERR_NULL;
     if ((x_rec == nullptr) != (xa_rec == nullptr)) return NCN_ERR_NULL;
     if (!known_dtype(y_dtype) || !known_dtype(dy_dtype) || !known_dtype(dx_dtype)) return NCN_ERR_DTYPE;
     if (n_levels > 1 && dx_dtype != NCN_F32) return NCN_ERR_ALIAS;
@@ -1019,7 +1063,7 @@ int ncn_backward_radix(const void* y, const void* ya, int y_dtype, const void* d
         xa_rec = reinterpret_cast<float*>(cb + plane_bytes);
     }
     if (!aligned16(y) || !aligned16(ya) || !aligned16(dy) || !aligned16(dya) || !aligned16(dx) || !aligned16(dxa) ||
-        !aligned16(x_rec) || !aligned16(xa_rec) || !aligned16(W) || !aligned16(dW) || !aligned16(workspace))
+        !aligned16(x_rec) || !aligned16(xa_rec) || !w.aligned(n_levels) || !aligned16(dW) || !aligned16(workspace))
         return NCN_ERR_ALIGN;
     const int path = kernel_path_for(shape, activation, alpha, m);
     if (path == 0) return NCN_ERR_UNSUPPORTED;
@@ -1033,7 +1077,7 @@ int ncn_backward_radix(const void* y, const void* ya, int y_dtype, const void* d
     const int64_t wstride = 2 * shape->E;
     const std::vector<RadixPass> passes = plan_radix(shape, first_level, n_levels, true, path == 2);
     // last pass first; the first one to run reads y, ya, dy, dya, the others run in place on x_rec, xa_rec, dx, dxa
-    DwReducer reducer(partials, level1, wstride, s);
+    DwReducer reducer(partials, level1, wstride, w.bf16, s);
     for (size_t e = 0; e < passes.size(); ++e) {
         const RadixPass& ps = passes[passes.size() - 1 - e];
         const bool top = (e == 0);
@@ -1050,7 +1094,7 @@ int ncn_backward_radix(const void* y, const void* ya, int y_dtype, const void* d
             a.g0 = top ? dy : dx; a.g1 = top ? dya : dxa; a.g_dtype = top ? dy_dtype : NCN_F32;
             a.out0 = dx; a.out1 = dxa; a.out_dtype = dx_dtype;
             a.aux0 = drop_rec ? nullptr : x_rec; a.aux1 = drop_rec ? nullptr : xa_rec;
-            a.W = W + ps.first * wstride;
+            w.set(a, ps.first);
             a.dw_partials = region;
             err = run_backward_kernel(a, p, false, headwise, s);
         } else {
@@ -1059,13 +1103,13 @@ int ncn_backward_radix(const void* y, const void* ya, int y_dtype, const void* d
             a.g0 = top ? dy : dx; a.g1 = top ? dya : dxa; a.g_dtype = top ? dy_dtype : NCN_F32;
             a.out0 = dx; a.out1 = dxa; a.out_dtype = dx_dtype;
             a.aux0 = drop_rec ? nullptr : x_rec; a.aux1 = drop_rec ? nullptr : xa_rec;
-            a.W = W + ps.first * wstride;
+            w.set(a, ps.first, ps.count);
             a.dw_partials = region;
             fill_step_table(a.tab, shape->n_cache, alpha, m, activation);
             err = launch_fused_radix(kBackward, a, shape, ps, s, headwise);
         }
         if (err != hipSuccess) return (int)err;
-        reducer.add(region, rows, ps.count, dW + ps.first * wstride);
+        reducer.add(region, rows, ps.count, w.out_at(dW, ps.first));
     }
     return (int)reducer.flush();
 }
@@ -1077,9 +1121,10 @@ int ncn_inverse_radix(const void* y, const void* ya, int in_dtype, void* x, void
     if (rc != NCN_OK) return rc;
     rc = check_radix(shape, first_level, n_levels);
     if (rc != NCN_OK) return rc;
-    if (!x || !xa || !y || !ya || !W) return NCN_ERR_NULL;
+    const Weights w(W, in_dtype, shape);
+    if (!x || !xa || !y || !ya || w.null(n_levels)) return NCN_ERR_NULL;
     if (!known_dtype(in_dtype) || !known_dtype(out_dtype)) return NCN_ERR_DTYPE;
-    if (!aligned16(x) || !aligned16(xa) || !aligned16(y) || !aligned16(ya) || !aligned16(W)) return NCN_ERR_ALIGN;
+    if (!aligned16(x) || !aligned16(xa) || !aligned16(y) || !aligned16(ya) || !w.aligned(n_levels)) return NCN_ERR_ALIGN;
     const int path = kernel_path_for(shape, activation, alpha, m);
     if (path == 0) return NCN_ERR_UNSUPPORTED;
     ncn_shape as_wide;
@@ -1087,7 +1132,6 @@ int ncn_inverse_radix(const void* y, const void* ya, int in_dtype, void* x, void
     if (headwise) shape = &as_wide;
     const Plan p = make_plan(shape, path, any_tile_for(shape, path, alpha, m));
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const int64_t wstride = 2 * shape->E;
     const std::vector<RadixPass> passes = plan_radix(shape, first_level, n_levels, false, path == 2);
     for (size_t e = 0; e < passes.size(); ++e) {   // last pass first; every pass is closed: in place after the first
         const RadixPass& ps = passes[passes.size() - 1 - e];
@@ -1099,13 +1143,13 @@ int ncn_inverse_radix(const void* y, const void* ya, int in_dtype, void* x, void
             fill_common(a, shape, p, 0, alpha, m, activation, g, 0);
             a.in0 = top ? y : x; a.in1 = top ? ya : xa; a.in_dtype = top ? in_dtype : out_dtype;
             a.out0 = x; a.out1 = xa; a.out_dtype = out_dtype;
-            a.W = W + ps.first * wstride;
+            w.set(a, ps.first);
             err = run_forward_kernel(kInverse, a, p, false, headwise, s);
         } else {
             FusedArgs a{};
             a.in0 = top ? y : x; a.in1 = top ? ya : xa; a.in_dtype = top ? in_dtype : out_dtype;
             a.out0 = x; a.out1 = xa; a.out_dtype = out_dtype;
-            a.W = W + ps.first * wstride;
+            w.set(a, ps.first, ps.count);
             fill_step_table(a.tab, shape->n_cache, alpha, m, activation);
             err = launch_fused_radix(kInverse, a, shape, ps, s, headwise);
         }

@@ -56,7 +56,7 @@ struct StageArgs {
     void* out1;
     float* aux0;
     float* aux1;
-    const float* W;      // [2E] of this stage
+    const void* W;       // [2E] of this stage, float32 or (w_bf16) bfloat16
     float* dw_partials;  // backward: [partial rows][2E]
     const int32_t* table;    // [N] slot -> position, or null
     const int32_t* ctx_len;  // [batch] live slots per batch entry, or null
@@ -71,6 +71,7 @@ struct StageArgs {
     int32_t in_dtype, g_dtype, out_dtype;
     int32_t activation;
     int32_t edge;
+    int32_t w_bf16;
     uint32_t radix_stride;   // n_cache^level: groups are the radix-n digit groups of that level (0: not used)
     uint32_t any_tile;       // ncn_anyshape_kernels.h: R | F << 8 | log2(lanes per row) << 16 | log2(row lanes) << 24
     StepTable tab;

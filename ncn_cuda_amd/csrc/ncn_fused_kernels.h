@@ -72,12 +72,12 @@ struct FusedArgs {
     void* out1;        //          ya             dxa
     float* aux0;       // forward: optional float32 copy of y     backward: x_rec (inputs of the pass's first stage)
     float* aux1;       //          optional float32 copy of ya              xa_rec
-    const float* W;    // [n_stages][2E], first stage of the pass first
+    const void* W[kFusedMaxStages];   // [2E] of each stage of the pass, first stage first; float32 or (w_bf16) bfloat16
     float* dw_partials;  // backward: [gridDim.x / n_head][n_stages][2E]
     const int32_t* ctx_len;  // LENGTHS builds: [batch] live slots per batch entry (in the group order of each stage)
     int64_t N, E;
     int32_t n_head, n_stages;
-    int32_t in_dtype, g_dtype, out_dtype;
+    int32_t in_dtype, g_dtype, out_dtype, w_bf16;
     uint32_t ring_magic;      // 0 when `ring` is a power of two, else ceil(2^32 / ring): closed passes divide by the ring
     // RADIX builds read: class_stride = n^a in rows, ring = n^k rows per window, window = rows / n_cache,
     // class_groups = workgroup-loads per batch entry, sub_stride[j] = n^j in rows, closed = 1
@@ -315,9 +315,14 @@ __device__ __forceinline__ void fused_store_rows_scaled(const FusedArgs& A, cons
 // the pass's weights times gamma, [stage][Wi | Wj][EC] of this workgroup's head, into LDS
 template <int EC, int NW>
 __device__ __forceinline__ void fused_load_weights(const FusedArgs& A, int head, float* w_lds) {
-    for (int k = threadIdx.x; k < A.n_stages * 2 * EC; k += 64 * NW) {
-        const int st = k / (2 * EC), rem = k - st * 2 * EC, half = rem / EC, f = rem - half * EC;
-        w_lds[k] = A.tab.gamma * A.W[(int64_t)st * 2 * A.E + (int64_t)half * A.E + (int64_t)head * EC + f];
+    // a wave per stage, so that the stage's pointer is a scalar load
+    for (int st = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); st < A.n_stages; st += NW) {
+        const void* w = A.W[st];
+        const int dtype = A.w_bf16 ? NCN_BF16 : NCN_F32;
+        for (int k = threadIdx.x & 63; k < 2 * EC; k += 64) {
+            const int half = k / EC, f = k - half * EC;
+            w_lds[st * 2 * EC + k] = A.tab.gamma * load_elem(w, dtype, (int64_t)half * A.E + (int64_t)head * EC + f);
+        }
     }
 }
 

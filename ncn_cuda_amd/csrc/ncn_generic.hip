@@ -53,6 +53,15 @@ __device__ __forceinline__ GenericLane generic_lane(const StageArgs& A, uint32_t
     return L;
 }
 
+__device__ __forceinline__ void generic_load_weights(const StageArgs& A, int head, float* Wi, float* Wj) {
+    const int dtype = A.w_bf16 ? NCN_BF16 : NCN_F32;
+    for (int f = threadIdx.x; f < A.head_dim; f += 64) {
+        Wi[f] = load_elem(A.W, dtype, (int64_t)head * A.head_dim + f);
+        Wj[f] = load_elem(A.W, dtype, A.E + (int64_t)head * A.head_dim + f);
+    }
+    __syncthreads();
+}
+
 #define LDS(arr, f) lds[((arr) * ec + (f)) * 64 + lane]
 #define LDS_AT(arr, f, l) lds[((arr) * ec + (f)) * 64 + (l)]
 
@@ -62,8 +71,8 @@ __global__ void __launch_bounds__(64) generic_forward_kernel(const StageArgs A, 
     const int lane = threadIdx.x, head = blockIdx.y, ec = A.head_dim;
     const float alpha = A.tab.alpha, m = A.tab.m, om = 1.f - A.tab.m, oa = 1.f - A.tab.alpha;
     const float inv_m = 1.f / m, k_ba = om / m;
-    const float* Wi = A.W + (int64_t)head * ec;
-    const float* Wj = Wi + A.E;
+    __shared__ float Wi[kGenericMaxHeadDim], Wj[kGenericMaxHeadDim];
+    generic_load_weights(A, head, Wi, Wj);
     enum { X = 0, XA = 1 };
     for (uint32_t t = blockIdx.x; t < A.total_tiles; t += gridDim.x) {
         const GenericLane L = generic_lane(A, t, lane, head);
@@ -120,8 +129,8 @@ __global__ void __launch_bounds__(64) generic_backward_kernel(const StageArgs A)
     const int lane = threadIdx.x, head = blockIdx.y, ec = A.head_dim;
     const float alpha = A.tab.alpha, m = A.tab.m, om = 1.f - A.tab.m, oa = 1.f - A.tab.alpha;
     const float inv_m = 1.f / m, k_ba = om / m, k1 = om * om, k2 = om, kh1 = m * om;
-    const float* Wi = A.W + (int64_t)head * ec;
-    const float* Wj = Wi + A.E;
+    __shared__ float Wi[kGenericMaxHeadDim], Wj[kGenericMaxHeadDim];
+    generic_load_weights(A, head, Wi, Wj);
     enum { X = 0, XA = 1, G = 2, H = 3, U = 4, DWI = 5, DWJ = 6 };
     for (int f = 0; f < ec; ++f) LDS(DWI, f) = LDS(DWJ, f) = 0.f;
     for (uint32_t t = blockIdx.x; t < A.total_tiles; t += gridDim.x) {
@@ -220,7 +229,7 @@ __global__ void __launch_bounds__(1024) reduce_rows_kernel(const ReduceJob J) {
 #pragma unroll
         for (int w = 0; w < 16; w += 4)
             total += (red[w][threadIdx.x] + red[w + 1][threadIdx.x]) + (red[w + 2][threadIdx.x] + red[w + 3][threadIdx.x]);
-        g.out[col0 + threadIdx.x] = total;
+        store_elem(g.out, J.out_dtype, col0 + threadIdx.x, total);
     }
 }
 
@@ -230,7 +239,7 @@ __global__ void __launch_bounds__(1024) reduce_rows_kernel(const ReduceJob J) {
 // blocks, so it takes narrow blocks with many row lanes); the order of additions is fixed.
 template <int RL>
 __device__ __forceinline__ void reduce_rows(const float* __restrict__ in, int r0, int r1, int64_t row_stride, int64_t cols,
-                                            float* __restrict__ out) {
+                                            void* __restrict__ out, int out_dtype) {
     constexpr int CW = 256 / RL;
     __shared__ float red[RL][CW];
     const int cx = threadIdx.x % CW, ry = threadIdx.x / CW;
@@ -246,7 +255,7 @@ __device__ __forceinline__ void reduce_rows(const float* __restrict__ in, int r0
         float total = 0.f;
 #pragma unroll
         for (int k = 0; k < RL; k += 4) total += (red[k][cx] + red[k + 1][cx]) + (red[k + 2][cx] + red[k + 3][cx]);
-        out[col] = total;
+        store_elem(out, out_dtype, col, total);
     }
 }
 
@@ -259,13 +268,13 @@ __global__ void __launch_bounds__(256) reduce_chunks_kernel(const ReduceJob J, f
     const int chunk = blockIdx.y - g.chunk0;
     const int r0 = chunk * kReduceRowsPerBlock;
     reduce_rows<kReduceLevel1Lanes>(g.in, r0, min(g.rows, r0 + kReduceRowsPerBlock), g.cols, g.cols,
-                                    level1 + g.level1_offset + chunk * g.cols);
+                                    level1 + g.level1_offset + chunk * g.cols, NCN_F32);
 }
 
 __global__ void __launch_bounds__(256) reduce_segments_kernel(const ReduceJob J, const float* __restrict__ level1) {
     const ReduceSegment& g = J.seg[blockIdx.y];
     const int chunks = (g.rows + kReduceRowsPerBlock - 1) / kReduceRowsPerBlock;
-    reduce_rows<kReduceLevel2Lanes>(level1 + g.level1_offset, 0, chunks, g.cols, g.cols, g.out);
+    reduce_rows<kReduceLevel2Lanes>(level1 + g.level1_offset, 0, chunks, g.cols, g.cols, g.out, J.out_dtype);
 }
 
 // Rows past a batch entry's context length take no part in the stage: they pass through.

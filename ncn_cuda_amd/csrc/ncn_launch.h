@@ -49,7 +49,7 @@ constexpr int kReduceMaxStages = 8;
 constexpr int kReduceLevel1Rows = kMaxGridX / kReduceRowsPerBlock + kReduceMaxStages;
 struct ReduceSegment {
     const float* in;        // [rows][cols], dense
-    float* out;             // [cols]
+    void* out;              // [cols] of the job's out_dtype
     int64_t cols;           // stages of the launch * 2E
     int64_t level1_offset;  // floats before this segment's chunk sums in the level-1 scratch
     int rows;
@@ -58,6 +58,7 @@ struct ReduceSegment {
 struct ReduceJob {
     ReduceSegment seg[kReduceMaxSegments];
     int n;
+    int out_dtype;
 };
 // out[col] of every segment = sum of its rows, in a fixed order; level1 is scratch of kReduceLevel1Rows * 2E floats.
 hipError_t launch_reduce_job(const ReduceJob& job, float* level1, hipStream_t s);

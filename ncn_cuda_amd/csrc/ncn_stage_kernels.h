@@ -70,14 +70,17 @@ __device__ __forceinline__ int tile_offsets(const StageArgs& A, uint32_t t, int 
     return live;
 }
 
+// A lane's weights times gamma.
 template <int F>
-__device__ __forceinline__ void load_w(const float* W, int64_t E, int head, int ec, int fl, float (&wi)[F],
-                                       float (&wj)[F]) {
-    const float* w = W + (int64_t)head * ec + fl * F;
+__device__ __forceinline__ void load_w(const StageArgs& A, int head, int ec, int fl, float (&wi)[F], float (&wj)[F]) {
+    const int64_t at = (int64_t)head * ec + fl * F;
+    const int dtype = A.w_bf16 ? NCN_BF16 : NCN_F32;
+    load_frag<F>(A.W, dtype, at, true, wi);
+    load_frag<F>(A.W, dtype, at + A.E, true, wj);
 #pragma unroll
     for (int f = 0; f < F; ++f) {
-        wi[f] = w[f];
-        wj[f] = w[E + f];
+        wi[f] *= A.tab.gamma;
+        wj[f] *= A.tab.gamma;
     }
 }
 
@@ -446,18 +449,15 @@ __device__ __forceinline__ void backward_steps(float (&Y)[R][F], float (&B)[R][F
     float4* slots = bcast_lds + (T::LR == 1 ? 0 : wave * (F / 4) * 64);                         \
     const int fl = lane % T::LF;                                                                \
     float wi[F], wj[F];                                                                         \
-    load_w<F>(A.W, A.E, head, EC, fl, wi, wj);                                                  \
-    bool w_raw = true;
+    bool w_todo = true;
 
-// The weights are scaled by gamma once, after the loads of the wave's first tile have been issued: scaling them in the
-// prologue would wait for them before the tile's own loads are even on their way (one memory latency after the other).
-#define NCN_SCALE_W_ONCE                                                                        \
-    if (w_raw) {                                                                                \
-        w_raw = false;                                                                          \
-        _Pragma("unroll") for (int f = 0; f < F; ++f) {                                         \
-            wi[f] *= A.tab.gamma;                                                               \
-            wj[f] *= A.tab.gamma;                                                               \
-        }                                                                                       \
+// The weights are loaded once, after the loads of the wave's first tile have been issued: their branch on the type waits
+// for them, and in the prologue that wait would come before the tile's own loads are even on their way (one memory
+// latency after the other).
+#define NCN_LOAD_W_ONCE                                                                         \
+    if (w_todo) {                                                                               \
+        w_todo = false;                                                                         \
+        load_w<F>(A, head, EC, fl, wi, wj);                                                     \
     }
 
 // Row rr of this lane is live when its slot is below the group's live rows (always, or never, without lengths).
@@ -507,7 +507,7 @@ __global__ void __launch_bounds__(kBlockThreads, (TANH_ONLY && !INDEXED && R == 
         float x[R][F], a[R][F];
         issue_tile<R, F>(A.in0, in_dtype, off, x);
         issue_tile<R, F>(A.in1, in_dtype, off, a);
-        NCN_SCALE_W_ONCE
+        NCN_LOAD_W_ONCE
         finish_tile<R, F>(in_dtype, x);
         finish_tile<R, F>(in_dtype, a);
         NCN_PASS_DEAD_ROWS(A.out0, A.out1, out_dtype, x, a)
@@ -539,7 +539,7 @@ __global__ void __launch_bounds__(kBlockThreads) stage_inverse_kernel(const Stag
         float y[R][F], b[R][F];
         issue_tile<R, F>(A.in0, in_dtype, off, y, A.plane);
         issue_tile<R, F>(A.in1, in_dtype, off, b, A.plane);
-        NCN_SCALE_W_ONCE
+        NCN_LOAD_W_ONCE
         finish_tile<R, F>(in_dtype, y);
         finish_tile<R, F>(in_dtype, b);
         NCN_PASS_DEAD_ROWS(A.out0, A.out1, out_dtype, y, b)
@@ -586,7 +586,7 @@ __global__ void __launch_bounds__(kBlockThreads, (TANH_ONLY && R * F <= 16 && F 
 #pragma unroll
                 for (int f = 0; f < F; ++f) H[rr][f] = 0.f;
         }
-        NCN_SCALE_W_ONCE
+        NCN_LOAD_W_ONCE
         finish_tile<R, F>(in_dtype, Y);
         finish_tile<R, F>(in_dtype, B);
         finish_tile<R, F>(g_dtype, G);
@@ -632,7 +632,7 @@ __global__ void __launch_bounds__(kBlockThreads, (TANH_ONLY && R * F <= 16 && F 
 #undef NCN_ROW_LIVE
 #undef NCN_ZERO_DEAD_ROWS
 #undef NCN_PASS_DEAD_ROWS
-#undef NCN_SCALE_W_ONCE
+#undef NCN_LOAD_W_ONCE
 #undef NCN_WAVE_PROLOGUE
 
 }  // namespace ncn

@@ -96,8 +96,13 @@ def _prep(t):
     return t
 
 
-def _w32(W):
-    return _prep(W.detach().reshape(-1).to(torch.float32))
+def _weights(W, as_they_are=True):
+    """The weights as the library takes them and the flag that says so: float32, or bfloat16 where the call may read
+    (and, in a backward, write) them so."""
+    flat = W.detach().reshape(-1)
+    if flat.dtype == torch.bfloat16 and as_they_are:
+        return _prep(flat), _lib.NCN_W_BF16
+    return _prep(flat.to(torch.float32)), 0
 
 
 def _stream(dev):
@@ -193,7 +198,7 @@ def forward_stages(x, xa, W, alpha, activation, cache_dim, nhead, first_stage, n
     dev = _require_gpu(x, xa, W)
     indexed = group_index is not None or ctx_len is not None
     gi, cl = _grouping(group_index, ctx_len, x.shape[0], x.shape[1], n_stages, dev, check_tables)
-    x, xa, w = _prep(x.detach()), _prep(xa.detach()), _w32(W)
+    x, xa, (w, wflag) = _prep(x.detach()), _prep(xa.detach()), _weights(W)
     out_dtype = x.dtype if out_dtype is None else out_dtype
     if out is not None and out_dtype not in _DTYPES:
         raise TypeError(f"out_dtype must be float32 or bfloat16, got {out_dtype}")
@@ -224,7 +229,7 @@ def forward_stages(x, xa, W, alpha, activation, cache_dim, nhead, first_stage, n
     ws, ws_bytes = None, 0
     if indexed:
         with torch.cuda.device(dev):
-            rc = lib.ncn_forward_indexed(_ptr(x), _ptr(xa), _DTYPES[x.dtype], _ptr(y), _ptr(ya), out_code,
+            rc = lib.ncn_forward_indexed(_ptr(x), _ptr(xa), _DTYPES[x.dtype] | wflag, _ptr(y), _ptr(ya), out_code,
                                          _ptr(aux[0]), _ptr(aux[1]), _ptr(w), _ptr(gi), _ptr(cl), ctypes.byref(shape),
                                          int(first_stage), int(n_stages), float(alpha), float(m), int(activation),
                                          _stream(dev))
@@ -234,7 +239,7 @@ def forward_stages(x, xa, W, alpha, activation, cache_dim, nhead, first_stage, n
         ws_bytes = lib.ncn_workspace_bytes_stages(ctypes.byref(shape), int(first_stage), int(n_stages), int(activation), 0)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev) if ws_bytes else None
     with torch.cuda.device(dev):
-        rc = lib.ncn_forward(_ptr(x), _ptr(xa), _DTYPES[x.dtype], _ptr(y), _ptr(ya), out_code,
+        rc = lib.ncn_forward(_ptr(x), _ptr(xa), _DTYPES[x.dtype] | wflag, _ptr(y), _ptr(ya), out_code,
                              _ptr(aux[0]), _ptr(aux[1]), _ptr(w), _ptr(ws), ctypes.c_size_t(ws_bytes),
                              ctypes.byref(shape), int(first_stage), int(n_stages), float(alpha), float(m),
                              int(activation), _stream(dev))
@@ -258,9 +263,10 @@ def forward_stages_saving(x, xa, W, alpha, activation, cache_dim, nhead, stage, 
 
 
 def backward_stages(y, ya, dy, dya, W, alpha, activation, cache_dim, nhead, first_stage, n_stages, *, m=M_DEFAULT,
-                    grad_dtype=None, want_inputs=True, group_index=None, ctx_len=None, check_tables=True):
+                    grad_dtype=None, want_inputs=True, group_index=None, ctx_len=None, check_tables=True,
+                    dw_dtype=torch.float32):
     """Reversible backward of stages first_stage+n_stages-1 .. first_stage from the outputs y, ya of the last one.
-    dya may be None (zeros).  y, ya may be the two-plane tensors [2, batch, N, E] of forward_stages(save_residual=True)
+    dya may be None (zeros).  dw_dtype: float32, or bfloat16 with bfloat16 weights.  y, ya may be the two-plane tensors [2, batch, N, E] of forward_stages(save_residual=True)
     (one stage).  Returns (x_rec, xa_rec, dx, dxa, dW[n_stages, 2E]); x_rec/xa_rec are None when
     want_inputs is False (with several stages the state between them then travels through the workspace and the
     last stage to run writes no reconstructed inputs)."""
@@ -284,7 +290,8 @@ def backward_stages(y, ya, dy, dya, W, alpha, activation, cache_dim, nhead, firs
     else:
         y, ya = _prep(y.detach()), _prep(ya.detach())
         y_code = _DTYPES[y.dtype]
-    dy, w = _prep(dy.detach()), _w32(W)
+    dy, (w, wflag) = _prep(dy.detach()), _weights(W, dw_dtype == torch.bfloat16)
+    y_code |= wflag
     dya = _prep(dya.detach()) if dya is not None else None
     grad_dtype = dy.dtype if grad_dtype is None else grad_dtype
     need_state = want_inputs
@@ -296,7 +303,9 @@ def backward_stages(y, ya, dy, dya, W, alpha, activation, cache_dim, nhead, firs
     x_rec = torch.empty(dy.shape, dtype=torch.float32, device=dev) if need_state else None
     xa_rec = torch.empty(dy.shape, dtype=torch.float32, device=dev) if need_state else None
     E = dy.shape[2]
-    dW = torch.empty(n_stages, 2 * E, dtype=torch.float32, device=dev)
+    if dw_dtype != torch.float32 and not (dw_dtype == torch.bfloat16 and W.dtype == torch.bfloat16):
+        raise TypeError(f"dw_dtype must be float32, or bfloat16 with bfloat16 weights, got {dw_dtype} for W of {W.dtype}")
+    dW = torch.empty(n_stages, 2 * E, dtype=dw_dtype, device=dev)
     lib = _lib.load()
     if indexed:
         # lengths without a table keep the stride permutation: with the multi-stage figure the library runs its
@@ -338,13 +347,13 @@ def inverse_stages(y, ya, W, alpha, activation, cache_dim, nhead, first_stage, n
     dev = _require_gpu(y, ya, W)
     indexed = group_index is not None or ctx_len is not None
     gi, cl = _grouping(group_index, ctx_len, y.shape[0], y.shape[1], n_stages, dev, check_tables)
-    y, ya, w = _prep(y.detach()), _prep(ya.detach()), _w32(W)
+    y, ya, (w, wflag) = _prep(y.detach()), _prep(ya.detach()), _weights(W)
     out_dtype = y.dtype if out_dtype is None else out_dtype
     x = torch.empty(y.shape, dtype=out_dtype, device=dev)
     xa = torch.empty(y.shape, dtype=out_dtype, device=dev)
     if indexed:
         with torch.cuda.device(dev):
-            rc = _lib.load().ncn_inverse_indexed(_ptr(y), _ptr(ya), _DTYPES[y.dtype], _ptr(x), _ptr(xa),
+            rc = _lib.load().ncn_inverse_indexed(_ptr(y), _ptr(ya), _DTYPES[y.dtype] | wflag, _ptr(x), _ptr(xa),
                                                  _DTYPES[out_dtype], _ptr(w), _ptr(gi), _ptr(cl), ctypes.byref(shape),
                                                  int(first_stage), int(n_stages), float(alpha), float(m),
                                                  int(activation), _stream(dev))
@@ -357,14 +366,14 @@ def inverse_stages(y, ya, W, alpha, activation, cache_dim, nhead, first_stage, n
     if ws_bytes:
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
         with torch.cuda.device(dev):
-            rc = lib.ncn_inverse_ws(_ptr(y), _ptr(ya), _DTYPES[y.dtype], _ptr(x), _ptr(xa), _DTYPES[out_dtype],
+            rc = lib.ncn_inverse_ws(_ptr(y), _ptr(ya), _DTYPES[y.dtype] | wflag, _ptr(x), _ptr(xa), _DTYPES[out_dtype],
                                     _ptr(w), _ptr(ws), ctypes.c_size_t(ws_bytes), ctypes.byref(shape),
                                     int(first_stage), int(n_stages), float(alpha), float(m), int(activation),
                                     _stream(dev))
         _lib.check(rc, "ncn_inverse_ws")
         return x, xa
     with torch.cuda.device(dev):
-        rc = lib.ncn_inverse(_ptr(y), _ptr(ya), _DTYPES[y.dtype], _ptr(x), _ptr(xa), _DTYPES[out_dtype],
+        rc = lib.ncn_inverse(_ptr(y), _ptr(ya), _DTYPES[y.dtype] | wflag, _ptr(x), _ptr(xa), _DTYPES[out_dtype],
                              _ptr(w), ctypes.byref(shape), int(first_stage), int(n_stages), float(alpha),
                              float(m), int(activation), _stream(dev))
     _lib.check(rc, "ncn_inverse")
@@ -378,12 +387,12 @@ def forward_radix(x, xa, W, alpha, activation, cache_dim, nhead, first_level, n_
     float32 unless out_dtype says otherwise (values between passes live in the outputs)."""
     shape = validate(x, xa, W, cache_dim, nhead, activation, 0, n_levels, alpha=alpha, m=m)
     dev = _require_gpu(x, xa, W)
-    x, xa, w = _prep(x.detach()), _prep(xa.detach()), _w32(W)
+    x, xa, (w, wflag) = _prep(x.detach()), _prep(xa.detach()), _weights(W)
     out_dtype = torch.float32 if out_dtype is None else out_dtype
     y = torch.empty(x.shape, dtype=out_dtype, device=dev)
     ya = torch.empty(x.shape, dtype=out_dtype, device=dev)
     with torch.cuda.device(dev):
-        rc = _lib.load().ncn_forward_radix(_ptr(x), _ptr(xa), _DTYPES[x.dtype], _ptr(y), _ptr(ya), _DTYPES[out_dtype],
+        rc = _lib.load().ncn_forward_radix(_ptr(x), _ptr(xa), _DTYPES[x.dtype] | wflag, _ptr(y), _ptr(ya), _DTYPES[out_dtype],
                                            _ptr(None), _ptr(None), _ptr(w), ctypes.byref(shape), int(first_level),
                                            int(n_levels), float(alpha), float(m), int(activation), _stream(dev))
     if rc == -2:
@@ -397,11 +406,11 @@ def inverse_radix(y, ya, W, alpha, activation, cache_dim, nhead, first_level, n_
     """x, xa (float32) with forward_radix(x, xa, ...) == (y, ya)."""
     shape = validate(y, ya, W, cache_dim, nhead, activation, 0, n_levels, what="y", alpha=alpha, m=m)
     dev = _require_gpu(y, ya, W)
-    y, ya, w = _prep(y.detach()), _prep(ya.detach()), _w32(W)
+    y, ya, (w, wflag) = _prep(y.detach()), _prep(ya.detach()), _weights(W)
     x = torch.empty(y.shape, dtype=torch.float32, device=dev)
     xa = torch.empty(y.shape, dtype=torch.float32, device=dev)
     with torch.cuda.device(dev):
-        rc = _lib.load().ncn_inverse_radix(_ptr(y), _ptr(ya), _DTYPES[y.dtype], _ptr(x), _ptr(xa), _lib.NCN_F32, _ptr(w),
+        rc = _lib.load().ncn_inverse_radix(_ptr(y), _ptr(ya), _DTYPES[y.dtype] | wflag, _ptr(x), _ptr(xa), _lib.NCN_F32, _ptr(w),
                                            ctypes.byref(shape), int(first_level), int(n_levels), float(alpha), float(m),
                                            int(activation), _stream(dev))
     if rc == -2:
@@ -421,7 +430,7 @@ def backward_radix(y, ya, dy, dya, W, alpha, activation, cache_dim, nhead, first
     if dy.dtype not in _DTYPES or (dya is not None and dya.dtype != dy.dtype):
         raise TypeError("dy and dya must both be float32 or bfloat16")
     dev = _require_gpu(y, ya, dy, dya, W)
-    y, ya, dy, w = _prep(y.detach()), _prep(ya.detach()), _prep(dy.detach()), _w32(W)
+    y, ya, dy, (w, _) = _prep(y.detach()), _prep(ya.detach()), _prep(dy.detach()), _weights(W, False)
     dya = _prep(dya.detach()) if dya is not None else None
     f32 = torch.float32
     dx, dxa = torch.empty(y.shape, dtype=f32, device=dev), torch.empty(y.shape, dtype=f32, device=dev)

@@ -1,0 +1,73 @@
+"""bfloat16 weights read, and their gradients written, by the kernels themselves: bit for bit what the same call gives on
+the weights converted to float32 (the conversion is exact) and on its float32 dW rounded once."""
+import ctypes
+
+import pytest
+import torch
+
+from oracle import ncn_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def M():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from ncn_cuda_amd import ncn_cuda_module
+    return ncn_cuda_module
+
+
+# (n_cache, E, heads, groups, stages, alpha)
+CASES = [(16, 128, 4, 4, 1, 0.9),   # register kernels, tiles of 4 x 4
+         (4, 128, 2, 6, 1, 0.9),    # 2 x 8
+         (8, 32, 32, 4, 1, 0.9),    # heads of one feature
+         (5, 30, 2, 5, 1, 0.9),     # no powers of two
+         (5, 30, 2, 5, 1, 0.0),     # generic kernels (alpha outside the scaled state)
+         (2, 64, 2, 32, 5, 0.9),    # two-row multi-stage passes
+         (4, 64, 2, 64, 4, 0.9)]    # multi-stage passes
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "n%d_E%d_C%d_g%d_L%d_a%g" % c)
+def test_bfloat16_weights(M, case):
+    n, E, C, groups, L, alpha = case
+    x, xa, Ws, dy, dya = (t.cuda() if isinstance(t, torch.Tensor) else [w.cuda() for w in t]
+                          for t in O.make_inputs(3, n * groups, E, L, n, seed=n + E, xa_zero=False))
+    W = torch.stack(Ws).bfloat16()
+    W32 = W.float()
+    y, ya = M.forward_stages(x, xa, W, alpha, 0, n, C, 0, L)
+    y32, ya32 = M.forward_stages(x, xa, W32, alpha, 0, n, C, 0, L)
+    assert torch.equal(y, y32) and torch.equal(ya, ya32)
+    for a, b in zip(M.inverse_stages(y, ya, W, alpha, 0, n, C, 0, L), M.inverse_stages(y, ya, W32, alpha, 0, n, C, 0, L)):
+        assert torch.equal(a, b)
+    kw = dict(want_inputs=False)
+    want = M.backward_stages(y, ya, dy, dya, W32, alpha, 0, n, C, 0, L, **kw)
+    got = M.backward_stages(y, ya, dy, dya, W, alpha, 0, n, C, 0, L, dw_dtype=torch.bfloat16, **kw)
+    assert torch.equal(got[2], want[2]) and torch.equal(got[3], want[3])
+    assert got[4].dtype == torch.bfloat16 and torch.equal(got[4], want[4].bfloat16())
+    got = M.backward_stages(y, ya, dy, dya, W, alpha, 0, n, C, 0, L, **kw)   # float32 dW of bfloat16 weights
+    assert torch.equal(got[4], want[4])
+
+
+@pytest.mark.parametrize("case", [CASES[0], CASES[5], CASES[6]], ids=lambda c: "n%d_E%d_C%d_g%d_L%d_a%g" % c)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_one_array_per_stage(M, case, dtype):
+    """NCN_W_ARRAYS: the weights of every stage where they are."""
+    from ncn_cuda_amd import _lib
+    n, E, C, groups, L, alpha = case
+    x, xa, Ws, _, _ = (t.cuda() if isinstance(t, torch.Tensor) else [w.cuda().to(dtype) for w in t]
+                       for t in O.make_inputs(2, n * groups, E, L, n, seed=n, xa_zero=False))
+    want = M.forward_stages(x, xa, torch.stack(Ws), alpha, 0, n, C, 0, L)
+    y, ya = torch.empty_like(x), torch.empty_like(x)
+    shape = _lib.NcnShape(2, n * groups, E, C, n)
+    lib = _lib.load()
+    ws = torch.empty(max(16, lib.ncn_workspace_bytes_stages(ctypes.byref(shape), 0, L, 0, 0)), dtype=torch.uint8, device="cuda")
+    ptrs = (ctypes.c_void_p * L)(*[w.data_ptr() for w in Ws])
+    flags = _lib.NCN_W_ARRAYS | (_lib.NCN_W_BF16 if dtype == torch.bfloat16 else 0)
+    args = lambda p: (x.data_ptr(), xa.data_ptr(), _lib.NCN_F32 | flags, y.data_ptr(), ya.data_ptr(), _lib.NCN_F32, None,
+                      None, p, ws.data_ptr(), ws.numel(), ctypes.byref(shape), 0, L, alpha, 0.9, 0,
+                      torch.cuda.current_stream().cuda_stream)
+    assert lib.ncn_forward(*args(ctypes.cast(ptrs, ctypes.c_void_p))) == 0
+    assert torch.equal(y, want[0]) and torch.equal(ya, want[1])
+    ptrs[L - 1] = None
+    assert lib.ncn_forward(*args(ctypes.cast(ptrs, ctypes.c_void_p))) == -1   # NCN_ERR_NULL, nothing launched
