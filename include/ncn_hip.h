@@ -300,6 +300,37 @@ int ncn_inverse_radix(const void* y, const void* ya, int in_dtype,
 int ncn_plan_radix(const ncn_shape* shape, int first_level, int n_levels, int activation, int backward, int32_t* out,
                    int max_passes);
 
+/*
+ * A stack that is trained, one call per direction: stages first_stage .. first_stage+n_stages-1 with the activations
+ * kept in float32 wherever the passes of both directions profit from it, so that the backward undoes at most max_range
+ * stages from a kept value.  Everything between the stages is float32 whatever the types of x, y, dy, dx.
+ * Replaces the chain of one autograd node per module of NCNNetCuda (ncn_cuda/ncn_pytorch_wrapper_v2.py:107-117).
+ *
+ * ncn_stack_plan returns the number R <= max_saves of ranges that the stages are cut into and writes out[0], out[1], the
+ * workspace bytes of the two calls (grad_dtype: the dx_dtype of the backward).  0: nothing to gain or not supported
+ * (shapes and scalars of the generic kernels, one stage, more than 256): use ncn_forward and ncn_backward.
+ *
+ * ncn_stack_forward: W as ncn_forward (flags on in_dtype).  saves: float32 [R-1][2][batch,N,E] with float32 outputs,
+ * [R][2][batch,N,E] with bfloat16 ones.  y, ya must not be x, xa (NCN_ERR_ALIAS).
+ * ncn_stack_backward: y, ya are the float32 outputs of the forward, NULL where they were bfloat16; saves as the forward
+ * left them; w_dtype: float32 or NCN_W_BF16 | NCN_F32, with NCN_W_ARRAYS as in ncn_forward.  dx, dxa must not be dy, dya.
+ * Both take the same max_range, max_saves and shape as ncn_stack_plan did.
+ */
+int ncn_stack_plan(const ncn_shape* shape, int first_stage, int n_stages, float alpha, float m, int activation,
+                   int max_range, int max_saves, int grad_dtype, int64_t* out);
+int ncn_stack_forward(const void* x, const void* xa, int in_dtype,
+                      void* y, void* ya, int out_dtype, float* saves,
+                      const void* W, void* workspace, size_t workspace_bytes,
+                      const ncn_shape* shape, int first_stage, int n_stages, int max_range, int max_saves,
+                      float alpha, float m, int activation, void* stream);
+int ncn_stack_backward(const float* y, const float* ya, const float* saves,
+                       const void* dy, const void* dya, int dy_dtype,
+                       void* dx, void* dxa, int dx_dtype,
+                       const void* W, void* dW, int w_dtype, void* workspace, size_t workspace_bytes,
+                       const ncn_shape* shape, int first_stage, int n_stages, int max_range, int max_saves,
+                       float alpha, float m, int activation, void* stream);
+
+
 /* Bytes of scratch ncn_backward needs for this shape (0 on an invalid shape).  No reference counterpart:
  * the reference allocates a [batch,N,2E] partial-dW tensor per call (ncn_bwd_cuda_kernel.cu:251). */
 size_t ncn_workspace_bytes(const ncn_shape* shape);

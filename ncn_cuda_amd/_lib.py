@@ -17,7 +17,7 @@ EXPORTS = ("ncn_forward", "ncn_backward", "ncn_inverse", "ncn_forward_indexed", 
            "ncn_inverse_indexed", "ncn_inverse_ws", "ncn_forward_radix", "ncn_backward_radix", "ncn_inverse_radix", "ncn_plan_radix", "ncn_workspace_bytes", "ncn_workspace_bytes_stages",
            "ncn_plan_passes", "ncn_kernel_path",
            "ncn_check_shape", "ncn_error_string", "ncn_version", "ncn_backward_static", "ncn_static_scratch_bytes", "ncn_kernel_path_scalars",
-           "ncn_build_id", "ncn_probe_issue", "ncn_probe_issue_info")
+           "ncn_stack_plan", "ncn_stack_forward", "ncn_stack_backward", "ncn_build_id", "ncn_probe_issue", "ncn_probe_issue_info")
 
 
 class NcnShape(ctypes.Structure):
@@ -93,6 +93,14 @@ def load():
                                        shp, i, i, fl, fl, i, vp]
     lib.ncn_inverse_radix.restype = i
     lib.ncn_inverse_radix.argtypes = [vp, vp, i, vp, vp, i, f32p, shp, i, i, fl, fl, i, vp]
+    i64p = ctypes.POINTER(ctypes.c_int64)
+    lib.ncn_stack_plan.restype = i
+    lib.ncn_stack_plan.argtypes = [shp, i, i, fl, fl, i, i, i, i, i64p]
+    lib.ncn_stack_forward.restype = i
+    lib.ncn_stack_forward.argtypes = [vp, vp, i, vp, vp, i, f32p, vp, vp, ctypes.c_size_t, shp, i, i, i, i, fl, fl, i, vp]
+    lib.ncn_stack_backward.restype = i
+    lib.ncn_stack_backward.argtypes = [f32p, f32p, f32p, vp, vp, i, vp, vp, i, vp, vp, i, vp, ctypes.c_size_t, shp, i, i, i, i,
+                                       fl, fl, i, vp]
     lib.ncn_plan_radix.restype = i
     lib.ncn_plan_radix.argtypes = [shp, i, i, i, i, ctypes.POINTER(ctypes.c_int32), i]
     lib.ncn_workspace_bytes.restype = ctypes.c_size_t

@@ -1158,6 +1158,226 @@ int ncn_inverse_radix(const void* y, const void* ya, int in_dtype, void* x, void
     return NCN_OK;
 }
 
+// ---- a trained stack: one call per direction, activations kept where the passes of both directions begin ----------
+// The plan of a stack and the buffers that follow from it; the same for the query and the two calls.
+struct StackCall {
+    ncn_shape as_wide;
+    const ncn_shape* shape;
+    bool headwise;
+    std::vector<StackRange> ranges;
+    size_t plane;        // one float32 activation array
+    int fwd_passes_max;  // passes of the longest range
+    int bwd_passes_max, bwd_passes;
+    int row_cap;         // rows of the dW partial buffer
+
+    // false: no such cut, or kernels without this entry (the caller uses ncn_forward and ncn_backward).  A program asks for
+    // the same stack step after step: the last plan of a thread is kept, it depends on sizes only.
+    bool plan(const ncn_shape* sh, int first, int count, int activation, float alpha, float m, int max_range, int max_saves) {
+        const int path = kernel_path_for(sh, activation, alpha, m);
+        // (the tables of plan_stack grow with the square of the stages)
+        if (path != 2 || count < 2 || count > 256 || max_range < 1 || max_saves < 1) return false;
+        headwise = headwise_call(sh, path, &as_wide);
+        shape = headwise ? &as_wide : sh;
+        const bool multi = fused_supported(shape, activation);
+        struct Kept {
+            int64_t batch = 0, N = 0, E = 0;
+            int n_head = 0, n_cache = 0, first = 0, count = 0, multi = 0, max_range = 0, max_saves = 0;
+            std::vector<StackRange> ranges;
+        };
+        thread_local Kept kept;
+        if (kept.batch != shape->batch || kept.N != shape->N || kept.E != shape->E || kept.n_head != shape->n_head ||
+            kept.n_cache != shape->n_cache || kept.first != first || kept.count != count || kept.multi != (int)multi ||
+            kept.max_range != max_range || kept.max_saves != max_saves) {
+            kept.batch = 0;   // not valid while it changes
+            kept.ranges = plan_stack(shape, first, count, multi, max_range, max_saves);
+            kept.N = shape->N; kept.E = shape->E; kept.n_head = shape->n_head; kept.n_cache = shape->n_cache;
+            kept.first = first; kept.count = count; kept.multi = multi;
+            kept.max_range = max_range; kept.max_saves = max_saves;
+            kept.batch = shape->batch;
+        }
+        ranges = kept.ranges;
+        if (ranges.empty()) return false;
+        plane = temp_bytes(shape, false) / 2;
+        fwd_passes_max = bwd_passes_max = bwd_passes = 0;
+        int64_t rows = 0;
+        const Plan single = make_plan(shape, 2, AnyTile{0, 0, 0, 0});
+        for (const StackRange& r : ranges) {
+            if ((int)r.fwd.size() > fwd_passes_max) fwd_passes_max = (int)r.fwd.size();
+            if ((int)r.bwd.size() > bwd_passes_max) bwd_passes_max = (int)r.bwd.size();
+            bwd_passes += (int)r.bwd.size();
+            for (const FusedPass& p : r.bwd)
+                rows += p.single ? (int64_t)single.partial_rows : fused_items(shape, p) / shape->n_head * p.count;
+        }
+        if (rows > kFusedRowCapMax) rows = kFusedRowCapMax;
+        row_cap = rows < kMaxGridX ? kMaxGridX : (int)rows;
+        return true;
+    }
+    // pairs of arrays in the workspace: the forward's passes that are not kept go through one; the backward's gradients
+    // through one (two where dx, dxa cannot hold them in between), reconstructed inputs inside a range through two more
+    size_t forward_bytes() const { return fwd_passes_max > 1 ? 2 * plane : 0; }
+    int gradient_pairs(bool out_f32) const { return bwd_passes < 2 ? 0 : bwd_passes == 2 || out_f32 ? 1 : 2; }
+    int state_pairs() const { return bwd_passes_max < 2 ? 0 : bwd_passes_max == 2 ? 1 : 2; }
+    size_t backward_bytes(bool out_f32) const {
+        return partial_buffer_bytes(shape, row_cap) + 2 * plane * (size_t)(gradient_pairs(out_f32) + state_pairs());
+    }
+};
+
+int ncn_stack_plan(const ncn_shape* shape, int first_stage, int n_stages, float alpha, float m, int activation,
+                   int max_range, int max_saves, int grad_dtype, int64_t* out) {
+    const int rc = check_shape(shape, first_stage, n_stages, activation);
+    if (rc != NCN_OK) return rc;
+    if (!out) return NCN_ERR_NULL;
+    if (!known_dtype(grad_dtype)) return NCN_ERR_DTYPE;
+    StackCall c;
+    if (!c.plan(shape, first_stage, n_stages, activation, alpha, m, max_range, max_saves)) return 0;
+    out[0] = (int64_t)c.forward_bytes();
+    out[1] = (int64_t)c.backward_bytes(grad_dtype == NCN_F32);
+    return (int)c.ranges.size();
+}
+
+int ncn_stack_forward(const void* x, const void* xa, int in_dtype, void* y, void* ya, int out_dtype, float* saves,
+                      const void* W, void* workspace, size_t workspace_bytes, const ncn_shape* shape, int first_stage,
+                      int n_stages, int max_range, int max_saves, float alpha, float m, int activation, void* stream) {
+    const int rc = check_shape(shape, first_stage, n_stages, activation);
+    if (rc != NCN_OK) return rc;
+    const Weights w(W, in_dtype, shape);
+    if (!x || !xa || !y || !ya || w.null(n_stages)) return NCN_ERR_NULL;
+    if (!known_dtype(in_dtype) || !known_dtype(out_dtype)) return NCN_ERR_DTYPE;
+    if (!aligned16(x) || !aligned16(xa) || !aligned16(y) || !aligned16(ya) || !aligned16(saves) || !aligned16(workspace) ||
+        !w.aligned(n_stages))
+        return NCN_ERR_ALIGN;
+    if (x == y || xa == ya || x == ya || xa == y) return NCN_ERR_ALIAS;
+    StackCall c;
+    if (!c.plan(shape, first_stage, n_stages, activation, alpha, m, max_range, max_saves)) return NCN_ERR_UNSUPPORTED;
+    shape = c.shape;
+    const size_t nr = c.ranges.size();
+    if ((nr > 1 || out_dtype != NCN_F32) && !saves) return NCN_ERR_NULL;
+    if (c.forward_bytes() && (!workspace || workspace_bytes < c.forward_bytes())) return NCN_ERR_WORKSPACE;
+    const Plan p = make_plan(shape, 2, AnyTile{0, 0, 0, 0});
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const int64_t elements = shape->batch * shape->N * shape->E;
+    void* const t0 = workspace;
+    void* const t1 = workspace ? static_cast<char*>(workspace) + c.plane : nullptr;
+    const void *cur0 = x, *cur1 = xa;
+    int cur_dtype = in_dtype;
+    for (size_t r = 0; r < nr; ++r) {
+        // float32 outputs of the last range are kept as they are; bfloat16 ones leave beside a float32 copy
+        const bool last_range = r + 1 == nr;
+        void* kept0 = last_range && out_dtype == NCN_F32 ? y : saves + (int64_t)(2 * r) * elements;
+        void* kept1 = last_range && out_dtype == NCN_F32 ? ya : saves + (int64_t)(2 * r + 1) * elements;
+        const std::vector<FusedPass>& passes = c.ranges[r].fwd;
+        const size_t np = passes.size();
+        for (size_t k = 0; k < np; ++k) {
+            const FusedPass& ps = passes[k];
+            const bool to_kept = ((np - 1 - k) % 2) == 0;   // in turns, so that the range's last pass ends where it is kept
+            const bool both = last_range && k + 1 == np && out_dtype != NCN_F32;
+            void* d0 = to_kept ? kept0 : t0;
+            void* d1 = to_kept ? kept1 : t1;
+            hipError_t err;
+            auto fill = [&](auto& a) {
+                a.in0 = cur0; a.in1 = cur1; a.in_dtype = cur_dtype;
+                a.out0 = both ? y : d0; a.out1 = both ? ya : d1;
+                a.out_dtype = both ? out_dtype : NCN_F32;
+                a.aux0 = both ? static_cast<float*>(d0) : nullptr;
+                a.aux1 = both ? static_cast<float*>(d1) : nullptr;
+            };
+            if (ps.single) {
+                StageArgs a{};
+                fill_common(a, shape, p, first_stage + ps.first, alpha, m, activation);
+                fill(a);
+                w.set(a, ps.first);
+                err = run_forward_kernel(kForward, a, p, true, c.headwise, s);
+            } else {
+                FusedArgs a{};
+                fill(a);
+                w.set(a, ps.first, ps.count);
+                fill_step_table(a.tab, shape->n_cache, alpha, m, activation);
+                err = launch_fused(kForward, a, shape, ps, s, kMaxGridX, c.headwise);
+            }
+            if (err != hipSuccess) return (int)err;
+            cur0 = d0; cur1 = d1; cur_dtype = NCN_F32;
+        }
+    }
+    return NCN_OK;
+}
+
+int ncn_stack_backward(const float* y, const float* ya, const float* saves, const void* dy, const void* dya, int dy_dtype,
+                       void* dx, void* dxa, int dx_dtype, const void* W, void* dW, int w_dtype, void* workspace,
+                       size_t workspace_bytes, const ncn_shape* shape, int first_stage, int n_stages, int max_range,
+                       int max_saves, float alpha, float m, int activation, void* stream) {
+    const int rc = check_shape(shape, first_stage, n_stages, activation);
+    if (rc != NCN_OK) return rc;
+    const Weights w(W, w_dtype, shape);
+    if (w_dtype != NCN_F32 || !known_dtype(dy_dtype) || !known_dtype(dx_dtype)) return NCN_ERR_DTYPE;
+    if (!dy || !dx || !dxa || w.null(n_stages) || !dW || ((y == nullptr) != (ya == nullptr))) return NCN_ERR_NULL;
+    if (!aligned16(y) || !aligned16(ya) || !aligned16(saves) || !aligned16(dy) || !aligned16(dya) || !aligned16(dx) ||
+        !aligned16(dxa) || !aligned16(dW) || !aligned16(workspace) || !w.aligned(n_stages))
+        return NCN_ERR_ALIGN;
+    if (dx == dy || dxa == dy || (dya && (dx == dya || dxa == dya))) return NCN_ERR_ALIAS;
+    StackCall c;
+    if (!c.plan(shape, first_stage, n_stages, activation, alpha, m, max_range, max_saves)) return NCN_ERR_UNSUPPORTED;
+    shape = c.shape;
+    const size_t nr = c.ranges.size();
+    if ((nr > 1 || !y) && !saves) return NCN_ERR_NULL;
+    if (!workspace || workspace_bytes < c.backward_bytes(dx_dtype == NCN_F32)) return NCN_ERR_WORKSPACE;
+    const Plan p = make_plan(shape, 2, AnyTile{0, 0, 0, 0});
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const int64_t elements = shape->batch * shape->N * shape->E, two_e = 2 * shape->E;
+    float* partials = static_cast<float*>(workspace);
+    char* tail = static_cast<char*>(workspace) + partial_buffer_bytes(shape, c.row_cap);
+    auto pair = [&](int k, int half) -> void* { return tail + (size_t)(2 * k + half) * c.plane; };
+    const int gp = c.gradient_pairs(dx_dtype == NCN_F32);
+    DwReducer reducer(partials, partials + (int64_t)c.row_cap * two_e, two_e, w.bf16, s, c.row_cap);
+    const void *cg = dy, *cga = dya;
+    int cg_dtype = dy_dtype, left = c.bwd_passes;
+    for (size_t r = nr; r-- > 0;) {
+        const bool from_y = r + 1 == nr && y;
+        const void* cy = from_y ? y : saves + (int64_t)(2 * r) * elements;
+        const void* cya = from_y ? ya : saves + (int64_t)(2 * r + 1) * elements;
+        const std::vector<FusedPass>& passes = c.ranges[r].bwd;
+        for (size_t k = passes.size(); k-- > 0;) {
+            const FusedPass& ps = passes[k];
+            --left;   // passes still to run: gradients travel in turns so that the last pass writes dx, dxa
+            const bool to_out = left == 0 || (left % 2 == 0 && dx_dtype == NCN_F32);
+            const int slot = left % 2 ? 0 : 1;
+            void* dg = to_out ? dx : pair(slot, 0);
+            void* dga = to_out ? dxa : pair(slot, 1);
+            // the first pass of a range hands no reconstructed inputs on: the range before it has kept its outputs
+            float* rec = k == 0 ? nullptr : static_cast<float*>(pair(gp + (int)(k - 1) % 2, 0));
+            float* reca = k == 0 ? nullptr : static_cast<float*>(pair(gp + (int)(k - 1) % 2, 1));
+            const int rows = ps.single ? p.partial_rows : fused_grid(shape, ps, true, c.row_cap) / shape->n_head;
+            float* region;
+            hipError_t err = reducer.reserve(rows, ps.count, &region);
+            if (err != hipSuccess) return (int)err;
+            auto fill = [&](auto& a) {
+                a.in0 = cy; a.in1 = cya; a.in_dtype = NCN_F32;
+                a.g0 = cg; a.g1 = cga; a.g_dtype = cg_dtype;
+                a.out0 = dg; a.out1 = dga; a.out_dtype = to_out ? dx_dtype : NCN_F32;
+                a.aux0 = rec; a.aux1 = reca;
+                a.dw_partials = region;
+            };
+            if (ps.single) {
+                StageArgs a{};
+                fill_common(a, shape, p, first_stage + ps.first, alpha, m, activation);
+                fill(a);
+                w.set(a, ps.first);
+                err = run_backward_kernel(a, p, true, c.headwise, s);
+            } else {
+                FusedArgs a{};
+                fill(a);
+                w.set(a, ps.first, ps.count);
+                fill_step_table(a.tab, shape->n_cache, alpha, m, activation);
+                err = launch_fused(kBackward, a, shape, ps, s, c.row_cap, c.headwise);
+            }
+            if (err != hipSuccess) return (int)err;
+            reducer.add(region, rows, ps.count, w.out_at(dW, ps.first));
+            cy = rec; cya = reca;
+            cg = dg; cga = dga; cg_dtype = to_out ? dx_dtype : NCN_F32;
+        }
+    }
+    return (int)reducer.flush();
+}
+
 int ncn_plan_radix(const ncn_shape* shape, int first_level, int n_levels, int activation, int backward, int32_t* out,
                    int max_passes) {
     int rc = check_shape(shape, 0, n_levels, activation);

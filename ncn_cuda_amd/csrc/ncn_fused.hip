@@ -64,77 +64,67 @@ bool fused_supported(const ncn_shape* sh, int activation) {
     return false;
 }
 
-// Cuts stages [first, first + count) into passes, ascending.  Window capacity in sub-blocks is a power of two.
-std::vector<FusedPass> plan_fused(const ncn_shape* sh, int first, int count, bool backward) {
-    std::vector<FusedPass> passes;
-    const int nc = sh->n_cache, ec = (int)(sh->E / sh->n_head);
-    const uint32_t groups = (uint32_t)(sh->N / nc);
-    const size_t state = nc == 2 ? pair_state_bytes(backward) : fused_state_bytes(backward);
-    const uint32_t cap_rows = (uint32_t)(state / ((backward ? 4 : 2) * ec * sizeof(float)));
-    uint32_t cap = floor_pow2(cap_rows / nc);
-    if (cap > groups) cap = floor_pow2(groups);
-    if (cap < 4) return passes;
-    const uint32_t groups_pow2 = groups & (~groups + 1u);   // the power of two in the number of groups
-    std::vector<uint32_t> s(count);
-    for (int k = 0; k < count; ++k) s[k] = stage_stride_of(first + k, groups);
+namespace {
 
-    // backward keeps a dW slot per wave and stage in LDS: 7 stages leave room for two workgroups per CU at heads of up
-    // to 32 features; the two-row kernels at heads of 64 take as many stages as still let two workgroups share a CU
-    // (3), at heads of 128 not even two stages would and a CU runs one workgroup of up to 7 stages
-    int max_stages = backward ? kFusedMaxStages - 1 : kFusedMaxStages;
-    if (backward && nc == 2) {
-        const size_t budget = 80 * 1024, fixed = pair_state_bytes(true) / 2 + (size_t)kFusedMaxStages * 2 * ec * sizeof(float);
-        const size_t per_stage = (size_t)kPairWavesBwd * 2 * ec * sizeof(float);
-        const int fit = fixed < budget ? (int)((budget - fixed) / per_stage) : 0;
-        if (fit >= 2 && fit < max_stages) max_stages = fit;
+// Prices and shapes the passes over stages [a, b) of a range (counted from `first`).  Window capacity in sub-blocks is a
+// power of two.
+class PassPlanner {
+  public:
+    PassPlanner(const ncn_shape* sh, int first, int count, bool backward)
+        : nc_(sh->n_cache), ec_((int)(sh->E / sh->n_head)), groups_((uint32_t)(sh->N / sh->n_cache)), backward_(backward),
+          s_(count) {
+        const size_t state = nc_ == 2 ? pair_state_bytes(backward) : fused_state_bytes(backward);
+        cap_rows_ = (uint32_t)(state / ((backward ? 4 : 2) * ec_ * sizeof(float)));
+        cap_ = floor_pow2(cap_rows_ / nc_);
+        if (cap_ > groups_) cap_ = floor_pow2(groups_);
+        groups_pow2_ = groups_ & (~groups_ + 1u);   // the power of two in the number of groups
+        for (int k = 0; k < count; ++k) s_[k] = stage_stride_of(first + k, groups_);
+
+        // backward keeps a dW slot per wave and stage in LDS: 7 stages leave room for two workgroups per CU at heads of up
+        // to 32 features; the two-row kernels at heads of 64 take as many stages as still let two workgroups share a CU
+        // (3), at heads of 128 not even two stages would and a CU runs one workgroup of up to 7 stages
+        max_stages_ = backward ? kFusedMaxStages - 1 : kFusedMaxStages;
+        if (backward && nc_ == 2) {
+            const size_t budget = 80 * 1024, fixed = pair_state_bytes(true) / 2 + (size_t)kFusedMaxStages * 2 * ec_ * sizeof(float);
+            const size_t per_stage = (size_t)kPairWavesBwd * 2 * ec_ * sizeof(float);
+            const int fit = fixed < budget ? (int)((budget - fixed) / per_stage) : 0;
+            if (fit >= 2 && fit < max_stages_) max_stages_ = fit;
+        }
     }
-    // What a pass costs, in the time one array of the activations' size takes to cross HBM at copy speed.  Traffic: the
-    // pass reads `arrays_in` arrays of its windows (window / own times the data) and writes `arrays_out` arrays of its
-    // owned rows; in the backward the pass that holds the call's first stage runs last and writes the two gradients
-    // only (callers that want the reconstructed inputs pay two arrays more than priced here).  Issue: every stage costs
-    // `per_stage` such units of instruction issue on all groups of its windows (measured per kernel family on
-    // x[128, 8192, 128]: a two-row backward stage 0.143 ms against 0.102 ms per array, a two-row forward stage 0.078 ms;
-    // the four-row kernels in proportion to their instruction counts).  The two overlap, better the more they differ:
-    // the cube root of the sum of cubes follows the measured pass times to 5 % (a closed backward pass, whose windows
-    // are the most scattered in memory, takes 1.1 times that).
-    const double arrays_in = backward ? 4.0 : 2.0;
-    const double per_stage = nc == 2 ? (backward ? 1.4 : 0.76) : (backward ? 3.6 : 2.0);
-    auto priced = [&](int a, double redundancy, int stages, bool closed) -> double {
-        const double arrays_out = backward ? (a == 0 ? 2.0 : 4.0) : 2.0;
-        const double traffic = arrays_in * redundancy + arrays_out;
-        const double issue = per_stage * stages * redundancy;
-        return std::cbrt(traffic * traffic * traffic + issue * issue * issue) * (closed && backward ? 1.1 : 1.0);
-    };
-    // stages [a, b) as one pass; returns its cost (see above), or < 0 if impossible
-    auto make = [&](int a, int b, FusedPass& p) -> double {
-        if (b - a > max_stages || b - a < 2) return -1.0;
+    int max_stages() const { return max_stages_; }
+    // a one-stage launch is bound by its traffic: every array once.  writes_state (backward): the launch hands the
+    // reconstructed inputs on.
+    double single(bool writes_state) const { return backward_ ? (writes_state ? 8.0 : 6.0) : 4.0; }
+    // stages [a, b) as one pass; returns its cost, or < 0 if impossible
+    double make(int a, int b, bool writes_state, FusedPass& p) const {
+        if (cap_ < 4 || b - a > max_stages_ || b - a < 2) return -1.0;
         // S0: the largest power of two that divides every non-zero stride of the pass and the number of groups (with a
         // power of two of groups the strides are powers of two and this is the smallest of them; with 3 * 2^k groups
         // and the like the strides past 2^k wrap to odd multiples of 2^k)
         uint32_t s0 = 0;
         for (int k = a; k < b; ++k)
-            if (s[k]) {
-                const uint32_t low = s[k] & (~s[k] + 1u);
+            if (s_[k]) {
+                const uint32_t low = s_[k] & (~s_[k] + 1u);
                 if (!s0 || low < s0) s0 = low;
             }
-        if (s0 > groups_pow2) s0 = groups_pow2;
+        if (s0 > groups_pow2_) s0 = groups_pow2_;
         if (!s0) {  // only contiguous-block stages: any class structure works, take full windows
-            s0 = groups_pow2;
-            while (s0 > 1 && groups / s0 < cap) s0 /= 2;
+            s0 = groups_pow2_;
+            while (s0 > 1 && groups_ / s0 < cap_) s0 /= 2;
         }
         p.first = a;
         p.count = b - a;
         p.single = 0;
         p.class_stride = s0;
-        p.ring = groups / s0;
+        p.ring = groups_ / s0;
         uint32_t sum = 0;
         for (int k = a; k < b; ++k) {
-            if (s[k] % s0) return -1.0;
-            p.sub_stride[k - a] = s[k] / s0;
-            sum += s[k] / s0;
+            if (s_[k] % s0) return -1.0;
+            p.sub_stride[k - a] = s_[k] / s0;
+            sum += s_[k] / s0;
         }
-        if (p.ring <= cap_rows / nc) {  // closed: whole rings of adjacent classes, a power of two of them per window
-            uint32_t rings = floor_pow2((cap_rows / nc) / p.ring);
+        if (p.ring <= cap_rows_ / nc_) {  // closed: whole rings of adjacent classes, a power of two of them per window
+            uint32_t rings = floor_pow2((cap_rows_ / nc_) / p.ring);
             if (rings > s0) rings = s0;
             p.closed = 1;
             p.window = rings * p.ring;
@@ -142,47 +132,147 @@ std::vector<FusedPass> plan_fused(const ncn_shape* sh, int first, int count, boo
             p.own = p.window;
             p.tiles_per_ring = 1;
             p.class_groups = s0 / rings;
-            return priced(a, 1.0, b - a, true);
+            return priced(writes_state, 1.0, b - a, true);
         }
         p.closed = 0;
-        p.window = cap;
-        p.halo = (uint32_t)(nc - 1) * sum;
-        if (2 * p.halo >= cap) return -1.0;
-        p.own = cap - 2 * p.halo;
-        if (p.own * 4 < cap * 3) return -1.0;  // more than a third of the window would be redundant work
+        p.window = cap_;
+        p.halo = (uint32_t)(nc_ - 1) * sum;
+        if (2 * p.halo >= cap_) return -1.0;
+        p.own = cap_ - 2 * p.halo;
+        if (p.own * 4 < cap_ * 3) return -1.0;  // more than a third of the window would be redundant work
         p.tiles_per_ring = (p.ring + p.own - 1) / p.own;
         p.class_groups = s0;
-        return priced(a, (double)cap / p.own, b - a, false);
-    };
-
-    // cheapest cut of the range into passes (a one-stage launch is bound by its traffic: every array once)
-    std::vector<double> best(count + 1, 1e30);
-    std::vector<int> from(count + 1, -1);
-    std::vector<FusedPass> how(count + 1);
-    best[0] = 0.0;
-    for (int b = 1; b <= count; ++b) {
-        const double single = arrays_in + (backward ? (b == 1 ? 2.0 : 4.0) : 2.0);
-        if (best[b - 1] + single < best[b]) {
-            best[b] = best[b - 1] + single;
-            from[b] = b - 1;
-            FusedPass p{};
-            p.first = b - 1;
-            p.count = 1;
-            p.single = 1;
-            how[b] = p;
-        }
-        for (int a = b - 2; a >= 0 && b - a <= max_stages; --a) {
-            FusedPass p{};
-            const double c = make(a, b, p);
-            if (c >= 0.0 && best[a] + c < best[b] - 1e-9) {
-                best[b] = best[a] + c;
-                from[b] = a;
-                how[b] = p;
-            }
-        }
+        return priced(writes_state, (double)cap_ / p.own, b - a, false);
     }
-    for (int b = count; b > 0; b = from[b]) passes.insert(passes.begin(), how[b]);
+
+  private:
+    // What a pass costs, in the time one array of the activations' size takes to cross HBM at copy speed.  Traffic: the
+    // pass reads 4 (forward 2) arrays of its windows (window / own times the data) and writes as many of its
+    // owned rows; a backward pass that hands no reconstructed inputs on writes the two gradients
+    // only (callers that want the reconstructed inputs pay two arrays more than priced here).  Issue: every stage costs
+    // `per_stage` such units of instruction issue on all groups of its windows (measured per kernel family on
+    // x[128, 8192, 128]: a two-row backward stage 0.143 ms against 0.102 ms per array, a two-row forward stage 0.078 ms;
+    // the four-row kernels in proportion to their instruction counts).  The two overlap, better the more they differ:
+    // the cube root of the sum of cubes follows the measured pass times to 5 % (a closed backward pass, whose windows
+    // are the most scattered in memory, takes 1.1 times that).
+    double priced(bool writes_state, double redundancy, int stages, bool closed) const {
+        const double arrays_in = backward_ ? 4.0 : 2.0, arrays_out = backward_ && writes_state ? 4.0 : 2.0;
+        const double per_stage = nc_ == 2 ? (backward_ ? 1.4 : 0.76) : (backward_ ? 3.6 : 2.0);
+        const double traffic = arrays_in * redundancy + arrays_out;
+        const double issue = per_stage * stages * redundancy;
+        return std::cbrt(traffic * traffic * traffic + issue * issue * issue) * (closed && backward_ ? 1.1 : 1.0);
+    }
+
+    int nc_, ec_;
+    uint32_t groups_, cap_rows_, cap_, groups_pow2_;
+    bool backward_;
+    int max_stages_;
+    std::vector<uint32_t> s_;
+};
+
+// One direction of a range whose planning tables are asked for again and again: the cheapest cut of [from, b) into
+// passes for every b, the pass at `from` handing no reconstructed inputs on.
+struct CheapestCut {
+    int from;
+    std::vector<double> cost;   // [b - from]
+    std::vector<int> last;      // where the last pass of [from, b) begins
+    template <class PassCost>
+    CheapestCut(int from_, int to, int max_stages, PassCost pass_cost)
+        : from(from_), cost(to - from_ + 1, 1e30), last(to - from_ + 1, -1) {
+        cost[0] = 0.0;
+        for (int b = from + 1; b <= to; ++b)
+            for (int a = b - 1; a >= from && (b - a == 1 || b - a <= max_stages); --a) {
+                const double c = pass_cost(a, b, a != from);
+                if (c >= 0.0 && cost[a - from] + c < cost[b - from] - 1e-9) {
+                    cost[b - from] = cost[a - from] + c;
+                    last[b - from] = a;
+                }
+            }
+    }
+};
+
+FusedPass pass_of(const PassPlanner& planner, int a, int b) {
+    FusedPass p{};
+    if (b - a > 1) {
+        planner.make(a, b, true, p);
+    } else {
+        p.first = a;
+        p.count = 1;
+        p.single = 1;
+    }
+    return p;
+}
+
+std::vector<FusedPass> passes_of(const PassPlanner& planner, const CheapestCut& cut, int to) {
+    std::vector<FusedPass> passes;
+    for (int b = to; b > cut.from; b = cut.last[b - cut.from])
+        passes.insert(passes.begin(), pass_of(planner, cut.last[b - cut.from], b));
     return passes;
+}
+
+}  // namespace
+
+// Cuts stages [first, first + count) into passes, ascending.
+std::vector<FusedPass> plan_fused(const ncn_shape* sh, int first, int count, bool backward) {
+    const PassPlanner planner(sh, first, count, backward);
+    FusedPass p{};
+    const CheapestCut cut(0, count, planner.max_stages(), [&](int a, int b, bool writes_state) {
+        return b - a == 1 ? planner.single(writes_state) : planner.make(a, b, writes_state, p);
+    });
+    return passes_of(planner, cut, count);
+}
+
+// Where a stack that is trained keeps its activations.  The forward hands the values between two passes through memory
+// anyway: kept, they spare the backward the two arrays that a pass which starts there would otherwise write (and
+// the next one read back all the same).  Where both directions' passes begin and end is chosen together, by the prices
+// above: of x[64, 2048, 128], groups of 4, 6 stages, the forward runs {0,1} {2} {3} {4,5} either way, and the backward's
+// one-stage launches write 2 instead of 4 arrays: a training step of it in bfloat16 870 -> 772 us, with the conversions of
+// the results and weights that the passes now do themselves; x[32, 1024, 128] float32, 5 stages, 253 -> 227.  kKeep is what a kept range must gain to be worth its memory.
+std::vector<StackRange> plan_stack(const ncn_shape* sh, int first, int count, bool multi_stage, int max_range, int max_saves) {
+    constexpr double kKeep = 0.25;
+    const PassPlanner fwd(sh, first, count, false), bwd(sh, first, count, true);
+    const int F = multi_stage ? fwd.max_stages() : 1, B = multi_stage ? bwd.max_stages() : 1;
+    // prices of every pass, made once: [a][length], backward with and without handing the state on
+    std::vector<double> fc((size_t)count * (kFusedMaxStages + 1), -1.0), bc(2 * fc.size(), -1.0);
+    auto at = [](int a, int len) { return (size_t)a * (kFusedMaxStages + 1) + len; };
+    for (int a = 0; a < count; ++a)
+        for (int len = 1; len <= kFusedMaxStages && a + len <= count; ++len) {
+            FusedPass p{};
+            if (len <= F) fc[at(a, len)] = len == 1 ? fwd.single(false) : fwd.make(a, a + len, false, p);
+            if (len <= B)
+                for (int w = 0; w < 2; ++w)
+                    bc[2 * at(a, len) + w] = len == 1 ? bwd.single(w != 0) : bwd.make(a, a + len, w != 0, p);
+        }
+    std::vector<CheapestCut> fcut, bcut;
+    for (int a = 0; a < count; ++a) {
+        const int to = a + max_range < count ? a + max_range : count;
+        fcut.emplace_back(a, to, F, [&](int u, int v, bool) { return fc[at(u, v - u)]; });
+        bcut.emplace_back(a, to, B, [&](int u, int v, bool w) { return bc[2 * at(u, v - u) + (w ? 1 : 0)]; });
+    }
+    // best[k][b]: [0, b) in k ranges
+    if (max_saves > count) max_saves = count;
+    std::vector<std::vector<double>> best(max_saves + 1, std::vector<double>(count + 1, 1e30));
+    std::vector<std::vector<int>> from(max_saves + 1, std::vector<int>(count + 1, -1));
+    best[0][0] = 0.0;
+    for (int k = 1; k <= max_saves; ++k)
+        for (int b = k; b <= count; ++b)
+            for (int a = b - 1; a >= 0 && b - a <= max_range; --a) {
+                const double c = best[k - 1][a] + fcut[a].cost[b - a] + bcut[a].cost[b - a] + kKeep;
+                if (c < best[k][b] - 1e-9) {
+                    best[k][b] = c;
+                    from[k][b] = a;
+                }
+            }
+    int k = 0;
+    for (int j = 1; j <= max_saves; ++j)
+        if (best[j][count] < 1e29 && (k == 0 || best[j][count] < best[k][count])) k = j;
+    std::vector<StackRange> ranges(k);
+    for (int b = count; k > 0; --k) {
+        const int a = from[k][b];
+        ranges[k - 1] = StackRange{passes_of(fwd, fcut[a], b), passes_of(bwd, bcut[a], b)};
+        b = a;
+    }
+    return ranges;
 }
 
 int64_t fused_items(const ncn_shape* sh, const FusedPass& p) {

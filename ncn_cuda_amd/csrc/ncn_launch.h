@@ -155,6 +155,14 @@ struct FusedPass {
 };
 bool fused_supported(const ncn_shape* sh, int activation);
 std::vector<FusedPass> plan_fused(const ncn_shape* sh, int first, int count, bool backward);
+// Consecutive stages of a trained stack whose last outputs are kept for the backward: the passes of both directions, in
+// ascending order, numbered relative to the planned stages.
+struct StackRange {
+    std::vector<FusedPass> fwd, bwd;
+};
+// At most max_saves ranges of at most max_range stages (empty if there is no such cut).  multi_stage: whether the shape has
+// multi-stage passes; without them every pass is one stage.
+std::vector<StackRange> plan_stack(const ncn_shape* sh, int first, int count, bool multi_stage, int max_range, int max_saves);
 // windows of a pass (== workgroups, when every workgroup takes one)
 int64_t fused_items(const ncn_shape* sh, const FusedPass& p);
 // row_cap: rows of the dW partial buffer a backward pass may fill (grid / n_head rows per stage)

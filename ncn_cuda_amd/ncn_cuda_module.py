@@ -339,6 +339,65 @@ def backward_stages(y, ya, dy, dya, W, alpha, activation, cache_dim, nhead, firs
     return x_rec, xa_rec, dx, dxa, dW
 
 
+class StackPlan:
+    """Where a trained stack keeps its activations (ncn_stack_plan): arguments that both directions share."""
+
+    def __init__(self, shape, first_stage, n_stages, alpha, m, activation, max_range, max_saves, io_dtype):
+        self.args = (int(first_stage), int(n_stages), int(max_range), int(max_saves), float(alpha), float(m), int(activation))
+        self.shape = shape
+        self.io_dtype = io_dtype
+        out = (ctypes.c_int64 * 2)()
+        self.ranges = _lib.load().ncn_stack_plan(ctypes.byref(shape), self.args[0], self.args[1], self.args[4], self.args[5],
+                                                 self.args[6], self.args[2], self.args[3], _DTYPES[io_dtype], out)
+        self.forward_bytes, self.backward_bytes = out[0], out[1]
+
+
+def stack_forward(x, xa, W, alpha, activation, cache_dim, nhead, first_stage, n_stages, max_range, save_budget, *, m=M_DEFAULT):
+    """The forward of a stack that will be trained: (plan, y, ya, saves), y and ya in the dtype of x, `saves` the float32
+    activations that stack_backward reads beside (float32) or in place of (bfloat16) y, ya; at most max_range stages lie
+    between two of them.  save_budget bounds their bytes where max_range leaves a choice.  None: no such plan."""
+    shape = validate(x, xa, W, cache_dim, nhead, activation, first_stage, n_stages, alpha=alpha, m=m)
+    dev = _require_gpu(x, xa, W)
+    max_saves = max(int(save_budget) // (8 * x.numel()), -(-int(n_stages) // int(max_range)))
+    plan = StackPlan(shape, first_stage, n_stages, alpha, m, activation, max_range, min(max_saves, int(n_stages)), x.dtype)
+    if plan.ranges <= 0:
+        return None
+    x, xa, (w, wflag) = _prep(x.detach()), _prep(xa.detach()), _weights(W)
+    y, ya = torch.empty(x.shape, dtype=x.dtype, device=dev), torch.empty(x.shape, dtype=x.dtype, device=dev)
+    kept = plan.ranges - (x.dtype == torch.float32)
+    saves = torch.empty((kept, 2) + tuple(x.shape), dtype=torch.float32, device=dev) if kept else None
+    ws = torch.empty(plan.forward_bytes, dtype=torch.uint8, device=dev) if plan.forward_bytes else None
+    with torch.cuda.device(dev):
+        rc = _lib.load().ncn_stack_forward(_ptr(x), _ptr(xa), _DTYPES[x.dtype] | wflag, _ptr(y), _ptr(ya), _DTYPES[x.dtype],
+                                           _ptr(saves), _ptr(w), _ptr(ws), ctypes.c_size_t(plan.forward_bytes),
+                                           ctypes.byref(shape), *plan.args, _stream(dev))
+    _lib.check(rc, "ncn_stack_forward")
+    return plan, y, ya, saves
+
+
+def stack_backward(plan, y, ya, saves, dy, dya, W):
+    """dx, dxa (in the dtype of the stack's inputs) and dW[n_stages, 2E] (in that of W) of a stack_forward call; y, ya its
+    float32 outputs or None.  dya may be None (zeros)."""
+    like = y if y is not None else saves[0, 0]
+    if dy.shape != like.shape or (dya is not None and dya.shape != dy.shape):
+        raise ValueError("dy/dya must have the shape of y")
+    if dy.dtype not in _DTYPES or (dya is not None and dya.dtype != dy.dtype):
+        raise TypeError("dy and dya must both be float32 or bfloat16")
+    dev = _require_gpu(y, ya, saves, dy, dya, W)
+    y, ya, saves = (None if t is None else _prep(t.detach()) for t in (y, ya, saves))
+    dy, dya, (w, wflag) = _prep(dy.detach()), None if dya is None else _prep(dya.detach()), _weights(W)
+    dx, dxa = torch.empty(dy.shape, dtype=plan.io_dtype, device=dev), torch.empty(dy.shape, dtype=plan.io_dtype, device=dev)
+    dW = torch.empty(plan.args[1], 2 * dy.shape[2], dtype=w.dtype, device=dev)
+    ws = torch.empty(plan.backward_bytes, dtype=torch.uint8, device=dev)
+    with torch.cuda.device(dev):
+        rc = _lib.load().ncn_stack_backward(_ptr(y), _ptr(ya), _ptr(saves), _ptr(dy), _ptr(dya), _DTYPES[dy.dtype], _ptr(dx),
+                                            _ptr(dxa), _DTYPES[plan.io_dtype], _ptr(w), _ptr(dW), wflag, _ptr(ws),
+                                            ctypes.c_size_t(plan.backward_bytes), ctypes.byref(plan.shape), *plan.args,
+                                            _stream(dev))
+    _lib.check(rc, "ncn_stack_backward")
+    return dx, dxa, dW
+
+
 def inverse_stages(y, ya, W, alpha, activation, cache_dim, nhead, first_stage, n_stages, *, m=M_DEFAULT,
                    out_dtype=None, group_index=None, ctx_len=None, check_tables=True, scratch=True):
     """x, xa with forward_stages(x, xa, ...) == (y, ya).  scratch: with several stages, allocate the scratch that lets

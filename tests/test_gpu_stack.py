@@ -1,0 +1,78 @@
+"""ncn_stack_forward / ncn_stack_backward (a trained stack in one call per direction) against the float64 oracle: every
+pairing of kept ranges with passes, both element types, group counts without multi-stage passes, heads of one feature."""
+import ctypes
+
+import pytest
+import torch
+
+from oracle import ncn_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+# batch, N, E, heads, n_cache, stages, max_range, max_saves; ranges expected
+CASES = [
+    ((2, 1024, 128, 4, 4, 5, 6, 5), None),    # ranges of one and two stages
+    ((2, 2048, 64, 2, 4, 6, 6, 1), 1),        # one range: scratch between passes, states handed on inside it
+    ((1, 2048, 64, 2, 4, 7, 6, 2), 2),        # two ranges, one of them of several passes
+    ((2, 8192, 64, 2, 2, 13, 13, 1), 1),      # three backward passes in one range
+    ((1, 8192, 32, 1, 2, 14, 13, 2), 2),
+    ((2, 1020, 64, 2, 4, 5, 6, 5), 5),        # an odd number of groups: one launch per stage, every output kept
+    ((2, 1018, 64, 2, 2, 4, 13, 1), 1),       # the same with nothing kept between the stages
+    ((1, 16, 32, 4, 2, 3, 13, 3), None),      # the smallest rings
+    ((1, 512, 64, 64, 2, 7, 13, 7), None),    # heads of one feature
+]
+
+
+@pytest.fixture(scope="module")
+def M():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from ncn_cuda_amd import ncn_cuda_module
+    return ncn_cuda_module
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("case,ranges", CASES, ids=lambda c: "_".join(map(str, c)) if isinstance(c, tuple) else "")
+def test_stack(M, case, ranges, dtype):
+    batch, N, E, C, n, L, max_range, max_saves = case
+    x, xa, Ws, dy, dya = O.make_inputs(batch, N, E, L, n, seed=sum(case), xa_zero=False, dtype=dtype)
+    d = torch.float64
+    ref = O.net_autograd(x.to(d), xa.to(d), [w.to(d) for w in Ws], dy.to(d), dya.to(d), 0.9, n, C, first_stage=1)
+    W = torch.stack([w.reshape(-1) for w in Ws]).cuda()
+    plan, y, ya, saves = M.stack_forward(x.cuda(), xa.cuda(), W, 0.9, 0, n, C, 1, L, max_range,
+                                         8 * x.numel() * max_saves)
+    assert plan.ranges == ranges or (ranges is None and 1 <= plan.ranges <= max_saves)
+    f32 = dtype == torch.float32
+    kept = (y, ya) if f32 else (None, None)
+    # float32: 1.2e-6 per unit of rounding, amplified by 1/m at each of the steps between two kept values (13 stages of
+    # groups of two rows at most); bfloat16 results are rounded once, by at most half a unit of their eight significant
+    # bits: 2^-8 of a value
+    tol = 1.2e-6 * 0.9 ** -(n * min(max_range, L)) if f32 else 2.0 ** -8
+    for grad_a in (dya.cuda(), None):
+        r = ref if grad_a is not None else O.net_autograd(x.to(d), xa.to(d), [w.to(d) for w in Ws], dy.to(d),
+                                                          torch.zeros_like(dya).to(d), 0.9, n, C, first_stage=1)
+        dx, dxa, dW = M.stack_backward(plan, *kept, saves, dy.cuda(), grad_a, W)
+        for name, got, want in (("y", y, r[0]), ("ya", ya, r[1]), ("dx", dx, r[2]), ("dxa", dxa, r[3])):
+            assert got.dtype == dtype
+            assert O.rel_err(got, want) < tol, name
+        for l in range(L):
+            assert dW.dtype == dtype and O.rel_err(dW[l], r[4][l].reshape(-1)) < tol, l
+
+
+def test_refusals(M):
+    """Outputs that are the inputs, a workspace that is too small: refused before any launch."""
+    from ncn_cuda_amd import _lib
+    x = torch.zeros(1, 64, 32, device="cuda")
+    xa, y, W = torch.zeros_like(x), torch.zeros_like(x), torch.zeros(3, 64, device="cuda")
+    sh = _lib.NcnShape(1, 64, 32, 1, 2)
+    lib = _lib.load()
+
+    def forward(out):
+        return lib.ncn_stack_forward(M._ptr(x), M._ptr(xa), 0, M._ptr(out), M._ptr(y), 0, None, M._ptr(W), None,
+                                     ctypes.c_size_t(0), ctypes.byref(sh), 0, 3, 13, 1, 0.9, 0.9, 0, M._stream(x.device))
+
+    assert "carry the state" in _lib.error_string(forward(x))
+    rc = lib.ncn_stack_backward(M._ptr(y), M._ptr(y), None, M._ptr(x), None, 0, M._ptr(xa), M._ptr(xa), 0, M._ptr(W),
+                                M._ptr(W), 0, None, ctypes.c_size_t(0), ctypes.byref(sh), 0, 3, 13, 1, 0.9, 0.9, 0,
+                                M._stream(x.device))
+    assert "workspace" in _lib.error_string(rc)
