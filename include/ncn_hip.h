@@ -11,7 +11,7 @@
  *     (reference: default stream + cudaDeviceSynchronize, ncn_fwd_cuda_kernel.cu:158);
  *   - every entry point returns 0 or an error code (reference: no checks at all);
  *   - activations and gradients may be float32 or bfloat16 in memory; all arithmetic is float32;
- *     W and dW are always float32;
+ *     W and dW are float32, or both bfloat16 (NCN_W_BF16);
  *   - `m`, hard-coded to 0.9 in the reference (ncn_fwd_cuda_kernel.cu:72), is an argument;
  *   - several consecutive stages can be run by one call (n_stages > 1), later stages in place.
  *
