@@ -18,11 +18,14 @@ struct Weights {
     const void* base;
     int64_t two_e;
     bool bf16, arrays;
-    // takes the flags out of dtype
+    // takes the flags out of dtype; a dtype with other bits set (a negative one, say) carries no flags and stays as it is
+    // for the check of the element type: W must not be read as an array of pointers for it
     Weights(const void* W, int& dtype, const ncn_shape* sh) : base(W), two_e(2 * sh->E) {
-        bf16 = (dtype & NCN_W_BF16) != 0;
-        arrays = (dtype & NCN_W_ARRAYS) != 0;
-        dtype &= ~(NCN_W_BF16 | NCN_W_ARRAYS);
+        constexpr int kFlags = NCN_W_BF16 | NCN_W_ARRAYS;
+        const int flags = (dtype & ~(kFlags | 0xff)) == 0 ? dtype & kFlags : 0;
+        bf16 = (flags & NCN_W_BF16) != 0;
+        arrays = (flags & NCN_W_ARRAYS) != 0;
+        dtype &= ~flags;
     }
     size_t size() const { return bf16 ? 2 : 4; }
     const void* at(int stage) const {

@@ -120,6 +120,32 @@ def test_entry_points_reject_bad_arguments_before_touching_the_gpu(lib):
     assert h.ncn_backward(*args, p, ctypes.c_size_t(ws8), ctypes.byref(sh8), 0, 2, 0.9, 0.9, 0, z) == -8  # needs x_rec
 
 
+@pytest.mark.parametrize("dtype", [-1, -256, 0x400, 0x700, 1 << 30, 5, 0x300 | 7])
+def test_unknown_first_element_type_is_refused_without_reading_the_weights(lib, dtype):
+    """The flags of the weights travel in the first element type: a value with other bits set is no element type, and W is
+    not taken for an array of pointers (it is not readable on the host here).  0x300 | 7 carries the flags: W is read."""
+    h = lib.load()
+    sh = _shape(lib, 2, 64, 32, 4, 4)
+    p, z = ctypes.c_void_p(4096), ctypes.c_void_p(0)
+    W = p if dtype & ~0x3ff or not dtype & 0x200 else ctypes.cast((ctypes.c_void_p * 2)(4096, 4096), ctypes.c_void_p)
+    dims = (ctypes.byref(sh), 0, 2, 0.9, 0.9, 0, z)
+    ws = (p, ctypes.c_size_t(1 << 40))
+    grads = (p, p, 0, p, p, 0, p, p)   # dy, dya, dx, dxa, x_rec, xa_rec
+    assert h.ncn_forward(p, p, dtype, p, p, 0, z, z, W, z, ctypes.c_size_t(0), *dims) == -3
+    assert h.ncn_inverse(p, p, dtype, p, p, 0, W, *dims) == -3
+    assert h.ncn_inverse_ws(p, p, dtype, p, p, 0, W, *ws, *dims) == -3
+    assert h.ncn_backward(p, p, dtype, *grads, W, p, *ws, *dims) == -3
+    assert h.ncn_forward_indexed(p, p, dtype, p, p, 0, z, z, W, p, p, *dims) == -3
+    assert h.ncn_inverse_indexed(p, p, dtype, p, p, 0, W, p, p, *dims) == -3
+    assert h.ncn_backward_indexed(p, p, dtype, *grads, W, p, *ws, p, p, *dims) == -3
+    assert h.ncn_forward_radix(p, p, dtype, p, p, 0, z, z, W, *dims) == -3
+    assert h.ncn_inverse_radix(p, p, dtype, p, p, 0, W, *dims) == -3
+    assert h.ncn_backward_radix(p, p, dtype, *grads, W, p, *ws, *dims) == -3
+    q, stack = ctypes.c_void_p(8192), (ctypes.byref(sh), 0, 2, 13, 2, 0.9, 0.9, 0, z)
+    assert h.ncn_stack_forward(p, p, dtype, q, q, 0, p, W, *ws, *stack) == -3
+    assert h.ncn_stack_backward(p, p, p, p, p, 0, q, q, 0, W, p, dtype, *ws, *stack) == -3
+
+
 def test_indexed_entry_points_reject_bad_arguments_before_touching_the_gpu(lib):
     h = lib.load()
     sh = _shape(lib, 2, 64, 32, 4, 4)
