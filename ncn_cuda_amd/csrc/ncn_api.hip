@@ -1,6 +1,7 @@
 // C ABI of libncn_hip.so: argument validation, stage sequencing and launches.  See include/ncn_hip.h.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <mutex>
 
@@ -1179,6 +1180,9 @@ struct StackCall {
         const int path = kernel_path_for(sh, activation, alpha, m);
         // (the tables of plan_stack grow with the square of the stages)
         if (path != 2 || count < 2 || count > 256 || max_range < 1 || max_saves < 1) return false;
+        // bounds past the stages bound nothing (and a stage number plus one of them must not overflow)
+        max_range = std::min(max_range, count);
+        max_saves = std::min(max_saves, count);
         headwise = headwise_call(sh, path, &as_wide);
         shape = headwise ? &as_wide : sh;
         const bool multi = fused_supported(shape, activation);

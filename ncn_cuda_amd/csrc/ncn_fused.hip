@@ -250,7 +250,6 @@ std::vector<StackRange> plan_stack(const ncn_shape* sh, int first, int count, bo
         bcut.emplace_back(a, to, B, [&](int u, int v, bool w) { return bc[2 * at(u, v - u) + (w ? 1 : 0)]; });
     }
     // best[k][b]: [0, b) in k ranges
-    if (max_saves > count) max_saves = count;
     std::vector<std::vector<double>> best(max_saves + 1, std::vector<double>(count + 1, 1e30));
     std::vector<std::vector<int>> from(max_saves + 1, std::vector<int>(count + 1, -1));
     best[0][0] = 0.0;

@@ -160,7 +160,7 @@ std::vector<FusedPass> plan_fused(const ncn_shape* sh, int first, int count, boo
 struct StackRange {
     std::vector<FusedPass> fwd, bwd;
 };
-// At most max_saves ranges of at most max_range stages (empty if there is no such cut).  multi_stage: whether the shape has
+// At most max_saves ranges of at most max_range stages, both at most `count` (empty if there is no such cut).  multi_stage: whether the shape has
 // multi-stage passes; without them every pass is one stage.
 std::vector<StackRange> plan_stack(const ncn_shape* sh, int first, int count, bool multi_stage, int max_range, int max_saves);
 // windows of a pass (== workgroups, when every workgroup takes one)

@@ -399,6 +399,26 @@ def test_multi_stage_plan_declines_ineligible_shapes(lib):
     assert [p[2] for p in fwd][-1] == 2 and len(fwd) <= 4
 
 
+@pytest.mark.parametrize("dims", [(2, 1024, 128, 4, 4, 5), (1, 256, 32, 4, 2, 8), (2, 1020, 64, 2, 4, 3)])
+def test_stack_plan_takes_bounds_of_any_size(lib, dims):
+    """max_range and max_saves up to the largest int bound no more than the number of stages does."""
+    h = lib.load()
+    batch, N, E, C, n, L = dims
+    sh, most = _shape(lib, batch, N, E, C, n), 2 ** 31 - 1
+
+    def plan(max_range, max_saves):
+        out = (ctypes.c_int64 * 2)()
+        ranges = h.ncn_stack_plan(ctypes.byref(sh), 0, L, 0.9, 0.9, 0, max_range, max_saves, 0, out)
+        return ranges, out[0], out[1]
+
+    want = plan(L, L)
+    assert 1 <= want[0] <= L
+    for max_range, max_saves in ((most, most), (most, L), (L, most), (L + 1, most - 1)):
+        assert plan(max_range, max_saves) == want
+    assert plan(most, 1)[0] == 1 and plan(1, most)[0] == L
+    assert plan(0, most)[0] == plan(-1, most)[0] == plan(most, 0)[0] == 0
+
+
 def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     """No fallback: if libncn_hip.so is absent and cannot be built, the binding raises instead of computing something
     else."""
