@@ -214,7 +214,9 @@ __device__ __forceinline__ void headwise_backward_core(float (&Y)[R][F], float (
     float4* slots = bcast_lds + (T::LR == 1 ? 0 : wave * (F / 4) * 64);                         \
     const int fl = lane % T::LF;                                                                \
     float wi[F], wj[F];                                                                         \
-    load_w<F>(A, head, EC, fl, wi, wj);
+    issue_w<F>(A, head, EC, fl, wi, wj);                                                        \
+    finish_w<F>(A, wi);                                                                         \
+    finish_w<F>(A, wj);
 
 #define NCN_HW_ROW_LIVE(rr) ((int)(((lane / T::LF) % T::LR) * R + (rr)) < live)
 

@@ -70,7 +70,38 @@ __device__ __forceinline__ int tile_offsets(const StageArgs& A, uint32_t t, int 
     return live;
 }
 
-// A lane's weights times gamma.
+// A lane's weights, still as loaded: float32 all four words of a chunk, bfloat16 the first two (the last two are loaded from
+// the same place).  No branch on the type, whose sides would wait for the loads: in the prologue of a kernel they are only
+// requested.  (With such a branch after the tile's loads, and nine registers more, forwards of mixed types took 88 instead of
+// 82 us at 32 x 4096 x 128, groups of 16.)
+template <int F>
+__device__ __forceinline__ void issue_w(const StageArgs& A, int head, int ec, int fl, float (&wi)[F], float (&wj)[F]) {
+    const int log2_size = A.w_bf16 ? 1 : 2, second = A.w_bf16 ? 0 : 8;
+    const char* const wi_at = static_cast<const char*>(A.W) + (((int64_t)head * ec + fl * F) << log2_size);
+    const char* const wj_at = wi_at + (A.E << log2_size);
+    const int chunk = 4 << log2_size;
+#pragma unroll
+    for (int k = 0; k < F / 4; ++k) {
+        const float2 i0 = *reinterpret_cast<const float2*>(wi_at + k * chunk), i1 = *reinterpret_cast<const float2*>(wi_at + k * chunk + second);
+        const float2 j0 = *reinterpret_cast<const float2*>(wj_at + k * chunk), j1 = *reinterpret_cast<const float2*>(wj_at + k * chunk + second);
+        wi[4 * k] = i0.x; wi[4 * k + 1] = i0.y; wi[4 * k + 2] = i1.x; wi[4 * k + 3] = i1.y;
+        wj[4 * k] = j0.x; wj[4 * k + 1] = j0.y; wj[4 * k + 2] = j1.x; wj[4 * k + 3] = j1.y;
+    }
+}
+// .. as float32, times gamma
+template <int F>
+__device__ __forceinline__ void finish_w(const StageArgs& A, float (&w)[F]) {
+#pragma unroll
+    for (int k = 0; k < F / 4; ++k) {
+        const uint32_t w0 = __float_as_uint(w[4 * k]), w1 = __float_as_uint(w[4 * k + 1]);
+        w[4 * k] = A.tab.gamma * (A.w_bf16 ? __uint_as_float(w0 << 16) : w[4 * k]);
+        w[4 * k + 1] = A.tab.gamma * (A.w_bf16 ? __uint_as_float(w0 & 0xffff0000u) : w[4 * k + 1]);
+        w[4 * k + 2] = A.tab.gamma * (A.w_bf16 ? __uint_as_float(w1 << 16) : w[4 * k + 2]);
+        w[4 * k + 3] = A.tab.gamma * (A.w_bf16 ? __uint_as_float(w1 & 0xffff0000u) : w[4 * k + 3]);
+    }
+}
+
+// Both at once, where nothing is to be loaded in between.
 template <int F>
 __device__ __forceinline__ void load_w(const StageArgs& A, int head, int ec, int fl, float (&wi)[F], float (&wj)[F]) {
     const int64_t at = (int64_t)head * ec + fl * F;
@@ -449,15 +480,15 @@ __device__ __forceinline__ void backward_steps(float (&Y)[R][F], float (&B)[R][F
     float4* slots = bcast_lds + (T::LR == 1 ? 0 : wave * (F / 4) * 64);                         \
     const int fl = lane % T::LF;                                                                \
     float wi[F], wj[F];                                                                         \
-    bool w_todo = true;
+    bool w_raw = true;
 
-// The weights are loaded once, after the loads of the wave's first tile have been issued: their branch on the type waits
-// for them, and in the prologue that wait would come before the tile's own loads are even on their way (one memory
-// latency after the other).
-#define NCN_LOAD_W_ONCE                                                                         \
-    if (w_todo) {                                                                               \
-        w_todo = false;                                                                         \
-        load_w<F>(A, head, EC, fl, wi, wj);                                                     \
+// The weights are scaled by gamma once, after the loads of the wave's first tile have been issued: scaling them in the
+// prologue would wait for them before the tile's own loads are even on their way (one memory latency after the other).
+#define NCN_FINISH_W_ONCE                                                                       \
+    if (w_raw) {                                                                                \
+        w_raw = false;                                                                          \
+        finish_w<F>(A, wi);                                                                     \
+        finish_w<F>(A, wj);                                                                     \
     }
 
 // Row rr of this lane is live when its slot is below the group's live rows (always, or never, without lengths).
@@ -499,6 +530,7 @@ __device__ __forceinline__ int dtype_of(int from_args, int when_bf16) {
 template <int NC, int EC, int R, int F, bool TANH_ONLY = true, bool INDEXED = false, int TYPES = kAnyTypes>
 __global__ void __launch_bounds__(kBlockThreads, (TANH_ONLY && !INDEXED && R == 4 && F == 4) ? 5 : 1) stage_forward_kernel(const StageArgs A) {
     NCN_WAVE_PROLOGUE
+    issue_w<F>(A, head, EC, fl, wi, wj);
     const int in_dtype = dtype_of<TYPES>(A.in_dtype, NCN_BF16);
     const int out_dtype = TYPES == kBf16Types && A.out_dtype != NCN_BF16X2 ? NCN_BF16 : dtype_of<TYPES>(A.out_dtype, NCN_BF16X2);
     for (uint32_t t = gwave / A.n_head; t < A.total_tiles; t += tile_step) {
@@ -507,7 +539,7 @@ __global__ void __launch_bounds__(kBlockThreads, (TANH_ONLY && !INDEXED && R == 
         float x[R][F], a[R][F];
         issue_tile<R, F>(A.in0, in_dtype, off, x);
         issue_tile<R, F>(A.in1, in_dtype, off, a);
-        NCN_LOAD_W_ONCE
+        NCN_FINISH_W_ONCE
         finish_tile<R, F>(in_dtype, x);
         finish_tile<R, F>(in_dtype, a);
         NCN_PASS_DEAD_ROWS(A.out0, A.out1, out_dtype, x, a)
@@ -532,6 +564,7 @@ __global__ void __launch_bounds__(kBlockThreads, (TANH_ONLY && !INDEXED && R == 
 template <int NC, int EC, int R, int F, bool TANH_ONLY = true, bool INDEXED = false, int TYPES = kAnyTypes>
 __global__ void __launch_bounds__(kBlockThreads) stage_inverse_kernel(const StageArgs A) {
     NCN_WAVE_PROLOGUE
+    issue_w<F>(A, head, EC, fl, wi, wj);
     const int in_dtype = dtype_of<TYPES>(A.in_dtype, NCN_BF16), out_dtype = dtype_of<TYPES>(A.out_dtype, NCN_BF16);
     for (uint32_t t = gwave / A.n_head; t < A.total_tiles; t += tile_step) {
         int64_t off[R];
@@ -539,7 +572,7 @@ __global__ void __launch_bounds__(kBlockThreads) stage_inverse_kernel(const Stag
         float y[R][F], b[R][F];
         issue_tile<R, F>(A.in0, in_dtype, off, y, A.plane);
         issue_tile<R, F>(A.in1, in_dtype, off, b, A.plane);
-        NCN_LOAD_W_ONCE
+        NCN_FINISH_W_ONCE
         finish_tile<R, F>(in_dtype, y);
         finish_tile<R, F>(in_dtype, b);
         NCN_PASS_DEAD_ROWS(A.out0, A.out1, out_dtype, y, b)
@@ -564,6 +597,9 @@ __global__ void __launch_bounds__(kBlockThreads) stage_inverse_kernel(const Stag
 template <int NC, int EC, int R, int F, bool TANH_ONLY = true, bool INDEXED = false, bool LOOP = true, int TYPES = kAnyTypes>
 __global__ void __launch_bounds__(kBlockThreads, (TANH_ONLY && R * F <= 16 && F == 4) ? 4 : (TYPES != kAnyTypes && R * F == 32) ? 2 : 1) stage_backward_kernel(const StageArgs A) {
     NCN_WAVE_PROLOGUE
+    // the builds for one type keep nothing in registers while the tile is loaded: they are at their limit of registers
+    constexpr bool kEarlyW = LOOP || TYPES == kAnyTypes;
+    if constexpr (kEarlyW) issue_w<F>(A, head, EC, fl, wi, wj);
     const int in_dtype = dtype_of<TYPES>(A.in_dtype, NCN_BF16X2), g_dtype = dtype_of<TYPES>(A.g_dtype, NCN_BF16);
     const int out_dtype = dtype_of<TYPES>(A.out_dtype, NCN_BF16);
     float dwi[F], dwj[F];
@@ -586,7 +622,11 @@ __global__ void __launch_bounds__(kBlockThreads, (TANH_ONLY && R * F <= 16 && F 
 #pragma unroll
                 for (int f = 0; f < F; ++f) H[rr][f] = 0.f;
         }
-        NCN_LOAD_W_ONCE
+        if constexpr (kEarlyW) {
+            NCN_FINISH_W_ONCE
+        } else {
+            load_w<F>(A, head, EC, fl, wi, wj);
+        }
         finish_tile<R, F>(in_dtype, Y);
         finish_tile<R, F>(in_dtype, B);
         finish_tile<R, F>(g_dtype, G);
@@ -632,7 +672,7 @@ __global__ void __launch_bounds__(kBlockThreads, (TANH_ONLY && R * F <= 16 && F 
 #undef NCN_ROW_LIVE
 #undef NCN_ZERO_DEAD_ROWS
 #undef NCN_PASS_DEAD_ROWS
-#undef NCN_LOAD_W_ONCE
+#undef NCN_FINISH_W_ONCE
 #undef NCN_WAVE_PROLOGUE
 
 }  // namespace ncn

@@ -21,6 +21,7 @@ def M():
 # (n_cache, E, heads, groups, stages, alpha)
 CASES = [(16, 128, 4, 4, 1, 0.9),   # register kernels, tiles of 4 x 4
          (4, 128, 2, 6, 1, 0.9),    # 2 x 8
+         (16, 256, 4, 3, 1, 0.9),   # 4 x 8, an odd number of groups
          (8, 32, 32, 4, 1, 0.9),    # heads of one feature
          (5, 30, 2, 5, 1, 0.9),     # no powers of two
          (5, 30, 2, 5, 1, 0.0),     # generic kernels (alpha outside the scaled state)
@@ -49,7 +50,27 @@ def test_bfloat16_weights(M, case):
     assert torch.equal(got[4], want[4])
 
 
-@pytest.mark.parametrize("case", [CASES[0], CASES[5], CASES[6]], ids=lambda c: "n%d_E%d_C%d_g%d_L%d_a%g" % c)
+@pytest.mark.parametrize("types", [(torch.bfloat16, torch.float32), (torch.float32, torch.bfloat16)], ids=["bf16-f32", "f32-bf16"])
+@pytest.mark.parametrize("act", [0, 1])
+@pytest.mark.parametrize("n,E,C,groups", [(16, 128, 4, 5), (16, 256, 4, 3), (4, 64, 4, 7), (8, 32, 32, 3)])
+def test_bfloat16_weights_with_mixed_types(M, n, E, C, groups, act, types):
+    """The builds for every element type: results of another type than the inputs, with and without a table."""
+    first, second = types
+    x, xa, Ws, dy, dya = (t.cuda() if isinstance(t, torch.Tensor) else t[0].cuda()
+                          for t in O.make_inputs(2, n * groups, E, 1, n, seed=n + E, xa_zero=False))
+    W = Ws.bfloat16()
+    table = torch.randperm(n * groups, generator=torch.Generator().manual_seed(1)).to(torch.int32).cuda()
+    for kw in ({}, dict(group_index=table)):
+        def both(f):
+            for a, b in zip(f(W), f(W.float())):
+                assert (a is None and b is None) or torch.equal(a, b)
+        both(lambda w: M.forward_stages(x.to(first), xa.to(first), w, 0.9, act, n, C, 1, 1, out_dtype=second, **kw))
+        both(lambda w: M.inverse_stages(x.to(first), xa.to(first), w, 0.9, act, n, C, 1, 1, out_dtype=second, **kw))
+        both(lambda w: M.backward_stages(x.to(first), xa.to(first), dy.to(second), dya.to(second), w, 0.9, act, n, C, 1, 1,
+                                         grad_dtype=first, **kw))
+
+
+@pytest.mark.parametrize("case", [CASES[0], CASES[6], CASES[7]], ids=lambda c: "n%d_E%d_C%d_g%d_L%d_a%g" % c)
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_one_array_per_stage(M, case, dtype):
     """NCN_W_ARRAYS: the weights of every stage where they are."""
