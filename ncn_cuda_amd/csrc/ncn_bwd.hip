@@ -1,9 +1,9 @@
 // Instantiations and dispatch of the register-resident reversible backward stage kernel.
-// Compiled six times: as it stands for the stride permutation, and through ncn_bwd_indexed.hip (NCN_INDEXED_BUILD = 1)
+// Compiled eight times: as it stands for the stride permutation, and through ncn_bwd_indexed.hip (NCN_INDEXED_BUILD = 1)
 // for launches that carry a grouping table or context lengths; each of the two takes every element type and activation,
-// with a loop over tiles, and hands tanh launches of one storage type whose grid has a wave for every tile on to its
-// builds for that type, which have no loop (ncn_bwd_f32.hip, ncn_bwd_bf16.hip, ncn_bwd_indexed_f32.hip,
-// ncn_bwd_indexed_bf16.hip: NCN_TYPES_BUILD).
+// with a loop over tiles, and hands launches whose grid has a wave for every tile on to its builds without the loop
+// (NCN_TYPES_BUILD): tanh of one storage type to ncn_bwd_f32.hip, ncn_bwd_bf16.hip, ncn_bwd_indexed_f32.hip and
+// ncn_bwd_indexed_bf16.hip, everything else to ncn_bwd_once.hip and ncn_bwd_indexed_once.hip.
 #include "ncn_configs.h"
 #include "ncn_launch.h"
 #include "ncn_stage_kernels.h"
@@ -20,15 +20,16 @@ namespace ncn {
 template <>
 hipError_t launch_stage_backward<NCN_INDEXED_BUILD != 0, NCN_TYPES_BUILD>(const StageArgs& a, int grid_x, hipStream_t s) {
     constexpr bool kIndexed = NCN_INDEXED_BUILD != 0;
-    constexpr int kTypes = NCN_TYPES_BUILD;
-    constexpr bool kLoop = kTypes == kAnyTypes;
+    constexpr bool kLoop = NCN_TYPES_BUILD == kAnyTypes;
+    constexpr int kTypes = NCN_TYPES_BUILD == kAnyTypesOnce ? kAnyTypes : NCN_TYPES_BUILD;
     const dim3 grid(grid_x), block(kBlockThreads);
     const bool tanh_only = a.activation == NCN_ACT_TANH;
-    if constexpr (kTypes == kAnyTypes) {
+    if constexpr (kLoop) {
         if ((uint64_t)a.total_tiles * (uint64_t)a.n_head <= (uint64_t)grid_x * kWavesPerBlock) {   // a wave for every tile
             const int types = stage_types(kBackward, a);
             if (types == kF32Types) return launch_stage_backward<kIndexed, kF32Types>(a, grid_x, s);
             if (types == kBf16Types) return launch_stage_backward<kIndexed, kBf16Types>(a, grid_x, s);
+            return launch_stage_backward<kIndexed, kAnyTypesOnce>(a, grid_x, s);
         }
     }
 #define NCN_LAUNCH(KERNEL) hipLaunchKernelGGL(KERNEL, grid, block, 0, s, a)

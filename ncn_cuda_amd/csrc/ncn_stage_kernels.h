@@ -73,7 +73,7 @@ __device__ __forceinline__ int tile_offsets(const StageArgs& A, uint32_t t, int 
 // A lane's weights, still as loaded: float32 all four words of a chunk, bfloat16 the first two (the last two are loaded from
 // the same place).  No branch on the type, whose sides would wait for the loads: in the prologue of a kernel they are only
 // requested.  (With such a branch after the tile's loads, and nine registers more, forwards of mixed types took 88 instead of
-// 82 us at 32 x 4096 x 128, groups of 16.)
+// 85 us at 32 x 4096 x 128, groups of 16.)
 template <int F>
 __device__ __forceinline__ void issue_w(const StageArgs& A, int head, int ec, int fl, float (&wi)[F], float (&wj)[F]) {
     const int log2_size = A.w_bf16 ? 1 : 2, second = A.w_bf16 ? 0 : 8;
