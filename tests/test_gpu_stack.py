@@ -59,6 +59,39 @@ def test_stack(M, case, ranges, dtype):
             assert dW.dtype == dtype and O.rel_err(dW[l], r[4][l].reshape(-1)) < tol, l
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("batch,N,E,C,n,L", [(16, 2048, 128, 4, 4, 6),     # multi-stage passes
+                                             (16, 2046, 128, 4, 2, 13)])   # an odd number of groups: one launch per stage
+@pytest.mark.parametrize("how", ["no_grad", "no_leaf"])
+def test_no_activations_are_kept_without_gradients(M, batch, N, E, C, n, L, dtype, how):
+    """The whole-net node under no_grad, or on tensors that want no gradient: nothing is kept for a backward.  At most a pair
+    for the outputs, a float32 pair that the passes end in and one that they run through; the training plan of the second
+    shape keeps 13 pairs."""
+    from ncn_cuda_amd.modules import fused_ncn_net
+    x, xa, Ws, _, _ = O.make_inputs(batch, N, E, L, n, seed=5, xa_zero=False, dtype=dtype)
+    ref = O.net_forward(x.double(), xa.double(), [w.double() for w in Ws], 0.9, n, C)
+    x, xa, Ws = x.cuda(), xa.cuda(), [w.cuda().requires_grad_(how == "no_grad") for w in Ws]
+
+    def run():
+        if how == "no_leaf":
+            return fused_ncn_net(x, xa, Ws, 0.9, 0, n, C)
+        with torch.no_grad():
+            return fused_ncn_net(x, xa, Ws, 0.9, 0, n, C)
+
+    run()
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    y, ya = run()
+    peak = torch.cuda.max_memory_allocated() - before
+    pair = 2 * x.numel()
+    assert peak <= pair * (4 + 4 + (2 if dtype == torch.bfloat16 else 0)) + (1 << 20)
+    assert not y.requires_grad and y.dtype == dtype
+    # float32: rounding of the sums, 13 stages at most; bfloat16: the outputs are rounded once
+    tol = 2e-6 if dtype == torch.float32 else 2.0 ** -8
+    assert O.rel_err(y, ref[0]) < tol and O.rel_err(ya, ref[1]) < tol
+
+
 def test_refusals(M):
     """Outputs that are the inputs, a workspace that is too small: refused before any launch."""
     from ncn_cuda_amd import _lib
