@@ -515,20 +515,54 @@ __device__ __forceinline__ int dtype_of(int from_args, int when_bf16) {
     return TYPES == kF32Types ? NCN_F32 : TYPES == kBf16Types ? when_bf16 : from_args;
 }
 
-// Rows past a context length take no part in the stage: they pass through, stored as they were loaded.  (A launch of
-// its own for them, one element per lane, cost 38 us per stage and direction on 32 x 4096 x 128 bfloat16 with a quarter
-// of the rows past their lengths, 0.22 of the 0.89 ms of a three-stage training step.)
-#define NCN_PASS_DEAD_ROWS(base0, base1, dtype, p, q)                                           \
-    if (INDEXED && __any(live >= 0 && live < NC)) {                                             \
+// Rows past a context length take no part in the stage: they pass through.  (A launch of its own for them, one element per
+// lane, cost 38 us per stage and direction on 32 x 4096 x 128 bfloat16 with a quarter of the rows past their lengths, 0.22 of
+// the 0.89 ms of a three-stage training step.)  The builds for one type store them as they were loaded.  In the builds for
+// every type that costs registers in every wave, with and without such rows: there they are read again behind the tile's own
+// stores (backward of relu behind a table, float32, 32 x 2048 x 256, groups of 16 rows, heads of 64 features: 598 against 338 us).
+#define NCN_STORE_DEAD_ROWS(base0, base1, dtype, p, q)                                          \
+    if (INDEXED && TYPES != kAnyTypes && A.ctx_len && __any(live >= 0 && live < NC)) {          \
         _Pragma("unroll") for (int rr = 0; rr < R; ++rr) {                                      \
             const bool dead = live >= 0 && !NCN_ROW_LIVE(rr);                                   \
             store_frag<F>(base0, dtype, off[rr], dead, p[rr], A.plane);                         \
             store_frag<F>(base1, dtype, off[rr], dead, q[rr], A.plane);                         \
         }                                                                                       \
     }
+struct PassPair {   // in0, in1 (null: zeros) -> out0, out1 (null: nothing)
+    const void *in0, *in1;
+    int in_dtype;
+    void *out0, *out1;
+    int out_dtype;
+};
+// A row is read before it is written: outputs may be the inputs, as for the rows that take part.
+template <int R, int F>
+__device__ __forceinline__ void pass_rows(const int64_t (&off)[R], const bool (&dead)[R], int64_t plane, const PassPair& p, const PassPair& q) {
+#pragma unroll
+    for (int rr = 0; rr < R; ++rr) {
+        float p0[F], p1[F], q0[F], q1[F];
+        load_frag<F>(p.in0, p.in_dtype, off[rr], dead[rr], p0, plane);
+        load_frag<F>(p.in1, p.in_dtype, off[rr], dead[rr] && p.in1, p1, plane);
+        load_frag<F>(q.in0, q.in_dtype, off[rr], dead[rr] && q.out0, q0, plane);
+        load_frag<F>(q.in1, q.in_dtype, off[rr], dead[rr] && q.out0, q1, plane);
+        store_frag<F>(p.out0, p.out_dtype, off[rr], dead[rr], p0, plane);
+        store_frag<F>(p.out1, p.out_dtype, off[rr], dead[rr], p1, plane);
+        store_frag<F>(q.out0, q.out_dtype, off[rr], dead[rr] && q.out0, q0);
+        store_frag<F>(q.out1, q.out_dtype, off[rr], dead[rr] && q.out0, q1);
+        __builtin_amdgcn_sched_barrier(0);   // one row in registers at a time
+    }
+}
+#define NCN_PASS_DEAD_ROWS(p, q)                                                                \
+    if (INDEXED && TYPES == kAnyTypes && A.ctx_len && __any(live >= 0 && live < NC)) {          \
+        bool dead[R];                                                                           \
+        _Pragma("unroll") for (int rr = 0; rr < R; ++rr) {                                      \
+            dead[rr] = live >= 0 && !NCN_ROW_LIVE(rr);                                          \
+            asm volatile("" : "+v"(off[rr]));   /* or the addresses of the loads stay in registers until here */ \
+        }                                                                                       \
+        pass_rows<R, F>(off, dead, A.plane, p, q);                                              \
+    }
 
 template <int NC, int EC, int R, int F, bool TANH_ONLY = true, bool INDEXED = false, int TYPES = kAnyTypes>
-__global__ void __launch_bounds__(kBlockThreads, (TANH_ONLY && !INDEXED && R == 4 && F == 4) ? 5 : 1) stage_forward_kernel(const StageArgs A) {
+__global__ void __launch_bounds__(kBlockThreads, (R == 4 && F == 4) ? 5 : 1) stage_forward_kernel(const StageArgs A) {
     NCN_WAVE_PROLOGUE
     issue_w<F>(A, head, EC, fl, wi, wj);
     const int in_dtype = dtype_of<TYPES>(A.in_dtype, NCN_BF16);
@@ -542,8 +576,8 @@ __global__ void __launch_bounds__(kBlockThreads, (TANH_ONLY && !INDEXED && R == 
         NCN_FINISH_W_ONCE
         finish_tile<R, F>(in_dtype, x);
         finish_tile<R, F>(in_dtype, a);
-        NCN_PASS_DEAD_ROWS(A.out0, A.out1, out_dtype, x, a)
-        if (A.aux0) { NCN_PASS_DEAD_ROWS(A.aux0, A.aux1, NCN_F32, x, a) }
+        NCN_STORE_DEAD_ROWS(A.out0, A.out1, out_dtype, x, a)
+        if (A.aux0) { NCN_STORE_DEAD_ROWS(A.aux0, A.aux1, NCN_F32, x, a) }
         NCN_ZERO_DEAD_ROWS(x, a, true)
         scale_tile<R, F>(x, a, A.tab.kappa, A.tab.a_scale);
         forward_core<NC, EC, R, F, TANH_ONLY, INDEXED>(x, a, wi, wj, A.tab, lane, slots, live);
@@ -558,11 +592,13 @@ __global__ void __launch_bounds__(kBlockThreads, (TANH_ONLY && !INDEXED && R == 
                 store_frag<F>(A.aux1, NCN_F32, off[rr], valid, a[rr]);
             }
         }
+        NCN_PASS_DEAD_ROWS((PassPair{A.in0, A.in1, in_dtype, A.out0, A.out1, out_dtype}),
+                           (PassPair{A.in0, A.in1, in_dtype, A.aux0, A.aux1, NCN_F32}))
     }
 }
 
 template <int NC, int EC, int R, int F, bool TANH_ONLY = true, bool INDEXED = false, int TYPES = kAnyTypes>
-__global__ void __launch_bounds__(kBlockThreads) stage_inverse_kernel(const StageArgs A) {
+__global__ void __launch_bounds__(kBlockThreads, (R == 4 && F == 4) ? 5 : 1) stage_inverse_kernel(const StageArgs A) {
     NCN_WAVE_PROLOGUE
     issue_w<F>(A, head, EC, fl, wi, wj);
     const int in_dtype = dtype_of<TYPES>(A.in_dtype, NCN_BF16), out_dtype = dtype_of<TYPES>(A.out_dtype, NCN_BF16);
@@ -575,7 +611,7 @@ __global__ void __launch_bounds__(kBlockThreads) stage_inverse_kernel(const Stag
         NCN_FINISH_W_ONCE
         finish_tile<R, F>(in_dtype, y);
         finish_tile<R, F>(in_dtype, b);
-        NCN_PASS_DEAD_ROWS(A.out0, A.out1, out_dtype, y, b)
+        NCN_STORE_DEAD_ROWS(A.out0, A.out1, out_dtype, y, b)
         NCN_ZERO_DEAD_ROWS(y, b, true)
         scale_tile<R, F>(y, b, A.tab.kappa, A.tab.b_scale);
         inverse_core<NC, EC, R, F, TANH_ONLY, INDEXED>(y, b, wi, wj, A.tab, lane, slots, live);
@@ -586,6 +622,7 @@ __global__ void __launch_bounds__(kBlockThreads) stage_inverse_kernel(const Stag
             store_frag<F>(A.out0, out_dtype, off[rr], valid, y[rr]);
             store_frag<F>(A.out1, out_dtype, off[rr], valid, b[rr]);
         }
+        NCN_PASS_DEAD_ROWS((PassPair{A.in0, A.in1, in_dtype, A.out0, A.out1, out_dtype}), (PassPair{}))
     }
 }
 
@@ -595,10 +632,10 @@ __global__ void __launch_bounds__(kBlockThreads) stage_inverse_kernel(const Stag
 // offsets are not carried in registers across it (the loop build spills 6 of them per lane at R x F = 16, which a
 // launch bound by its traffic pays for), and the steps come out in an order that issues better.
 template <int NC, int EC, int R, int F, bool TANH_ONLY = true, bool INDEXED = false, bool LOOP = true, int TYPES = kAnyTypes>
-__global__ void __launch_bounds__(kBlockThreads, (TANH_ONLY && R * F <= 16 && F == 4) ? 4 : (TYPES != kAnyTypes && R * F == 32) ? 2 : 1) stage_backward_kernel(const StageArgs A) {
+__global__ void __launch_bounds__(kBlockThreads, (TANH_ONLY && R * F <= 16 && F == 4) ? 4 : ((TYPES != kAnyTypes || (INDEXED && (TANH_ONLY || !LOOP))) && R * F == 32) ? 2 : 1) stage_backward_kernel(const StageArgs A) {
     NCN_WAVE_PROLOGUE
-    // the builds for one type keep nothing in registers while the tile is loaded: they are at their limit of registers
-    constexpr bool kEarlyW = LOOP || TYPES == kAnyTypes;
+    // the builds without a loop keep nothing in registers while the tile is loaded: at their limit of registers, they spill
+    constexpr bool kEarlyW = LOOP;
     if constexpr (kEarlyW) issue_w<F>(A, head, EC, fl, wi, wj);
     const int in_dtype = dtype_of<TYPES>(A.in_dtype, NCN_BF16X2), g_dtype = dtype_of<TYPES>(A.g_dtype, NCN_BF16);
     const int out_dtype = dtype_of<TYPES>(A.out_dtype, NCN_BF16);
@@ -631,8 +668,8 @@ __global__ void __launch_bounds__(kBlockThreads, (TANH_ONLY && R * F <= 16 && F 
         finish_tile<R, F>(in_dtype, B);
         finish_tile<R, F>(g_dtype, G);
         if (A.g1) finish_tile<R, F>(g_dtype, H);
-        NCN_PASS_DEAD_ROWS(A.out0, A.out1, out_dtype, G, H)
-        if (A.aux0) { NCN_PASS_DEAD_ROWS(A.aux0, A.aux1, NCN_F32, Y, B) }
+        NCN_STORE_DEAD_ROWS(A.out0, A.out1, out_dtype, G, H)
+        if (A.aux0) { NCN_STORE_DEAD_ROWS(A.aux0, A.aux1, NCN_F32, Y, B) }
         NCN_ZERO_DEAD_ROWS(Y, B, false)
         NCN_ZERO_DEAD_ROWS(G, H, false)
         backward_steps<NC, EC, R, F, false, TANH_ONLY, INDEXED>(Y, B, G, H, wi, wj, dwi, dwj, 1.0f, A.tab, lane, slots,
@@ -652,6 +689,8 @@ __global__ void __launch_bounds__(kBlockThreads, (TANH_ONLY && R * F <= 16 && F 
                 store_frag<F>(A.aux1, NCN_F32, off[rr], valid, B[rr]);
             }
         }
+        NCN_PASS_DEAD_ROWS((PassPair{A.g0, A.g1, g_dtype, A.out0, A.out1, out_dtype}),
+                           (PassPair{A.in0, A.in1, in_dtype, A.aux0, A.aux1, NCN_F32}))
     } while (LOOP && (t += tile_step) < A.total_tiles);
 
     // dW: lanes holding the same feature chunk -> one value; this wave owns slot (gwave / n_head, head).
@@ -671,6 +710,7 @@ __global__ void __launch_bounds__(kBlockThreads, (TANH_ONLY && R * F <= 16 && F 
 }
 #undef NCN_ROW_LIVE
 #undef NCN_ZERO_DEAD_ROWS
+#undef NCN_STORE_DEAD_ROWS
 #undef NCN_PASS_DEAD_ROWS
 #undef NCN_FINISH_W_ONCE
 #undef NCN_WAVE_PROLOGUE
