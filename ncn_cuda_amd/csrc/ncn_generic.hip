@@ -219,10 +219,11 @@ __global__ void __launch_bounds__(64) generic_backward_kernel(const StageArgs A)
 // its wave and the block's 16 waves are summed, all in a fixed order.  Bound by the latency of its few rounds of loads.
 // Workgroups go round the XCDs in turn, so the four blocks that share the 128-byte lines of 32 columns are numbered
 // eight apart: their lines are fetched into one L2 instead of four (16384 x 256: 10 against 34 us).
-// Against the two launches below, back to back: 2.4 : 4.8 us up to 1024 rows, 4.1 : 5.0 at 4096 x 256, 5.1 : 5.4 at
-// 6144 x 256, 6.2 : 7.5 at 4096 x 1792 and 12.2 : 11.1 at 6144 x 1792, 10 : 7.7 at 16384 x 256 -- hence up to
-// kReduceOneLaunchRows.
-constexpr int kReduceColumns = 8, kReduceOneLaunchRows = 4096;
+// Against the two launches below, a backward call of one stage, whose partial rows other XCDs have just written: 1024 rows
+// (8 x 4096 x 128, groups of 16, bfloat16) 48.9 : 50.7 us, 2048 rows (16 x 4096 x 128) 80.6 : 81.1, 4096 rows (32 x 2048 x 128,
+// groups of 4) 39.0 : 37.0 -- hence up to kReduceOneLaunchRows.  (Launched again and again on rows that lie in L2 it is ahead up
+// to 4096 rows.)
+constexpr int kReduceColumns = 8, kReduceOneLaunchRows = 2048;
 __device__ __forceinline__ uint32_t reduce_column_block(uint32_t x, uint32_t n) {
     const uint32_t base = x & ~31u;
     return base + 32u <= n ? base + (x & 7u) * 4u + (x >> 3 & 3u) : x;

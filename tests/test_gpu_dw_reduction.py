@@ -1,4 +1,4 @@
-"""Sum of the dW partial rows: one launch up to 4096 rows, two beyond; row counts around its block of 128 rows and around
+"""Sum of the dW partial rows: one launch up to 2048 rows, two beyond; row counts around its block of 128 rows and around
 the switch, column counts that end inside a block of 8 columns or fill blocks of 32 (numbered for the XCDs)."""
 import pytest
 import torch
@@ -17,7 +17,7 @@ def M():
 
 
 # (batch entries = wave tiles of a single head = partial rows, E, heads): 2E columns
-CASES = [(1, 4, 1), (127, 4, 1), (132, 4, 1), (4096, 4, 1), (4100, 4, 1), (3, 15, 3), (5, 64, 2), (260, 128, 4), (4097, 15, 3)]
+CASES = [(1, 4, 1), (127, 4, 1), (132, 4, 1), (2048, 4, 1), (2049, 15, 3), (2052, 4, 1), (4096, 4, 1), (4100, 4, 1), (3, 15, 3), (5, 64, 2), (260, 128, 4), (4097, 15, 3)]
 
 
 @pytest.mark.parametrize("batch,E,C", CASES)
