@@ -21,9 +21,9 @@
 
 namespace ncn {
 
-// sums over the lanes {lane ^ k * 2^LO : k} for the levels LO <= level < HI, LO = 0 or (FROM0 = false) `lo`
+// Sums across lanes, the levels (lane bits) known at run time and the same for the wave: over the 2^hi lanes of a row ..
 template <int N>
-__device__ __forceinline__ void any_sum_rows(float (&v)[N], int hi) {   // over the 2^hi lanes of a row
+__device__ __forceinline__ void any_sum_rows(float (&v)[N], int hi) {
 #define NCN_LEVEL(S)                                                    \
     _Pragma("unroll") for (int k = 0; k < N; ++k) v[k] += lane_xor<S, true>(v[k]);
     if (hi > 0) {
@@ -40,8 +40,9 @@ __device__ __forceinline__ void any_sum_rows(float (&v)[N], int hi) {   // over 
         }
     }
 }
+// .. and over the lanes that differ in the bits lo .. hi-1
 template <int N>
-__device__ __forceinline__ void any_sum_span(float (&v)[N], int lo, int hi) {   // over lane bits lo .. hi-1
+__device__ __forceinline__ void any_sum_span(float (&v)[N], int lo, int hi) {
     if (lo >= hi) return;
     if (lo <= 0) { NCN_LEVEL(1) }
     if (lo <= 1 && hi > 1) { NCN_LEVEL(2) }
@@ -128,13 +129,18 @@ __device__ __forceinline__ void any_finish(int dtype, float (&v)[R][F]) {
 #pragma unroll
         for (int f = 0; f < F; ++f) v[rr][f] = __uint_as_float(__float_as_uint(v[rr][f]) << 16);
 }
+// Rows that do not run become zero, features that do not exist `missing`: zero, or for x (y), which every row sum multiplies,
+// any other number.  Their weights are zero, so they add nothing to a sum; but an infinite sum times zero would be NaN, which
+// the next sum spreads over the row, where times one it saturates the activation as it does in the features that exist.
 template <int R, int F, bool LENGTHS>
-__device__ __forceinline__ void any_zero_padding(const AnyLane<R, F, LENGTHS>& L, float (&v)[R][F]) {
+__device__ __forceinline__ void any_fill_padding(const AnyLane<R, F, LENGTHS>& L, float (&v)[R][F], float missing = 0.f) {
 #pragma unroll
     for (int rr = 0; rr < R; ++rr)
 #pragma unroll
-        for (int f = 0; f < F; ++f) v[rr][f] = L.run(rr) && L.has[f] ? v[rr][f] : 0.f;
+        for (int f = 0; f < F; ++f) v[rr][f] = !L.run(rr) ? 0.f : L.has[f] ? v[rr][f] : missing;
 }
+// for a tile whose steps are undone, which multiplies by 1/m each time: where (1/m)^n would leave the range of float32, zero
+__device__ __forceinline__ float any_missing_undone(const StepTable& S) { return S.m_pow_n > 1e-30f ? 1.f : 0.f; }
 // both arrays of a pair, the rows that take part in the steps (DEAD = false) or those that pass through
 template <bool DEAD, int R, int F, bool LENGTHS>
 __device__ __forceinline__ void any_store(const StageArgs& A, const AnyLane<R, F, LENGTHS>& L, void* base0, void* base1, int dtype,
@@ -229,8 +235,8 @@ __global__ void __launch_bounds__(kBlockThreads, R * F <= 16 ? 4 : R * F <= 20 ?
             any_store<true>(A, L, A.out0, A.out1, A.out_dtype, x, a);
             if (!INVERSE && A.aux0) any_store<true>(A, L, A.aux0, A.aux1, NCN_F32, x, a);
         }
-        any_zero_padding(L, x);
-        any_zero_padding(L, a);
+        any_fill_padding(L, x, INVERSE ? any_missing_undone(S) : 1.f);
+        any_fill_padding(L, a);
         scale_tile<R, F>(x, a, S.kappa, INVERSE ? S.b_scale : S.a_scale);
 #pragma unroll 1
         for (int k = 0; k < lr; ++k) {
@@ -305,10 +311,10 @@ __global__ void __launch_bounds__(kBlockThreads, R * F <= 10 ? 4 : R * F <= 16 ?
             any_store<true>(A, L, A.out0, A.out1, A.out_dtype, G, P);
             if (A.aux0) any_store<true>(A, L, A.aux0, A.aux1, NCN_F32, Y, B);
         }
-        any_zero_padding(L, Y);
-        any_zero_padding(L, B);
-        any_zero_padding(L, G);
-        any_zero_padding(L, P);
+        any_fill_padding(L, Y, any_missing_undone(S));
+        any_fill_padding(L, B);
+        any_fill_padding(L, G);
+        any_fill_padding(L, P);
         // as if the steps that a group cut by a context length skips had been done: G, P carry m^-t
         const float isc = LENGTHS && L.live < A.n_cache ? pow_steps(S.im, A.n_cache - L.live) : 1.0f;
 #pragma unroll

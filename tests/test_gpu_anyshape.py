@@ -90,6 +90,29 @@ def test_table_and_lengths(M, case):
     assert torch.equal(dx[0].cpu(), dy[0]) and torch.equal(xr[0].cpu(), x[0])
 
 
+@pytest.mark.parametrize("value", [float("inf"), -float("inf")])
+@pytest.mark.parametrize("n,ec,C", [(5, 7, 2), (3, 7, 3), (12, 22, 2), (4, 18, 2)])   # heads that end inside their tile
+def test_infinite_inputs(M, n, ec, C, value):
+    """An infinite input makes row sums infinite, which saturate tanh: where the oracle's results are finite so are the
+    kernel's, although the features that pad a tile see the same sums (zero times them would be NaN)."""
+    d, group = torch.float64, slice(0, n)   # stage 0: the group of the infinite value
+    for seed in range(40):   # most weights make the sum NaN at once: inf - inf
+        x, xa, Ws, _, _ = O.make_inputs(2, n * 4, ec * C, 1, n, seed=seed, xa_zero=False)
+        x[:, 2, 1] = value
+        ref = O.net_forward(x.to(d), xa.to(d), [Ws[0].to(d)], 0.9, n, C)
+        finite = torch.isfinite(ref[1][:, group, :ec])
+        if finite.float().mean() > 0.5 and not finite.all():
+            break
+    assert finite.any() and not finite.all()
+    W = Ws[0].cuda()
+    y, ya = M.forward_stages(x.cuda(), xa.cuda(), W, 0.9, 0, n, C, 0, 1)
+    for a, b in ((y, ref[0]), (ya, ref[1])):
+        a, b = a.cpu()[:, group, :ec].to(d), b[:, group, :ec]
+        assert torch.equal(torch.isfinite(a), torch.isfinite(b))
+        ok = torch.isfinite(b)
+        assert (a - b)[ok].norm() < TOL * b[ok].norm()
+
+
 @pytest.mark.parametrize("case", [CASES[3], CASES[4]], ids=lambda c: "n%d_e%d_C%d_g%d_b%d" % c)
 def test_bfloat16(M, case):
     n, ec, C, groups, batch = case
