@@ -352,21 +352,49 @@ class StackPlan:
         self.forward_bytes, self.backward_bytes = out[0], out[1]
 
 
+# Kept activations past this size are held to a quarter of the device memory that torch has not handed out.
+_SAVES_LOOK_AT_MEMORY = 1 << 30
+
+
+def _saves_within(budget, wanted, dev):
+    """Bytes that a stack which would like to keep `wanted` may keep."""
+    if min(budget, wanted) <= _SAVES_LOOK_AT_MEMORY:
+        return budget
+    left = torch.cuda.get_device_properties(dev).total_memory - torch.cuda.memory_allocated(dev)
+    return min(budget, max(left // 4, 0))
+
+
 def stack_forward(x, xa, W, alpha, activation, cache_dim, nhead, first_stage, n_stages, max_range, save_budget, *, m=M_DEFAULT):
     """The forward of a stack that will be trained: (plan, y, ya, saves), y and ya in the dtype of x, `saves` the float32
     activations that stack_backward reads beside (float32) or in place of (bfloat16) y, ya; at most max_range stages lie
-    between two of them.  save_budget bounds their bytes where max_range leaves a choice.  None: no such plan."""
+    between two of them.  save_budget bounds their bytes where max_range leaves a choice; so do, past 1 GiB, a quarter of the
+    memory that is not allocated, and an allocation that fails: the plan with the fewest kept activations is then taken.  None: no
+    such plan."""
     shape = validate(x, xa, W, cache_dim, nhead, activation, first_stage, n_stages, alpha=alpha, m=m)
     dev = _require_gpu(x, xa, W)
-    max_saves = max(int(save_budget) // (8 * x.numel()), -(-int(n_stages) // int(max_range)))
-    plan = StackPlan(shape, first_stage, n_stages, alpha, m, activation, max_range, min(max_saves, int(n_stages)), x.dtype)
+    pair, fewest = 8 * x.numel(), -(-int(n_stages) // int(max_range))
+    max_saves = min(max(_saves_within(int(save_budget), pair * int(n_stages), dev) // pair, fewest), int(n_stages))
+    plan = StackPlan(shape, first_stage, n_stages, alpha, m, activation, max_range, max_saves, x.dtype)
     if plan.ranges <= 0:
         return None
     x, xa, (w, wflag) = _prep(x.detach()), _prep(xa.detach()), _weights(W)
     y, ya = torch.empty(x.shape, dtype=x.dtype, device=dev), torch.empty(x.shape, dtype=x.dtype, device=dev)
-    kept = plan.ranges - (x.dtype == torch.float32)
-    saves = torch.empty((kept, 2) + tuple(x.shape), dtype=torch.float32, device=dev) if kept else None
-    ws = torch.empty(plan.forward_bytes, dtype=torch.uint8, device=dev) if plan.forward_bytes else None
+
+    def scratch(plan):
+        kept = plan.ranges - (x.dtype == torch.float32)
+        saves = torch.empty((kept, 2) + tuple(x.shape), dtype=torch.float32, device=dev) if kept else None
+        return saves, torch.empty(plan.forward_bytes, dtype=torch.uint8, device=dev) if plan.forward_bytes else None
+
+    got = None
+    try:
+        got = scratch(plan)
+    except torch.OutOfMemoryError:
+        if max_saves <= fewest:
+            raise
+    if got is None:   # (past the except clause, which holds on to what was allocated)
+        plan = StackPlan(shape, first_stage, n_stages, alpha, m, activation, max_range, fewest, x.dtype)
+        got = scratch(plan)
+    saves, ws = got
     with torch.cuda.device(dev):
         rc = _lib.load().ncn_stack_forward(_ptr(x), _ptr(xa), _DTYPES[x.dtype] | wflag, _ptr(y), _ptr(ya), _DTYPES[x.dtype],
                                            _ptr(saves), _ptr(w), _ptr(ws), ctypes.c_size_t(plan.forward_bytes),

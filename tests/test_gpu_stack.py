@@ -92,6 +92,46 @@ def test_no_activations_are_kept_without_gradients(M, batch, N, E, C, n, L, dtyp
     assert O.rel_err(y, ref[0]) < tol and O.rel_err(ya, ref[1]) < tol
 
 
+@pytest.mark.parametrize("why", ["little_left", "allocation_fails"])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+def test_fewer_activations_are_kept_where_memory_is_short(M, monkeypatch, dtype, why):
+    """A stack that would keep every stage's outputs keeps the fewest when little device memory is left, or when the
+    allocation fails; its gradients are as good."""
+    batch, N, E, C, n, L = 2, 1018, 64, 2, 2, 13     # 509 groups: one launch per stage
+    x, xa, Ws, dy, dya = O.make_inputs(batch, N, E, L, n, seed=1, xa_zero=False, dtype=dtype)
+    d = torch.float64
+    ref = O.net_autograd(x.to(d), xa.to(d), [w.to(d) for w in Ws], dy.to(d), dya.to(d), 0.9, n, C)
+    W = torch.stack([w.reshape(-1) for w in Ws]).cuda()
+    x, xa, dy, dya = x.cuda(), xa.cuda(), dy.cuda(), dya.cuda()
+    call = lambda: M.stack_forward(x, xa, W, 0.9, 0, n, C, 0, L, 13, 32 << 30)
+    assert call()[0].ranges == L
+    failed = []
+    if why == "little_left":
+        monkeypatch.setattr(M, "_SAVES_LOOK_AT_MEMORY", 0)
+        total = torch.cuda.get_device_properties(x.device).total_memory
+        monkeypatch.setattr(torch.cuda, "memory_allocated", lambda dev=None: total - 16 * x.numel())
+    else:
+        real = torch.empty
+
+        def empty(*size, **kw):
+            if len(size) == 1 and isinstance(size[0], tuple) and len(size[0]) == 5 and size[0][0] > 1:
+                failed.append(size[0])
+                raise torch.OutOfMemoryError("no memory")
+            return real(*size, **kw)
+
+        monkeypatch.setattr(torch, "empty", empty)
+    plan, y, ya, saves = call()
+    assert plan.ranges == 1 and (saves is None if dtype == torch.float32 else saves.shape[0] == 1)
+    assert bool(failed) == (why == "allocation_fails")
+    kept = (y, ya) if dtype == torch.float32 else (None, None)
+    dx, dxa, dW = M.stack_backward(plan, *kept, saves, dy, dya, W)
+    tol = 1.2e-6 * 0.9 ** -(n * L) if dtype == torch.float32 else 2.0 ** -8   # as in test_stack
+    for got, want in ((y, ref[0]), (ya, ref[1]), (dx, ref[2]), (dxa, ref[3])):
+        assert O.rel_err(got, want) < tol
+    for l in range(L):
+        assert O.rel_err(dW[l], ref[4][l].reshape(-1)) < tol
+
+
 def test_refusals(M):
     """Outputs that are the inputs, a workspace that is too small: refused before any launch."""
     from ncn_cuda_amd import _lib
