@@ -2,6 +2,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <mutex>
 
@@ -1168,14 +1169,15 @@ struct StackCall {
     ncn_shape as_wide;
     const ncn_shape* shape;
     bool headwise;
-    std::vector<StackRange> ranges;
+    const std::vector<StackRange>* ranges;   // of this thread's kept plans
     size_t plane;        // one float32 activation array
     int fwd_passes_max;  // passes of the longest range
     int bwd_passes_max, bwd_passes;
     int row_cap;         // rows of the dW partial buffer
 
     // false: no such cut, or kernels without this entry (the caller uses ncn_forward and ncn_backward).  A program asks for
-    // the same stack step after step: the last plan of a thread is kept, it depends on sizes only.
+    // the same few stacks step after step: a thread keeps the last kKeptPlans plans, which depend on sizes only.
+    static constexpr unsigned kKeptPlans = 8;
     bool plan(const ncn_shape* sh, int first, int count, int activation, float alpha, float m, int max_range, int max_saves) {
         const int path = kernel_path_for(sh, activation, alpha, m);
         // (the tables of plan_stack grow with the square of the stages)
@@ -1186,29 +1188,28 @@ struct StackCall {
         headwise = headwise_call(sh, path, &as_wide);
         shape = headwise ? &as_wide : sh;
         const bool multi = fused_supported(shape, activation);
+        using Key = std::array<int64_t, 10>;
         struct Kept {
-            int64_t batch = 0, N = 0, E = 0;
-            int n_head = 0, n_cache = 0, first = 0, count = 0, multi = 0, max_range = 0, max_saves = 0;
+            Key key{};   // N = 0: nothing kept
             std::vector<StackRange> ranges;
         };
-        thread_local Kept kept;
-        if (kept.batch != shape->batch || kept.N != shape->N || kept.E != shape->E || kept.n_head != shape->n_head ||
-            kept.n_cache != shape->n_cache || kept.first != first || kept.count != count || kept.multi != (int)multi ||
-            kept.max_range != max_range || kept.max_saves != max_saves) {
-            kept.batch = 0;   // not valid while it changes
-            kept.ranges = plan_stack(shape, first, count, multi, max_range, max_saves);
-            kept.N = shape->N; kept.E = shape->E; kept.n_head = shape->n_head; kept.n_cache = shape->n_cache;
-            kept.first = first; kept.count = count; kept.multi = multi;
-            kept.max_range = max_range; kept.max_saves = max_saves;
-            kept.batch = shape->batch;
+        thread_local std::array<Kept, kKeptPlans> kept;
+        thread_local unsigned next = 0;
+        const Key key{shape->batch, shape->N, shape->E, shape->n_head, shape->n_cache, first, count, multi, max_range, max_saves};
+        Kept* found = std::find_if(kept.begin(), kept.end(), [&](const Kept& k) { return k.key == key; });
+        if (found == kept.end()) {
+            found = &kept[next++ % kKeptPlans];
+            found->key = Key{};   // not valid while it changes
+            found->ranges = plan_stack(shape, first, count, multi, max_range, max_saves);
+            found->key = key;
         }
-        ranges = kept.ranges;
-        if (ranges.empty()) return false;
+        ranges = &found->ranges;
+        if (ranges->empty()) return false;
         plane = temp_bytes(shape, false) / 2;
         fwd_passes_max = bwd_passes_max = bwd_passes = 0;
         int64_t rows = 0;
         const Plan single = make_plan(shape, 2, AnyTile{0, 0, 0, 0});
-        for (const StackRange& r : ranges) {
+        for (const StackRange& r : *ranges) {
             if ((int)r.fwd.size() > fwd_passes_max) fwd_passes_max = (int)r.fwd.size();
             if ((int)r.bwd.size() > bwd_passes_max) bwd_passes_max = (int)r.bwd.size();
             bwd_passes += (int)r.bwd.size();
@@ -1239,7 +1240,7 @@ int ncn_stack_plan(const ncn_shape* shape, int first_stage, int n_stages, float 
     if (!c.plan(shape, first_stage, n_stages, activation, alpha, m, max_range, max_saves)) return 0;
     out[0] = (int64_t)c.forward_bytes();
     out[1] = (int64_t)c.backward_bytes(grad_dtype == NCN_F32);
-    return (int)c.ranges.size();
+    return (int)c.ranges->size();
 }
 
 int ncn_stack_forward(const void* x, const void* xa, int in_dtype, void* y, void* ya, int out_dtype, float* saves,
@@ -1257,7 +1258,7 @@ int ncn_stack_forward(const void* x, const void* xa, int in_dtype, void* y, void
     StackCall c;
     if (!c.plan(shape, first_stage, n_stages, activation, alpha, m, max_range, max_saves)) return NCN_ERR_UNSUPPORTED;
     shape = c.shape;
-    const size_t nr = c.ranges.size();
+    const size_t nr = c.ranges->size();
     if ((nr > 1 || out_dtype != NCN_F32) && !saves) return NCN_ERR_NULL;
     if (c.forward_bytes() && (!workspace || workspace_bytes < c.forward_bytes())) return NCN_ERR_WORKSPACE;
     const Plan p = make_plan(shape, 2, AnyTile{0, 0, 0, 0});
@@ -1272,7 +1273,7 @@ int ncn_stack_forward(const void* x, const void* xa, int in_dtype, void* y, void
         const bool last_range = r + 1 == nr;
         void* kept0 = last_range && out_dtype == NCN_F32 ? y : saves + (int64_t)(2 * r) * elements;
         void* kept1 = last_range && out_dtype == NCN_F32 ? ya : saves + (int64_t)(2 * r + 1) * elements;
-        const std::vector<FusedPass>& passes = c.ranges[r].fwd;
+        const std::vector<FusedPass>& passes = (*c.ranges)[r].fwd;
         const size_t np = passes.size();
         for (size_t k = 0; k < np; ++k) {
             const FusedPass& ps = passes[k];
@@ -1324,7 +1325,7 @@ int ncn_stack_backward(const float* y, const float* ya, const float* saves, cons
     StackCall c;
     if (!c.plan(shape, first_stage, n_stages, activation, alpha, m, max_range, max_saves)) return NCN_ERR_UNSUPPORTED;
     shape = c.shape;
-    const size_t nr = c.ranges.size();
+    const size_t nr = c.ranges->size();
     if ((nr > 1 || !y) && !saves) return NCN_ERR_NULL;
     if (!workspace || workspace_bytes < c.backward_bytes(dx_dtype == NCN_F32)) return NCN_ERR_WORKSPACE;
     const Plan p = make_plan(shape, 2, AnyTile{0, 0, 0, 0});
@@ -1341,7 +1342,7 @@ int ncn_stack_backward(const float* y, const float* ya, const float* saves, cons
         const bool from_y = r + 1 == nr && y;
         const void* cy = from_y ? y : saves + (int64_t)(2 * r) * elements;
         const void* cya = from_y ? ya : saves + (int64_t)(2 * r + 1) * elements;
-        const std::vector<FusedPass>& passes = c.ranges[r].bwd;
+        const std::vector<FusedPass>& passes = (*c.ranges)[r].bwd;
         for (size_t k = passes.size(); k-- > 0;) {
             const FusedPass& ps = passes[k];
             --left;   // passes still to run: gradients travel in turns so that the last pass writes dx, dxa

@@ -419,6 +419,23 @@ def test_stack_plan_takes_bounds_of_any_size(lib, dims):
     assert plan(0, most)[0] == plan(-1, most)[0] == plan(most, 0)[0] == 0
 
 
+def test_stack_plans_of_several_nets_are_kept_apart(lib):
+    """More stacks than a thread keeps plans for, asked for in turn: every answer is that stack's own."""
+    h = lib.load()
+
+    def plan(n, L, N, saves):
+        out = (ctypes.c_int64 * 2)()
+        sh = _shape(lib, 2, N, 64, 2, n)
+        return h.ncn_stack_plan(ctypes.byref(sh), 0, L, 0.9, 0.9, 0, 26 // n, saves, 0, out), out[0], out[1]
+
+    asked = [(n, L, N, saves) for n in (2, 4) for L in (5, 9) for N in (1020, 2048, 4096) for saves in (3, 9)]
+    first = [plan(*a) for a in asked]
+    assert len(set(first)) > 8
+    assert [plan(*a) for a in asked] == first
+    for a, want in list(zip(asked, first))[::-1]:
+        assert plan(*a) == want == plan(*a)
+
+
 def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     """No fallback: if libncn_hip.so is absent and cannot be built, the binding raises instead of computing something
     else."""
