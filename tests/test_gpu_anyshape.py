@@ -8,25 +8,50 @@ from oracle import ncn_oracle as O
 
 pytestmark = pytest.mark.gpu
 
-# (n_cache, head width, heads, groups, batch): tile R x F, lanes per row x row lanes
+# (n_cache, head width, heads, groups, batch): tile R x F, lanes per row x row lanes (as _tile says)
 CASES = [
     (3, 3, 3, 7, 3),     # 3x3, 1x1, a wave tile of 64 groups, three heads
     (1, 5, 2, 70, 2),    # 2x5, 1x1, one row of two that exist
     (5, 1, 5, 1, 2),     # 5x3, 1x1, one feature of three; one group
     (6, 10, 1, 5, 4),    # 3x5, 2x2, one head
     (7, 40, 4, 3, 2),    # 2x5, 8x4, seven rows of eight
-    (4, 20, 2, 9, 2),    # power-of-two rows, 4x3 or 4x4 with padded features
+    (4, 20, 2, 9, 2),    # 2x5, 4x2, power-of-two rows, nothing padded
     (8, 12, 4, 4, 2),    # 4x3, 4x2
-    (9, 7, 2, 3, 2),     # 5x4 does not fit better: padded both ways
-    (10, 56, 2, 3, 2),   # 16 lanes per row
-    (13, 16, 2, 3, 2),   # power-of-two width, 13 rows
-    (16, 24, 3, 2, 2),   # three heads (a wave of the block works on the next tile)
+    (9, 7, 2, 3, 2),     # 3x4, 2x4, rows and features padded
+    (10, 56, 2, 3, 2),   # 3x4, 16x4
+    (13, 16, 2, 3, 2),   # 4x4, 4x4, power-of-two width, 13 rows of 16
+    (16, 24, 3, 2, 2),   # 4x3, 8x4, three heads (a wave of the block works on the next tile)
     (20, 56, 1, 2, 2),   # 5x4, 16x4: only a tile of 20 elements holds the group
     (20, 64, 1, 2, 1),   # 5x4, 16x4 exactly
     (48, 12, 1, 2, 1),   # 3x3, 4x16: every lane of the wave in one group
-    (24, 64, 1, 2, 1),   # 4x.. no tile: generic kernels
+    (2, 46, 1, 5, 2),    # 2x3, 16x1, 46 features of 48
+    (2, 7, 3, 41, 2),    # 2x4, 2x1, 32 groups to a wave tile
+    (25, 36, 1, 2, 1),   # 4x5, 8x8
+    (33, 36, 1, 2, 1),   # 5x5, 8x8: the largest tile, rows and features padded
+    (40, 40, 2, 1, 2),   # 5x5, 8x8 exactly
+    (24, 64, 1, 2, 1),   # no tile: generic kernels
 ]
 TOL = 1e-5
+
+
+def _tile(n, ec):
+    """The tile that any_tile() (csrc/ncn_launch.h) takes: (R, F, lanes per row, row lanes), or None."""
+    best = None
+    for r in range(2, 6):
+        for f in range(3, 6):
+            lf = max(0, (-(-ec // f) - 1).bit_length())
+            lr = max(0, (-(-n // r) - 1).bit_length())
+            if lf + lr > 6 or lf > 5:
+                continue
+            cost = ((20 * r * f + 4 * r * lf + 2 * f * lr + 10 * f) << (lf + lr)) * (4 if r * f > 16 else 1)
+            if best is None or cost < best[0]:
+                best = (cost, (r, f, 1 << lf, 1 << lr))
+    return best and best[1]
+
+
+def test_every_tile_has_a_case():
+    tiles = [_tile(n, ec) for n, ec, _, _, _ in CASES]
+    assert {t[:2] for t in tiles if t} == {(r, f) for r in range(2, 6) for f in range(3, 6)} and None in tiles
 
 
 def _tolerance(n):
@@ -69,25 +94,39 @@ def test_stage(M, case, act):
             assert O.rel_err(a, b) < rtol
 
 
-@pytest.mark.parametrize("case", [CASES[0], CASES[4], CASES[11]], ids=lambda c: "n%d_e%d_C%d_g%d_b%d" % c)
-def test_table_and_lengths(M, case):
+def _with(*shapes):
+    return [c for c in CASES if c[:2] in shapes]
+
+
+# the last one: the generic kernels, with their second launch for the groups that lengths cut and the rows passed through
+@pytest.mark.parametrize("case", _with((3, 3), (7, 40), (20, 56), (2, 7), (25, 36), (33, 36), (24, 64)), ids=lambda c: "n%d_e%d_C%d_g%d_b%d" % c)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+def test_table_and_lengths(M, case, dtype):
     """A random table, lengths that cut a group, end between groups, are zero and the whole of N."""
     n, ec, C, groups, batch = case
     batch, N = 4, n * groups
-    x, xa, Ws, dy, dya = O.make_inputs(batch, N, ec * C, 1, n, seed=7, xa_zero=False)
+    x, xa, Ws, dy, dya = O.make_inputs(batch, N, ec * C, 1, n, seed=7, xa_zero=False, dtype=dtype)
     table = torch.randperm(N, generator=torch.Generator().manual_seed(3))
     lens = [0, N, n * (groups // 2), N - 1]
     d = torch.float64
     ref = O.net_autograd_indexed(x.to(d), xa.to(d), [Ws[0].to(d)], dy.to(d), dya.to(d), 0.9, n, C, [table], lens)
-    gt, gl = table.to(torch.int32).cuda(), torch.tensor(lens, dtype=torch.int32).cuda()
+    kw = dict(group_index=table.to(torch.int32).cuda(), ctx_len=torch.tensor(lens, dtype=torch.int32).cuda())
     W = Ws[0].cuda()
-    y, ya = M.forward_stages(x.cuda(), xa.cuda(), W, 0.9, 0, n, C, 0, 1, group_index=gt, ctx_len=gl)
-    assert O.rel_err(y, ref[0]) < TOL and O.rel_err(ya, ref[1]) < TOL
+    # bfloat16: what is stored is rounded once, by at most 2^-8 of a value; the float32 copies of y, ya are saved
+    stored = lambda tol: tol if dtype == torch.float32 else max(tol, 2.0 ** -8)
+    y, ya, sy, sya = M.forward_stages_saving(x.cuda(), xa.cuda(), W, 0.9, 0, n, C, 0, **kw)
+    assert O.rel_err(y, ref[0]) < stored(TOL) and O.rel_err(ya, ref[1]) < stored(TOL)
     assert torch.equal(y[0].cpu(), x[0]) and torch.equal(ya[0].cpu(), xa[0])
-    xr, xar, dx, dxa, dW = M.backward_stages(y, ya, dy.cuda(), dya.cuda(), W, 0.9, 0, n, C, 0, 1, group_index=gt, ctx_len=gl)
+    xr, xar, dx, dxa, dW = M.backward_stages(sy, sya, dy.cuda(), dya.cuda(), W, 0.9, 0, n, C, 0, 1, **kw)
     tol = _tolerance(n)
-    assert O.rel_err(dx, ref[2]) < tol and O.rel_err(dxa, ref[3]) < tol and O.rel_err(dW[0], ref[4][0]) < tol
-    assert torch.equal(dx[0].cpu(), dy[0]) and torch.equal(xr[0].cpu(), x[0])
+    assert dx.dtype == dtype and dW.dtype == torch.float32
+    assert O.rel_err(dx, ref[2]) < stored(tol) and O.rel_err(dxa, ref[3]) < stored(tol) and O.rel_err(dW[0], ref[4][0]) < tol
+    assert torch.equal(dx[0].cpu(), dy[0]) and torch.equal(xr[0].cpu(), x[0].float())
+    # the saved outputs are undone: their float32 rounding, amplified by (1/m)^n
+    ix, ixa = M.inverse_stages(sy, sya, W, 0.9, 0, n, C, 0, 1, **kw)
+    rtol = max(3e-5, 6e-6 * 0.9 ** -n)
+    for a, b in ((xr, x), (xar, xa), (ix, x), (ixa, xa)):
+        assert O.rel_err(a, b) < rtol
 
 
 @pytest.mark.parametrize("value", [float("inf"), -float("inf")])

@@ -296,7 +296,7 @@ def test_backward_with_the_smaller_workspace_loops_over_windows(M):
     (1, 256, 32, 1, 2, 0, 8),      # one pass covers the range
     (2, 1024, 128, 4, 4, 0, 5),    # multi-stage passes and one-stage launches mixed
     (2, 512, 32, 2, 8, 0, 4),      # one-stage launches only
-    (2, 96, 20, 2, 3, 1, 3),       # the generic kernels
+    (2, 96, 20, 2, 3, 1, 3),       # register tiles for odd shapes
     (3, 1024, 32, 32, 2, 0, 11),   # heads of one feature: several multi-stage passes
 ], ids=lambda c: "b%d_N%d_E%d_C%d_n%d_s%d_L%d" % c)
 @pytest.mark.parametrize("grouping", ["closed", "lengths", "table"])

@@ -66,7 +66,7 @@ def test_golden_forward_backward(M, name):
     assert (xar.cpu() - g["xa"]).abs().max().item() < TOL_F32 * max(1.0, g["x"].abs().max().item())
 
 
-# (batch, N, E, C, n, L): every register-kernel head width and group size, ragged tails, the generic kernel
+# (batch, N, E, C, n, L): every register-kernel head width and group size, ragged tails, register tiles for odd shapes
 SHAPES = [
     (3, 64, 16, 4, 2, 4),      # Ec=4
     (2, 96, 32, 4, 4, 3),      # Ec=8, groups=24 (not a power of two)
@@ -78,9 +78,9 @@ SHAPES = [
     (2, 64, 256, 2, 2, 3),     # Ec=128, n=2
     (5, 40, 32, 1, 2, 3),      # Ec=32, one head, 20 groups: partial wave tile
     (2, 64, 64, 4, 16, 6),     # stride wraps to 0 again (L > log2(groups)+1)
-    (2, 36, 20, 2, 3, 3),      # generic kernel: n=3, Ec=10
-    (1, 128, 6, 2, 64, 2),     # generic kernel: n=64, Ec=3
-    (2, 14, 12, 4, 1, 2),      # generic kernel: n=1
+    (2, 36, 20, 2, 3, 3),      # odd shape: n=3, Ec=10
+    (1, 128, 6, 2, 64, 2),     # odd shape: n=64, Ec=3
+    (2, 14, 12, 4, 1, 2),      # odd shape: n=1
     (3, 40, 8, 8, 2, 3),       # one feature per head (E == n_head), four heads to a lane: n=2, 8 heads to a row, partial wave tile
     (2, 64, 16, 16, 4, 4),     # one feature per head, n=4, 16 heads to a row
     (2, 64, 12, 12, 8, 2),     # one feature per head, n=8, E = 3 * 4: 4 heads to a row
@@ -89,7 +89,7 @@ SHAPES = [
     (1, 128, 4, 4, 64, 2),     # one feature per head, n=64, E = 4
     (1, 128, 32, 32, 64, 1),   # one feature per head, n=64, 32 heads to a row: eight heads to a lane
     (2, 32, 48, 48, 2, 2),     # one feature per head, E = 3 * 16
-    (2, 32, 6, 6, 4, 2),       # one feature per head, E not a multiple of 4: generic kernel
+    (2, 32, 6, 6, 4, 2),       # one feature per head, E not a multiple of 4: odd shape
 ]
 
 
@@ -194,11 +194,11 @@ def test_dya_none_equals_zeros(M):
 
 
 @pytest.mark.parametrize("shape", [(2, 32, 16, 2, 4, 3), (2, 128, 128, 4, 16, 2), (2, 36, 20, 2, 3, 3), (2, 64, 16, 16, 8, 2)],
-                         ids=["register_n4_Ec8", "register_n16_Ec32", "generic_n3_Ec10", "register_n8_Ec1"])
+                         ids=["register_n4_Ec8", "register_n16_Ec32", "odd_n3_Ec10", "register_n8_Ec1"])
 @pytest.mark.parametrize("act", [1, 2, -1, 3], ids=["relu", "sigmoid", "linear", "leaky_relu"])
 def test_other_activations_vs_oracle(M, act, shape):
     """relu / sigmoid / linear (codes of ncn_fwd_cuda_kernel.cu:86-95) and the Triton kernels' leaky relu
-    (ncn_triton.py:22-28) on the register kernels and on the generic kernel; the oracle's branches for them are pinned by
+    (ncn_triton.py:22-28) on the register kernels of both kinds; the oracle's branches for them are pinned by
     scalar loops, identities and finite differences (tests/test_oracle_properties.py).
     relu and leaky relu have a kink at T = 0, where a float32 recomputation may pick the other slope: the small shapes
     use a seed whose every |T| stays above 1e-4 (checked in float64), the large one inputs whose T keeps one sign per

@@ -1,5 +1,5 @@
-"""Seeded sweep over small random problems: every kernel path (register tiles, generic LDS kernel, multi-stage
-passes, table / context-length builds) against the float64 oracle.  Shapes include n_cache = 1, n_cache = 64, one
+"""Seeded sweep over small random problems: every kernel path that alpha = 0.9 takes (register tiles of both
+kinds, generic LDS kernel where none fits, multi-stage passes, table / context-length builds) against the float64 oracle.  Shapes include n_cache = 1, n_cache = 64, one
 feature per head, one group, one batch entry, group counts that are not powers of two."""
 import random
 
@@ -41,7 +41,7 @@ def _cases(seed, count, acts=None):
 
 def _one_feature_cases(seed, count):
     """Heads of one feature (E == n_head) on the group sizes and widths their register kernels exist for, and some
-    they do not (E not a multiple of 4, n_cache not a power of two: generic kernels)."""
+    they do not (E not a multiple of 4, n_cache not a power of two: register tiles for odd shapes)."""
     rng = random.Random(seed)
     out = []
     while len(out) < count:

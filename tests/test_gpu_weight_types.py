@@ -88,7 +88,23 @@ def test_one_array_per_stage(M, case, dtype):
     args = lambda p: (x.data_ptr(), xa.data_ptr(), _lib.NCN_F32 | flags, y.data_ptr(), ya.data_ptr(), _lib.NCN_F32, None,
                       None, p, ws.data_ptr(), ws.numel(), ctypes.byref(shape), 0, L, alpha, 0.9, 0,
                       torch.cuda.current_stream().cuda_stream)
-    assert lib.ncn_forward(*args(ctypes.cast(ptrs, ctypes.c_void_p))) == 0
+    array = ctypes.cast(ptrs, ctypes.c_void_p)
+    assert lib.ncn_forward(*args(array)) == 0
     assert torch.equal(y, want[0]) and torch.equal(ya, want[1])
+    # .. in the inverse and the backward, whose dW is one array
+    st = torch.cuda.current_stream().cuda_stream
+    want_x = M.inverse_stages(y, ya, torch.stack(Ws), alpha, 0, n, C, 0, L)
+    ix, ixa = torch.empty_like(x), torch.empty_like(x)
+    assert lib.ncn_inverse_ws(y.data_ptr(), ya.data_ptr(), flags, ix.data_ptr(), ixa.data_ptr(), _lib.NCN_F32, array, ws.data_ptr(),
+                              ws.numel(), ctypes.byref(shape), 0, L, alpha, 0.9, 0, st) == 0
+    assert torch.equal(ix, want_x[0]) and torch.equal(ixa, want_x[1])
+    _, _, want_dx, want_dxa, want_dW = M.backward_stages(y, ya, x, xa, torch.stack(Ws), alpha, 0, n, C, 0, L, want_inputs=False,
+                                                         dw_dtype=dtype)
+    dx, dxa, dW = torch.empty_like(x), torch.empty_like(x), torch.empty(L, 2 * E, dtype=dtype, device="cuda")
+    bws = torch.empty(lib.ncn_workspace_bytes_stages(ctypes.byref(shape), 0, L, 0, 2 if L > 1 else 1), dtype=torch.uint8, device="cuda")
+    assert lib.ncn_backward(y.data_ptr(), ya.data_ptr(), flags, x.data_ptr(), xa.data_ptr(), _lib.NCN_F32, dx.data_ptr(),
+                            dxa.data_ptr(), _lib.NCN_F32, None, None, array, dW.data_ptr(), bws.data_ptr(), bws.numel(),
+                            ctypes.byref(shape), 0, L, alpha, 0.9, 0, st) == 0
+    assert torch.equal(dx, want_dx) and torch.equal(dxa, want_dxa) and torch.equal(dW, want_dW)
     ptrs[L - 1] = None
-    assert lib.ncn_forward(*args(ctypes.cast(ptrs, ctypes.c_void_p))) == -1   # NCN_ERR_NULL, nothing launched
+    assert lib.ncn_forward(*args(array)) == -1   # NCN_ERR_NULL, nothing launched

@@ -79,7 +79,7 @@ def test_backward_static_matches_backward_on_two_calls_in_a_row():
     a, b = _call_both(lib, _lib, (2, 96, 32, 4, 4), 3, seed=4)
     for u, v in zip(a, b):
         assert torch.isfinite(v).all() and O.rel_err(v, u) < 1e-5
-    # generic kernels (n_cache = 3) use the scratch too
+    # register tiles for odd shapes (n_cache = 3) use the scratch too
     a, b = _call_both(lib, _lib, (2, 36, 20, 2, 3), 1, seed=5)
     for u, v in zip(a, b):
         assert torch.isfinite(v).all() and O.rel_err(v, u) < 1e-5
