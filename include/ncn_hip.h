@@ -77,7 +77,7 @@ extern "C" {
 #define NCN_ERR_UNSUPPORTED (-6) /* n_cache > 64, or head width too large for the generic kernel; also alpha outside
                                     [1e-3, 1e3] or m outside [1e-3, 0.999] at head widths above 64 (see ncn_kernel_path_scalars) */
 #define NCN_ERR_ALIGN (-7)       /* a pointer is not 16-byte aligned (4-byte for the int32 tables) */
-#define NCN_ERR_ALIAS (-8)       /* n_stages > 1 needs the state buffers the call would carry it in */
+#define NCN_ERR_ALIAS (-8)       /* n_stages > 1 needs the state buffers the call would carry it in; ncn_stack_*: outputs are inputs */
 #define NCN_ERR_STATIC_LIMIT (-9) /* ncn_backward_static: the shape needs more scratch than the library holds */
 
 /* Shape of one problem; shared by all entry points. */

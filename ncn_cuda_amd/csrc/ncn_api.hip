@@ -362,8 +362,8 @@ size_t temp_bytes(const ncn_shape* sh, bool backward) {
 }
 
 // The backward launches of one call write their dW partial rows side by side into the partial buffer and are summed
-// together: two reduction launches per call instead of two per launch, as long as the buffer (kMaxGridX rows of 2E)
-// and the job (kReduceMaxSegments launches, kReduceMaxStages stages) hold them.
+// together: one reduction (one launch, or two past kReduceOneLaunchRows rows) per call instead of one per launch, as long as
+// the buffer (kMaxGridX rows of 2E) and the job (kReduceMaxSegments launches, kReduceMaxStages stages) hold them.
 class DwReducer {
   public:
     DwReducer(float* partials, float* level1, int64_t two_e, bool out_bf16, hipStream_t s, int row_cap = kMaxGridX)
@@ -486,7 +486,7 @@ const char* ncn_error_string(int code) {
         case NCN_ERR_WORKSPACE: return "workspace is NULL or smaller than ncn_workspace_bytes()";
         case NCN_ERR_UNSUPPORTED: return "unsupported shape: n_cache must be <= 64 and the head width <= 64 (128 for power-of-two n_cache <= 16)";
         case NCN_ERR_ALIGN: return "a pointer is not 16-byte aligned (4-byte for group_index and ctx_len)";
-        case NCN_ERR_ALIAS: return "n_stages > 1 needs float32 dx, dxa and either x_rec, xa_rec or the workspace of ncn_workspace_bytes_stages(.., 2) to carry the state";
+        case NCN_ERR_ALIAS: return "outputs that are the call's own inputs (ncn_stack_*), or n_stages > 1 without float32 dx, dxa and either x_rec, xa_rec or the workspace of ncn_workspace_bytes_stages(.., 2) to carry the state";
         case NCN_ERR_STATIC_LIMIT: return "ncn_backward_static: E is above 256, the limit of the library's own scratch";
         default: break;
     }

@@ -12,7 +12,7 @@
     X(2, 128, 2, 8) X(4, 128, 2, 8) X(8, 128, 4, 8) X(16, 128, 4, 8)
 
 // The shapes X(n_cache, head width) with multi-stage (LDS-resident) builds, under the stride permutation, with context
-// lengths and for the radix-n levels alike.  Groups of 8 rows and more are bound by arithmetic even stage by stage
-// (measured 10 % slower through LDS) and have none.
+// lengths and for the radix-n levels alike.  Groups of 8 rows and more have none: from 16 rows on a stage is bound by its
+// instruction issue; at 8, issue and traffic of a one-stage launch are about equal, and passes through LDS measured 10 % slower.
 #define NCN_FOR_EACH_FUSED_CONFIG(X) \
     X(2, 8) X(4, 8) X(2, 16) X(4, 16) X(2, 32) X(4, 32) X(2, 64) X(4, 64) X(2, 128) X(4, 128)

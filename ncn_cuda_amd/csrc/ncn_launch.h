@@ -38,7 +38,8 @@ constexpr int kGenericArrays = 7;
 constexpr int kMaxGridX = 16384;
 // Upper bound on gridDim.x of a forward / inverse launch (no partial rows to pay for).
 constexpr int kMaxForwardGridX = 1 << 18;
-// dW partial rows are summed in two levels: chunks of kReduceRowsPerBlock rows, then the chunk sums.
+// dW partial rows are summed in one launch where no segment has more than kReduceOneLaunchRows (ncn_generic.hip), else in two
+// levels: chunks of kReduceRowsPerBlock rows, then the chunk sums.
 constexpr int kReduceRowsPerBlock = 32;
 // One reduction job sums up to kReduceMaxSegments partial arrays (one per backward launch of a call) that lie side by
 // side in the partial buffer and hold at most kReduceMaxStages stages between them.
@@ -121,7 +122,7 @@ struct AnyTile {
 };
 // The tile whose wave issues the least for a group: padded elements times what one costs (some 20 instructions), plus
 // the sums across lanes (2 R over the lanes of a row, F over the row lanes) and the pivot row's own terms, per lane.  Tiles
-// of more than 16 elements (two waves per SIMD, spills) only where the group fits no smaller one.
+// of more than 16 elements (two or three waves per SIMD) only where the group fits no smaller one.
 inline AnyTile any_tile(int nc, int ec) {
     AnyTile best{0, 0, 0, 0};
     int best_cost = 0;

@@ -59,6 +59,49 @@ def test_stack(M, case, ranges, dtype):
             assert dW.dtype == dtype and O.rel_err(dW[l], r[4][l].reshape(-1)) < tol, l
 
 
+@pytest.mark.parametrize("act", [1, 2, 3, -1])
+@pytest.mark.parametrize("case", [CASES[1][0], CASES[3][0], CASES[5][0]], ids=lambda c: "_".join(map(str, c)))
+def test_other_activations(M, case, act):
+    batch, N, E, C, n, L, max_range, max_saves = case
+    make = O.make_inputs_signed_regimes if act in (1, 3) else O.make_inputs   # relu: away from its kink
+    x, xa, Ws, dy, dya = make(batch, N, E, L, n, seed=sum(case))
+    d = torch.float64
+    ref = O.net_autograd(x.to(d), xa.to(d), [w.to(d) for w in Ws], dy.to(d), dya.to(d), 0.9, n, C, activation=act)
+    W = torch.stack([w.reshape(-1) for w in Ws]).cuda()
+    plan, y, ya, saves = M.stack_forward(x.cuda(), xa.cuda(), W, 0.9, act, n, C, 0, L, max_range, 8 * x.numel() * max_saves)
+    dx, dxa, dW = M.stack_backward(plan, y, ya, saves, dy.cuda(), dya.cuda(), W)
+    tol = 1.2e-6 * 0.9 ** -(n * min(max_range, L))   # as in test_stack
+    for name, got, want in (("y", y, ref[0]), ("ya", ya, ref[1]), ("dx", dx, ref[2]), ("dxa", dxa, ref[3]),
+                            *(("dW%d" % l, dW[l], ref[4][l].reshape(-1)) for l in range(L))):
+        assert O.rel_err(got, want) < tol, name
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("n", [2, 4])
+def test_results_depend_on_the_inputs_alone(M, n, dtype):
+    """The same bits again whatever the memory holds that scratch, saves and outputs are allocated from (NaN here), and with a
+    pass on other inputs in between."""
+    from ncn_cuda_amd.modules import fused_ncn_net
+    batch, N, E, C, L = 4, 2048, 64, 2, 6
+
+    def inputs(seed):
+        x, xa, Ws, dy, _ = O.make_inputs(batch, N, E, L, n, seed=seed, xa_zero=False, dtype=dtype)
+        return [t.cuda().requires_grad_() for t in (x, xa, *Ws)], dy.cuda()
+
+    def run(leaves, dy):
+        y, ya = fused_ncn_net(leaves[0], leaves[1], leaves[2:], 0.9, 0, n, C)
+        return [y, ya, *torch.autograd.grad(y, leaves, dy)]
+
+    leaves, dy = inputs(3)
+    first = [t.detach().clone() for t in run(leaves, dy)]
+    for again in range(3):
+        run(*inputs(4 + again))
+        poison = [torch.full((1 << k,), float("nan"), device="cuda") for k in range(6, 24) for _ in range(4)]
+        del poison
+        for a, b in zip(run(leaves, dy), first):
+            assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
 @pytest.mark.parametrize("batch,N,E,C,n,L", [(16, 2048, 128, 4, 4, 6),     # multi-stage passes
                                              (16, 2046, 128, 4, 2, 13)])   # an odd number of groups: one launch per stage
@@ -144,7 +187,7 @@ def test_refusals(M):
         return lib.ncn_stack_forward(M._ptr(x), M._ptr(xa), 0, M._ptr(out), M._ptr(y), 0, None, M._ptr(W), None,
                                      ctypes.c_size_t(0), ctypes.byref(sh), 0, 3, 13, 1, 0.9, 0.9, 0, M._stream(x.device))
 
-    assert "carry the state" in _lib.error_string(forward(x))
+    assert forward(x) == -8 and "call's own inputs" in _lib.error_string(forward(x))   # NCN_ERR_ALIAS
     rc = lib.ncn_stack_backward(M._ptr(y), M._ptr(y), None, M._ptr(x), None, 0, M._ptr(xa), M._ptr(xa), 0, M._ptr(W),
                                 M._ptr(W), 0, None, ctypes.c_size_t(0), ctypes.byref(sh), 0, 3, 13, 1, 0.9, 0.9, 0,
                                 M._stream(x.device))
