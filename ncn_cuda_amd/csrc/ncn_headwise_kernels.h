@@ -283,7 +283,7 @@ __global__ void __launch_bounds__(kBlockThreads) headwise_forward_kernel(const S
 // LOOP = false is for launches with a wave for every tile, as in stage_backward_kernel: the build with the loop
 // carries the tile's addresses across it and spills at R x F = 16.
 template <int NC, int EC, int R, int F, bool TANH_ONLY, bool INDEXED, bool LOOP = true>
-__global__ void __launch_bounds__(kBlockThreads, (TANH_ONLY && !INDEXED && R * F <= 16) ? 4 : 1) headwise_backward_kernel(const StageArgs A) {
+__global__ void __launch_bounds__(kBlockThreads, (TANH_ONLY && !INDEXED && R * F <= 16) ? 4 : (TANH_ONLY && INDEXED && R * F == 32) ? 2 : 1) headwise_backward_kernel(const StageArgs A) {
     NCN_HW_PROLOGUE
     float dwi[F], dwj[F];
 #pragma unroll
