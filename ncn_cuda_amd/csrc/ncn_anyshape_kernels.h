@@ -4,9 +4,9 @@
 // citations), with a geometry that is chosen per launch instead of compiled in: a lane holds an R x F tile (R = 2..5
 // rows, F = 3..5 features), a row is spread over LF = 2^lf_log2 lanes and a group over
 // LR = 2^lr_log2 row lanes, so that R * LR covers n_cache rows and F * LF the head's features with little padding
-// (any_tile() in ncn_launch.h; 5 rows of 40 features: R = 3, F = 5, LF = 8, LR = 2, one row of six padded).  What does not exist
-// is zero: padded features have zero weights and stay zero; padded rows have zero gradients, which stay zero, and never
-// are a pivot.  The feature of a lane's register f is f * LF + (lane % LF): a load instruction reads LF consecutive
+// (any_tile() in ncn_launch.h; 5 rows of 40 features: R = 3, F = 5, LF = 8, LR = 2, one row of six padded).  Padded
+// features have zero weights and zero gradients, which stay zero; padded rows have zero gradients, which stay zero, and
+// never are a pivot.  The feature of a lane's register f is f * LF + (lane % LF): a load instruction reads LF consecutive
 // elements of a row, at any alignment, where F consecutive ones per lane would touch every line F times over.
 //
 // What bounds it: vector issue, as for the shapes of powers of two; the levels of the cross-lane sums are taken under

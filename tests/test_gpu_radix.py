@@ -41,6 +41,8 @@ CASES = [
     (2, 768, 64, 2, 4, 0, 3),      # n = 4, N = 12 * 4^3: 12 windows, 4 per load forward, 2 per load backward
     (2, 512, 32, 2, 8, 0, 3),      # n = 8: no LDS passes, closed-form positions in the one-stage register kernels
     (2, 81, 10, 2, 3, 0, 4),       # n = 3, head width 5: register tiles for odd shapes
+    (2, 150, 21, 3, 5, 1, 1),      # n = 5, level 1 of 6 * 5^2, head width 7: tiles with padded features
+    (3, 72, 20, 1, 6, 0, 2),       # n = 6, levels 0 and 1 of 2 * 6^2
     (2, 128, 256, 2, 2, 2, 3),     # head width 128: register kernels, one level per launch
     (2, 64, 16, 16, 2, 0, 6),      # one feature per head, laid out as one head of 16: levels in LDS like heads of 16
     (2, 1024, 64, 64, 4, 0, 5),    # the same at n = 4, two "heads" of 32
