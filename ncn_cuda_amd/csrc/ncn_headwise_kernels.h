@@ -282,6 +282,9 @@ __global__ void __launch_bounds__(kBlockThreads) headwise_forward_kernel(const S
 
 // LOOP = false is for launches with a wave for every tile, as in stage_backward_kernel: the build with the loop
 // carries the tile's addresses across it and spills at R x F = 16.
+// Launch bounds: four waves per SIMD fit at tiles of up to 16 elements.  At 4 x 8 the INDEXED build, which stores the rows past a
+// length as they are loaded, would take 272 registers and one wave: held to two it takes 376 instead of 535 us at 32 x 2048 x
+// 128, groups of 64, with a table (388 instead of 534 with lengths too).
 template <int NC, int EC, int R, int F, bool TANH_ONLY, bool INDEXED, bool LOOP = true>
 __global__ void __launch_bounds__(kBlockThreads, (TANH_ONLY && !INDEXED && R * F <= 16) ? 4 : (TANH_ONLY && INDEXED && R * F == 32) ? 2 : 1) headwise_backward_kernel(const StageArgs A) {
     NCN_HW_PROLOGUE
