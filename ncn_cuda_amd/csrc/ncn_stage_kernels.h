@@ -101,7 +101,7 @@ __device__ __forceinline__ void finish_w(const StageArgs& A, float (&w)[F]) {
     }
 }
 
-// Both at once, where nothing is to be loaded in between.
+// Both at once, for the backward without a loop, which has no register to keep raw weights in while its tile is loaded.
 template <int F>
 __device__ __forceinline__ void load_w(const StageArgs& A, int head, int ec, int fl, float (&wi)[F], float (&wj)[F]) {
     const int64_t at = (int64_t)head * ec + fl * F;
@@ -561,6 +561,8 @@ __device__ __forceinline__ void pass_rows(const int64_t (&off)[R], const bool (&
         pass_rows<R, F>(off, dead, A.plane, p, q);                                              \
     }
 
+// Tiles of 4 x 4 run five waves per SIMD (96 registers): most builds need 82 to 95 by themselves, a few ended two above (relu
+// behind a table, 32 x 2048 x 128, groups of 32: 141 us with four waves, 132 with five).
 template <int NC, int EC, int R, int F, bool TANH_ONLY = true, bool INDEXED = false, int TYPES = kAnyTypes>
 __global__ void __launch_bounds__(kBlockThreads, (R == 4 && F == 4) ? 5 : 1) stage_forward_kernel(const StageArgs A) {
     NCN_WAVE_PROLOGUE
@@ -626,8 +628,10 @@ __global__ void __launch_bounds__(kBlockThreads, (R == 4 && F == 4) ? 5 : 1) sta
     }
 }
 
-// Tiles of up to 16 elements per lane fit 128 VGPRs (4 waves per SIMD) when the compiler is asked to.  Larger tiles,
-// the multi-activation build and the builds that mask steps would spill, so they are left alone.
+// Tiles of up to 16 elements per lane fit 128 VGPRs (4 waves per SIMD) when the compiler is asked to.  Tiles of 32 are held to two
+// waves per SIMD in the builds for one type and in those that mask steps, which would end a few registers above 256 (relu
+// behind a table: one wave, 598 us where two take 338; see above).  The other builds for every activation would spill and
+// are left alone.
 // LOOP = false is for launches with a wave for every tile: without the loop around them the tile's addresses and
 // offsets are not carried in registers across it (the loop build spills 6 of them per lane at R x F = 16, which a
 // launch bound by its traffic pays for), and the steps come out in an order that issues better.
