@@ -11,7 +11,7 @@
 //
 // What bounds it: vector issue, as for the shapes of powers of two; the levels of the cross-lane sums are taken under
 // wave-uniform branches because LF and LR are not known at compile time.  One lane per row with the state in LDS (the
-// generic kernels, which still take what fits no tile and scalars outside the scaled state) leaves three quarters of
+// generic kernels, which still take what fits no tile, scalars outside the scaled state and m < 0.85) leaves three quarters of
 // the time to LDS traffic and its barriers.
 // 16 x 1005 x 160 float32, groups of 5 rows, heads of 40: forward 113 -> 17.6 us, backward 519 -> 31.7 us per stage.
 #pragma once
