@@ -179,5 +179,72 @@ def build(verbose=False, force=True):
             fcntl.flock(lock, fcntl.LOCK_UN)
 
 
+# ---- the autograd nodes in native code (csrc/ncn_torch.cpp), the one part that is built against torch -------------
+TORCH_SOURCE = "ncn_torch.cpp"
+TORCH_LIB_PATH = os.path.join(PKG_DIR, "_ncn_torch.so")
+TORCH_ID_MARKER = "NCN_TORCH_ID="
+TORCH_FLAGS = ["-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1"]
+TORCH_LIBS = ["c10", "c10_hip", "torch_cpu", "torch", "torch_python"]
+
+
+def torch_source_id():
+    """Hash of what _ncn_torch.so is made from: its source, the C ABI's header, its flags, and the torch and Python it is for."""
+    import torch
+    h = hashlib.sha256()
+    h.update(_read(os.path.join(CSRC, TORCH_SOURCE)) + b"\0" + _read(os.path.join(INCLUDE, "ncn_hip.h")) + b"\0")
+    h.update(" ".join(TORCH_FLAGS + TORCH_LIBS + [torch.__version__, sys.version.split()[0]]).encode())
+    return h.hexdigest()[:16]
+
+
+def torch_library_id(path=None):
+    """The id compiled into _ncn_torch.so (read from the file, nothing is loaded), or None."""
+    try:
+        data = _read(TORCH_LIB_PATH if path is None else path)
+    except OSError:
+        return None
+    k = data.find(TORCH_ID_MARKER.encode())
+    return data[k + len(TORCH_ID_MARKER):k + len(TORCH_ID_MARKER) + 16].decode("ascii", "replace") if k >= 0 else None
+
+
+def have_cxx():
+    return shutil.which("g++") is not None
+
+
+def build_torch(verbose=False, force=True):
+    """Compile _ncn_torch.so; force=False only if its id is not that of the source beside it."""
+    import sysconfig
+
+    import torch
+    with open(LOCK_PATH, "w") as lock:
+        fcntl.flock(lock, fcntl.LOCK_EX)
+        try:
+            want = torch_source_id()
+            if not force and torch_library_id() == want:
+                return False
+            if not have_cxx():
+                raise RuntimeError("g++ not found: cannot build _ncn_torch.so")
+            root = os.path.dirname(torch.__file__)
+            rocm = os.path.dirname(os.path.dirname(os.path.realpath(_hipcc())))
+            include = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
+                       sysconfig.get_paths()["include"], os.path.join(rocm, "include"), "/opt/rocm/include"]
+            tmp = f"{TORCH_LIB_PATH}.{os.getpid()}.tmp"
+            cmd = ["g++", *TORCH_FLAGS, f'-DNCN_TORCH_ID_TEXT="{TORCH_ID_MARKER}{want}"',
+                   f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+                   *(a for i in include for a in ("-isystem", i)), os.path.join(CSRC, TORCH_SOURCE), "-o", tmp,
+                   "-L", os.path.join(root, "lib"), *("-l" + x for x in TORCH_LIBS)]
+            proc = subprocess.run(cmd, capture_output=True, text=True)
+            if proc.returncode != 0:
+                if os.path.exists(tmp):
+                    os.unlink(tmp)
+                raise RuntimeError(f"g++ failed on {TORCH_SOURCE}:\n{proc.stdout}\n{proc.stderr}")
+            os.replace(tmp, TORCH_LIB_PATH)
+            if verbose:
+                print(f"built {TORCH_LIB_PATH} ({os.path.getsize(TORCH_LIB_PATH)} bytes, id {want})", file=sys.stderr)
+            return True
+        finally:
+            fcntl.flock(lock, fcntl.LOCK_UN)
+
+
 if __name__ == "__main__":
     build(verbose=True, force="--incremental" not in sys.argv)
+    build_torch(verbose=True, force="--incremental" not in sys.argv)

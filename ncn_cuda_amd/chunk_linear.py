@@ -21,7 +21,7 @@ radix_group_table the radix-n digit grouping of ncn_triton/group_tensors.py:8-18
 """
 import torch
 
-from . import ncn_cuda_module
+from . import _native, ncn_cuda_module
 
 __all__ = ["FusedLinearChunkNCNFunction", "fused_chunk_linear_ncn", "stride_group_table", "radix_group_table"]
 
@@ -90,4 +90,9 @@ class FusedLinearChunkNCNFunction(torch.autograd.Function):
 
 def fused_chunk_linear_ncn(x, xa, W, group_tensor, ctxlen_tensor, ALPHA, ACTIVATION, NHEAD, CACHE, l):
     """(yi, ya) of one stage; same argument order as ncn_triton_old.py:362-387."""
+    if not torch.compiler.is_compiling() and isinstance(x, torch.Tensor) and x.dim() == 3 and \
+            ncn_cuda_module.table_was_checked(group_tensor, x.shape[1]):
+        got = _native.ext().table_stage(x, xa, W, group_tensor, ctxlen_tensor, ALPHA, _activation_code(ACTIVATION), CACHE, NHEAD)
+        if got is not None:
+            return got
     return FusedLinearChunkNCNFunction.apply(x, xa, W, group_tensor, ctxlen_tensor, ALPHA, ACTIVATION, NHEAD, CACHE, l)

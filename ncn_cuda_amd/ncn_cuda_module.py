@@ -129,14 +129,19 @@ def validate_grouping(group_index, ctx_len, batch, N, n_stages):
 _checked_tables = {}   # id(tensor) -> (weak reference, version counter, N) of tables found good; dies with the tensor
 
 
+def table_was_checked(group_index, N):
+    """Whether check_group_table has found this tensor, as it is now, to be good."""
+    seen = _checked_tables.get(id(group_index))
+    return seen is not None and seen[0]() is group_index and seen[1:] == (group_index._version, int(N))
+
+
 def check_group_table(group_index, N):
     """Raises ValueError unless every row of the table is a permutation of 0 .. N-1 (the kernels clamp bad entries
     but cannot repair a table).  Works on CPU or GPU tensors; on the GPU it synchronises, so a table that passed is
     remembered (the tensor object with its version counter) and not sorted again while it stays unchanged."""
-    key = id(group_index)
-    seen = _checked_tables.get(key)
-    if seen is not None and seen[0]() is group_index and seen[1:] == (group_index._version, int(N)):
+    if table_was_checked(group_index, N):
         return
+    key = id(group_index)
     t = group_index.reshape(-1, N).to(torch.int64)
     want = torch.arange(N, dtype=torch.int64, device=t.device).expand_as(t)
     if not torch.equal(torch.sort(t, dim=1).values, want):

@@ -15,7 +15,7 @@ import math
 import torch
 from torch import nn
 
-from .modules import NCNFunction
+from .modules import fused_ncn_cuda_v2
 
 __all__ = ["activation_code", "fused_ncn_triton", "NCNModuleTriton", "NCNNetTriton", "NCNNetTestTriton"]
 
@@ -30,7 +30,7 @@ def activation_code(name):
 
 def fused_ncn_triton(x, xa, W, ALPHA, ACTIVATION, NHEAD, CACHE, MODULE_L):
     """(yi, ya) of stage MODULE_L; argument order of ncn_triton.py:333-349."""
-    return NCNFunction.apply(x, xa, W, ALPHA, activation_code(ACTIVATION), CACHE, NHEAD, MODULE_L)
+    return fused_ncn_cuda_v2(x, xa, W, ALPHA, activation_code(ACTIVATION), CACHE, NHEAD, MODULE_L)
 
 
 class NCNModuleTriton(nn.Module):

@@ -542,3 +542,19 @@ def test_probe_entry_points_validate_their_arguments(lib):
     assert h.ncn_probe_issue(99, 8, 8, 16, p, None) == -2
     assert h.ncn_probe_issue(0, 3, 8, 16, p, None) == -2      # chains: 1, 4 or 8
     assert h.ncn_probe_issue(0, 8, 3, 16, p, None) == -2      # waves per SIMD: 1, 2, 4 or 8
+
+
+def test_native_nodes_leave_cpu_calls_to_the_python_nodes():
+    import torch
+
+    from ncn_cuda_amd import _build, _native
+    assert _build.torch_library_id() == _build.torch_source_id()
+    ext = _native.ext()
+    x, W = torch.zeros(1, 4, 4), torch.zeros(8)
+    assert ext.stage(x, x, W, 0.9, 0, 2, 1, 0) is None
+    assert ext.stack(x, x, [W, W], 0.9, 0, 2, 1, 0, 13, 1 << 30, 1 << 30) is None
+    assert ext.radix(x, x, [W], 0.9, 0, 2, 1, 0) is None
+    assert ext.table_stage(x, x, W, torch.arange(4, dtype=torch.int32), None, 0.9, 0, 2, 1) is None
+    for bad in ((), (1,) * 3, (0,) * len(_native.ENTRIES), None):
+        with pytest.raises((TypeError, ValueError)):
+            ext.bind(bad)
