@@ -26,7 +26,7 @@ ID_SOURCE = "ncn_build_id.hip"
 SOURCES = ["ncn_api.hip", "ncn_fwd.hip", "ncn_bwd.hip", "ncn_fwd_f32.hip", "ncn_fwd_bf16.hip",
            "ncn_bwd_once.hip", "ncn_bwd_f32.hip", "ncn_bwd_bf16.hip", "ncn_fwd_indexed.hip", "ncn_fwd_indexed_f32.hip", "ncn_fwd_indexed_bf16.hip",
            "ncn_bwd_indexed.hip", "ncn_bwd_indexed_once.hip", "ncn_bwd_indexed_f32.hip", "ncn_bwd_indexed_bf16.hip",
-           "ncn_headwise.hip", "ncn_headwise_indexed.hip", "ncn_headwise_bwd.hip", "ncn_headwise_bwd_indexed.hip", "ncn_anyshape.hip", "ncn_anyshape_bwd.hip", "ncn_anyshape_lengths.hip", "ncn_anyshape_bwd_lengths.hip", "ncn_generic.hip", "ncn_fused.hip", "ncn_fused_radix.hip", "ncn_fused_lengths.hip", "ncn_fused_headwise.hip", "ncn_fused_headwise_lengths.hip",
+           "ncn_headwise.hip", "ncn_headwise_indexed.hip", "ncn_headwise_bwd.hip", "ncn_headwise_bwd_indexed.hip", "ncn_anyshape.hip", "ncn_anyshape_bwd.hip", "ncn_anyshape_lengths.hip", "ncn_anyshape_bwd_lengths.hip", "ncn_split.hip", "ncn_generic.hip", "ncn_fused.hip", "ncn_fused_radix.hip", "ncn_fused_lengths.hip", "ncn_fused_headwise.hip", "ncn_fused_headwise_lengths.hip",
            "ncn_fused_radix_headwise.hip", "ncn_probe.hip", ID_SOURCE]
 # packed-fp32 VALU instructions are switched off for device code on purpose (flag is device-only;
 # the host pass prints a harmless "not a recognized feature" note).
@@ -48,7 +48,7 @@ EXTRA_FLAGS = {"ncn_fused.hip": MAX_ILP, "ncn_fused_radix.hip": MAX_ILP, "ncn_fu
                "ncn_bwd_indexed_bf16.hip": MAX_ILP, "ncn_fwd_f32.hip": MAX_ILP, "ncn_fwd_bf16.hip": MAX_ILP,
                "ncn_fwd_indexed_f32.hip": MAX_ILP, "ncn_fwd_indexed_bf16.hip": MAX_ILP,
                "ncn_headwise.hip": MAX_ILP, "ncn_headwise_indexed.hip": MAX_ILP, "ncn_headwise_bwd.hip": MAX_ILP,
-               "ncn_headwise_bwd_indexed.hip": MAX_ILP}
+               "ncn_headwise_bwd_indexed.hip": MAX_ILP, "ncn_split.hip": MAX_ILP}
 
 
 def _hipcc():

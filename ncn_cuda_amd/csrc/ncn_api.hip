@@ -133,6 +133,7 @@ uint32_t stage_stride(int stage, uint32_t groups) {
 
 struct Plan {
     int path;
+    bool split;        // path 2 on the kernels for few groups (ncn_split_kernels.h), with a partial row per wave tile
     AnyTile any;       // path 1 on the register tiles of ncn_anyshape_kernels.h (any.r != 0), else the generic kernels
     int groups_per_tile;
     uint32_t groups, tiles_per_inst, total_tiles;
@@ -143,18 +144,25 @@ struct Plan {
 
 // reserve_rows: rows of the dW partial buffer kept free for another launch of the same stage
 // row_cap: rows of the dW partial buffer the caller has (kMaxGridX in a workspace of ncn_workspace_bytes)
-Plan make_plan(const ncn_shape* sh, int path, const AnyTile& any, int reserve_rows = 0, int row_cap = kMaxGridX) {
+// may_split: may_split_call() of the launches that are planned
+Plan make_plan(const ncn_shape* sh, int path, const AnyTile& any, bool may_split, int reserve_rows = 0, int row_cap = kMaxGridX) {
     Plan p;
     const int max_rows = row_cap - reserve_rows;
     p.path = path;
+    p.split = may_split && path == 2 && sh->batch * sh->N * sh->E <= split_max_elements(sh->n_cache);
     p.any = any;
     const int ec = (int)(sh->E / sh->n_head);
     p.groups_per_tile = any.r ? 64 >> (any.lf_log2 + any.lr_log2)
+                        : p.split ? split_groups_per_tile(sh->n_cache, ec)
                               : (p.path == 2) ? fast_groups_per_tile(sh->n_cache, ec) : generic_groups_per_tile(sh->n_cache);
     p.groups = (uint32_t)(sh->N / sh->n_cache);
     p.tiles_per_inst = (p.groups + p.groups_per_tile - 1) / p.groups_per_tile;
     p.total_tiles = (uint32_t)(sh->batch * p.tiles_per_inst);
-    if (p.path == 2 || any.r) {
+    if (p.split && p.total_tiles > (uint32_t)max_rows) return make_plan(sh, path, any, false, reserve_rows, row_cap);
+    if (p.split) {
+        p.grid_x = p.grid_fwd = 0;   // launch_split makes its own
+        p.partial_rows = (int)p.total_tiles;
+    } else if (p.path == 2 || any.r) {
         // 4 waves per block, wave w works on head w % n_head: the grid holds a multiple of n_head waves and at
         // most kMaxGridX partial rows (one per n_head consecutive waves)
         const int C = sh->n_head;
@@ -310,9 +318,13 @@ const ncn_shape* planning_shape(const ncn_shape* sh, ncn_shape* as_wide) {
     return headwise_call(sh, 2, as_wide) ? as_wide : sh;
 }
 
+// Whether launches of a call may go to the kernels for few groups.
+bool may_split_call(int activation, bool headwise) { return activation == NCN_ACT_TANH && !headwise; }
+
 // One stage.  Register kernels: the plain builds know the stride permutation only, the others read the launch's table,
 // radix level and context lengths.
 hipError_t run_forward_kernel(Pass pass, const StageArgs& a, const Plan& p, bool plain, bool headwise, hipStream_t s) {
+    if (p.split) return launch_split(pass, a, !plain, s);
     if (p.any.r) return launch_any_forward(pass, a, p.grid_fwd, s);
     if (p.path != 2) return launch_generic(pass, a, a.n_head, p.grid_fwd, s);
     if (headwise)
@@ -320,6 +332,7 @@ hipError_t run_forward_kernel(Pass pass, const StageArgs& a, const Plan& p, bool
     return plain ? launch_stage_forward<false>(pass, a, p.grid_fwd, s) : launch_stage_forward<true>(pass, a, p.grid_fwd, s);
 }
 hipError_t run_backward_kernel(const StageArgs& a, const Plan& p, bool plain, bool headwise, hipStream_t s) {
+    if (p.split) return launch_split(kBackward, a, !plain, s);
     if (p.any.r) return launch_any_backward(a, p.grid_x, s);
     if (p.path != 2) return launch_generic(kBackward, a, a.n_head, p.grid_x, s);
     if (headwise) return plain ? launch_headwise_backward(a, p.grid_x, s) : launch_headwise_backward_indexed(a, p.grid_x, s);
@@ -554,7 +567,7 @@ static int forward_impl(const void* x, const void* xa, int in_dtype, void* y, vo
     if (!aligned16(x) || !aligned16(xa) || !aligned16(y) || !aligned16(ya) || !w.aligned(n_stages) || !aligned16(y32) ||
         !aligned16(ya32) || !aligned16(workspace))
         return NCN_ERR_ALIGN;
-    const Plan p = make_plan(shape, path, any_tile_for(shape, path, alpha, m));
+    const Plan p = make_plan(shape, path, any_tile_for(shape, path, alpha, m), may_split_call(activation, headwise));
     hipStream_t s = static_cast<hipStream_t>(stream);
 
     // several stages: LDS-resident passes when the shape allows and the buffers permit the ping-pong
@@ -677,7 +690,7 @@ static int inverse_impl(const void* y, const void* ya, int in_dtype, void* x, vo
     if (!known_dtype_or_x2(in_dtype, n_stages, path) || !known_dtype(out_dtype)) return NCN_ERR_DTYPE;
     if (!aligned16(x) || !aligned16(xa) || !aligned16(y) || !aligned16(ya) || !w.aligned(n_stages) || !aligned16(workspace))
         return NCN_ERR_ALIGN;
-    const Plan p = make_plan(shape, path, any_tile_for(shape, path, alpha, m));
+    const Plan p = make_plan(shape, path, any_tile_for(shape, path, alpha, m), may_split_call(activation, headwise));
     hipStream_t s = static_cast<hipStream_t>(stream);
 
     // several stages: LDS-resident passes, last pass of the range first.  Without scratch to ping-pong with, the
@@ -807,7 +820,7 @@ static int backward_impl(const void* y, const void* ya, int y_dtype, const void*
     // partial rows of the generic kernel's second launch
     const AnyTile any = any_tile_for(shape, path, alpha, m);
     const int extra_rows = (grouping.ctx_len && path != 2 && !any.r) ? edge_rows(shape) : 0;
-    const Plan p = make_plan(shape, path, any, extra_rows, row_cap);
+    const Plan p = make_plan(shape, path, any, may_split_call(activation, headwise), extra_rows, row_cap);
     hipStream_t s = static_cast<hipStream_t>(stream);
     float* partials = static_cast<float*>(workspace);
     float* level1 = partials + (int64_t)row_cap * 2 * shape->E;
@@ -1016,7 +1029,7 @@ int ncn_forward_radix(const void* x, const void* xa, int in_dtype, void* y, void
     ncn_shape as_wide;
     const bool headwise = headwise_call(shape, path, &as_wide);
     if (headwise) shape = &as_wide;
-    const Plan p = make_plan(shape, path, any_tile_for(shape, path, alpha, m));
+    const Plan p = make_plan(shape, path, any_tile_for(shape, path, alpha, m), may_split_call(activation, headwise));
     hipStream_t s = static_cast<hipStream_t>(stream);
     const std::vector<RadixPass> passes = plan_radix(shape, first_level, n_levels, false, path == 2);
     // every pass is closed: the first reads x, xa and the later ones run in place on y, ya; passes of several levels
@@ -1080,7 +1093,7 @@ int ncn_backward_radix(const void* y, const void* ya, int y_dtype, const void* d
     ncn_shape as_wide;
     const bool headwise = headwise_call(shape, path, &as_wide);
     if (headwise) shape = &as_wide;
-    const Plan p = make_plan(shape, path, any_tile_for(shape, path, alpha, m));
+    const Plan p = make_plan(shape, path, any_tile_for(shape, path, alpha, m), may_split_call(activation, headwise));
     hipStream_t s = static_cast<hipStream_t>(stream);
     float* partials = static_cast<float*>(workspace);
     float* level1 = partials + (int64_t)kMaxGridX * 2 * shape->E;
@@ -1140,7 +1153,7 @@ int ncn_inverse_radix(const void* y, const void* ya, int in_dtype, void* x, void
     ncn_shape as_wide;
     const bool headwise = headwise_call(shape, path, &as_wide);
     if (headwise) shape = &as_wide;
-    const Plan p = make_plan(shape, path, any_tile_for(shape, path, alpha, m));
+    const Plan p = make_plan(shape, path, any_tile_for(shape, path, alpha, m), may_split_call(activation, headwise));
     hipStream_t s = static_cast<hipStream_t>(stream);
     const std::vector<RadixPass> passes = plan_radix(shape, first_level, n_levels, false, path == 2);
     for (size_t e = 0; e < passes.size(); ++e) {   // last pass first; every pass is closed: in place after the first
@@ -1173,7 +1186,7 @@ int ncn_inverse_radix(const void* y, const void* ya, int in_dtype, void* x, void
 struct StackCall {
     ncn_shape as_wide;
     const ncn_shape* shape;
-    bool headwise;
+    bool headwise, may_split;
     const std::vector<StackRange>* ranges;   // of this thread's kept plans
     size_t plane;        // one float32 activation array
     int fwd_passes_max;  // passes of the longest range
@@ -1213,7 +1226,8 @@ struct StackCall {
         plane = temp_bytes(shape, false) / 2;
         fwd_passes_max = bwd_passes_max = bwd_passes = 0;
         int64_t rows = 0;
-        const Plan single = make_plan(shape, 2, AnyTile{0, 0, 0, 0});
+        may_split = may_split_call(activation, headwise);
+        const Plan single = one_stage();
         for (const StackRange& r : *ranges) {
             if ((int)r.fwd.size() > fwd_passes_max) fwd_passes_max = (int)r.fwd.size();
             if ((int)r.bwd.size() > bwd_passes_max) bwd_passes_max = (int)r.bwd.size();
@@ -1225,6 +1239,7 @@ struct StackCall {
         row_cap = rows < kMaxGridX ? kMaxGridX : (int)rows;
         return true;
     }
+    Plan one_stage() const { return make_plan(shape, 2, AnyTile{0, 0, 0, 0}, may_split); }   // of the passes of one stage
     // pairs of arrays in the workspace: the forward's passes that are not kept go through one; the backward's gradients
     // through one (two where dx, dxa cannot hold them in between), reconstructed inputs inside a range through two more
     size_t forward_bytes() const { return fwd_passes_max > 1 ? 2 * plane : 0; }
@@ -1266,7 +1281,7 @@ int ncn_stack_forward(const void* x, const void* xa, int in_dtype, void* y, void
     const size_t nr = c.ranges->size();
     if ((nr > 1 || out_dtype != NCN_F32) && !saves) return NCN_ERR_NULL;
     if (c.forward_bytes() && (!workspace || workspace_bytes < c.forward_bytes())) return NCN_ERR_WORKSPACE;
-    const Plan p = make_plan(shape, 2, AnyTile{0, 0, 0, 0});
+    const Plan p = c.one_stage();
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int64_t elements = shape->batch * shape->N * shape->E;
     void* const t0 = workspace;
@@ -1333,7 +1348,7 @@ int ncn_stack_backward(const float* y, const float* ya, const float* saves, cons
     const size_t nr = c.ranges->size();
     if ((nr > 1 || !y) && !saves) return NCN_ERR_NULL;
     if (!workspace || workspace_bytes < c.backward_bytes(dx_dtype == NCN_F32)) return NCN_ERR_WORKSPACE;
-    const Plan p = make_plan(shape, 2, AnyTile{0, 0, 0, 0});
+    const Plan p = c.one_stage();
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int64_t elements = shape->batch * shape->N * shape->E, two_e = 2 * shape->E;
     float* partials = static_cast<float*>(workspace);

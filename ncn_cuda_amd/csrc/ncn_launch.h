@@ -101,6 +101,17 @@ NCN_DECLARE(true, kAnyTypes) NCN_DECLARE(true, kF32Types) NCN_DECLARE(true, kBf1
 #undef NCN_DECLARE
 template <> hipError_t launch_stage_backward<false, kAnyTypesOnce>(const StageArgs&, int, hipStream_t);
 template <> hipError_t launch_stage_backward<true, kAnyTypesOnce>(const StageArgs&, int, hipStream_t);
+// Launches with few groups (ncn_split_kernels.h): tanh, one row fragment of 4 features per lane.
+// Up to 2^20 elements (four waves of them per SIMD, one of the register tiles) they are as fast or faster in both directions
+// from groups of 8 rows on: us of a launch on the register tiles : here, heads of 32, float32, backward with its reduction,
+//   groups of 32   2^19: 15.6 : 10.2, backward 38.8 : 25.0   2^20: 16.9 : 16.4, 41.6 : 35.6   2^21: 27.6 : 28.2, 53.9 : 61.7
+//   groups of 16   2^19: 9.4 : 6.5, 21.1 : 16.1              2^20: 10.7 : 9.9, 23.3 : 22.9    2^21: 16.8 : 16.7, 32.3 : 37.6
+//   groups of 8    2^19: 6.4 : 4.6, 12.9 : 10.6              2^20: 7.5 : 6.5, 14.8 : 14.5     2^21: 11.6 : 10.6, 21.8 : 25.1
+// Smaller groups have short chains (their tile is 2 x 4): groups of 4, 2^18: 3.7 : 3.3, 7.4 : 6.8; 2^19: 4.1 : 3.8, 8.0 : 8.7.
+constexpr int64_t split_max_elements(int n_cache) { return n_cache >= 8 ? 1 << 20 : 1 << 18; }
+int split_groups_per_tile(int nc, int ec);
+// indexed: the builds that honour a.table, a.radix_stride and a.ctx_len
+hipError_t launch_split(Pass pass, const StageArgs& a, bool indexed, hipStream_t s);
 // Heads of one feature (ncn_headwise_kernels.h): `a` carries the geometry of E / w heads of w features, w =
 // headwise_width(E), for which the grid was planned as well; the second form honours a.table, a.radix_stride and
 // a.ctx_len.
