@@ -194,7 +194,7 @@ hipError_t launch_fused_headwise(Pass pass, const FusedArgs& a, int nc, int ec, 
 hipError_t launch_fused_headwise_lengths(Pass pass, const FusedArgs& a, int nc, int ec, int grid, size_t lds, hipStream_t s);
 
 
-// ---- multi-stage passes over radix-n levels, ncn_fused_radix.hip ---------------------------------------------
+// ---- multi-stage passes over radix-n levels, ncn_radix.hip ---------------------------------------------
 struct RadixPass {
     int first, count;  // levels [first, first + count) relative to the range that was planned
     int single;        // 1: one level, run with the one-stage kernel
@@ -209,6 +209,13 @@ std::vector<RadixPass> plan_radix(const ncn_shape* sh, int first, int count, boo
 int radix_grid(const ncn_shape* sh, const RadixPass& p, bool backward);
 hipError_t launch_fused_radix(Pass pass, FusedArgs& a, const ncn_shape* sh, const RadixPass& p, hipStream_t s,
                               bool headwise = false);
-hipError_t launch_fused_radix_headwise(Pass pass, const FusedArgs& a, int nc, int ec, int grid, size_t lds, hipStream_t s);
+// the builds, by kind (ncn_radix_build.hip and the units that include it)
+template <bool HEADWISE, bool BACKWARD, bool TANH>
+hipError_t launch_radix(Pass pass, const FusedArgs& a, int nc, int ec, int grid, hipStream_t s);
+#define NCN_DECLARE(H, B) \
+    template <> hipError_t launch_radix<H, B, true>(Pass, const FusedArgs&, int, int, int, hipStream_t); \
+    template <> hipError_t launch_radix<H, B, false>(Pass, const FusedArgs&, int, int, int, hipStream_t);
+NCN_DECLARE(false, false) NCN_DECLARE(false, true) NCN_DECLARE(true, false) NCN_DECLARE(true, true)
+#undef NCN_DECLARE
 
 }  // namespace ncn

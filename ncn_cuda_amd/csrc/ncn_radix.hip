@@ -1,34 +1,25 @@
 // Planning and launching of multi-stage passes over levels of the radix-n digit grouping
-// (ncn_triton/group_tensors.py:8-18); the kernels are the RADIX builds of ncn_fused_kernels.h.
+// (ncn_triton/group_tensors.py:8-18); the kernels are those of ncn_radix_kernels.h,
+// built in ncn_radix_build.hip.
+#include <climits>
 #include <cmath>
 #include <vector>
 
-#include "ncn_fused_dispatch.h"
+#include "ncn_configs.h"
+#include "ncn_fused_kernels.h"
+#include "ncn_launch.h"
 
 namespace ncn {
 
 namespace {
 
-// shapes with a radix build: digits are extracted with shifts, so n_cache is 2 or 4 (tile shapes of the one-stage table)
+// shapes with a radix build: digits are bits of a row number, so n_cache is 2 or 4
 #define NCN_FOR_EACH_RADIX_CONFIG(X) NCN_FOR_EACH_FUSED_CONFIG(X)
-
-constexpr int kRadixMaxGrid = 4096;
 
 uint32_t floor_pow2(uint32_t v) {
     uint32_t p = 1;
     while (p * 2 <= v) p *= 2;
     return p;
-}
-
-size_t radix_lds_bytes(int nc, int ec, bool backward, uint32_t rows, int n_stages) {
-    const TileShape t = fast_tile(nc, ec);
-    const int lr = nc / t.r;
-    size_t bytes = (size_t)(backward ? 4 : 2) * rows * ec * sizeof(float);
-    bytes += (size_t)kFusedMaxStages * 2 * ec * sizeof(float);
-    const int nw = backward ? kFusedWavesBwd : kFusedWavesFwd;
-    if (lr > 1) bytes += (size_t)nw * t.f * 64 * sizeof(float);
-    if (backward) bytes += (size_t)nw * n_stages * 2 * ec * sizeof(float);
-    return bytes;
 }
 
 int64_t ipow(int64_t b, int e) {
@@ -83,12 +74,10 @@ std::vector<RadixPass> plan_radix(const ncn_shape* sh, int first, int count, boo
 
 int radix_grid(const ncn_shape* sh, const RadixPass& p, bool backward) {
     const int64_t items = sh->batch * (int64_t)p.loads * sh->n_head;
-    int64_t cap = kRadixMaxGrid;
-    if (backward) {
-        const int64_t by_rows = (int64_t)kMaxGridX / p.count * sh->n_head;
-        if (by_rows < cap) cap = by_rows;
-    }
-    int64_t g = items < cap ? items : cap;
+    if (!backward) return items <= INT_MAX ? (int)items : 0;   // a workgroup for every item
+    // .. in the backward where the dW scratch has a partial row for each
+    const int64_t by_rows = (int64_t)kMaxGridX / p.count * sh->n_head;
+    int64_t g = items < by_rows ? items : by_rows;
     g = g / sh->n_head * sh->n_head;
     if (g < sh->n_head) g = sh->n_head;
     return (int)g;
@@ -115,9 +104,13 @@ hipError_t launch_fused_radix(Pass pass, FusedArgs& a, const ncn_shape* sh, cons
     a.scale_dn = (float)std::pow((double)a.tab.m, (double)(nc * p.count));
     a.scale_up = (float)std::pow((double)a.tab.m, -(double)(nc * p.count));
     const int grid = radix_grid(sh, p, backward);
-    const size_t lds = radix_lds_bytes(nc, ec, backward, p.rows, p.count);
-    if (headwise) return launch_fused_radix_headwise(pass, a, nc, ec, grid, lds, s);
-    return launch_fused_shape<true, false, false>(pass, a, nc, ec, grid, lds, s);
+    const bool tanh_only = a.tab.activation == NCN_ACT_TANH;
+#define NCN_PICK(HEADWISE, BACKWARD, TANH) \
+    if (headwise == HEADWISE && backward == BACKWARD && tanh_only == TANH) return launch_radix<HEADWISE, BACKWARD, TANH>(pass, a, nc, ec, grid, s);
+    NCN_PICK(false, false, true) NCN_PICK(false, true, true) NCN_PICK(false, false, false) NCN_PICK(false, true, false)
+    NCN_PICK(true, false, true) NCN_PICK(true, true, true) NCN_PICK(true, false, false) NCN_PICK(true, true, false)
+#undef NCN_PICK
+    return hipErrorInvalidConfiguration;
 }
 
 }  // namespace ncn

@@ -1,0 +1,91 @@
+"""The multi-level radix kernels (ncn_radix_kernels.h) against the float64 oracle: every head width and group size, passes of two
+levels up to the most that a workgroup holds, so that the levels run in registers, after exchanges of register and lane bits and
+after the exchange through LDS, windows that are no power of two, every kind of launch."""
+import pytest
+import torch
+
+from oracle import ncn_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def M():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from ncn_cuda_amd import ncn_cuda_module
+    return ncn_cuda_module
+
+
+def check(M, batch, N, ec, C, n, first, L, act=0, dtype=torch.float32):
+    E = ec * C
+    make = O.make_inputs_signed_regimes if act in (1, 3) else O.make_inputs   # away from the kink
+    x, xa, Ws, dy, dya = make(batch, N, E, L, n, seed=N + ec) if act in (1, 3) else make(batch, N, E, L, n, seed=N + ec, xa_zero=False)
+    x, xa, dy, dya = (t.to(dtype) for t in (x, xa, dy, dya))
+    d = torch.float64
+    tables = [O.radix_group_table(N, n, first + l) for l in range(L)]
+    ref = O.net_autograd_indexed(x.to(d), xa.to(d), [w.to(d) for w in Ws], dy.to(d), dya.to(d), 0.9, n, C, tables, activation=act)
+    W = torch.stack([w.reshape(-1) for w in Ws]).cuda()
+    x, xa, dy, dya = (t.cuda() for t in (x, xa, dy, dya))
+    args = (W, 0.9, act, n, C, first, L)
+    y, ya = M.forward_radix(x, xa, *args)
+    rx, rxa, dx, dxa, dW = M.backward_radix(y, ya, dy, dya, *args)
+    _, _, dx2, dxa2, dW2 = M.backward_radix(y, ya, dy, dya, *args, want_inputs=False)
+    ix, ixa = M.inverse_radix(y, ya, *args)
+    # rounding of the sums, amplified by 1/m at every step undone (as in test_gpu_stack); reconstruction as in test_gpu_parity
+    tol = max(1e-5, 1.2e-6 * 0.9 ** -(n * L))
+    assert O.rel_err(y, ref[0]) < 1e-5 and O.rel_err(ya, ref[1]) < 1e-5
+    assert O.rel_err(dx, ref[2]) < tol and O.rel_err(dxa, ref[3]) < tol
+    for l in range(L):
+        assert O.rel_err(dW[l], ref[4][l].reshape(-1)) < tol, l
+    for got, want in ((rx, x), (rxa, xa), (ix, x), (ixa, xa)):
+        assert O.rel_err(got, want) < 12e-6 * 0.9 ** -(n * L)
+    assert torch.equal(dx, dx2) and torch.equal(dxa, dxa2) and torch.equal(dW, dW2)
+
+
+@pytest.mark.parametrize("levels", [2, 3, 5, "most"])
+@pytest.mark.parametrize("ec", [8, 16, 32, 64, 128])
+@pytest.mark.parametrize("n", [2, 4])
+def test_levels(M, n, ec, levels):
+    most = {2: {8: 10, 16: 9, 32: 8, 64: 7, 128: 6}, 4: {8: 5, 16: 4, 32: 4, 64: 3, 128: 3}}[n][ec]
+    L = most if levels == "most" else min(levels, most)
+    check(M, 2, 3 * n ** L, ec, 2, n, 0, L)          # three windows of every level
+
+
+@pytest.mark.parametrize("n,ec,first,L", [(2, 32, 3, 6), (4, 32, 1, 3), (2, 8, 1, 9), (4, 64, 1, 2)])
+def test_levels_that_do_not_start_at_the_first(M, n, ec, first, L):
+    check(M, 1, 5 * n ** (first + L), ec, 3, n, first, L)
+
+
+@pytest.mark.parametrize("act", [1, 2, 3, -1])
+@pytest.mark.parametrize("n,ec,L", [(2, 32, 7), (4, 32, 3), (2, 128, 5), (4, 16, 4)])
+def test_other_activations(M, n, ec, L, act):
+    check(M, 2, 3 * n ** L, ec, 2, n, 0, L, act)
+
+
+@pytest.mark.parametrize("n,E,L,act", [(2, 32, 8, 0), (4, 64, 4, 0), (2, 8, 9, 2), (4, 16, 3, -1)])
+def test_heads_of_one_feature(M, n, E, L, act):
+    check(M, 2, 3 * n ** L, 1, E, n, 0, L, act)
+
+
+@pytest.mark.parametrize("n,ec,L", [(2, 32, 8), (4, 32, 4)])
+def test_bfloat16_inputs_and_gradients(M, n, ec, L):
+    check(M, 2, n ** L, ec, 2, n, 0, L, dtype=torch.bfloat16)
+
+
+@pytest.mark.parametrize("n,L", [(2, 7), (4, 4)])
+def test_more_windows_than_partial_rows(M, n, L):
+    """The backward then loops over windows; each half of the batch has a workgroup for every window."""
+    batch, N, E = 16384 // L + 100, 512, 8
+    gen = torch.Generator(device="cuda").manual_seed(0)
+    x, xa, dy, dya = (torch.randn(batch, N, E, generator=gen, device="cuda") for _ in range(4))
+    W = torch.randn(L, 2 * E, generator=gen, device="cuda") / n ** 0.5
+    args = (W, 0.9, 0, n, 1, 0, L)
+    y, ya = M.forward_radix(x, xa, *args)
+    _, _, dx, dxa, dW = M.backward_radix(y, ya, dy, dya, *args, want_inputs=False)
+    halves = [M.backward_radix(*(t[s].contiguous() for t in (y, ya, dy, dya)), *args, want_inputs=False)
+              for s in (slice(0, batch // 2), slice(batch // 2, batch))]
+    assert torch.equal(dx, torch.cat([h[2] for h in halves])) and torch.equal(dxa, torch.cat([h[3] for h in halves]))
+    want = sum(h[4].double() for h in halves)
+    # sums of 2^20 products in float32, in other orders
+    assert ((dW.double() - want).norm() / want.norm()) < 1e-5
