@@ -160,6 +160,19 @@ __device__ __forceinline__ FusedItem fused_item(const FusedArgs& A, uint32_t ite
     return it;
 }
 
+// The item of workgroup `blk` of a launch with a workgroup for every item.  Workgroups go to the 8 XCDs in turn, each with an L2
+// of its own, and the heads of a window share 128-byte lines where a head's slice of a row is shorter: in groups of 8 windows, the
+// heads of one are given to workgroups 8 apart, i.e. to one XCD.  Training passes, us without : with: heads of 8 features (32 bytes),
+// x[64, 4096, 32], groups of two, 12 stages 422 : 309, 12 radix levels 405 : 267, groups of four, 6 stages 446 : 348; heads of 16,
+// x[64, 4096, 64], 12 stages 538 : 513; heads of 32, whose float32 slices are whole lines, the same either way.  (Workgroups that
+// loop over items keep their own order: every item of one must be of one head.)
+__device__ __forceinline__ uint32_t fused_deal(const FusedArgs& A, uint32_t blk) {
+    const uint32_t heads = A.n_head, windows = A.total_items / heads;
+    const uint32_t first = blk / (8u * heads) * 8u, r = blk - first * heads;
+    const uint32_t n = min(8u, windows - first), head = r / n;
+    return (first + r - head * n) * heads + head;
+}
+
 // element offset (without the feature) of local row `lr` = (window sub-block qi) * NC + slot
 template <int NC, bool RADIX>
 __device__ __forceinline__ int64_t fused_row_offset(const FusedArgs& A, const FusedItem& it, uint32_t lr) {
@@ -330,18 +343,19 @@ __global__ void __launch_bounds__(64 * kFusedWavesFwd) fused_forward_kernel(cons
     float* as = lds + rows * EC;
     float* w_lds = as + rows * EC;                              // [kFusedMaxStages][2][EC]
     float4* slots = reinterpret_cast<float4*>(w_lds + kFusedMaxStages * 2 * EC) + wave * (F / 4) * 64;
-    fused_load_weights<EC, NW>(A, blockIdx.x % A.n_head, w_lds);   // every item of this workgroup has this head
+    const uint32_t item0 = gridDim.x == A.total_items ? fused_deal(A, blockIdx.x) : blockIdx.x;
+    fused_load_weights<EC, NW>(A, item0 % A.n_head, w_lds);   // every item of this workgroup has this head
 
     // trips of 64 * NW threads over the float4 chunks of the largest window the LDS budget allows
     constexpr int K = (int)((kFusedStateBytesFwd / 2 / sizeof(float4) + 64 * NW - 1) / (64 * NW));
     uint4 rx[K], ra[K];
-    if (blockIdx.x < A.total_items) {
+    if (item0 < A.total_items) {
         int64_t off[K];
-        fused_window_offsets<NC, EC, NW, K>(A, fused_item<NC, EC, false>(A, blockIdx.x), rows, off);
+        fused_window_offsets<NC, EC, NW, K>(A, fused_item<NC, EC, false>(A, item0), rows, off);
         fused_fetch_rows<K>(A.in0, A.in_dtype, off, rx);
         fused_fetch_rows<K>(A.in1, A.in_dtype, off, ra);
     }
-    for (uint32_t item = blockIdx.x; item < A.total_items; item += gridDim.x) {
+    for (uint32_t item = item0; item < A.total_items; item += gridDim.x) {
         const FusedItem it = fused_item<NC, EC, false>(A, item);
         const int32_t len = LENGTHS ? max(0, min(A.ctx_len[it.batch], (int32_t)A.N)) : 0;
         fused_commit_rows<NC, EC, NW, K>(rx, A.in_dtype, xs, rows, A.tab.kappa);
@@ -419,7 +433,8 @@ __global__ void __launch_bounds__(64 * kFusedWavesBwd, TANH_ONLY ? (R * F <= 8 ?
     const int dw_wave_stride = A.n_stages * 2 * EC;
     float* dw_mine = dw_all + wave * dw_wave_stride;
     for (int k = lane; k < dw_wave_stride; k += 64) dw_mine[k] = 0.f;
-    const int head = blockIdx.x % A.n_head;   // == head of every item of this workgroup (gridDim.x % n_head == 0)
+    const uint32_t item0 = gridDim.x == A.total_items ? fused_deal(A, blockIdx.x) : blockIdx.x;
+    const int head = item0 % A.n_head;   // == head of every item of this workgroup (gridDim.x % n_head == 0)
     fused_load_weights<EC, NW>(A, head, w_lds);
 
     // The step code leaves no registers to carry a window across the stages, but between two items they are free:
@@ -455,13 +470,13 @@ __global__ void __launch_bounds__(64 * kFusedWavesBwd, TANH_ONLY ? (R * F <= 8 ?
             }
         }
     };
-    if (blockIdx.x < A.total_items) {
+    if (item0 < A.total_items) {
         Raw first;
-        fetch(blockIdx.x, first);
+        fetch(item0, first);
         commit(first);
     }
     __syncthreads();
-    for (uint32_t item = blockIdx.x; item < A.total_items; item += gridDim.x) {
+    for (uint32_t item = item0; item < A.total_items; item += gridDim.x) {
         const FusedItem it = fused_item<NC, EC, false>(A, item);
         const int32_t len = LENGTHS ? max(0, min(A.ctx_len[it.batch], (int32_t)A.N)) : 0;
         for (int st = A.n_stages - 1; st >= 0; --st) {
@@ -582,8 +597,8 @@ __global__ void __launch_bounds__(64 * kFusedWavesBwd, TANH_ONLY ? (R * F <= 8 ?
         }
         __syncthreads();
     }
-    // one partial row per workgroup and stage; workgroup b owns slot (b / n_head, head b % n_head)
-    float* prow = A.dw_partials + (int64_t)(blockIdx.x / A.n_head) * A.n_stages * (2 * A.E);
+    // one partial row per workgroup and stage; the workgroup of item i owns slot (i / n_head, head i % n_head)
+    float* prow = A.dw_partials + (int64_t)(item0 / A.n_head) * A.n_stages * (2 * A.E);
     for (int k = threadIdx.x; k < A.n_stages * 2 * EC; k += 64 * NW) {
         const int st = k / (2 * EC), rem = k - st * 2 * EC, half = rem / EC, f = rem - half * EC;
         float sum = 0.f;

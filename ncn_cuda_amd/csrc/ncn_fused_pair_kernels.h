@@ -140,11 +140,11 @@ __global__ void __launch_bounds__(64 * kFusedWavesFwd, NCN_PAIR_FWD_WAVES) pair_
     float* xs1 = lds;                               // slot-1 rows, [sub-block][EC]
     float* as1 = xs1 + ARR;
     float* w_lds = as1 + ARR;                       // [kFusedMaxStages][2][EC]
-    fused_load_weights<EC, NW>(A, blockIdx.x % A.n_head, w_lds);
+    const uint32_t item = fused_deal(A, blockIdx.x);   // the launch has a workgroup for every window
+    fused_load_weights<EC, NW>(A, item % A.n_head, w_lds);
     const float a_in = INVERSE ? A.tab.b_scale : A.tab.a_scale, a_out = INVERSE ? A.tab.inv_b_scale : A.tab.inv_a_scale;
 
     constexpr int K1 = (int)((kPairStateBytesFwd / 4 / sizeof(float4) + 64 * NW - 1) / (64 * NW));   // half the rows
-    const uint32_t item = blockIdx.x;   // the launch has a workgroup for every window
     if (item < A.total_items) {
         const FusedItem it = fused_item<NC, EC, false>(A, item);
         const int32_t len = LENGTHS ? max(0, min(A.ctx_len[it.batch], (int32_t)A.N)) : 0;
@@ -335,7 +335,8 @@ __global__ void __launch_bounds__(64 * kPairWavesBwd, TANH_ONLY ? NCN_PAIR_BWD_W
     const int dw_wave_stride = A.n_stages * 2 * EC;
     float* dw_mine = dw_all + wave * dw_wave_stride;
     for (int k = lane; k < dw_wave_stride; k += 64) dw_mine[k] = 0.f;
-    const int head = blockIdx.x % A.n_head;   // == head of every item of this workgroup (gridDim.x % n_head == 0)
+    const uint32_t item0 = LOOP ? blockIdx.x : fused_deal(A, blockIdx.x);
+    const int head = item0 % A.n_head;   // == head of every item of this workgroup (gridDim.x % n_head == 0)
     fused_load_weights<EC, NW>(A, head, w_lds);
 
     constexpr int K1 = (int)((kPairStateBytesBwd / 8 / sizeof(float4) + 64 * NW - 1) / (64 * NW));   // half the rows
@@ -401,14 +402,14 @@ __global__ void __launch_bounds__(64 * kPairWavesBwd, TANH_ONLY ? NCN_PAIR_BWD_W
                 }
             }
     };
-    if (blockIdx.x < A.total_items) {
+    if (item0 < A.total_items) {
         Raw first;
-        fetch(blockIdx.x, first);
-        load_slot0(blockIdx.x);
+        fetch(item0, first);
+        load_slot0(item0);
         commit(first);
     }
     __syncthreads();
-    uint32_t item = blockIdx.x;
+    uint32_t item = item0;
     if (item < A.total_items) do {
         const FusedItem it = fused_item<NC, EC, false>(A, item);
         const int32_t len = LENGTHS ? max(0, min(A.ctx_len[it.batch], (int32_t)A.N)) : 0;
@@ -550,8 +551,8 @@ __global__ void __launch_bounds__(64 * kPairWavesBwd, TANH_ONLY ? NCN_PAIR_BWD_W
         }
         __syncthreads();
     } while (LOOP && (item += gridDim.x) < A.total_items);
-    // one partial row per workgroup and stage; workgroup b owns slot (b / n_head, head b % n_head)
-    float* prow = A.dw_partials + (int64_t)(blockIdx.x / A.n_head) * A.n_stages * (2 * A.E);
+    // one partial row per workgroup and stage; the workgroup of item i owns slot (i / n_head, head i % n_head)
+    float* prow = A.dw_partials + (int64_t)(item0 / A.n_head) * A.n_stages * (2 * A.E);
     for (int k = threadIdx.x; k < A.n_stages * 2 * EC; k += 64 * NW) {
         const int st = k / (2 * EC), rem = k - st * 2 * EC, half = rem / EC, f = rem - half * EC;
         float sum = 0.f;

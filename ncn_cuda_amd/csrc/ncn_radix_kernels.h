@@ -345,7 +345,7 @@ __global__ void __launch_bounds__((64 * RadixShape<NC, EC, false>::NW), TANH_ONL
     float* w_lds = reinterpret_cast<float*>(fused_lds4);                  // [kFusedMaxStages][2][EC]
     float4* exch = fused_lds4 + kFusedMaxStages * 2 * EC / 4;             // one array of the workgroup
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), fl = lane % S::LF;
-    const FusedItem it = fused_item<NC, EC, true>(A, blockIdx.x);         // the launch has a workgroup for every item
+    const FusedItem it = fused_item<NC, EC, true>(A, fused_deal(A, blockIdx.x));   // the launch has a workgroup for every item
     int64_t off[S::R];
     radix_offsets<S, NC, 0, 0, INVERSE>(A, it, lane, wave, fl, off);
     uint4 rx[S::R * S::H], ra[S::R * S::H];
@@ -499,10 +499,11 @@ __global__ void __launch_bounds__((64 * RadixShape<NC, EC, true>::NW), TANH_ONLY
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), fl = lane % S::LF;
     const int dw_stride = A.n_stages * 2 * EC;
     float* dw_mine = dw_all + wave * dw_stride;
-    const int head = blockIdx.x % A.n_head;   // of every item of this workgroup (gridDim.x % n_head == 0)
+    const uint32_t item0 = LOOP ? blockIdx.x : fused_deal(A, blockIdx.x);
+    const int head = item0 % A.n_head;   // of every item of this workgroup (gridDim.x % n_head == 0)
     if (LOOP)
         for (int k = lane; k < dw_stride; k += 64) dw_mine[k] = 0.f;
-    uint32_t item = blockIdx.x;
+    uint32_t item = item0;
     do {
         const FusedItem it = fused_item<NC, EC, true>(A, item);
         int64_t off[S::R];
@@ -512,7 +513,7 @@ __global__ void __launch_bounds__((64 * RadixShape<NC, EC, true>::NW), TANH_ONLY
         radix_fetch<S>(A.in1, A.in_dtype, off, rb);
         radix_fetch<S>(A.g0, A.g_dtype, off, rg);
         radix_fetch<S>(A.g1, A.g_dtype, off, rh);
-        if (item == blockIdx.x) fused_load_weights<EC, S::NW>(A, head, w_lds);
+        if (item == item0) fused_load_weights<EC, S::NW>(A, head, w_lds);
         K k{A, it, w_lds, dw_mine, exch, lane, wave, fl};
         radix_commit<S>(ry, A.in_dtype, A.tab.kappa, k.Y);
         radix_commit<S>(rb, A.in_dtype, A.tab.b_scale, k.B);
@@ -537,8 +538,8 @@ __global__ void __launch_bounds__((64 * RadixShape<NC, EC, true>::NW), TANH_ONLY
         k.run();
     } while (LOOP && (item += gridDim.x) < A.total_items);
     __syncthreads();
-    // one partial row per workgroup and stage; workgroup b owns slot (b / n_head, head b % n_head)
-    float* prow = A.dw_partials + (int64_t)(blockIdx.x / A.n_head) * A.n_stages * (2 * A.E);
+    // one partial row per workgroup and stage; the workgroup of item i owns slot (i / n_head, head i % n_head)
+    float* prow = A.dw_partials + (int64_t)(item0 / A.n_head) * A.n_stages * (2 * A.E);
     for (int k = threadIdx.x; k < A.n_stages * 2 * EC; k += 64 * S::NW) {
         const int st = k / (2 * EC), rem = k - st * 2 * EC, half = rem / EC, f = rem - half * EC;
         float sum = 0.f;
