@@ -164,9 +164,12 @@ __device__ __forceinline__ FusedItem fused_item(const FusedArgs& A, uint32_t ite
 // of its own, and the heads of a window share 128-byte lines where a head's slice of a row is shorter: in groups of 8 windows, the
 // heads of one are given to workgroups 8 apart, i.e. to one XCD.  Training passes, us without : with: heads of 8 features (32 bytes),
 // x[64, 4096, 32], groups of two, 12 stages 422 : 309, 12 radix levels 405 : 267, groups of four, 6 stages 446 : 348; heads of 16,
-// x[64, 4096, 64], 12 stages 538 : 513; heads of 32, whose float32 slices are whole lines, the same either way.  (Workgroups that
+// x[64, 4096, 64], 12 stages 538 : 513; heads of 32, whose float32 slices are whole lines, the same either
+// way, and the divisions cost an inverse call of 36 us one more: they keep their order.  (Workgroups that
 // loop over items keep their own order: every item of one must be of one head.)
+template <int EC>
 __device__ __forceinline__ uint32_t fused_deal(const FusedArgs& A, uint32_t blk) {
+    if (EC * sizeof(float) >= 128) return blk;
     const uint32_t heads = A.n_head, windows = A.total_items / heads;
     const uint32_t first = blk / (8u * heads) * 8u, r = blk - first * heads;
     const uint32_t n = min(8u, windows - first), head = r / n;
@@ -343,7 +346,7 @@ __global__ void __launch_bounds__(64 * kFusedWavesFwd) fused_forward_kernel(cons
     float* as = lds + rows * EC;
     float* w_lds = as + rows * EC;                              // [kFusedMaxStages][2][EC]
     float4* slots = reinterpret_cast<float4*>(w_lds + kFusedMaxStages * 2 * EC) + wave * (F / 4) * 64;
-    const uint32_t item0 = gridDim.x == A.total_items ? fused_deal(A, blockIdx.x) : blockIdx.x;
+    const uint32_t item0 = gridDim.x == A.total_items ? fused_deal<EC>(A, blockIdx.x) : blockIdx.x;
     fused_load_weights<EC, NW>(A, item0 % A.n_head, w_lds);   // every item of this workgroup has this head
 
     // trips of 64 * NW threads over the float4 chunks of the largest window the LDS budget allows
@@ -433,7 +436,7 @@ __global__ void __launch_bounds__(64 * kFusedWavesBwd, TANH_ONLY ? (R * F <= 8 ?
     const int dw_wave_stride = A.n_stages * 2 * EC;
     float* dw_mine = dw_all + wave * dw_wave_stride;
     for (int k = lane; k < dw_wave_stride; k += 64) dw_mine[k] = 0.f;
-    const uint32_t item0 = gridDim.x == A.total_items ? fused_deal(A, blockIdx.x) : blockIdx.x;
+    const uint32_t item0 = gridDim.x == A.total_items ? fused_deal<EC>(A, blockIdx.x) : blockIdx.x;
     const int head = item0 % A.n_head;   // == head of every item of this workgroup (gridDim.x % n_head == 0)
     fused_load_weights<EC, NW>(A, head, w_lds);
 

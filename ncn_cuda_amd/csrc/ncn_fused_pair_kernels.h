@@ -140,7 +140,7 @@ __global__ void __launch_bounds__(64 * kFusedWavesFwd, NCN_PAIR_FWD_WAVES) pair_
     float* xs1 = lds;                               // slot-1 rows, [sub-block][EC]
     float* as1 = xs1 + ARR;
     float* w_lds = as1 + ARR;                       // [kFusedMaxStages][2][EC]
-    const uint32_t item = fused_deal(A, blockIdx.x);   // the launch has a workgroup for every window
+    const uint32_t item = fused_deal<EC>(A, blockIdx.x);   // the launch has a workgroup for every window
     fused_load_weights<EC, NW>(A, item % A.n_head, w_lds);
     const float a_in = INVERSE ? A.tab.b_scale : A.tab.a_scale, a_out = INVERSE ? A.tab.inv_b_scale : A.tab.inv_a_scale;
 
@@ -335,7 +335,7 @@ __global__ void __launch_bounds__(64 * kPairWavesBwd, TANH_ONLY ? NCN_PAIR_BWD_W
     const int dw_wave_stride = A.n_stages * 2 * EC;
     float* dw_mine = dw_all + wave * dw_wave_stride;
     for (int k = lane; k < dw_wave_stride; k += 64) dw_mine[k] = 0.f;
-    const uint32_t item0 = LOOP ? blockIdx.x : fused_deal(A, blockIdx.x);
+    const uint32_t item0 = LOOP ? blockIdx.x : fused_deal<EC>(A, blockIdx.x);
     const int head = item0 % A.n_head;   // == head of every item of this workgroup (gridDim.x % n_head == 0)
     fused_load_weights<EC, NW>(A, head, w_lds);
 

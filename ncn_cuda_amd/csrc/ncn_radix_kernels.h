@@ -345,7 +345,7 @@ __global__ void __launch_bounds__((64 * RadixShape<NC, EC, false>::NW), TANH_ONL
     float* w_lds = reinterpret_cast<float*>(fused_lds4);                  // [kFusedMaxStages][2][EC]
     float4* exch = fused_lds4 + kFusedMaxStages * 2 * EC / 4;             // one array of the workgroup
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), fl = lane % S::LF;
-    const FusedItem it = fused_item<NC, EC, true>(A, fused_deal(A, blockIdx.x));   // the launch has a workgroup for every item
+    const FusedItem it = fused_item<NC, EC, true>(A, fused_deal<EC>(A, blockIdx.x));   // the launch has a workgroup for every item
     int64_t off[S::R];
     radix_offsets<S, NC, 0, 0, INVERSE>(A, it, lane, wave, fl, off);
     uint4 rx[S::R * S::H], ra[S::R * S::H];
@@ -499,7 +499,7 @@ __global__ void __launch_bounds__((64 * RadixShape<NC, EC, true>::NW), TANH_ONLY
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), fl = lane % S::LF;
     const int dw_stride = A.n_stages * 2 * EC;
     float* dw_mine = dw_all + wave * dw_stride;
-    const uint32_t item0 = LOOP ? blockIdx.x : fused_deal(A, blockIdx.x);
+    const uint32_t item0 = LOOP ? blockIdx.x : fused_deal<EC>(A, blockIdx.x);
     const int head = item0 % A.n_head;   // of every item of this workgroup (gridDim.x % n_head == 0)
     if (LOOP)
         for (int k = lane; k < dw_stride; k += 64) dw_mine[k] = 0.f;
