@@ -34,10 +34,17 @@ hipError_t launch_any_forward(Pass pass, const StageArgs& a, int grid_x, hipStre
     const bool tanh_only = a.activation == NCN_ACT_TANH;
 #define NCN_LAUNCH(KERNEL) hipLaunchKernelGGL(KERNEL, dim3(grid_x), dim3(kBlockThreads), 0, s, a)
 #if NCN_ANYSHAPE_BACKWARD
+    const bool loop = (uint64_t)a.total_tiles * (uint64_t)a.n_head > (uint64_t)grid_x * kWavesPerBlock;   // more tiles than waves
 #define NCN_CASE(R, F)                                                                  \
     if (r == R && f == F) {                                                             \
-        if (tanh_only) NCN_LAUNCH((any_backward_kernel<R, F, true, kLengths>));                   \
-        else NCN_LAUNCH((any_backward_kernel<R, F, false, kLengths>));                            \
+        if constexpr (R * F <= 15) {                                                    \
+            if (tanh_only && !loop) {                                                   \
+                NCN_LAUNCH((any_backward_kernel<R, F, true, kLengths, false>));         \
+                return hipGetLastError();                                               \
+            }                                                                           \
+        }                                                                               \
+        if (tanh_only) NCN_LAUNCH((any_backward_kernel<R, F, true, kLengths, true>));        \
+        else NCN_LAUNCH((any_backward_kernel<R, F, false, kLengths, true>));                      \
         return hipGetLastError();                                                       \
     }
 #else

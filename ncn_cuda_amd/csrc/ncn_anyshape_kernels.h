@@ -57,8 +57,8 @@ __device__ __forceinline__ void any_sum_span(float (&v)[N], int lo, int hi) {
 template <int R, int F, bool LENGTHS>
 struct AnyLane {
     int lfl, lrl, fl, rl, gw;   // log2 of lanes per row and row lanes per group; this lane's place
-    int feat[F];                // feature of register f, clamped into the head
-    bool has[F];                // that feature exists
+    int head_dim;
+    bool whole;                 // head_dim is a multiple of F: register f of lane fl is feature fl * F + f, else (f << lfl) + fl
     int64_t entry;              // element offset of the tile's batch entry (wave-uniform)
     uint32_t row[R];            // elements from there to the row's head slice: 32-bit offsets from a scalar base
     int live;                   // live rows of the lane's group, -1 past the last group
@@ -68,30 +68,49 @@ struct AnyLane {
         fl = lane & ((1 << lfl) - 1);
         rl = (lane >> lfl) & ((1 << lrl) - 1);
         gw = lane >> (lfl + lrl);
-#pragma unroll
-        for (int f = 0; f < F; ++f) {
-            const int k = (f << lfl) + fl;
-            has[f] = k < A.head_dim;
-            feat[f] = min(k, A.head_dim - 1);
-        }
+        head_dim = A.head_dim;
+        whole = head_dim % F == 0;
     }
+    // feature of register f, clamped into the head, and whether it exists: made again where they are needed, for they would
+    // take 2 F registers across the steps
+    __device__ __forceinline__ int feat0() const { return min(fl * F, head_dim - F); }   // first of a lane's features, when whole
+    __device__ __forceinline__ int feat(int f) const { return whole ? feat0() + f : min((f << lfl) + fl, head_dim - 1); }
+    __device__ __forceinline__ bool has(int f) const { return whole ? fl * F < head_dim : (f << lfl) + fl < head_dim; }
     __device__ __forceinline__ void rows(const StageArgs& A, uint32_t t, int head) {
         const uint32_t b = t / A.tiles_per_inst;
         const uint32_t group = (t - b * A.tiles_per_inst) * (64u >> (lfl + lrl)) + gw;
         const bool valid = group < A.groups;
         live = !valid ? -1 : LENGTHS ? live_rows(A, b, group) : A.n_cache;
         entry = (int64_t)b * A.N * A.E;
+        // slot_position() of every row, with one branch on the kind of grouping around them all: a branch per row would wait
+        // for the arguments, and behind a table for memory, row by row
+        const uint32_t g = valid ? group : 0u, n = A.n_cache;
+        uint32_t pos[R];
+        if (A.table) {
 #pragma unroll
-        for (int rr = 0; rr < R; ++rr) {
-            const uint32_t slot = min(rl * R + rr, A.n_cache - 1);
-            row[rr] = (uint32_t)slot_position(A, valid ? group : 0u, slot) * (uint32_t)A.E + head * A.head_dim;
+            for (int rr = 0; rr < R; ++rr) pos[rr] = A.table[(int64_t)g * n + min((uint32_t)(rl * R + rr), n - 1u)];
+#pragma unroll
+            for (int rr = 0; rr < R; ++rr) pos[rr] = (uint32_t)max(0, min((int32_t)pos[rr], (int32_t)A.N - 1));
+        } else if (A.radix_stride) {
+            const uint32_t s = A.radix_stride, hi = g / s;
+#pragma unroll
+            for (int rr = 0; rr < R; ++rr) pos[rr] = (hi * n + min((uint32_t)(rl * R + rr), n - 1u)) * s + (g - hi * s);
+        } else {
+#pragma unroll
+            for (int rr = 0; rr < R; ++rr) {
+                const uint32_t slot = min((uint32_t)(rl * R + rr), n - 1u);
+                pos[rr] = stage_block(A, g, slot) * n + slot;
+            }
         }
+#pragma unroll
+        for (int rr = 0; rr < R; ++rr) row[rr] = pos[rr] * (uint32_t)A.E + head * A.head_dim;
     }
     // Between the loads and the stores of a tile: the compiler would otherwise keep the R x F element offsets it made for
     // the loads in registers across the steps instead of making them again.
     __device__ __forceinline__ void forget_offsets() {
 #pragma unroll
         for (int rr = 0; rr < R; ++rr) asm volatile("" : "+v"(row[rr]));
+        asm volatile("" : "+v"(fl));
     }
     // the row is one of the group's: it takes part in the steps (run) or lies past a context length (pass)
     __device__ __forceinline__ bool run(int rr) const { return rl * R + rr < live; }
@@ -102,23 +121,73 @@ struct AnyLane {
 
 template <typename T>
 __device__ __forceinline__ T* any_at(T* entry, uint32_t elem) {
-    return reinterpret_cast<T*>(reinterpret_cast<uintptr_t>(entry) + (uint32_t)(elem * sizeof(T)));
+    // (by way of an integer the address would lose its address space, and every load and store become a flat one)
+    return reinterpret_cast<T*>(const_cast<char*>(reinterpret_cast<const char*>(entry)) + (uint32_t)(elem * sizeof(T)));
 }
+
+// The weights of a lane times gamma, zero in features that do not exist.  All requested before any is waited for.
+template <int R, int F, bool LENGTHS>
+__device__ __forceinline__ void any_weights(const StageArgs& A, const AnyLane<R, F, LENGTHS>& L, int head, float (&wi)[F], float (&wj)[F]) {
+    const int64_t at = (int64_t)head * A.head_dim;
+    if (A.w_bf16) {
+        const uint16_t *i = static_cast<const uint16_t*>(A.W) + at, *j = i + A.E;
+        uint32_t ri[F], rj[F];
+#pragma unroll
+        for (int f = 0; f < F; ++f) { ri[f] = i[L.feat(f)]; rj[f] = j[L.feat(f)]; }
+#pragma unroll
+        for (int f = 0; f < F; ++f) { wi[f] = bf16_to_f32(ri[f]); wj[f] = bf16_to_f32(rj[f]); }
+    } else {
+        const float *i = static_cast<const float*>(A.W) + at, *j = i + A.E;
+#pragma unroll
+        for (int f = 0; f < F; ++f) { wi[f] = i[L.feat(f)]; wj[f] = j[L.feat(f)]; }
+    }
+#pragma unroll
+    for (int f = 0; f < F; ++f) {
+        wi[f] = L.has(f) ? A.tab.gamma * wi[f] : 0.f;
+        wj[f] = L.has(f) ? A.tab.gamma * wj[f] : 0.f;
+    }
+}
+
+// A lane's F adjacent features of a row, at any element: loads and stores of up to four words where the head is a whole number of
+// lanes.  Launches on x[16, 1005, 160], heads of 40, groups of 5, float32, us: one word at a time by flat instructions, over eight
+// rows each, with the weights one latency after the other and a loop over tiles: forward 17.3, backward 33.3 (20 of them without
+// its steps); weights behind the tile and no loop 17.0 and 30.7; adjacent features 15.8 and 28.3; global instructions 15.5 and 26.3.
+template <typename T, int F>
+struct __attribute__((packed, aligned(sizeof(T)))) AnyFrag {
+    T v[F];
+};
 
 // The loads of a tile, as raw words (converted by any_finish), so that those of all arrays of a tile are under way together.
 template <int R, int F, bool LENGTHS>
 __device__ __forceinline__ void any_issue(const void* base, int dtype, const AnyLane<R, F, LENGTHS>& L, float (&v)[R][F]) {
-    if (dtype == NCN_F32) {
+    if (L.whole) {
+        const uint32_t f0 = L.feat0();
+        if (dtype == NCN_F32) {
+#pragma unroll
+            for (int rr = 0; rr < R; ++rr) {
+                const auto q = *reinterpret_cast<const AnyFrag<float, F>*>(any_at(static_cast<const float*>(base) + L.entry, L.row[rr] + f0));
+#pragma unroll
+                for (int f = 0; f < F; ++f) v[rr][f] = q.v[f];
+            }
+        } else {
+#pragma unroll
+            for (int rr = 0; rr < R; ++rr) {
+                const auto q = *reinterpret_cast<const AnyFrag<uint16_t, F>*>(any_at(static_cast<const uint16_t*>(base) + L.entry, L.row[rr] + f0));
+#pragma unroll
+                for (int f = 0; f < F; ++f) v[rr][f] = __uint_as_float(q.v[f]);
+            }
+        }
+    } else if (dtype == NCN_F32) {
 #pragma unroll
         for (int rr = 0; rr < R; ++rr)
 #pragma unroll
-            for (int f = 0; f < F; ++f) v[rr][f] = *any_at(static_cast<const float*>(base) + L.entry, L.row[rr] + L.feat[f]);
+            for (int f = 0; f < F; ++f) v[rr][f] = *any_at(static_cast<const float*>(base) + L.entry, L.row[rr] + L.feat(f));
     } else {
 #pragma unroll
         for (int rr = 0; rr < R; ++rr)
 #pragma unroll
             for (int f = 0; f < F; ++f)
-                v[rr][f] = __uint_as_float(*any_at(static_cast<const uint16_t*>(base) + L.entry, L.row[rr] + L.feat[f]));
+                v[rr][f] = __uint_as_float(*any_at(static_cast<const uint16_t*>(base) + L.entry, L.row[rr] + L.feat(f)));
     }
 }
 template <int R, int F>
@@ -137,7 +206,7 @@ __device__ __forceinline__ void any_fill_padding(const AnyLane<R, F, LENGTHS>& L
 #pragma unroll
     for (int rr = 0; rr < R; ++rr)
 #pragma unroll
-        for (int f = 0; f < F; ++f) v[rr][f] = !L.run(rr) ? 0.f : L.has[f] ? v[rr][f] : missing;
+        for (int f = 0; f < F; ++f) v[rr][f] = !L.run(rr) ? 0.f : L.has(f) ? v[rr][f] : missing;
 }
 // for a tile whose steps are undone, which multiplies by 1/m each time: where (1/m)^n would leave the range of float32, zero
 __device__ __forceinline__ float any_missing_undone(const StepTable& S) { return S.m_pow_n > 1e-30f ? 1.f : 0.f; }
@@ -145,13 +214,39 @@ __device__ __forceinline__ float any_missing_undone(const StepTable& S) { return
 template <bool DEAD, int R, int F, bool LENGTHS>
 __device__ __forceinline__ void any_store(const StageArgs& A, const AnyLane<R, F, LENGTHS>& L, void* base0, void* base1, int dtype,
                                           const float (&p)[R][F], const float (&q)[R][F]) {
+    if (L.whole) {
+        const uint32_t f0 = L.feat0();
+#pragma unroll
+        for (int rr = 0; rr < R; ++rr)
+            if ((DEAD ? L.pass(A, rr) : L.run(rr)) && L.has(0)) {
+                const uint32_t at = L.row[rr] + f0;
+                if (dtype == NCN_F32) {
+                    AnyFrag<float, F> fp, fq;
+#pragma unroll
+                    for (int f = 0; f < F; ++f) { fp.v[f] = p[rr][f]; fq.v[f] = q[rr][f]; }
+                    *reinterpret_cast<AnyFrag<float, F>*>(any_at(static_cast<float*>(base0) + L.entry, at)) = fp;
+                    *reinterpret_cast<AnyFrag<float, F>*>(any_at(static_cast<float*>(base1) + L.entry, at)) = fq;
+                } else {
+                    AnyFrag<uint16_t, F> fp, fq;
+#pragma unroll
+                    for (int f = 0; f < F; ++f) {
+                        const uint32_t pq = pack_bf16x2(p[rr][f], q[rr][f]);
+                        fp.v[f] = (uint16_t)pq;
+                        fq.v[f] = (uint16_t)(pq >> 16);
+                    }
+                    *reinterpret_cast<AnyFrag<uint16_t, F>*>(any_at(static_cast<uint16_t*>(base0) + L.entry, at)) = fp;
+                    *reinterpret_cast<AnyFrag<uint16_t, F>*>(any_at(static_cast<uint16_t*>(base1) + L.entry, at)) = fq;
+                }
+            }
+        return;
+    }
 #pragma unroll
     for (int rr = 0; rr < R; ++rr)
         if (DEAD ? L.pass(A, rr) : L.run(rr)) {
 #pragma unroll
             for (int f = 0; f < F; ++f)
-                if (L.has[f]) {
-                    const uint32_t at = L.row[rr] + L.feat[f];
+                if (L.has(f)) {
+                    const uint32_t at = L.row[rr] + L.feat(f);
                     if (dtype == NCN_F32) {
                         *any_at(static_cast<float*>(base0) + L.entry, at) = p[rr][f];
                         *any_at(static_cast<float*>(base1) + L.entry, at) = q[rr][f];
@@ -212,13 +307,7 @@ __device__ __forceinline__ void for_each_row(const Fn& f) {
     L.place(A, lane);                                                                           \
     const int lr = 1 << L.lrl;                                                                  \
     const StepTable& S = A.tab;                                                                 \
-    float wi[F], wj[F];                                                                         \
-    _Pragma("unroll") for (int f = 0; f < F; ++f) {                                             \
-        const int64_t at = (int64_t)head * A.head_dim + L.feat[f];                              \
-        const int w_dtype = A.w_bf16 ? NCN_BF16 : NCN_F32;                                      \
-        wi[f] = L.has[f] ? S.gamma * load_elem(A.W, w_dtype, at) : 0.f;                         \
-        wj[f] = L.has[f] ? S.gamma * load_elem(A.W, w_dtype, at + A.E) : 0.f;                   \
-    }
+    float wi[F], wj[F];
 
 // INVERSE = false: x, xa -> y, ya (optional float32 copies);  true: y, ya -> x, xa
 template <int R, int F, bool TANH_ONLY, bool INVERSE, bool LENGTHS>
@@ -229,6 +318,7 @@ __global__ void __launch_bounds__(kBlockThreads, R * F <= 16 ? 4 : R * F <= 20 ?
         float x[R][F], a[R][F];
         any_issue(A.in0, A.in_dtype, L, x);
         any_issue(A.in1, A.in_dtype, L, a);
+        any_weights(A, L, head, wi, wj);   // behind the tile's own loads: one latency, not two
         any_finish(A.in_dtype, x);
         any_finish(A.in_dtype, a);
         if (LENGTHS) {   // rows past a context length pass through
@@ -280,16 +370,26 @@ __global__ void __launch_bounds__(kBlockThreads, R * F <= 16 ? 4 : R * F <= 20 ?
     }
 }
 
-template <int R, int F, bool TANH_ONLY, bool LENGTHS>
-__global__ void __launch_bounds__(kBlockThreads, R * F <= 10 ? 4 : R * F <= 16 ? 3 : 2) any_backward_kernel(const StageArgs A) {
+// LOOP = false: launches with a wave for every tile (tiles of up to 15 elements, whose loop builds need 16 to 24 registers more;
+// larger ones spill without it).  Three rows of five features run three waves per SIMD: at four, 16 registers spill and a backward
+// launch of the figures above takes 29.3 us.
+template <int R, int F, bool TANH_ONLY, bool LENGTHS, bool LOOP>
+__global__ void __launch_bounds__(kBlockThreads, R * F <= (LOOP ? 10 : 12) ? 4 : R * F <= 16 ? 3 : 2) any_backward_kernel(const StageArgs A) {
     NCN_ANY_PROLOGUE
-    float dwi[F], dwj[F], wiku[F];
+    constexpr bool kKuW = LOOP || R * F <= 10;   // ku Wi' kept beside the weights, where there are registers for it
+    float dwi[F], dwj[F], wiku[kKuW ? F : 1];
 #pragma unroll
-    for (int f = 0; f < F; ++f) {
-        dwi[f] = dwj[f] = 0.f;
-        wiku[f] = S.ku * wi[f];
-    }
-    for (uint32_t t = gwave / A.n_head; t < A.total_tiles; t += tile_step) {
+    for (int f = 0; f < F; ++f) dwi[f] = dwj[f] = 0.f;
+    auto weights = [&]() {
+        any_weights(A, L, head, wi, wj);
+        if constexpr (kKuW) {
+#pragma unroll
+            for (int f = 0; f < F; ++f) wiku[f] = S.ku * wi[f];
+        }
+    };
+    if constexpr (LOOP) weights();
+    uint32_t t = gwave / A.n_head;
+    if (t < A.total_tiles) do {
         L.rows(A, t, head);
         float Y[R][F], B[R][F], G[R][F], P[R][F];
         any_issue(A.in0, A.in_dtype, L, Y);
@@ -303,6 +403,7 @@ __global__ void __launch_bounds__(kBlockThreads, R * F <= 10 ? 4 : R * F <= 16 ?
 #pragma unroll
                 for (int f = 0; f < F; ++f) P[rr][f] = 0.f;
         }
+        if constexpr (!LOOP) weights();   // behind the tile's own loads: one latency, not two
         any_finish(A.in_dtype, Y);
         any_finish(A.in_dtype, B);
         any_finish(A.g_dtype, G);
@@ -371,11 +472,12 @@ __global__ void __launch_bounds__(kBlockThreads, R * F <= 10 ? 4 : R * F <= 16 ?
 #pragma unroll
                 for (int rr = 0; rr < R; ++rr) {
                     const float rho_w = krho * rh[rr];
+                    const float rho_ku = kKuW ? rh[rr] : S.ku * rh[rr];
                     rhosum += rh[rr];
 #pragma unroll
                     for (int f = 0; f < F; ++f) {
                         dwi[f] = fmaf(rho_w, Y[rr][f], dwi[f]);
-                        G[rr][f] = fmaf(rh[rr], wiku[f], G[rr][f]);
+                        G[rr][f] = fmaf(rho_ku, kKuW ? wiku[f] : wi[f], G[rr][f]);
                         if (rr != jr) P[rr][f] = fmaf(S.om, G[rr][f], P[rr][f]);
                     }
                 }
@@ -408,7 +510,7 @@ __global__ void __launch_bounds__(kBlockThreads, R * F <= 10 ? 4 : R * F <= 16 ?
             scale_tile<R, F>(Y, B, S.inv_kappa, S.inv_b_scale);
             any_store<false>(A, L, A.aux0, A.aux1, NCN_F32, Y, B);
         }
-    }
+    } while (LOOP && (t += tile_step) < A.total_tiles);
     // dW: lanes holding the same features -> one value; this wave owns slot (gwave / n_head, head)
     any_sum_span<F>(dwi, L.lfl, 6);
     any_sum_span<F>(dwj, L.lfl, 6);
@@ -416,9 +518,9 @@ __global__ void __launch_bounds__(kBlockThreads, R * F <= 10 ? 4 : R * F <= 16 ?
         float* out = A.dw_partials + (int64_t)(gwave / A.n_head) * (2 * A.E) + (int64_t)head * A.head_dim;
 #pragma unroll
         for (int f = 0; f < F; ++f)
-            if (L.has[f]) {
-                out[L.feat[f]] = dwi[f];
-                out[A.E + L.feat[f]] = dwj[f];
+            if (L.has(f)) {
+                out[L.feat(f)] = dwi[f];
+                out[A.E + L.feat(f)] = dwj[f];
             }
     }
 }

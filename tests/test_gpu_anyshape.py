@@ -179,3 +179,23 @@ def test_bfloat16(M, case):
     _, _, dx, dxa, dW = M.backward_stages(sy, sya, dy.cuda(), dya.cuda(), W, 0.9, 0, n, C, 0, 1, want_inputs=False)
     for got, want in ((y, ref[0]), (ya, ref[1]), (dx, ref[2]), (dxa, ref[3]), (dW[0], ref[4][0])):
         assert O.rel_err(got, want) < 2e-2
+
+
+@pytest.mark.parametrize("n,ec,C", [(3, 3, 1), (5, 7, 2), (2, 10, 1)])   # heads that end with a lane, inside one, two lanes of five
+def test_more_tiles_than_partial_rows(n, ec, C):
+    """The backward then loops over tiles; each half of the batch has a wave for every tile."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from ncn_cuda_amd import ncn_cuda_module as M
+    batch, E = 16384 + 200, ec * C
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    x, xa, dy, dya = (torch.randn(batch, n, E, generator=gen, device="cuda") for _ in range(4))
+    W = torch.randn(2 * E, generator=gen, device="cuda") / n ** 0.5
+    y, ya = M.forward_stages(x, xa, W, 0.9, 0, n, C, 0, 1)
+    _, _, dx, dxa, dW = M.backward_stages(y, ya, dy, dya, W, 0.9, 0, n, C, 0, 1, want_inputs=False)
+    halves = [M.backward_stages(*(t[s].contiguous() for t in (y, ya, dy, dya)), W, 0.9, 0, n, C, 0, 1, want_inputs=False)
+              for s in (slice(0, batch // 2), slice(batch // 2, batch))]
+    # the builds with and without the loop round ku rh Wi' differently, by a few units in the last place
+    assert O.rel_err(dx, torch.cat([h[2] for h in halves])) < 1e-6 and O.rel_err(dxa, torch.cat([h[3] for h in halves])) < 1e-6
+    want = sum(h[4].double() for h in halves)
+    assert ((dW.double() - want).norm() / want.norm()) < 1e-5    # sums of some 10^5 products in float32, in other orders
