@@ -66,6 +66,7 @@ constexpr float kM = 0.9f;   // the m of the Python surface (ncn_cuda_module.M_D
 void check(int rc, const char* what) {
     TORCH_CHECK(rc == 0, what, " failed: ", lib.error_string(rc), " (code ", rc, ")");
 }
+bool is_activation(at::ScalarType t) { return t == at::kFloat || t == at::kBFloat16; }
 int code_of(at::ScalarType t) { return t == at::kFloat ? NCN_F32 : NCN_BF16; }
 int weight_flag(const Tensor& W) { return W.scalar_type() == at::kBFloat16 ? NCN_W_BF16 : 0; }
 void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
@@ -81,6 +82,39 @@ Tensor prepared(const Tensor& t) {
     if (!t.defined()) return t;
     Tensor c = t.detach().contiguous();
     return aligned(c) ? c : c.clone(at::MemoryFormat::Contiguous);
+}
+
+// ---- what reaches a backward -------------------------------------------------------------------------------------
+// Saved tensors come back from the caller's hooks, from anywhere and as anything, and a saved table or length is the caller's own
+// tensor: what a kernel could not read, or would read past the end of, is refused with the errors of the Python nodes.
+void on_device(const Tensor& t, const Tensor& like, const char* what) {
+    TORCH_CHECK(t.is_cuda() && t.device() == like.device(), "all tensors must live on one GPU: ", what, " is on ", t.device(),
+                ", the gradients on ", like.device());
+}
+Tensor returned(const Tensor& t, at::IntArrayRef sizes, const Tensor& like, const char* what) {
+    on_device(t, like, what);
+    TORCH_CHECK_VALUE(t.sizes().equals(sizes), what, " came back as ", t.sizes(), ", not as ", sizes);
+    TORCH_CHECK_TYPE(is_activation(t.scalar_type()), what, " must be float32 or bfloat16, came back as ", t.scalar_type());
+    return prepared(t);
+}
+// saved outputs of a call: [batch, N, E] of either type, or two bfloat16 planes of that
+Tensor returned_output(const Tensor& t, at::IntArrayRef sizes, const Tensor& like, const char* what) {
+    if (t.dim() != 4) return returned(t, sizes, like, what);
+    TORCH_CHECK_TYPE(t.scalar_type() == at::kBFloat16, what, ": two planes must be bfloat16, came back as ", t.scalar_type());
+    return returned(t, {2, sizes[0], sizes[1], sizes[2]}, like, what);
+}
+Tensor returned_weights(const Tensor& t, int64_t numel, const Tensor& like) {
+    on_device(t, like, "W");
+    TORCH_CHECK_VALUE(t.numel() == numel, "W must hold ", numel, " values, came back with ", t.numel());
+    TORCH_CHECK_TYPE(is_activation(t.scalar_type()), "W must be float32 or bfloat16, came back as ", t.scalar_type());
+    return prepared(t);
+}
+Tensor current_index(const Tensor& t, int64_t numel, const Tensor& like, const char* what) {
+    if (!t.defined()) return t;
+    on_device(t, like, what);
+    TORCH_CHECK_VALUE(t.numel() == numel, what, " must hold ", numel, " values, now holds ", t.numel());
+    TORCH_CHECK_TYPE(t.scalar_type() == at::kInt || t.scalar_type() == at::kLong, what, " must be int32 or int64, now is ", t.scalar_type());
+    return prepared(t.to(at::kInt));
 }
 
 // ---- what a call is ---------------------------------------------------------------------------------------------
@@ -114,7 +148,6 @@ bool usable(PyObject* o, Tensor& out) {
     out = t;
     return true;
 }
-bool is_activation(at::ScalarType t) { return t == at::kFloat || t == at::kBFloat16; }
 
 bool to_int(PyObject* o, int& out) {
     if (!PyLong_CheckExact(o)) return false;
@@ -188,11 +221,14 @@ Call kept(AutogradContext* ctx) {
                 static_cast<int>(v[7])};
 }
 // dy, dya as they arrive: missing ones stay missing but for a missing dy, which is zeros; false: there is nothing to do
-bool gradients(const variable_list& grads, Tensor& dy, Tensor& dya) {
-    dy = prepared(grads[0]);
-    dya = prepared(grads[1]);
-    if (!dy.defined() && !dya.defined()) return false;
+bool gradients(const variable_list& grads, const Call& c, Tensor& dy, Tensor& dya) {
+    const Tensor& first = grads[0].defined() ? grads[0] : grads[1];
+    if (!first.defined()) return false;
+    const int64_t sizes[] = {c.shape.batch, c.shape.N, c.shape.E};
+    if (grads[0].defined()) dy = returned(grads[0], sizes, first, "dy");
+    if (grads[1].defined()) dya = returned(grads[1], sizes, first, "dya");
     if (!dy.defined()) dy = at::zeros_like(dya);
+    TORCH_CHECK_TYPE(!dya.defined() || dya.scalar_type() == dy.scalar_type(), "dy and dya must both be float32 or bfloat16");
     return true;
 }
 
@@ -260,13 +296,15 @@ struct StageNode : torch::autograd::Function<StageNode> {
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
         Tensor dy, dya;
-        if (!gradients(grads, dy, dya)) return variable_list(5);
-        const variable_list saved = ctx->get_saved_variables();
-        const Tensor y = prepared(saved[0]), ya = prepared(saved[1]), W = prepared(saved[2]);
         const Call c = kept(ctx);
+        if (!gradients(grads, c, dy, dya)) return variable_list(5);
+        const variable_list saved = ctx->get_saved_variables();
+        const Tensor y = returned_output(saved[0], dy.sizes(), dy, "y"), ya = returned_output(saved[1], dy.sizes(), dy, "ya");
+        TORCH_CHECK_TYPE(y.sizes().equals(ya.sizes()) && y.scalar_type() == ya.scalar_type(), "y and ya came back as different kinds");
+        const Tensor W = returned_weights(saved[2], 2 * c.shape.E, dy);
         Grouping g;
-        if (ctx->saved_data.count("table")) g.table = ctx->saved_data["table"].toTensor();
-        if (ctx->saved_data.count("lengths")) g.lengths = ctx->saved_data["lengths"].toTensor();
+        if (ctx->saved_data.count("table")) g.table = current_index(ctx->saved_data["table"].toTensor(), c.shape.N, dy, "group_index");
+        if (ctx->saved_data.count("lengths")) g.lengths = current_index(ctx->saved_data["lengths"].toTensor(), c.shape.batch, dy, "ctx_len");
         const c10::DeviceGuard guard(dy.device());
         const at::ScalarType dtype = ctx->saved_data["bf16"].toBool() ? at::kBFloat16 : at::kFloat;
         const Tensor dx = empty(dy.sizes(), dtype, dy), dxa = empty(dy.sizes(), dtype, dy);
@@ -398,17 +436,26 @@ struct StackNode : torch::autograd::Function<StackNode> {
         ctx->set_materialize_grads(false);
         ctx->save_for_backward({W, saves, is_f32 ? y : Tensor(), is_f32 ? ya : Tensor()});
         keep(ctx, c);
-        ctx->saved_data["plan"] = std::vector<int64_t>{p.max_range, p.max_saves, p.backward_bytes, is_f32};
+        ctx->saved_data["plan"] = std::vector<int64_t>{p.max_range, p.max_saves, p.backward_bytes, is_f32, n_saves};
         ctx->saved_data["sizes"] = sizes_value(Ws);
         return {y, ya};
     }
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
         Tensor dy, dya;
         const Call c = kept(ctx);
-        if (!gradients(grads, dy, dya)) return variable_list(4 + c.count);
+        if (!gradients(grads, c, dy, dya)) return variable_list(4 + c.count);
         const variable_list saved = ctx->get_saved_variables();
-        const Tensor W = prepared(saved[0]), saves = prepared(saved[1]), y = prepared(saved[2]), ya = prepared(saved[3]);
         const std::vector<int64_t> p = ctx->saved_data["plan"].toIntVector();
+        // (other types than the library's are read as float32, as the Python node does)
+        const Tensor W = returned_weights(is_activation(saved[0].scalar_type()) ? saved[0] : saved[0].to(at::kFloat), 2 * c.shape.E * c.count, dy);
+        Tensor saves, y, ya;
+        if (p[4]) saves = returned(saved[1], {p[4], 2, dy.size(0), dy.size(1), dy.size(2)}, dy, "a kept activation");
+        if (p[3]) {
+            y = returned(saved[2], dy.sizes(), dy, "y");
+            ya = returned(saved[3], dy.sizes(), dy, "ya");
+        }
+        for (const Tensor& t : {saves, y, ya})
+            TORCH_CHECK_TYPE(!t.defined() || t.scalar_type() == at::kFloat, "a stack keeps float32, which came back as ", t.scalar_type());
         const c10::DeviceGuard guard(dy.device());
         const at::ScalarType dtype = p[3] ? at::kFloat : at::kBFloat16;
         const Tensor dx = empty(dy.sizes(), dtype, dy), dxa = empty(dy.sizes(), dtype, dy);
@@ -474,9 +521,11 @@ struct RadixNode : torch::autograd::Function<RadixNode> {
     static variable_list backward(AutogradContext* ctx, variable_list grads) {
         Tensor dy, dya;
         const Call c = kept(ctx);
-        if (!gradients(grads, dy, dya)) return variable_list(3 + c.count);
+        if (!gradients(grads, c, dy, dya)) return variable_list(3 + c.count);
         const variable_list saved = ctx->get_saved_variables();
-        const Tensor W = prepared(saved[0]), y = prepared(saved[1]), ya = prepared(saved[2]);
+        const Tensor W = prepared(returned_weights(saved[0], 2 * c.shape.E * c.count, dy).to(at::kFloat));
+        const Tensor y = returned(saved[1], dy.sizes(), dy, "y"), ya = returned(saved[2], dy.sizes(), dy, "ya");
+        TORCH_CHECK_TYPE(y.scalar_type() == ya.scalar_type(), "y and ya came back as different types");
         const c10::DeviceGuard guard(dy.device());
         const Tensor dx = empty(dy.sizes(), at::kFloat, dy), dxa = empty(dy.sizes(), at::kFloat, dy);
         const Tensor dW = empty({c.count, 2 * c.shape.E}, at::kFloat, dy);
@@ -484,7 +533,7 @@ struct RadixNode : torch::autograd::Function<RadixNode> {
         const size_t ws_bytes = lib.workspace_bytes(&c.shape) +
                                 (c.count > 1 ? 2 * ((static_cast<size_t>(dy.numel()) * 4 + 255) / 256 * 256) : 0);
         const Tensor ws = bytes(ws_bytes, dy);
-        check(lib.backward_radix(ptr(y), ptr(ya), NCN_F32, ptr(dy), ptr(dya), code_of(dy.scalar_type()), ptr(dx), ptr(dxa),
+        check(lib.backward_radix(ptr(y), ptr(ya), code_of(y.scalar_type()), ptr(dy), ptr(dya), code_of(dy.scalar_type()), ptr(dx), ptr(dxa),
                                  NCN_F32, nullptr, nullptr, f32(W), static_cast<float*>(ptr(dW)), ptr(ws), ws_bytes, &c.shape,
                                  c.first, c.count, c.alpha, kM, c.activation, stream_of(dy)),
               "ncn_backward_radix");

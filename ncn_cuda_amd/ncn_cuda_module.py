@@ -411,8 +411,21 @@ def stack_forward(x, xa, W, alpha, activation, cache_dim, nhead, first_stage, n_
 def stack_backward(plan, y, ya, saves, dy, dya, W):
     """dx, dxa (in the dtype of the stack's inputs) and dW[n_stages, 2E] (in that of W) of a stack_forward call; y, ya its
     float32 outputs or None.  dya may be None (zeros)."""
-    like = y if y is not None else saves[0, 0]
-    if dy.shape != like.shape or (dya is not None and dya.shape != dy.shape):
+    shape = (plan.shape.batch, plan.shape.N, plan.shape.E)
+    kept = plan.ranges - (plan.io_dtype == torch.float32)
+    # (saved tensors may have been through hooks of the caller's: the library reads them as the plan says)
+    for name, t, want in (("y", y, shape if plan.io_dtype == torch.float32 else None),
+                          ("ya", ya, shape if plan.io_dtype == torch.float32 else None),
+                          ("saves", saves, (kept, 2) + shape if kept else None)):
+        if want is None:
+            continue
+        if t is None or tuple(t.shape) != want:
+            raise ValueError(f"{name} must be {want}, got {None if t is None else tuple(t.shape)}")
+        if t.dtype != torch.float32:
+            raise TypeError(f"{name} must be float32, got {t.dtype}")
+    if W.numel() != plan.args[1] * 2 * shape[2]:
+        raise ValueError(f"W must hold {plan.args[1]} x 2E = {plan.args[1] * 2 * shape[2]} values, got {W.numel()}")
+    if tuple(dy.shape) != shape or (dya is not None and dya.shape != dy.shape):
         raise ValueError("dy/dya must have the shape of y")
     if dy.dtype not in _DTYPES or (dya is not None and dya.dtype != dy.dtype):
         raise TypeError("dy and dya must both be float32 or bfloat16")

@@ -157,6 +157,72 @@ def test_hooks_transforms_and_modes(P):
     assert not g.requires_grad
 
 
+# what a hook gives back in place of one saved tensor, and what that raises: from y, ya, W on, or (a stack) the kept activations
+UNPACKED = [("on the host", lambda t: t.cpu(), RuntimeError), ("half", lambda t: t.half(), (TypeError, ValueError)),
+            ("a part", lambda t: t.flatten()[:-4], ValueError), ("transposed", lambda t: t.transpose(0, -1)[..., :1], ValueError)]
+
+
+@pytest.mark.parametrize("what,unpack,error", UNPACKED, ids=[u[0].replace(" ", "_") for u in UNPACKED])
+@pytest.mark.parametrize("kind,n,L,dtype", [("stage", 16, 1, F), ("stage", 16, 1, H), ("stack", 2, 8, F), ("stack", 2, 8, H), ("radix", 2, 5, F),
+                                            ("lengths", 8, 1, F)], ids=lambda v: str(v).replace("torch.", ""))
+def test_saved_tensors_that_do_not_come_back_as_they_were(P, kind, n, L, dtype, what, unpack, error):
+    """Refused by either node before anything is launched: a kernel would read them past their end."""
+    for f in kinds(P, kind, n, 4):
+        x, xa, Ws, dy, dya = leaves(n, 8, 4, 32, L, dtype, F)
+        saved = []
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: saved.append(t) or t, lambda t: t):
+            f(x, xa, Ws)
+        for which in range(len(saved)):
+            if kind == "stack" and what == "half" and which == 0:
+                continue   # a stack reads weights of any type as float32
+            count = iter(range(100))
+            hooks = torch.autograd.graph.saved_tensors_hooks(lambda t: (next(count), t), lambda k: unpack(k[1]) if k[0] == which else k[1])
+            with hooks:
+                y, ya = f(x, xa, Ws)
+            with pytest.raises(error):
+                torch.autograd.grad([y, ya], [x, xa, *Ws], [dy, dya])
+
+
+@pytest.mark.parametrize("kind,n,L", [("stage", 16, 1), ("radix", 2, 5)])
+def test_saved_tensors_kept_as_bfloat16(P, kind, n, L):
+    """A hook that packs float32 into bfloat16: both nodes take the outputs in the type they come back in."""
+    native, python = kinds(P, kind, n, 4)
+    x, xa, Ws, dy, dya = leaves(n, 8, 4, 32, L, F, F)
+    got = []
+    for f in (native, python):
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t.to(H), lambda t: t):
+            y, ya = f(x, xa, Ws)
+        got.append(torch.autograd.grad([y, ya], [x, xa, *Ws], [dy, dya]))
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+
+
+def test_table_that_changes_before_the_backward(P):
+    """The table and the lengths are the caller's tensors: what they hold by then is read, if the kernels can read it."""
+    ext = P[3]
+    x, xa, Ws, dy, dya = leaves(8, 8, 4, 6, 1, F, F)
+    N = x.shape[1]
+    call = lambda table, lens: ext.table_stage(x, xa, Ws[0], table, lens, ALPHA, 0, 8, 4)
+    base = lambda: torch.randperm(N, generator=torch.Generator().manual_seed(1)).to(torch.int32).cuda()
+    lengths = lambda: torch.tensor([N - 3, N // 2], dtype=torch.int32).cuda()
+    want = torch.autograd.grad(call(base(), lengths()), [x, xa, Ws[0]], [dy, dya])
+    for change, error in [(lambda t: t.resize_(4 if t.numel() > 4 else 1), ValueError), (lambda t: setattr(t, "data", t.data.cpu()), RuntimeError),
+                          (lambda t: setattr(t, "data", t.data.float()), TypeError), (lambda t: setattr(t, "data", t.data.long()), None)]:
+        for which in (0, 1):
+            args = [base(), lengths()]
+            out = call(*args)
+            try:
+                change(args[which])
+            except RuntimeError:   # torch itself refuses: nothing changed
+                continue
+            if error is None:
+                for a, b in zip(torch.autograd.grad(out, [x, xa, Ws[0]], [dy, dya]), want):
+                    assert torch.equal(a, b)
+            else:
+                with pytest.raises(error):
+                    torch.autograd.grad(out, [x, xa, Ws[0]], [dy, dya])
+
+
 def test_streams_and_threads(P):
     import threading
     modules = P[0]

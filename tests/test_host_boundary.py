@@ -558,3 +558,29 @@ def test_native_nodes_leave_cpu_calls_to_the_python_nodes():
     for bad in ((), (1,) * 3, (0,) * len(_native.ENTRIES), None):
         with pytest.raises((TypeError, ValueError)):
             ext.bind(bad)
+
+
+def test_stack_backward_checks_what_was_kept():
+    """Kept activations may have been through hooks of the caller's: another size or type is refused, no GPU needed."""
+    import torch
+
+    from ncn_cuda_amd import _lib
+    from ncn_cuda_amd import ncn_cuda_module as M
+    shape = _lib.NcnShape(2, 4096, 32, 4, 2)
+    x, W = torch.zeros(2, 4096, 32), torch.zeros(12, 64)
+    for dtype in (torch.float32, torch.bfloat16):
+        plan = M.StackPlan(shape, 0, 12, 0.9, 0.9, 0, 13, 12, dtype)
+        kept = plan.ranges - (dtype == torch.float32)
+        assert plan.ranges > 1
+        good = dict(y=x, ya=x, saves=torch.zeros(kept, 2, 2, 4096, 32), dy=x, dya=None, W=W)
+        if dtype == torch.bfloat16:
+            good.update(y=None, ya=None)
+        with pytest.raises(RuntimeError, match="GPU only"):   # everything fits, but for the device
+            M.stack_backward(plan, **good)
+        bad = [("saves", good["saves"][:-1], ValueError), ("saves", good["saves"].half(), TypeError), ("saves", None, ValueError),
+               ("W", W[:-1], ValueError), ("dy", x[:1], ValueError), ("dya", x[:1], ValueError)]
+        if dtype == torch.float32:
+            bad += [("y", x[:1], ValueError), ("ya", x.bfloat16(), TypeError), ("y", None, ValueError)]
+        for name, value, error in bad:
+            with pytest.raises(error):
+                M.stack_backward(plan, **{**good, name: value})
