@@ -187,31 +187,59 @@ def build(verbose=False, force=True):
 TORCH_SOURCE = "ncn_torch.cpp"
 TORCH_LIB_PATH = os.path.join(PKG_DIR, "_ncn_torch.so")
 TORCH_ID_MARKER = "NCN_TORCH_ID="
+TORCH_FOR_MARKER = "NCN_TORCH_FOR="   # followed by the torch and the Python that the file was built for, and a semicolon
 TORCH_FLAGS = ["-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1"]
 TORCH_LIBS = ["c10", "c10_hip", "torch_cpu", "torch", "torch_python"]
 
 
 def torch_source_id():
     """Hash of what _ncn_torch.so is made from: its source, the C ABI's header, its flags, and the torch and Python it is for."""
-    import torch
     h = hashlib.sha256()
     h.update(_read(os.path.join(CSRC, TORCH_SOURCE)) + b"\0" + _read(os.path.join(INCLUDE, "ncn_hip.h")) + b"\0")
-    h.update(" ".join(TORCH_FLAGS + TORCH_LIBS + [torch.__version__, sys.version.split()[0]]).encode())
+    h.update(" ".join(TORCH_FLAGS + TORCH_LIBS + [torch_in_use()]).encode())
     return h.hexdigest()[:16]
 
 
-def torch_library_id(path=None):
-    """The id compiled into _ncn_torch.so (read from the file, nothing is loaded), or None."""
+def torch_in_use():
+    """The torch and the Python of this process."""
+    import torch
+    return f"{torch.__version__} {sys.version.split()[0]}"
+
+
+def _text_behind(marker, path, length=None):
     try:
         data = _read(TORCH_LIB_PATH if path is None else path)
     except OSError:
         return None
-    k = data.find(TORCH_ID_MARKER.encode())
-    return data[k + len(TORCH_ID_MARKER):k + len(TORCH_ID_MARKER) + 16].decode("ascii", "replace") if k >= 0 else None
+    k = data.find(marker.encode())
+    if k < 0:
+        return None
+    k += len(marker)
+    end = k + length if length else data.find(b";", k)
+    return data[k:end].decode("ascii", "replace")
+
+
+def torch_library_id(path=None):
+    """The id compiled into _ncn_torch.so (read from the file, nothing is loaded), or None."""
+    return _text_behind(TORCH_ID_MARKER, path, 16)
+
+
+def torch_library_for(path=None):
+    """What _ncn_torch.so was built for, as torch_in_use() says it (read from the file, nothing is loaded), or None."""
+    return _text_behind(TORCH_FOR_MARKER, path)
 
 
 def have_cxx():
     return shutil.which("g++") is not None
+
+
+def _rocm_includes():
+    """Where HIP's headers may be: no hipcc is needed to compile against them."""
+    homes = [os.environ.get("ROCM_PATH"), os.environ.get("ROCM_HOME")]
+    if shutil.which("hipcc"):
+        homes.append(os.path.dirname(os.path.dirname(os.path.realpath(shutil.which("hipcc")))))
+    found = [os.path.join(h, "include") for h in homes if h] + ["/opt/rocm/include"]
+    return [i for i in dict.fromkeys(found) if os.path.isdir(i)]
 
 
 def build_torch(verbose=False, force=True):
@@ -228,11 +256,11 @@ def build_torch(verbose=False, force=True):
             if not have_cxx():
                 raise RuntimeError("g++ not found: cannot build _ncn_torch.so")
             root = os.path.dirname(torch.__file__)
-            rocm = os.path.dirname(os.path.dirname(os.path.realpath(_hipcc())))
             include = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
-                       sysconfig.get_paths()["include"], os.path.join(rocm, "include"), "/opt/rocm/include"]
+                       sysconfig.get_paths()["include"], *_rocm_includes()]
             tmp = f"{TORCH_LIB_PATH}.{os.getpid()}.tmp"
             cmd = ["g++", *TORCH_FLAGS, f'-DNCN_TORCH_ID_TEXT="{TORCH_ID_MARKER}{want}"',
+                   f'-DNCN_TORCH_FOR_TEXT="{TORCH_FOR_MARKER}{torch_in_use()};"',
                    f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
                    *(a for i in include for a in ("-isystem", i)), os.path.join(CSRC, TORCH_SOURCE), "-o", tmp,
                    "-L", os.path.join(root, "lib"), *("-l" + x for x in TORCH_LIBS)]

@@ -28,22 +28,28 @@ _ext = None
 
 
 def ext():
-    """The extension module, loaded and bound once; built first if it is missing or made from other sources."""
+    """The extension module, loaded and bound once; built first if it is missing or made from other sources.  Where that cannot
+    be done the nodes in Python run instead, which is said once and remembered: the same kernels, more host time."""
     global _ext
     if _ext is None:
-        _ext = _load()
+        lib = _lib.load()   # the kernels themselves have no substitute: this raises
+        try:
+            _ext = _load(lib)
+        except Exception as exc:
+            print(f"ncn_cuda_amd: warning: autograd nodes run in Python, _ncn_torch.so cannot be used: {exc}", file=sys.stderr)
+            _ext = _PythonNodes
     return _ext
 
 
-def _load():
+def _load(lib):
     from . import _build
-    lib = _lib.load()
-    if _build.have_sources() and _build.torch_library_id() != _build.torch_source_id():
-        if not _build.have_cxx():
-            print("ncn_cuda_amd: warning: _ncn_torch.so is missing or not made for this source and torch, and there is no g++ "
-                  "here to build it: autograd nodes run in Python", file=sys.stderr)
-            return _PythonNodes
-        print("ncn_cuda_amd: building _ncn_torch.so with g++ (half a minute)", file=sys.stderr)
+    if not _build.have_sources():
+        made_for = _build.torch_library_for()
+        if made_for != _build.torch_in_use():
+            raise ImportError("it is missing" if made_for is None else f"it was built for torch and Python {made_for}")
+    elif _build.torch_library_id() != _build.torch_source_id():
+        if _build.have_cxx():
+            print("ncn_cuda_amd: building _ncn_torch.so with g++ (half a minute)", file=sys.stderr)
         _build.build_torch(force=False)
     from . import _ncn_torch
     _ncn_torch.bind(tuple(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in ENTRIES))

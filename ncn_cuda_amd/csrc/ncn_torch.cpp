@@ -34,6 +34,9 @@
 #ifndef NCN_TORCH_ID_TEXT
 #define NCN_TORCH_ID_TEXT "NCN_TORCH_ID=0000000000000000"
 #endif
+#ifndef NCN_TORCH_FOR_TEXT
+#define NCN_TORCH_FOR_TEXT "NCN_TORCH_FOR=unknown;"
+#endif
 
 namespace {
 
@@ -601,5 +604,6 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_ncn_torch", nullptr, -1, methods,
 }  // namespace
 
 extern "C" __attribute__((visibility("default"))) const char* ncn_torch_id() { return NCN_TORCH_ID_TEXT; }
+extern "C" __attribute__((visibility("default"))) const char* ncn_torch_for() { return NCN_TORCH_FOR_TEXT; }
 
 PyMODINIT_FUNC PyInit__ncn_torch() { return PyModule_Create(&module); }

@@ -584,3 +584,70 @@ def test_stack_backward_checks_what_was_kept():
         for name, value, error in bad:
             with pytest.raises(error):
                 M.stack_backward(plan, **{**good, name: value})
+
+
+def test_native_nodes_that_cannot_be_had_are_done_without(monkeypatch, capsys):
+    """Any failure to build, find or import _ncn_torch.so leaves the Python nodes in its place: said once, not tried again."""
+    import sys
+
+    from ncn_cuda_amd import _build, _lib, _native
+
+    def outcome(**patches):
+        with monkeypatch.context() as m:
+            m.setattr(_native, "_ext", None)
+            for name, value in patches.items():
+                m.setattr(_build, name, value)
+            capsys.readouterr()
+            got = _native.ext()
+            assert _native.ext() is got
+            return got, capsys.readouterr().err
+
+    builds = []
+
+    def fails(**kw):
+        builds.append(1)
+        raise OSError("read-only file system")
+
+    stale = dict(torch_library_id=lambda: "0" * 16, build_torch=fails)
+    got, said = outcome(**stale)
+    assert got is _native._PythonNodes and len(builds) == 1 and said.count("read-only file system") == 1
+    assert got.stage(1, 2, 3) is None and got.stack() is None
+    # no g++: build_torch says so
+    got, said = outcome(torch_library_id=lambda: None, have_cxx=lambda: False, torch_source_id=lambda: "1" * 16)
+    assert got is _native._PythonNodes and "g++ not found" in said
+    # without sources, a module for this torch is taken and no other is
+    assert _build.torch_library_for() == _build.torch_in_use()
+    got, said = outcome(have_sources=lambda: False)
+    assert got.__name__.endswith("_ncn_torch") and not said
+    got, said = outcome(have_sources=lambda: False, torch_in_use=lambda: "1.0 3.0")
+    assert got is _native._PythonNodes and "built for torch" in said
+    got, said = outcome(have_sources=lambda: False, torch_library_for=lambda: None)
+    assert got is _native._PythonNodes and "missing" in said
+    # an import that fails
+    with monkeypatch.context() as m:
+        m.setitem(sys.modules, "ncn_cuda_amd._ncn_torch", None)
+        m.delattr(sys.modules["ncn_cuda_amd"], "_ncn_torch", raising=False)
+        got, said = outcome()
+    assert got is _native._PythonNodes and said.count("warning") == 1
+    # the kernels have no substitute
+    with monkeypatch.context() as m, pytest.raises(RuntimeError, match="no kernels"):
+        m.setattr(_native, "_ext", None)
+        m.setattr(_lib, "load", lambda: (_ for _ in ()).throw(RuntimeError("no kernels")))
+        _native.ext()
+
+
+def test_native_nodes_are_compiled_without_hipcc(monkeypatch):
+    """Headers are all that is needed: the command that build_torch would run names them, and no hipcc is looked for."""
+    from ncn_cuda_amd import _build
+    monkeypatch.setattr(_build, "_hipcc", lambda: (_ for _ in ()).throw(RuntimeError("hipcc not found")))
+    monkeypatch.setattr(_build.shutil, "which", lambda name: None if name == "hipcc" else "/usr/bin/" + name)
+    monkeypatch.setattr(_build, "torch_library_id", lambda: None)
+    seen = []
+
+    class Refused:
+        returncode, stdout, stderr = 1, "", "stopped here"
+
+    monkeypatch.setattr(_build.subprocess, "run", lambda cmd, **kw: seen.append(cmd) or Refused)
+    with pytest.raises(RuntimeError, match="stopped here"):
+        _build.build_torch(force=True)
+    assert "/opt/rocm/include" in seen[0] and any(a.startswith("-DNCN_TORCH_FOR_TEXT=") for a in seen[0])
