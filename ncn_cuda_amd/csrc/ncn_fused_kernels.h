@@ -73,7 +73,7 @@ struct FusedArgs {
     int32_t in_dtype, g_dtype, out_dtype, w_bf16;
     uint32_t ring_magic;      // 0 when `ring` is a power of two, else ceil(2^32 / ring): closed passes divide by the ring
     // the radix kernels (ncn_radix_kernels.h) read: class_stride = n^a in rows, ring = n^k rows per window, window = rows /
-    // n_cache, class_groups = workgroup-loads per batch entry, closed = 1
+    // n_cache, class_groups = workgroup-loads per batch entry, or 0: entry_windows .. all_windows
     uint32_t class_stride;    // S0, in blocks
     uint32_t ring;            // sub-blocks per class = groups / S0 (a power of two, or an odd number times one)
     uint32_t window;          // sub-blocks held in LDS
@@ -85,6 +85,9 @@ struct FusedArgs {
     uint32_t total_items;     // batch * class_groups * tiles_per_ring * n_head
     uint32_t sub_stride[kFusedMaxStages];  // s_l / S0 per stage of the pass
     float scale_dn, scale_up;              // m^(n_cache * n_stages) and its reciprocal (backward: gradients leave as G m^T)
+    // radix kernels whose workgroups hold windows of several batch entries: windows of an entry, 0 or ceil(2^31 / entry_windows),
+    // and windows of all entries
+    uint32_t entry_windows, entry_magic, all_windows;
     StepTable tab;
 };
 

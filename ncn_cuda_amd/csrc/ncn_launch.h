@@ -200,8 +200,8 @@ struct RadixPass {
     int single;        // 1: one level, run with the one-stage kernel
     uint32_t s0;       // n^(first level of the pass): distance in rows between the rows of a window
     uint32_t span;     // n^count: rows of a window
-    uint32_t rows;     // rows a workgroup holds (a whole number of windows)
-    uint32_t loads;    // workgroup-loads per batch entry and head
+    uint32_t rows;     // rows of one batch entry that a workgroup holds (a whole number of windows)
+    uint32_t loads;    // workgroup-loads per batch entry and head, when it holds no others
 };
 bool radix_fused_supported(const ncn_shape* sh);
 // fused = false: one level per pass whatever the shape (calls whose scalars only the generic kernels take)

@@ -28,6 +28,26 @@ int64_t ipow(int64_t b, int e) {
     return r;
 }
 
+// Rows that a workgroup holds: its kernels keep them in registers (RadixShape::T bits of them)
+uint32_t capacity_rows(int ec, bool backward) {
+    return floor_pow2((uint32_t)(fused_state_bytes(backward) / ((backward ? 4 : 2) * ec * sizeof(float))));
+}
+
+// The workgroup-loads of a pass per head.  Windows of one batch entry (p.rows) leave a workgroup partly empty where their number
+// has no divisor that fills it; counted through all entries they need fewer workgroups, each of which takes the same time.
+struct RadixLoads {
+    uint32_t rows;     // per workgroup
+    int64_t loads;
+    bool across;       // .. of windows counted through all batch entries
+};
+RadixLoads radix_loads(const ncn_shape* sh, const RadixPass& p, bool backward) {
+    const uint32_t cap = capacity_rows((int)(sh->E / sh->n_head), backward);
+    const int64_t whole = sh->batch * (int64_t)p.loads, per = cap / p.span;
+    const int64_t across = (sh->batch * (sh->N / p.span) + per - 1) / per;
+    if (across < whole) return RadixLoads{cap, across, true};
+    return RadixLoads{p.rows, whole, false};
+}
+
 }  // namespace
 
 bool radix_fused_supported(const ncn_shape* sh) {
@@ -39,12 +59,12 @@ bool radix_fused_supported(const ncn_shape* sh) {
     return false;
 }
 
-// Levels [first, first + count) cut into passes of as many levels as fit the LDS budget (and the stage limits of the
+// Levels [first, first + count) cut into passes of as many levels as a workgroup's rows take (and the stage limits of the
 // kernels); a pass of one level is left to the one-stage kernel.  Every pass is closed.
 std::vector<RadixPass> plan_radix(const ncn_shape* sh, int first, int count, bool backward, bool fused) {
     std::vector<RadixPass> passes;
     const int nc = sh->n_cache, ec = (int)(sh->E / sh->n_head);
-    const uint32_t cap_rows = floor_pow2((uint32_t)(fused_state_bytes(backward) / ((backward ? 4 : 2) * ec * sizeof(float))));
+    const uint32_t cap_rows = capacity_rows(ec, backward);
     int kmax = 0;
     while (ipow(nc, kmax + 1) <= (int64_t)cap_rows) ++kmax;
     const int max_stages = backward ? kFusedMaxStages - 1 : kFusedMaxStages;
@@ -57,12 +77,11 @@ std::vector<RadixPass> plan_radix(const ncn_shape* sh, int first, int count, boo
         if (p.single) p.count = 1;
         p.s0 = (uint32_t)ipow(nc, first + a);
         p.span = (uint32_t)ipow(nc, p.count);
-        // A workgroup holds a whole number of windows, and every workgroup-load of a batch entry holds the same
-        // number: the largest divisor of the window count that the LDS budget takes (N = odd * n^k leaves an odd
-        // factor in the window count; a count that does not divide would leave the last windows unprocessed).
+        // A workgroup holds a whole number of windows, and every workgroup-load of a batch entry the same number: the largest
+        // divisor of the window count that it takes (N = odd * n^k leaves an odd factor in the window count).
         const uint32_t windows = (uint32_t)(sh->N / p.span);   // per batch entry and head
         uint32_t per_load = cap_rows / p.span;
-        if (per_load > windows) per_load = windows;            // N smaller than the LDS budget
+        if (per_load > windows) per_load = windows;            // N smaller than a workgroup
         while (windows % per_load) --per_load;
         p.rows = per_load * p.span;
         p.loads = windows / per_load;
@@ -73,8 +92,9 @@ std::vector<RadixPass> plan_radix(const ncn_shape* sh, int first, int count, boo
 }
 
 int radix_grid(const ncn_shape* sh, const RadixPass& p, bool backward) {
-    const int64_t items = sh->batch * (int64_t)p.loads * sh->n_head;
-    if (!backward) return items <= INT_MAX ? (int)items : 0;   // a workgroup for every item
+    const int64_t items = radix_loads(sh, p, backward).loads * sh->n_head;
+    // a workgroup for every item: filled ones need more than the card's memory before they exceed a grid
+    if (!backward) return items <= INT_MAX ? (int)items : 0;
     // .. in the backward where the dW scratch has a partial row for each
     const int64_t by_rows = (int64_t)kMaxGridX / p.count * sh->n_head;
     int64_t g = items < by_rows ? items : by_rows;
@@ -93,16 +113,15 @@ hipError_t launch_fused_radix(Pass pass, FusedArgs& a, const ncn_shape* sh, cons
     a.n_stages = p.count;
     a.class_stride = p.s0;
     a.ring = p.span;
-    a.window = p.rows / nc;
-    a.halo = 0;
-    a.own = a.window;
-    a.tiles_per_ring = 1;
-    a.closed = 1;
-    a.class_groups = p.loads;
-    a.total_items = (uint32_t)(sh->batch * (int64_t)p.loads * sh->n_head);
-    for (int k = 0; k < kFusedMaxStages; ++k) a.sub_stride[k] = k < p.count ? (uint32_t)ipow(nc, k) : 0;
+    const RadixLoads l = radix_loads(sh, p, backward);
+    const int64_t windows = sh->N / p.span, per = l.rows / p.span;
+    a.window = l.rows / nc;
+    a.class_groups = l.across ? 0 : p.loads;
+    a.entry_windows = (uint32_t)windows;
+    a.entry_magic = windows < per ? (uint32_t)(((1ull << 31) + windows - 1) / windows) : 0;   // (exact: window numbers < 2 per)
+    a.all_windows = (uint32_t)(sh->batch * windows);
+    a.total_items = (uint32_t)(l.loads * sh->n_head);
     a.scale_dn = (float)std::pow((double)a.tab.m, (double)(nc * p.count));
-    a.scale_up = (float)std::pow((double)a.tab.m, -(double)(nc * p.count));
     const int grid = radix_grid(sh, p, backward);
     const bool tanh_only = a.tab.activation == NCN_ACT_TANH;
 #define NCN_PICK(HEADWISE, BACKWARD, TANH) \

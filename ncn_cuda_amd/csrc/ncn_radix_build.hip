@@ -22,6 +22,9 @@ template <int NC, int EC>
 hipError_t launch_radix_shape(Pass pass, const FusedArgs& a, int grid, hipStream_t s) {
     constexpr bool kTanh = NCN_RADIX_TANH, kHeadwise = NCN_RADIX_HEADWISE;
     using S = RadixShape<NC, EC, NCN_RADIX_BACKWARD>;
+    // what plan_radix gives a workgroup is what it holds: all slots, and levels on whole digits of their bits
+    static_assert(((size_t)EC * sizeof(float) << S::T) * (NCN_RADIX_BACKWARD ? 4 : 2) == fused_state_bytes(NCN_RADIX_BACKWARD), "rows of a workgroup");
+    if (a.window * NC > (1u << S::T) || a.n_stages * S::DB > S::TU) return hipErrorInvalidConfiguration;
     const bool loop = (uint32_t)grid < a.total_items;
     void (*k)(const FusedArgs);
     size_t lds = (size_t)kFusedMaxStages * 2 * EC * sizeof(float) + ((size_t)EC * sizeof(float) << S::T);

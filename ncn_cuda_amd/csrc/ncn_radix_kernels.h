@@ -197,10 +197,53 @@ __device__ __forceinline__ void radix_weights(const float* w, int fl, float (&v)
     }
 }
 
-// Offsets of this lane's rows as they lie after `CHUNKS` exchanges of phase P0; a row that does not exist (a workgroup whose
-// windows are no power of two) gets row 0's and its bit of the result is 0.
+// The windows of a workgroup: of one batch entry where a divisor of their number fills it, else (class_groups 0) counted through
+// all batch entries, so that short sequences fill workgroups too.  x[4096, 32, 128], 5 levels of groups of two, forward, us: 32 rows
+// of the 256 that a workgroup holds 432, all of them FWD_NOW; x[512, 640, 128], 7 levels (windows of 128 rows, five to an entry)
+// 373, FWD_NOW2.
+struct RadixItem {
+    int head;
+    uint32_t window0, rows;   // first window, in its batch entry; rows that exist
+    int64_t base;             // element offset of (batch entry, row 0, head slice)
+};
+template <int NC, int EC>
+__device__ __forceinline__ RadixItem radix_item(const FusedArgs& A, uint32_t item) {
+    RadixItem it;
+    it.head = item % A.n_head;
+    const uint32_t load = item / A.n_head, per = (A.window * NC) >> log2u(A.ring);
+    uint32_t b;
+    it.rows = A.window * NC;
+    if (A.class_groups) {
+        b = load / A.class_groups;
+        it.window0 = (load - b * A.class_groups) * per;
+    } else {
+        const uint32_t w = load * per;
+        b = w / A.entry_windows;
+        it.window0 = w - b * A.entry_windows;
+        it.rows = min(per, A.all_windows - w) << log2u(A.ring);
+    }
+    it.base = (int64_t)b * A.N * A.E + (int64_t)it.head * EC;
+    return it;
+}
+// element offset (without the feature) of row lr of a workgroup
+__device__ __forceinline__ int64_t radix_row_offset(const FusedArgs& A, const RadixItem& it, uint32_t lr) {
+    const uint32_t lg_span = log2u(A.ring), lg_s0 = log2u(A.class_stride);
+    const uint32_t d = lr & (A.ring - 1u);
+    uint32_t u = it.window0 + (lr >> lg_span);
+    int64_t base = it.base;
+    if (A.class_groups == 0u) {   // u may lie in a later entry: the next, or, where a workgroup holds several, the u / entry_windows-th
+        const uint32_t k = A.entry_magic ? __umulhi(2u * u, A.entry_magic) : u >= A.entry_windows ? 1u : 0u;
+        u -= k * A.entry_windows;
+        base += (int64_t)k * (A.N * A.E);
+    }
+    const int64_t pos = (int64_t)(u & (A.class_stride - 1u)) + ((int64_t)d << lg_s0) + ((int64_t)(u >> lg_s0) << (lg_s0 + lg_span));
+    return base + pos * A.E;
+}
+
+// Offsets of this lane's rows as they lie after `CHUNKS` exchanges of phase P0; a row that does not exist (the windows of the
+// workgroup do not fill it) gets row 0's and its bit of the result is 0.
 template <class S, int NC, int P0, int CHUNKS, bool DESC>
-__device__ __forceinline__ uint32_t radix_offsets(const FusedArgs& A, const FusedItem& it, int lane, int wave, int fl,
+__device__ __forceinline__ uint32_t radix_offsets(const FusedArgs& A, const RadixItem& it, int lane, int wave, int fl,
                                                   int64_t (&off)[S::R]) {
     constexpr RadixMap m = radix_map<S>(P0, CHUNKS);
     const uint32_t base = radix_row<S::DB, DESC>(radix_lane_slot<S, P0, CHUNKS>(lane, wave), A.n_stages);
@@ -208,9 +251,9 @@ __device__ __forceinline__ uint32_t radix_offsets(const FusedArgs& A, const Fuse
 #pragma unroll
     for (int r = 0; r < S::R; ++r) {
         const uint32_t lr = base | radix_row<S::DB, DESC>(radix_reg_slot<S>(m, r), A.n_stages);
-        const bool ok = lr < A.window * NC;
+        const bool ok = lr < it.rows;
         exists |= ok ? 1u << r : 0u;
-        off[r] = fused_row_offset<NC, true>(A, it, ok ? lr : 0u) + fl * 4;
+        off[r] = radix_row_offset(A, it, ok ? lr : 0u) + fl * 4;
     }
     return exists;
 }
@@ -254,7 +297,7 @@ template <int NC, int EC, bool TANH_ONLY, bool INVERSE, bool HEADWISE>
 struct RadixForward {
     using S = RadixShape<NC, EC, false>;
     const FusedArgs& A;
-    const FusedItem& it;
+    const RadixItem& it;
     const float* w_lds;
     float4* exch;
     int lane, wave, fl;
@@ -345,7 +388,7 @@ __global__ void __launch_bounds__((64 * RadixShape<NC, EC, false>::NW), TANH_ONL
     float* w_lds = reinterpret_cast<float*>(fused_lds4);                  // [kFusedMaxStages][2][EC]
     float4* exch = fused_lds4 + kFusedMaxStages * 2 * EC / 4;             // one array of the workgroup
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), fl = lane % S::LF;
-    const FusedItem it = fused_item<NC, EC, true>(A, fused_deal<EC>(A, blockIdx.x));   // the launch has a workgroup for every item
+    const RadixItem it = radix_item<NC, EC>(A, fused_deal<EC>(A, blockIdx.x));   // the launch has a workgroup for every item
     int64_t off[S::R];
     radix_offsets<S, NC, 0, 0, INVERSE>(A, it, lane, wave, fl, off);
     uint4 rx[S::R * S::H], ra[S::R * S::H];
@@ -364,7 +407,7 @@ template <int NC, int EC, bool TANH_ONLY, bool LOOP, bool HEADWISE>
 struct RadixBackward {
     using S = RadixShape<NC, EC, true>;
     const FusedArgs& A;
-    const FusedItem& it;
+    const RadixItem& it;
     const float* w_lds;
     float* dw_mine;   // [n_stages][2][EC] of this wave
     float4* exch;
@@ -506,7 +549,7 @@ __global__ void __launch_bounds__((64 * RadixShape<NC, EC, true>::NW), TANH_ONLY
         for (int k = lane; k < dw_stride; k += 64) dw_mine[k] = 0.f;
     uint32_t item = item0;
     do {
-        const FusedItem it = fused_item<NC, EC, true>(A, item);
+        const RadixItem it = radix_item<NC, EC>(A, item);
         int64_t off[S::R];
         const uint32_t exists = radix_offsets<S, NC, 0, 0, true>(A, it, lane, wave, fl, off);
         uint4 ry[S::R * S::H], rb[S::R * S::H], rg[S::R * S::H], rh[S::R * S::H];

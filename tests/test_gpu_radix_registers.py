@@ -73,10 +73,40 @@ def test_bfloat16_inputs_and_gradients(M, n, ec, L):
     check(M, 2, n ** L, ec, 2, n, 0, L, dtype=torch.bfloat16)
 
 
-@pytest.mark.parametrize("n,L", [(2, 7), (4, 4)])
-def test_more_windows_than_partial_rows(M, n, L):
+# windows counted through batch entries: several entries to a workgroup, an entry that begins inside one and ends in the next, a
+# last workgroup that is not full; levels that do not start at the first; more and fewer windows to an entry than to a workgroup
+@pytest.mark.parametrize("batch,N,ec,n,first,L,act,dtype", [
+    (41, 4, 8, 2, 0, 2, 0, torch.float32), (130, 8, 32, 2, 0, 3, 0, torch.float32), (13, 80, 32, 2, 0, 4, 0, torch.float32),
+    (5, 640, 32, 2, 0, 7, 0, torch.float32), (7, 96, 64, 2, 0, 5, 0, torch.float32), (9, 48, 128, 2, 0, 4, 0, torch.float32),
+    (6, 96, 16, 2, 2, 3, 0, torch.float32), (11, 48, 32, 4, 0, 2, 0, torch.float32), (3, 192, 16, 4, 1, 2, 0, torch.bfloat16),
+    (50, 64, 8, 4, 0, 3, 2, torch.float32), (21, 96, 32, 2, 0, 5, -1, torch.bfloat16), (33, 56, 1, 2, 0, 3, 0, torch.float32),
+    (33, 112, 1, 4, 0, 2, 2, torch.float32)])
+def test_windows_of_several_batch_entries(M, batch, N, ec, n, first, L, act, dtype):
+    check(M, batch, N, ec, 16 if ec == 1 else 3, n, first, L, act, dtype)   # (heads of one feature are laid out as one of 16)
+
+
+@pytest.mark.parametrize("n,L,rows", [(2, 2, 4), (4, 2, 16)])
+def test_millions_of_short_sequences(M, n, L, rows):
+    """More windows than a grid holds workgroups: several to a workgroup."""
+    batch, C = (1 << 22) * 4 // rows, 4
+    gen = torch.Generator(device="cuda").manual_seed(0)
+    x = torch.randn(batch * (2 if n == 4 else 1), rows, 8 * C, generator=gen, device="cuda", dtype=torch.bfloat16)
+    W = torch.randn(L, 16 * C, generator=gen, device="cuda") / n ** 0.5
+    args = (W, 0.9, 0, n, C, 0, L)
+    y, ya = M.forward_radix(x, x, *args)
+    ix, ixa = M.inverse_radix(y, ya, *args)
+    for part in (slice(0, 1000), slice(len(x) // 2 - 500, len(x) // 2 + 500), slice(len(x) - 1001, None)):
+        py, pya = M.forward_radix(x[part].contiguous(), x[part].contiguous(), *args)
+        assert torch.equal(y[part], py) and torch.equal(ya[part], pya)
+        for a, b in zip(M.inverse_radix(py, pya, *args), (ix, ixa)):
+            assert torch.equal(a, b[part]) and O.rel_err(a, x[part].float()) < 12e-6 * 0.9 ** -(n * L)
+
+
+# the windows of an entry fill workgroups, or are counted through the entries
+@pytest.mark.parametrize("n,L,batch,N", [(2, 7, 16384 // 7 + 100, 512), (4, 4, 16384 // 4 + 100, 512), (2, 2, 360000, 12)])
+def test_more_windows_than_partial_rows(M, n, L, batch, N):
     """The backward then loops over windows; each half of the batch has a workgroup for every window."""
-    batch, N, E = 16384 // L + 100, 512, 8
+    E = 8
     gen = torch.Generator(device="cuda").manual_seed(0)
     x, xa, dy, dya = (torch.randn(batch, N, E, generator=gen, device="cuda") for _ in range(4))
     W = torch.randn(L, 2 * E, generator=gen, device="cuda") / n ** 0.5
