@@ -199,8 +199,8 @@ __device__ __forceinline__ void radix_weights(const float* w, int fl, float (&v)
 
 // The windows of a workgroup: of one batch entry where a divisor of their number fills it, else (class_groups 0) counted through
 // all batch entries, so that short sequences fill workgroups too.  x[4096, 32, 128], 5 levels of groups of two, forward, us: 32 rows
-// of the 256 that a workgroup holds 432, all of them FWD_NOW; x[512, 640, 128], 7 levels (windows of 128 rows, five to an entry)
-// 373, FWD_NOW2.
+// of the 256 that a workgroup holds 426, all of them 82; x[512, 640, 128], 7 levels (windows of 128 rows, five to an entry) 385
+// with one to a workgroup, 231 with two.
 struct RadixItem {
     int head;
     uint32_t window0, rows;   // first window, in its batch entry; rows that exist
