@@ -29,7 +29,7 @@ SOURCES = ["ncn_radix_fwd_act.hip", "ncn_radix_headwise_fwd_act.hip", "ncn_api.h
            "ncn_bwd_indexed.hip", "ncn_bwd_indexed_once.hip", "ncn_bwd_indexed_f32.hip", "ncn_bwd_indexed_bf16.hip",
            "ncn_headwise.hip", "ncn_headwise_indexed.hip", "ncn_headwise_bwd.hip", "ncn_headwise_bwd_indexed.hip", "ncn_anyshape.hip", "ncn_anyshape_bwd.hip", "ncn_anyshape_lengths.hip", "ncn_anyshape_bwd_lengths.hip", "ncn_split.hip", "ncn_generic.hip", "ncn_fused.hip", "ncn_fused_lengths.hip", "ncn_fused_headwise.hip", "ncn_fused_headwise_lengths.hip",
            "ncn_radix.hip", "ncn_radix_build.hip", "ncn_radix_bwd.hip", "ncn_radix_bwd_act.hip", "ncn_radix_headwise_fwd.hip",
-           "ncn_radix_headwise_bwd.hip", "ncn_radix_headwise_bwd_act.hip", "ncn_probe.hip", ID_SOURCE]
+           "ncn_radix_headwise_bwd.hip", "ncn_radix_headwise_bwd_act.hip", "ncn_radix_lds.hip", "ncn_radix_lds_headwise.hip", "ncn_probe.hip", ID_SOURCE]
 # packed-fp32 VALU instructions are switched off for device code on purpose (flag is device-only;
 # the host pass prints a harmless "not a recognized feature" note).
 HIPCC_FLAGS = ["-O3", "--offload-arch=gfx950", "-fPIC", "-std=c++17",
@@ -46,7 +46,7 @@ EXTRA_FLAGS = {"ncn_fused.hip": MAX_ILP, "ncn_fused_lengths.hip": MAX_ILP,
                "ncn_fused_headwise.hip": MAX_ILP, "ncn_fused_headwise_lengths.hip": MAX_ILP,
                "ncn_radix_build.hip": MAX_ILP, "ncn_radix_fwd_act.hip": MAX_ILP, "ncn_radix_bwd.hip": MAX_ILP, "ncn_radix_bwd_act.hip": MAX_ILP,
                "ncn_radix_headwise_fwd.hip": MAX_ILP, "ncn_radix_headwise_fwd_act.hip": MAX_ILP, "ncn_radix_headwise_bwd.hip": MAX_ILP,
-               "ncn_radix_headwise_bwd_act.hip": MAX_ILP,
+               "ncn_radix_headwise_bwd_act.hip": MAX_ILP, "ncn_radix_lds.hip": MAX_ILP, "ncn_radix_lds_headwise.hip": MAX_ILP,
                "ncn_fwd.hip": MAX_ILP, "ncn_fwd_indexed.hip": MAX_ILP, "ncn_bwd_indexed.hip": MAX_ILP,
                "ncn_bwd_once.hip": MAX_ILP, "ncn_bwd_indexed_once.hip": MAX_ILP, "ncn_bwd_f32.hip": MAX_ILP, "ncn_bwd_bf16.hip": MAX_ILP, "ncn_bwd_indexed_f32.hip": MAX_ILP,
                "ncn_bwd_indexed_bf16.hip": MAX_ILP, "ncn_fwd_f32.hip": MAX_ILP, "ncn_fwd_bf16.hip": MAX_ILP,

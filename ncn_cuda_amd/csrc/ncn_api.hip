@@ -1105,7 +1105,7 @@ int ncn_backward_radix(const void* y, const void* ya, int y_dtype, const void* d
         const RadixPass& ps = passes[passes.size() - 1 - e];
         const bool top = (e == 0);
         const bool drop_rec = no_rec && e + 1 == passes.size();
-        const int rows = ps.single ? p.partial_rows : radix_grid(shape, ps, true) / shape->n_head;
+        const int rows = ps.single ? p.partial_rows : radix_grid(shape, ps, true, activation == NCN_ACT_TANH) / shape->n_head;
         float* region;
         hipError_t err = reducer.reserve(rows, ps.count, &region);
         if (err != hipSuccess) return (int)err;

@@ -318,7 +318,7 @@ hipError_t launch_fused(Pass pass, FusedArgs& a, const ncn_shape* sh, const Fuse
     const size_t lds = fused_lds_bytes(nc, ec, backward, p.window, p.count);
     if (headwise) return launch_fused_headwise(pass, a, nc, ec, grid, lds, s);
     if (a.ctx_len) return launch_fused_lengths(pass, a, nc, ec, grid, lds, s);
-    return launch_fused_shape<false, false>(pass, a, nc, ec, grid, lds, s);
+    return launch_fused_shape<false, false, false>(pass, a, nc, ec, grid, lds, s);
 }
 
 }  // namespace ncn

@@ -11,12 +11,12 @@ namespace ncn {
 
 #if NCN_LENGTHS_BUILD
 hipError_t launch_fused_headwise_lengths(Pass pass, const FusedArgs& a, int nc, int ec, int grid, size_t lds, hipStream_t s) {
-    return launch_fused_shape<true, true>(pass, a, nc, ec, grid, lds, s);
+    return launch_fused_shape<false, true, true>(pass, a, nc, ec, grid, lds, s);
 }
 #else
 hipError_t launch_fused_headwise(Pass pass, const FusedArgs& a, int nc, int ec, int grid, size_t lds, hipStream_t s) {
     if (a.ctx_len) return launch_fused_headwise_lengths(pass, a, nc, ec, grid, lds, s);
-    return launch_fused_shape<false, true>(pass, a, nc, ec, grid, lds, s);
+    return launch_fused_shape<false, false, true>(pass, a, nc, ec, grid, lds, s);
 }
 #endif
 

@@ -25,6 +25,13 @@
 // the stages, p = (1-m) g + h in place of h), so true values exist only in HBM.  The pass's weights sit in LDS,
 // already scaled by gamma.  Backward sums each wave's dW share of a stage into a per-wave LDS
 // slot (one writer per slot, fixed order: deterministic) and leaves one partial row per workgroup and stage.
+//
+// RADIX builds of the same kernels run levels of the radix-n digit grouping (ncn_triton/group_tensors.py:8-18)
+// instead: level l groups the n_cache positions that differ only in base-n_cache digit l.  A run of levels a .. a+k-1
+// only ever mixes the positions lower + n^a * d + n^(a+k) * upper, d = 0 .. n^k - 1, of one (lower, upper): a closed
+// window of n^k rows, no halo at all, any pass may run in place.  A workgroup holds rows / n^k such windows; the LDS
+// row of digit string d is d itself, and level a+j pairs the rows whose d differ in digit j.  (n_cache 2 and 4
+// only: every size below is a power of two and the digit arithmetic is shifts.)
 #pragma once
 #include "ncn_headwise_kernels.h"
 
@@ -72,8 +79,9 @@ struct FusedArgs {
     int32_t n_head, n_stages;
     int32_t in_dtype, g_dtype, out_dtype, w_bf16;
     uint32_t ring_magic;      // 0 when `ring` is a power of two, else ceil(2^32 / ring): closed passes divide by the ring
-    // the radix kernels (ncn_radix_kernels.h) read: class_stride = n^a in rows, ring = n^k rows per window, window = rows /
-    // n_cache, class_groups = workgroup-loads per batch entry, or 0: entry_windows .. all_windows
+    // RADIX builds read: class_stride = n^a in rows, ring = n^k rows per window, window = rows / n_cache, class_groups =
+    // workgroup-loads per batch entry, sub_stride[j] = n^j in rows, closed = 1; the radix kernels (ncn_radix_kernels.h) the first
+    // four, class_groups 0 meaning entry_windows .. all_windows
     uint32_t class_stride;    // S0, in blocks
     uint32_t ring;            // sub-blocks per class = groups / S0 (a power of two, or an odd number times one)
     uint32_t window;          // sub-blocks held in LDS
@@ -206,8 +214,17 @@ __device__ __forceinline__ uint32_t fused_lds_place(uint32_t lr) {
 }
 
 // LDS row of slot i of the group whose slot-0 sub-block is window position qg
-template <int NC>
+// (RADIX: row of digit i at level log_n(sstride) of group qg; groups are numbered window by window)
+template <int NC, bool RADIX>
 __device__ __forceinline__ uint32_t fused_lds_row(const FusedArgs& A, uint32_t qg, uint32_t i, uint32_t sstride) {
+    if (RADIX) {
+        constexpr uint32_t lg_nc = NC == 2 ? 1u : 2u;
+        static_assert(NC == 2 || NC == 4, "digit arithmetic by shifts");
+        const uint32_t lg_span = log2u(A.ring), lg_sj = log2u(sstride);
+        const uint32_t gpw = A.ring >> lg_nc;                       // groups per window
+        const uint32_t wq = qg >> (lg_span - lg_nc), g = qg & (gpw - 1u);
+        return fused_lds_place<NC>((wq << lg_span) + ((g >> lg_sj) << (lg_sj + lg_nc)) + (i << lg_sj) + (g & (sstride - 1u)));
+    }
     const uint32_t qi = A.closed ? ring_wrap(A, qg, i * sstride) : qg + i * sstride;  // closed: inside the group's own ring
     return fused_lds_place<NC>(qi * NC + i);
 }
@@ -241,7 +258,7 @@ __device__ __forceinline__ void lds_store_frag(float* row, const float (&v)[F]) 
 // Window rows on their way from global memory to LDS: 4 features per thread and trip, kept as raw bits so that
 // nothing waits for the loads until fused_commit_rows turns them into floats.  A workgroup fetches the window of
 // its next item while it computes the current one.
-template <int NC, int EC, int NW, int K>
+template <int NC, int EC, int NW, int K, bool RADIX>
 __device__ __forceinline__ void fused_window_offsets(const FusedArgs& A, const FusedItem& it, uint32_t rows,
                                                      int64_t (&off)[K]) {
     constexpr uint32_t CPR = EC / 4;
@@ -250,7 +267,7 @@ __device__ __forceinline__ void fused_window_offsets(const FusedArgs& A, const F
         // a trip past the end re-reads the last chunk, which fused_commit_rows ignores
         const uint32_t c = min(threadIdx.x + k * 64 * NW, rows * CPR - 1u);
         const uint32_t lr = c / CPR, c4 = c - lr * CPR;
-        off[k] = fused_row_offset<NC, false>(A, it, lr) + c4 * 4;
+        off[k] = fused_row_offset<NC, RADIX>(A, it, lr) + c4 * 4;
     }
 }
 
@@ -298,7 +315,7 @@ __device__ __forceinline__ void fused_commit_rows(const uint4 (&raw)[K], int dty
 }
 
 // LDS -> global for the owned rows, each value times `scale`
-template <int NC, int EC, int NW>
+template <int NC, int EC, int NW, bool RADIX>
 __device__ __forceinline__ void fused_store_rows_scaled(const FusedArgs& A, const FusedItem& it, const float* src,
                                                         float scale, void* dst, int dtype, float* copy32) {
     constexpr uint32_t CPR = EC / 4;
@@ -309,7 +326,7 @@ __device__ __forceinline__ void fused_store_rows_scaled(const FusedArgs& A, cons
         lds_load_frag<4>(src + fused_lds_place<NC>(lr) * EC + c4 * 4, v);
 #pragma unroll
         for (int k = 0; k < 4; ++k) v[k] *= scale;
-        const int64_t off = fused_row_offset<NC, false>(A, it, lr) + c4 * 4;
+        const int64_t off = fused_row_offset<NC, RADIX>(A, it, lr) + c4 * 4;
         store_frag<4>(dst, dtype, off, true, v);
         if (copy32) store_frag<4>(copy32, NCN_F32, off, true, v);
     }
@@ -335,9 +352,10 @@ __device__ __forceinline__ void fused_load_weights(const FusedArgs& A, int head,
 // past the length stay in LDS as they came (a row may be live in one stage of the pass and past the length in another).
 // HEADWISE: heads of one feature laid out as heads of EC adjacent ones (ncn_headwise_kernels.h): the same windows, tiles
 // and weights, the step code without sums across a row's lanes.
-template <int NC, int EC, int R, int F, bool TANH_ONLY, bool INVERSE = false, bool LENGTHS = false,
+template <int NC, int EC, int R, int F, bool TANH_ONLY, bool RADIX = false, bool INVERSE = false, bool LENGTHS = false,
           bool HEADWISE = false>
 __global__ void __launch_bounds__(64 * kFusedWavesFwd) fused_forward_kernel(const FusedArgs A) {
+    static_assert(!(RADIX && LENGTHS), "context lengths go with the stride permutation");
     constexpr int NW = kFusedWavesFwd;
     using T = Tile<NC, EC, R, F>;
     extern __shared__ float4 fused_lds4[];
@@ -357,19 +375,19 @@ __global__ void __launch_bounds__(64 * kFusedWavesFwd) fused_forward_kernel(cons
     uint4 rx[K], ra[K];
     if (item0 < A.total_items) {
         int64_t off[K];
-        fused_window_offsets<NC, EC, NW, K>(A, fused_item<NC, EC, false>(A, item0), rows, off);
+        fused_window_offsets<NC, EC, NW, K, RADIX>(A, fused_item<NC, EC, RADIX>(A, item0), rows, off);
         fused_fetch_rows<K>(A.in0, A.in_dtype, off, rx);
         fused_fetch_rows<K>(A.in1, A.in_dtype, off, ra);
     }
     for (uint32_t item = item0; item < A.total_items; item += gridDim.x) {
-        const FusedItem it = fused_item<NC, EC, false>(A, item);
+        const FusedItem it = fused_item<NC, EC, RADIX>(A, item);
         const int32_t len = LENGTHS ? max(0, min(A.ctx_len[it.batch], (int32_t)A.N)) : 0;
         fused_commit_rows<NC, EC, NW, K>(rx, A.in_dtype, xs, rows, A.tab.kappa);
         fused_commit_rows<NC, EC, NW, K>(ra, A.in_dtype, as, rows, INVERSE ? A.tab.b_scale : A.tab.a_scale);
         __syncthreads();
         if (item + gridDim.x < A.total_items) {   // the next window travels while this one is computed
             int64_t off[K];
-            fused_window_offsets<NC, EC, NW, K>(A, fused_item<NC, EC, false>(A, item + gridDim.x), rows, off);
+            fused_window_offsets<NC, EC, NW, K, RADIX>(A, fused_item<NC, EC, RADIX>(A, item + gridDim.x), rows, off);
             fused_fetch_rows<K>(A.in0, A.in_dtype, off, rx);
             fused_fetch_rows<K>(A.in1, A.in_dtype, off, ra);
         }
@@ -387,7 +405,7 @@ __global__ void __launch_bounds__(64 * kFusedWavesFwd) fused_forward_kernel(cons
                 uint32_t row[R];
 #pragma unroll
                 for (int rr = 0; rr < R; ++rr) {
-                    row[rr] = fused_lds_row<NC>(A, valid ? qg : 0u, rl * R + rr, ss) * EC + fl * F;
+                    row[rr] = fused_lds_row<NC, RADIX>(A, valid ? qg : 0u, rl * R + rr, ss) * EC + fl * F;
                     lds_load_frag<F>(xs + row[rr], x[rr]);
                     lds_load_frag<F>(as + row[rr], a[rr]);
                 }
@@ -411,15 +429,16 @@ __global__ void __launch_bounds__(64 * kFusedWavesFwd) fused_forward_kernel(cons
             __syncthreads();
         }
         // out of the scaled form
-        fused_store_rows_scaled<NC, EC, NW>(A, it, xs, A.tab.inv_kappa, A.out0, A.out_dtype, A.aux0);
-        fused_store_rows_scaled<NC, EC, NW>(A, it, as, INVERSE ? A.tab.inv_b_scale : A.tab.inv_a_scale, A.out1,
+        fused_store_rows_scaled<NC, EC, NW, RADIX>(A, it, xs, A.tab.inv_kappa, A.out0, A.out_dtype, A.aux0);
+        fused_store_rows_scaled<NC, EC, NW, RADIX>(A, it, as, INVERSE ? A.tab.inv_b_scale : A.tab.inv_a_scale, A.out1,
                                                    A.out_dtype, A.aux1);
         __syncthreads();
     }
 }
 
-template <int NC, int EC, int R, int F, bool TANH_ONLY, bool LENGTHS = false, bool HEADWISE = false>
+template <int NC, int EC, int R, int F, bool TANH_ONLY, bool RADIX = false, bool LENGTHS = false, bool HEADWISE = false>
 __global__ void __launch_bounds__(64 * kFusedWavesBwd, TANH_ONLY ? (R * F <= 8 ? 4 : 2) : 1) fused_backward_kernel(const FusedArgs A) {
+    static_assert(!(RADIX && LENGTHS), "context lengths go with the stride permutation");
     constexpr int NW = kFusedWavesBwd;
     using T = Tile<NC, EC, R, F>;
     extern __shared__ float4 fused_lds4[];
@@ -452,7 +471,7 @@ __global__ void __launch_bounds__(64 * kFusedWavesBwd, TANH_ONLY ? (R * F <= 8 ?
     };
     auto fetch = [&](uint32_t item, Raw& r) {
         int64_t off[K];
-        fused_window_offsets<NC, EC, NW, K>(A, fused_item<NC, EC, false>(A, item), rows, off);
+        fused_window_offsets<NC, EC, NW, K, RADIX>(A, fused_item<NC, EC, RADIX>(A, item), rows, off);
         fused_fetch_rows<K>(A.in0, A.in_dtype, off, r.y);
         fused_fetch_rows<K>(A.in1, A.in_dtype, off, r.b);
         fused_fetch_rows<K>(A.g0, A.g_dtype, off, r.g);
@@ -483,7 +502,7 @@ __global__ void __launch_bounds__(64 * kFusedWavesBwd, TANH_ONLY ? (R * F <= 8 ?
     }
     __syncthreads();
     for (uint32_t item = item0; item < A.total_items; item += gridDim.x) {
-        const FusedItem it = fused_item<NC, EC, false>(A, item);
+        const FusedItem it = fused_item<NC, EC, RADIX>(A, item);
         const int32_t len = LENGTHS ? max(0, min(A.ctx_len[it.batch], (int32_t)A.N)) : 0;
         for (int st = A.n_stages - 1; st >= 0; --st) {
             const uint32_t ss = A.sub_stride[st];
@@ -501,7 +520,7 @@ __global__ void __launch_bounds__(64 * kFusedWavesBwd, TANH_ONLY ? (R * F <= 8 ?
                 uint32_t row[R];
 #pragma unroll
                 for (int rr = 0; rr < R; ++rr) {
-                    row[rr] = fused_lds_row<NC>(A, valid ? qg : 0u, rl * R + rr, ss) * EC + fl * F;
+                    row[rr] = fused_lds_row<NC, RADIX>(A, valid ? qg : 0u, rl * R + rr, ss) * EC + fl * F;
                     lds_load_frag<F>(ys + row[rr], Y[rr]);
                     lds_load_frag<F>(bs + row[rr], B[rr]);
                     lds_load_frag<F>(gs + row[rr], G[rr]);
@@ -575,7 +594,7 @@ __global__ void __launch_bounds__(64 * kFusedWavesBwd, TANH_ONLY ? (R * F <= 8 ?
             const uint32_t r0 = it.own_lo * NC, nrows = it.own_cnt * NC;
             for (uint32_t c = threadIdx.x; c < nrows * CPR; c += 64 * NW) {
                 const uint32_t lr = r0 + c / CPR, c4 = c % CPR;
-                const int64_t off = fused_row_offset<NC, false>(A, it, lr) + c4 * 4;
+                const int64_t off = fused_row_offset<NC, RADIX>(A, it, lr) + c4 * 4;
                 float g[4], h[4];
                 lds_load_frag<4>(gs + fused_lds_place<NC>(lr) * EC + c4 * 4, g);
                 lds_load_frag<4>(ps + fused_lds_place<NC>(lr) * EC + c4 * 4, h);
@@ -588,8 +607,8 @@ __global__ void __launch_bounds__(64 * kFusedWavesBwd, TANH_ONLY ? (R * F <= 8 ?
                 store_frag<4>(A.out1, A.out_dtype, off, true, h);
             }
             if (A.aux0) {
-                fused_store_rows_scaled<NC, EC, NW>(A, it, ys, A.tab.inv_kappa, A.aux0, NCN_F32, nullptr);
-                fused_store_rows_scaled<NC, EC, NW>(A, it, bs, A.tab.inv_b_scale, A.aux1, NCN_F32, nullptr);
+                fused_store_rows_scaled<NC, EC, NW, RADIX>(A, it, ys, A.tab.inv_kappa, A.aux0, NCN_F32, nullptr);
+                fused_store_rows_scaled<NC, EC, NW, RADIX>(A, it, bs, A.tab.inv_b_scale, A.aux1, NCN_F32, nullptr);
             }
         };
         if (item + gridDim.x < A.total_items) {   // the same for the whole workgroup

@@ -5,7 +5,7 @@
 namespace ncn {
 
 hipError_t launch_fused_lengths(Pass pass, const FusedArgs& a, int nc, int ec, int grid, size_t lds, hipStream_t s) {
-    return launch_fused_shape<true, false>(pass, a, nc, ec, grid, lds, s);
+    return launch_fused_shape<false, true, false>(pass, a, nc, ec, grid, lds, s);
 }
 
 }  // namespace ncn

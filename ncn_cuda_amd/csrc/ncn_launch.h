@@ -206,10 +206,15 @@ struct RadixPass {
 bool radix_fused_supported(const ncn_shape* sh);
 // fused = false: one level per pass whatever the shape (calls whose scalars only the generic kernels take)
 std::vector<RadixPass> plan_radix(const ncn_shape* sh, int first, int count, bool backward, bool fused = true);
-int radix_grid(const ncn_shape* sh, const RadixPass& p, bool backward);
+int radix_grid(const ncn_shape* sh, const RadixPass& p, bool backward, bool tanh);
 hipError_t launch_fused_radix(Pass pass, FusedArgs& a, const ncn_shape* sh, const RadixPass& p, hipStream_t s,
                               bool headwise = false);
-// the builds, by kind (ncn_radix_build.hip and the units that include it)
+// the builds that keep rows in LDS, heads of several features or of one (ncn_radix_lds.hip)
+template <bool HEADWISE>
+hipError_t launch_radix_lds(Pass pass, const FusedArgs& a, int nc, int ec, int grid, hipStream_t s);
+template <> hipError_t launch_radix_lds<false>(Pass, const FusedArgs&, int, int, int, hipStream_t);
+template <> hipError_t launch_radix_lds<true>(Pass, const FusedArgs&, int, int, int, hipStream_t);
+// those that keep them in registers, by kind (ncn_radix_build.hip and the units that include it)
 template <bool HEADWISE, bool BACKWARD, bool TANH>
 hipError_t launch_radix(Pass pass, const FusedArgs& a, int nc, int ec, int grid, hipStream_t s);
 #define NCN_DECLARE(H, B) \

@@ -1,6 +1,6 @@
 // Planning and launching of multi-stage passes over levels of the radix-n digit grouping
-// (ncn_triton/group_tensors.py:8-18); the kernels are those of ncn_radix_kernels.h,
-// built in ncn_radix_build.hip.
+// (ncn_triton/group_tensors.py:8-18); the kernels are those of ncn_radix_kernels.h, built in ncn_radix_build.hip, and in
+// launches with few workgroups the RADIX builds of ncn_fused_kernels.h (ncn_radix_lds.hip).
 #include <climits>
 #include <cmath>
 #include <vector>
@@ -39,13 +39,46 @@ struct RadixLoads {
     uint32_t rows;     // per workgroup
     int64_t loads;
     bool across;       // .. of windows counted through all batch entries
+    bool lds;          // for the kernels that keep rows in LDS
 };
-RadixLoads radix_loads(const ncn_shape* sh, const RadixPass& p, bool backward) {
+
+// Whether a launch of so many workgroups, of `rows` rows each, runs on the kernels that keep rows in LDS.  A lane of the register
+// kernels holds 16 elements and more, and a workgroup takes the same time however few of its rows exist; the LDS kernels spread the
+// rows there are over 8 waves, 8 elements to a lane, which is the shorter chain as long as every workgroup starts at once and has
+// at most half the rows that fit.  tanh, us, LDS : registers, forward | backward, N = rows, by workgroups:
+//   groups of two, heads of  8,  8 rows, 3 levels  64:  6.0 : 11.0 | 11.0 : 12.6   256:  6.1 : 11.4 | 11.3 : 12.9   512:  8.1 : 11.8 | 12.8 : 12.9
+//   groups of two, heads of 32,  8 rows, 3 levels  64:  5.9 :  9.4 | 10.7 : 10.9   256:  6.0 :  9.5 | 10.9 : 11.2   512:  7.4 :  9.6 | 12.1 : 11.3
+//   groups of two, heads of 32, 128 rows, 7 levels 64: 11.9 : 15.8 | 22.1 : 18.1   256: 13.1 : 16.8 | 24.0 : 19.6   512: 20.2 : 19.4 | 36.7 : 32.3
+//   groups of two, heads of 64,  8 rows, 3 levels  64:  7.1 :  9.4 | 13.9 : 11.4   256:  7.3 :  9.5 | 14.3 : 11.6   512: 12.6 :  9.7 | 24.3 : 12.0
+//   groups of four, heads of 32, 64 rows, 3 levels 64:  8.2 : 12.9 | 14.3 : 16.4   256:  8.8 : 13.4 | 15.2 : 17.3   512: 11.9 : 14.0 | 19.8 : 18.3
+// With all the rows that fit (groups of two, heads of 16, 8 levels of 512 rows forward and 256 backward) registers win from the
+// first workgroup on, by 10 and 11 %.
+//   The other activations spend more instructions on an element, which 8 waves of few elements overlap better: the time on registers
+// over that in LDS, relu, groups of two, by workgroups (512, 2048, 6000 unless named), forward heads of 16: 128 rows of 512 2.12, 0.78,
+// 0.59, 256 rows 1.97, 1.23, 0.99, all 512 rows 1.27, 1.12, 1.07 (sigmoid 1.14, 1.03, 0.95); heads of 64: 64: 1.38, 256: 1.36, 512:
+// 0.86; groups of four, heads of 8: 512 of 1024 rows 1.23, 0.82, 0.82, all of them 0.80.  Backward, heads of 32, all 128 rows: 64:
+// 1.28, 256: 1.24, 512: 0.77; heads of 64 0.87 at 64.
+bool rows_in_lds(int nc, int ec, bool backward, bool tanh, uint32_t rows, uint32_t cap, int64_t workgroups) {
+    const bool half = 2 * rows <= cap, quarter = 4 * rows <= cap;
+    if (tanh) {
+        if (!half) return false;
+        if (backward) return workgroups <= 256 && (ec <= 16 || (ec <= 32 && nc == 4));
+        return workgroups <= (ec <= 16 || (ec <= 32 && quarter) ? 512 : 256);
+    }
+    if (backward) return workgroups <= 256 && ec <= 32;
+    if (ec > 32) return workgroups <= 256;
+    if (nc == 4 && ec == 8 && !quarter) return half && workgroups <= 512;
+    return workgroups <= (quarter ? 512 : half ? 2048 : 4096);
+}
+
+RadixLoads radix_loads(const ncn_shape* sh, const RadixPass& p, bool backward, bool tanh) {
     const uint32_t cap = capacity_rows((int)(sh->E / sh->n_head), backward);
     const int64_t whole = sh->batch * (int64_t)p.loads, per = cap / p.span;
     const int64_t across = (sh->batch * (sh->N / p.span) + per - 1) / per;
-    if (across < whole) return RadixLoads{cap, across, true};
-    return RadixLoads{p.rows, whole, false};
+    if (rows_in_lds(sh->n_cache, (int)(sh->E / sh->n_head), backward, tanh, p.rows, cap, whole * sh->n_head))
+        return RadixLoads{p.rows, whole, false, true};
+    if (across < whole) return RadixLoads{cap, across, true, false};
+    return RadixLoads{p.rows, whole, false, false};
 }
 
 }  // namespace
@@ -91,8 +124,8 @@ std::vector<RadixPass> plan_radix(const ncn_shape* sh, int first, int count, boo
     return passes;
 }
 
-int radix_grid(const ncn_shape* sh, const RadixPass& p, bool backward) {
-    const int64_t items = radix_loads(sh, p, backward).loads * sh->n_head;
+int radix_grid(const ncn_shape* sh, const RadixPass& p, bool backward, bool tanh) {
+    const int64_t items = radix_loads(sh, p, backward, tanh).loads * sh->n_head;
     // a workgroup for every item: filled ones need more than the card's memory before they exceed a grid
     if (!backward) return items <= INT_MAX ? (int)items : 0;
     // .. in the backward where the dW scratch has a partial row for each
@@ -113,7 +146,9 @@ hipError_t launch_fused_radix(Pass pass, FusedArgs& a, const ncn_shape* sh, cons
     a.n_stages = p.count;
     a.class_stride = p.s0;
     a.ring = p.span;
-    const RadixLoads l = radix_loads(sh, p, backward);
+    const bool tanh = a.tab.activation == NCN_ACT_TANH;
+    const RadixLoads l = radix_loads(sh, p, backward, tanh);
+    const int grid = radix_grid(sh, p, backward, tanh);
     const int64_t windows = sh->N / p.span, per = l.rows / p.span;
     a.window = l.rows / nc;
     a.class_groups = l.across ? 0 : p.loads;
@@ -122,10 +157,16 @@ hipError_t launch_fused_radix(Pass pass, FusedArgs& a, const ncn_shape* sh, cons
     a.all_windows = (uint32_t)(sh->batch * windows);
     a.total_items = (uint32_t)(l.loads * sh->n_head);
     a.scale_dn = (float)std::pow((double)a.tab.m, (double)(nc * p.count));
-    const int grid = radix_grid(sh, p, backward);
-    const bool tanh_only = a.tab.activation == NCN_ACT_TANH;
+    if (l.lds) {
+        a.own = a.window;
+        a.tiles_per_ring = 1;
+        a.closed = 1;
+        for (int k = 0; k < p.count; ++k) a.sub_stride[k] = (uint32_t)ipow(nc, k);
+        a.scale_up = (float)std::pow((double)a.tab.m, -(double)(nc * p.count));
+        return headwise ? launch_radix_lds<true>(pass, a, nc, ec, grid, s) : launch_radix_lds<false>(pass, a, nc, ec, grid, s);
+    }
 #define NCN_PICK(HEADWISE, BACKWARD, TANH) \
-    if (headwise == HEADWISE && backward == BACKWARD && tanh_only == TANH) return launch_radix<HEADWISE, BACKWARD, TANH>(pass, a, nc, ec, grid, s);
+    if (headwise == HEADWISE && backward == BACKWARD && tanh == TANH) return launch_radix<HEADWISE, BACKWARD, TANH>(pass, a, nc, ec, grid, s);
     NCN_PICK(false, false, true) NCN_PICK(false, true, true) NCN_PICK(false, false, false) NCN_PICK(false, true, false)
     NCN_PICK(true, false, true) NCN_PICK(true, true, true) NCN_PICK(true, false, false) NCN_PICK(true, true, false)
 #undef NCN_PICK

@@ -11,10 +11,11 @@
 // and the waves of a workgroup (WB), and a level runs where its bits are register bits: all rows of a group in one lane, the
 // step code of ncn_stage_kernels.h without any exchange between rows.  Then register bits and lane bits change places:
 // v_permlane32_swap and v_permlane16_swap exchange the upper two lane bits with a register bit in one instruction per two
-// registers, DPP moves the lower ones.  What lies across waves comes in by one exchange of all rows through LDS for the five or
-// more levels before it.  (The kernels this replaces kept the rows in LDS, read and wrote them all at every level with a
+// registers, DPP moves the lower ones.  What lies across waves comes in by an exchange of all rows through LDS after the
+// RB + LB bits before it (heads of 32, groups of two: six levels forward, five backward; heads of 128, groups of four, backward:
+// one).  (The RADIX builds of ncn_fused_kernels.h keep the rows in LDS, read and write them all at every level with a
 // barrier after it: x[32, 8192, 128], 13 levels of groups of two, 8 + 5 forward and 7 + 6 backward, 231 us a pass forward and 459
-// backward; here 213 and 152, 345 and 316.)
+// backward; here 213 and 152, 345 and 316.  They run where there are few workgroups: rows_in_lds() in ncn_radix.hip.)
 //
 // What bounds it: of the 345 us of the backward pass over 7 levels its loads, stores and exchanges alone take 174, its
 // instructions at the rates they issue at some 210, and with four workgroups per CU, whose registers are full, the two overlap

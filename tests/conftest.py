@@ -47,6 +47,18 @@ def has_gpu():
     return torch.cuda.is_available()
 
 
+def kernels_of(call):
+    """What call() returns, and the names of the library's kernels that it launched, without their arguments."""
+    from torch.profiler import ProfilerActivity, profile
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA]) as seen:
+        result = call()
+        torch.cuda.synchronize()
+    names = {e.name.split("(ncn::")[0].split("ncn::")[-1] for e in seen.events() if "ncn::" in e.name}
+    assert names
+    return result, names
+
+
 def record_errors(kind, **values):
     """Appends one line of measured errors to the file $NCN_ERROR_REPORT names, if any: the figures that the tolerances of
     the tests that call it are set from (a margin over the worst case measured)."""

@@ -1,9 +1,11 @@
 """The multi-level radix kernels (ncn_radix_kernels.h) against the float64 oracle: every head width and group size, passes of two
 levels up to the most that a workgroup holds, so that the levels run in registers, after exchanges of register and lane bits and
-after the exchange through LDS, windows that are no power of two, every kind of launch."""
+after the exchange through LDS, windows that are no power of two, every kind of launch; and the kernels that keep rows in LDS
+(ncn_fused_kernels.h), which launches with few workgroups take."""
 import pytest
 import torch
 
+from conftest import kernels_of
 from oracle import ncn_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -17,7 +19,8 @@ def M():
     return ncn_cuda_module
 
 
-def check(M, batch, N, ec, C, n, first, L, act=0, dtype=torch.float32):
+def check(M, batch, N, ec, C, n, first, L, act=0, dtype=torch.float32, forward=None, backward=None):
+    """forward, backward: the kernels that the passes have to run on, "radix" (registers) or "fused" (LDS)."""
     E = ec * C
     make = O.make_inputs_signed_regimes if act in (1, 3) else O.make_inputs   # away from the kink
     x, xa, Ws, dy, dya = make(batch, N, E, L, n, seed=N + ec) if act in (1, 3) else make(batch, N, E, L, n, seed=N + ec, xa_zero=False)
@@ -28,8 +31,11 @@ def check(M, batch, N, ec, C, n, first, L, act=0, dtype=torch.float32):
     W = torch.stack([w.reshape(-1) for w in Ws]).cuda()
     x, xa, dy, dya = (t.cuda() for t in (x, xa, dy, dya))
     args = (W, 0.9, act, n, C, first, L)
-    y, ya = M.forward_radix(x, xa, *args)
-    rx, rxa, dx, dxa, dW = M.backward_radix(y, ya, dy, dya, *args)
+    (y, ya), ran = kernels_of(lambda: M.forward_radix(x, xa, *args))
+    multi_level = lambda names: {k.split("_")[0] for k in names} & {"radix", "fused"}   # (a last pass of one level has other kernels)
+    assert forward is None or multi_level(ran) == {forward}, ran
+    (rx, rxa, dx, dxa, dW), ran = kernels_of(lambda: M.backward_radix(y, ya, dy, dya, *args))
+    assert backward is None or multi_level(ran) == {backward}, ran
     _, _, dx2, dxa2, dW2 = M.backward_radix(y, ya, dy, dya, *args, want_inputs=False)
     ix, ixa = M.inverse_radix(y, ya, *args)
     # rounding of the sums, amplified by 1/m at every step undone (as in test_gpu_stack); reconstruction as in test_gpu_parity
@@ -50,6 +56,8 @@ def test_levels(M, n, ec, levels):
     most = {2: {8: 10, 16: 9, 32: 8, 64: 7, 128: 6}, 4: {8: 5, 16: 4, 32: 4, 64: 3, 128: 3}}[n][ec]
     L = most if levels == "most" else min(levels, most)
     check(M, 2, 3 * n ** L, ec, 2, n, 0, L)          # three windows of every level
+    # workgroups that are full in either direction
+    check(M, 1, 3 * 8192 // ec, ec, 2, n, 0, L, forward="radix", backward="radix")
 
 
 @pytest.mark.parametrize("n,ec,first,L", [(2, 32, 3, 6), (4, 32, 1, 3), (2, 8, 1, 9), (4, 64, 1, 2)])
@@ -61,6 +69,21 @@ def test_levels_that_do_not_start_at_the_first(M, n, ec, first, L):
 @pytest.mark.parametrize("n,ec,L", [(2, 32, 7), (4, 32, 3), (2, 128, 5), (4, 16, 4)])
 def test_other_activations(M, n, ec, L, act):
     check(M, 2, 3 * n ** L, ec, 2, n, 0, L, act)
+
+
+# the same on launches that are large enough for the registers
+@pytest.mark.parametrize("act", [1, 2, 3, -1])
+@pytest.mark.parametrize("n,ec,L,batch,N", [(2, 32, 6, 300, 64), (4, 16, 3, 300, 64), (2, 128, 4, 150, 48), (4, 64, 3, 150, 64), (2, 8, 3, 300, 24)])
+def test_other_activations_on_many_workgroups(M, n, ec, L, batch, N, act):
+    check(M, batch, N, ec, 2, n, 0, L, act, forward="radix", backward="radix")
+
+
+@pytest.mark.parametrize("n,ec,batch,N,L,act,backward", [(2, 8, 5, 80, 4, 0, "fused"), (2, 16, 3, 96, 5, 0, "fused"), (2, 32, 3, 96, 5, 0, "radix"),
+                                                         (2, 64, 2, 48, 4, 0, "radix"), (2, 128, 2, 24, 3, 0, "radix"), (4, 8, 3, 192, 3, 0, "fused"),
+                                                         (4, 32, 2, 48, 2, 0, "fused"), (4, 128, 2, 16, 2, 0, "radix"), (2, 32, 2, 256, 6, 2, "fused"),
+                                                         (4, 16, 2, 192, 3, 1, "fused"), (2, 64, 2, 128, 5, -1, "radix"), (2, 1, 3, 48, 4, 0, "fused")])
+def test_few_workgroups(M, n, ec, batch, N, L, act, backward):
+    check(M, batch, N, ec, 16 if ec == 1 else 2, n, 0, L, act, forward="fused", backward=backward)
 
 
 @pytest.mark.parametrize("n,E,L,act", [(2, 32, 8, 0), (4, 64, 4, 0), (2, 8, 9, 2), (4, 16, 3, -1)])
@@ -76,13 +99,14 @@ def test_bfloat16_inputs_and_gradients(M, n, ec, L):
 # windows counted through batch entries: several entries to a workgroup, an entry that begins inside one and ends in the next, a
 # last workgroup that is not full; levels that do not start at the first; more and fewer windows to an entry than to a workgroup
 @pytest.mark.parametrize("batch,N,ec,n,first,L,act,dtype", [
-    (41, 4, 8, 2, 0, 2, 0, torch.float32), (130, 8, 32, 2, 0, 3, 0, torch.float32), (13, 80, 32, 2, 0, 4, 0, torch.float32),
-    (5, 640, 32, 2, 0, 7, 0, torch.float32), (7, 96, 64, 2, 0, 5, 0, torch.float32), (9, 48, 128, 2, 0, 4, 0, torch.float32),
-    (6, 96, 16, 2, 2, 3, 0, torch.float32), (11, 48, 32, 4, 0, 2, 0, torch.float32), (3, 192, 16, 4, 1, 2, 0, torch.bfloat16),
-    (50, 64, 8, 4, 0, 3, 2, torch.float32), (21, 96, 32, 2, 0, 5, -1, torch.bfloat16), (33, 56, 1, 2, 0, 3, 0, torch.float32),
-    (33, 112, 1, 4, 0, 2, 2, torch.float32)])
+    (181, 4, 8, 2, 0, 2, 0, torch.float32), (190, 8, 32, 2, 0, 3, 0, torch.float32), (175, 80, 32, 2, 0, 4, 0, torch.float32),
+    (18, 640, 32, 2, 0, 7, 0, torch.float32), (91, 96, 64, 2, 0, 5, 0, torch.float32), (89, 48, 128, 2, 0, 4, 0, torch.float32),
+    (175, 96, 16, 2, 2, 3, 0, torch.float32), (173, 48, 32, 4, 0, 2, 0, torch.float32), (175, 192, 16, 4, 1, 2, 0, torch.bfloat16),
+    (181, 64, 8, 4, 0, 3, 2, torch.float32), (177, 48, 32, 2, 0, 4, -1, torch.bfloat16), (519, 56, 1, 2, 0, 3, 0, torch.float32),
+    (523, 16, 1, 4, 0, 2, 2, torch.float32)])
 def test_windows_of_several_batch_entries(M, batch, N, ec, n, first, L, act, dtype):
-    check(M, batch, N, ec, 16 if ec == 1 else 3, n, first, L, act, dtype)   # (heads of one feature are laid out as one of 16)
+    # (heads of one feature are laid out as one of 16)
+    check(M, batch, N, ec, 16 if ec == 1 else 3, n, first, L, act, dtype, forward="radix", backward="radix")
 
 
 @pytest.mark.parametrize("n,L,rows", [(2, 2, 4), (4, 2, 16)])
