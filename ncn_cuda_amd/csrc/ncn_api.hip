@@ -144,12 +144,12 @@ struct Plan {
 
 // reserve_rows: rows of the dW partial buffer kept free for another launch of the same stage
 // row_cap: rows of the dW partial buffer the caller has (kMaxGridX in a workspace of ncn_workspace_bytes)
-// may_split: may_split_call() of the launches that are planned
-Plan make_plan(const ncn_shape* sh, int path, const AnyTile& any, bool may_split, int reserve_rows = 0, int row_cap = kMaxGridX) {
+// split_limit: split_limit_of() the launches that are planned
+Plan make_plan(const ncn_shape* sh, int path, const AnyTile& any, int64_t split_limit, int reserve_rows = 0, int row_cap = kMaxGridX) {
     Plan p;
     const int max_rows = row_cap - reserve_rows;
     p.path = path;
-    p.split = may_split && path == 2 && sh->batch * sh->N * sh->E <= split_max_elements(sh->n_cache);
+    p.split = path == 2 && sh->batch * sh->N * sh->E <= split_limit;
     p.any = any;
     const int ec = (int)(sh->E / sh->n_head);
     p.groups_per_tile = any.r ? 64 >> (any.lf_log2 + any.lr_log2)
@@ -158,7 +158,7 @@ Plan make_plan(const ncn_shape* sh, int path, const AnyTile& any, bool may_split
     p.groups = (uint32_t)(sh->N / sh->n_cache);
     p.tiles_per_inst = (p.groups + p.groups_per_tile - 1) / p.groups_per_tile;
     p.total_tiles = (uint32_t)(sh->batch * p.tiles_per_inst);
-    if (p.split && p.total_tiles > (uint32_t)max_rows) return make_plan(sh, path, any, false, reserve_rows, row_cap);
+    if (p.split && p.total_tiles > (uint32_t)max_rows) return make_plan(sh, path, any, 0, reserve_rows, row_cap);
     if (p.split) {
         p.grid_x = p.grid_fwd = 0;   // launch_split makes its own
         p.partial_rows = (int)p.total_tiles;
@@ -318,8 +318,11 @@ const ncn_shape* planning_shape(const ncn_shape* sh, ncn_shape* as_wide) {
     return headwise_call(sh, 2, as_wide) ? as_wide : sh;
 }
 
-// Whether launches of a call may go to the kernels for few groups.
-bool may_split_call(int activation, bool headwise) { return activation == NCN_ACT_TANH && !headwise; }
+// Up to how many elements the launches of a call go to the kernels for few groups; 0: never.
+int64_t split_limit_of(const ncn_shape* sh, int activation, bool headwise, bool backward, bool indexed) {
+    if (activation != NCN_ACT_TANH || headwise) return 0;
+    return split_max_elements(sh->n_cache, (int)(sh->E / sh->n_head), backward, indexed);
+}
 
 // One stage.  Register kernels: the plain builds know the stride permutation only, the others read the launch's table,
 // radix level and context lengths.
@@ -567,7 +570,7 @@ static int forward_impl(const void* x, const void* xa, int in_dtype, void* y, vo
     if (!aligned16(x) || !aligned16(xa) || !aligned16(y) || !aligned16(ya) || !w.aligned(n_stages) || !aligned16(y32) ||
         !aligned16(ya32) || !aligned16(workspace))
         return NCN_ERR_ALIGN;
-    const Plan p = make_plan(shape, path, any_tile_for(shape, path, alpha, m), may_split_call(activation, headwise));
+    const Plan p = make_plan(shape, path, any_tile_for(shape, path, alpha, m), split_limit_of(shape, activation, headwise, false, !grouping.plain()));
     hipStream_t s = static_cast<hipStream_t>(stream);
 
     // several stages: LDS-resident passes when the shape allows and the buffers permit the ping-pong
@@ -690,7 +693,7 @@ static int inverse_impl(const void* y, const void* ya, int in_dtype, void* x, vo
     if (!known_dtype_or_x2(in_dtype, n_stages, path) || !known_dtype(out_dtype)) return NCN_ERR_DTYPE;
     if (!aligned16(x) || !aligned16(xa) || !aligned16(y) || !aligned16(ya) || !w.aligned(n_stages) || !aligned16(workspace))
         return NCN_ERR_ALIGN;
-    const Plan p = make_plan(shape, path, any_tile_for(shape, path, alpha, m), may_split_call(activation, headwise));
+    const Plan p = make_plan(shape, path, any_tile_for(shape, path, alpha, m), split_limit_of(shape, activation, headwise, false, !grouping.plain()));
     hipStream_t s = static_cast<hipStream_t>(stream);
 
     // several stages: LDS-resident passes, last pass of the range first.  Without scratch to ping-pong with, the
@@ -820,7 +823,7 @@ static int backward_impl(const void* y, const void* ya, int y_dtype, const void*
     // partial rows of the generic kernel's second launch
     const AnyTile any = any_tile_for(shape, path, alpha, m);
     const int extra_rows = (grouping.ctx_len && path != 2 && !any.r) ? edge_rows(shape) : 0;
-    const Plan p = make_plan(shape, path, any, may_split_call(activation, headwise), extra_rows, row_cap);
+    const Plan p = make_plan(shape, path, any, split_limit_of(shape, activation, headwise, true, !grouping.plain()), extra_rows, row_cap);
     hipStream_t s = static_cast<hipStream_t>(stream);
     float* partials = static_cast<float*>(workspace);
     float* level1 = partials + (int64_t)row_cap * 2 * shape->E;
@@ -1029,7 +1032,7 @@ int ncn_forward_radix(const void* x, const void* xa, int in_dtype, void* y, void
     ncn_shape as_wide;
     const bool headwise = headwise_call(shape, path, &as_wide);
     if (headwise) shape = &as_wide;
-    const Plan p = make_plan(shape, path, any_tile_for(shape, path, alpha, m), may_split_call(activation, headwise));
+    const Plan p = make_plan(shape, path, any_tile_for(shape, path, alpha, m), split_limit_of(shape, activation, headwise, false, true));
     hipStream_t s = static_cast<hipStream_t>(stream);
     const std::vector<RadixPass> passes = plan_radix(shape, first_level, n_levels, false, path == 2);
     // every pass is closed: the first reads x, xa and the later ones run in place on y, ya; passes of several levels
@@ -1093,7 +1096,7 @@ int ncn_backward_radix(const void* y, const void* ya, int y_dtype, const void* d
     ncn_shape as_wide;
     const bool headwise = headwise_call(shape, path, &as_wide);
     if (headwise) shape = &as_wide;
-    const Plan p = make_plan(shape, path, any_tile_for(shape, path, alpha, m), may_split_call(activation, headwise));
+    const Plan p = make_plan(shape, path, any_tile_for(shape, path, alpha, m), split_limit_of(shape, activation, headwise, true, true));
     hipStream_t s = static_cast<hipStream_t>(stream);
     float* partials = static_cast<float*>(workspace);
     float* level1 = partials + (int64_t)kMaxGridX * 2 * shape->E;
@@ -1153,7 +1156,7 @@ int ncn_inverse_radix(const void* y, const void* ya, int in_dtype, void* x, void
     ncn_shape as_wide;
     const bool headwise = headwise_call(shape, path, &as_wide);
     if (headwise) shape = &as_wide;
-    const Plan p = make_plan(shape, path, any_tile_for(shape, path, alpha, m), may_split_call(activation, headwise));
+    const Plan p = make_plan(shape, path, any_tile_for(shape, path, alpha, m), split_limit_of(shape, activation, headwise, false, true));
     hipStream_t s = static_cast<hipStream_t>(stream);
     const std::vector<RadixPass> passes = plan_radix(shape, first_level, n_levels, false, path == 2);
     for (size_t e = 0; e < passes.size(); ++e) {   // last pass first; every pass is closed: in place after the first
@@ -1186,7 +1189,8 @@ int ncn_inverse_radix(const void* y, const void* ya, int in_dtype, void* x, void
 struct StackCall {
     ncn_shape as_wide;
     const ncn_shape* shape;
-    bool headwise, may_split;
+    bool headwise;
+    int activation;
     const std::vector<StackRange>* ranges;   // of this thread's kept plans
     size_t plane;        // one float32 activation array
     int fwd_passes_max;  // passes of the longest range
@@ -1226,8 +1230,8 @@ struct StackCall {
         plane = temp_bytes(shape, false) / 2;
         fwd_passes_max = bwd_passes_max = bwd_passes = 0;
         int64_t rows = 0;
-        may_split = may_split_call(activation, headwise);
-        const Plan single = one_stage();
+        this->activation = activation;
+        const Plan single = one_stage(true);
         for (const StackRange& r : *ranges) {
             if ((int)r.fwd.size() > fwd_passes_max) fwd_passes_max = (int)r.fwd.size();
             if ((int)r.bwd.size() > bwd_passes_max) bwd_passes_max = (int)r.bwd.size();
@@ -1239,7 +1243,9 @@ struct StackCall {
         row_cap = rows < kMaxGridX ? kMaxGridX : (int)rows;
         return true;
     }
-    Plan one_stage() const { return make_plan(shape, 2, AnyTile{0, 0, 0, 0}, may_split); }   // of the passes of one stage
+    Plan one_stage(bool backward) const {   // of the passes of one stage
+        return make_plan(shape, 2, AnyTile{0, 0, 0, 0}, split_limit_of(shape, activation, headwise, backward, false));
+    }
     // pairs of arrays in the workspace: the forward's passes that are not kept go through one; the backward's gradients
     // through one (two where dx, dxa cannot hold them in between), reconstructed inputs inside a range through two more
     size_t forward_bytes() const { return fwd_passes_max > 1 ? 2 * plane : 0; }
@@ -1281,7 +1287,7 @@ int ncn_stack_forward(const void* x, const void* xa, int in_dtype, void* y, void
     const size_t nr = c.ranges->size();
     if ((nr > 1 || out_dtype != NCN_F32) && !saves) return NCN_ERR_NULL;
     if (c.forward_bytes() && (!workspace || workspace_bytes < c.forward_bytes())) return NCN_ERR_WORKSPACE;
-    const Plan p = c.one_stage();
+    const Plan p = c.one_stage(false);
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int64_t elements = shape->batch * shape->N * shape->E;
     void* const t0 = workspace;
@@ -1348,7 +1354,7 @@ int ncn_stack_backward(const float* y, const float* ya, const float* saves, cons
     const size_t nr = c.ranges->size();
     if ((nr > 1 || !y) && !saves) return NCN_ERR_NULL;
     if (!workspace || workspace_bytes < c.backward_bytes(dx_dtype == NCN_F32)) return NCN_ERR_WORKSPACE;
-    const Plan p = c.one_stage();
+    const Plan p = c.one_stage(true);
     hipStream_t s = static_cast<hipStream_t>(stream);
     const int64_t elements = shape->batch * shape->N * shape->E, two_e = 2 * shape->E;
     float* partials = static_cast<float*>(workspace);

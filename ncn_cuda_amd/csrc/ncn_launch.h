@@ -102,13 +102,30 @@ NCN_DECLARE(true, kAnyTypes) NCN_DECLARE(true, kF32Types) NCN_DECLARE(true, kBf1
 template <> hipError_t launch_stage_backward<false, kAnyTypesOnce>(const StageArgs&, int, hipStream_t);
 template <> hipError_t launch_stage_backward<true, kAnyTypesOnce>(const StageArgs&, int, hipStream_t);
 // Launches with few groups (ncn_split_kernels.h): tanh, one row fragment of 4 features per lane.
-// Up to 2^20 elements (four waves of them per SIMD, one of the register tiles) they are as fast or faster in both directions
-// from groups of 8 rows on: us of a launch on the register tiles : here, heads of 32, float32, backward with its reduction,
-//   groups of 32   2^19: 15.6 : 10.2, backward 38.8 : 25.0   2^20: 16.9 : 16.4, 41.6 : 35.6   2^21: 27.6 : 28.2, 53.9 : 61.7
-//   groups of 16   2^19: 9.4 : 6.5, 21.1 : 16.1              2^20: 10.7 : 9.9, 23.3 : 22.9    2^21: 16.8 : 16.7, 32.3 : 37.6
-//   groups of 8    2^19: 6.4 : 4.6, 12.9 : 10.6              2^20: 7.5 : 6.5, 14.8 : 14.5     2^21: 11.6 : 10.6, 21.8 : 25.1
-// Smaller groups have short chains (their tile is 2 x 4): groups of 4, 2^18: 3.7 : 3.3, 7.4 : 6.8; 2^19: 4.1 : 3.8, 8.0 : 8.7.
-constexpr int64_t split_max_elements(int n_cache) { return n_cache >= 8 ? 1 << 20 : 1 << 18; }
+// The time of a launch here over that on the register tiles, float32, backward with its reduction (bfloat16 is within 0.05 of it but
+// where named; behind a table):
+//                 forward, 2^19   3 2^18   2^20 elements    backward, 2^19   3 2^18   2^20             tiles : here at 2^20, us
+//   8 rows of  8      0.73  0.78  0.86 (table 0.83)            0.85  0.99  1.03 (table 0.97)            8.2 :  7.1, 14.1 : 14.6
+//   8 rows of 16      0.75  0.81  0.90 (0.88)                  0.87  0.98  1.07 (1.04)                  7.6 :  6.8, 13.6 : 14.5
+//   8 rows of 32      0.74  0.80  0.87 (0.85)                  0.80  0.91  1.00 (0.97)                  7.9 :  6.9, 14.8 : 14.8
+//  16 rows of 16      0.72  0.80  0.93 (0.89)                  0.78  0.90  1.04 (1.00)                 10.3 :  9.6, 20.3 : 21.2
+//  16 rows of 32      0.71  0.82  0.96 (0.90)                  0.77  0.86  1.01 (0.97)                 10.8 : 10.3, 22.7 : 22.9
+//  32 rows of  4      0.58  0.72  0.82 (0.83)                  0.68  0.84  1.00, bfloat16 1.08 (0.93)
+//  32 rows of 16      0.68  0.84  1.01 (0.95)                  0.79  0.91  1.09 (1.05)                 16.2 : 16.4, 35.1 : 38.2
+//  32 rows of 32      0.67  0.81  0.98 (0.90)                  0.65  0.73  0.88 (0.84)                 17.0 : 16.8, 40.4 : 35.4
+//  64 rows of  8      0.64  0.83  1.00 (0.99)                  0.71  0.85  1.03, bfloat16 1.07 (1.01)
+//  64 rows of 16      0.65  0.87  1.03, bfloat16 1.12 (0.93)   0.67  0.78  0.96 (0.93)
+// Heads of 64 and 128 (whose tiles hold 8 features per lane) and 64 rows of 32: at most 0.83 everywhere at 2^20.
+// Smaller groups have short chains (their tile is 2 x 4).  Two rows, heads up to 32: forward 0.92 to 0.98 up to 2^17, 0.91 to 1.04 at
+// 2^18, backward 0.91 to 1.02, 0.94 to 1.05; wider heads at most 0.97 at 2^18.  Four rows, 2^18: at most 0.98; 2^19: up to 1.08.
+constexpr int64_t split_max_elements(int n_cache, int head_dim, bool backward, bool indexed) {
+    if (n_cache == 2) return head_dim <= 32 ? 1 << 17 : 1 << 18;
+    if (n_cache == 4) return 1 << 18;
+    const bool even_earlier = backward ? (head_dim == 16 && n_cache <= 32) || (head_dim == 8 && (n_cache == 8 || n_cache == 64)) ||
+                                             (head_dim == 4 && n_cache == 32)
+                                       : (head_dim == 16 && n_cache >= 32) || (head_dim == 8 && n_cache == 64);
+    return !indexed && even_earlier ? 3 << 18 : 1 << 20;
+}
 int split_groups_per_tile(int nc, int ec);
 // indexed: the builds that honour a.table, a.radix_stride and a.ctx_len
 hipError_t launch_split(Pass pass, const StageArgs& a, bool indexed, hipStream_t s);

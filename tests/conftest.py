@@ -54,7 +54,7 @@ def kernels_of(call):
     with profile(activities=[ProfilerActivity.CUDA]) as seen:
         result = call()
         torch.cuda.synchronize()
-    names = {e.name.split("(ncn::")[0].split("ncn::")[-1] for e in seen.events() if "ncn::" in e.name}
+    names = {e.name.replace("(anonymous namespace)::", "").split("(ncn::")[0].split("ncn::")[-1] for e in seen.events() if "ncn::" in e.name}
     assert names
     return result, names
 
