@@ -175,6 +175,35 @@ def test_fewer_activations_are_kept_where_memory_is_short(M, monkeypatch, dtype,
         assert O.rel_err(dW[l], ref[4][l].reshape(-1)) < tol
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+def test_a_native_node_without_memory_leaves_the_call_to_the_python_node(M, dtype):
+    """The native node plans for every activation and runs out of memory; the call is then made with the fewest."""
+    from ncn_cuda_amd.modules import fused_ncn_net
+    batch, N, E, C, n, L = 64, 1018, 128, 4, 2, 13     # 66 MB a pair of float32 activations, one launch per stage
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    x, xa, dy, dya = (torch.randn(batch, N, E, generator=gen, device="cuda").to(dtype) for _ in range(4))
+    leaves = [x.requires_grad_(), xa.requires_grad_(), *((torch.randn(2 * E, generator=gen, device="cuda") / n ** 0.5).requires_grad_() for _ in range(L))]
+
+    def call():
+        y, ya = fused_ncn_net(leaves[0], leaves[1], leaves[2:], 0.9, 0, n, C)
+        return type(y.grad_fn).__name__, [y.detach(), ya.detach(), *torch.autograd.grad([y, ya], leaves, [dy, dya])]
+
+    name, want = call()
+    assert name != "NCNNetFunctionBackward"
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (600 << 20)) / total)   # the saves alone are 800 MB
+    try:
+        name, got = call()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert name == "NCNNetFunctionBackward"
+    tol = 1.2e-6 * 0.9 ** -(n * L) if dtype == torch.float32 else 2.0 ** -8   # as in test_stack
+    for a, b in zip(got, want):
+        assert O.rel_err(a, b) < tol
+
+
 def test_refusals(M):
     """Outputs that are the inputs, a workspace that is too small: refused before any launch."""
     from ncn_cuda_amd import _lib

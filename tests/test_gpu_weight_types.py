@@ -19,9 +19,13 @@ def M():
 
 
 # (n_cache, E, heads, groups, stages, alpha)
-CASES = [(16, 128, 4, 4, 1, 0.9),   # register kernels, tiles of 4 x 4
-         (4, 128, 2, 6, 1, 0.9),    # 2 x 8
-         (16, 256, 4, 3, 1, 0.9),   # 4 x 8, an odd number of groups
+CASES = [(16, 128, 4, 4, 1, 0.9),   # kernels for few groups, a group over two waves
+         (4, 128, 2, 6, 1, 0.9),    # .. in part of one
+         (16, 256, 4, 3, 1, 0.9),   # .. over four, an odd number of groups
+         (16, 128, 4, 173, 1, 0.9), # larger launches: register tiles of 4 x 4
+         (4, 128, 2, 173, 1, 0.9),  # 2 x 8
+         (2, 32, 4, 1367, 1, 0.9),  # 2 x 4
+         (16, 256, 4, 87, 1, 0.9),  # 4 x 8, an odd number of groups
          (8, 32, 32, 4, 1, 0.9),    # heads of one feature
          (5, 30, 2, 5, 1, 0.9),     # no powers of two
          (5, 30, 2, 5, 1, 0.0),     # generic kernels (alpha outside the scaled state)
@@ -52,7 +56,8 @@ def test_bfloat16_weights(M, case):
 
 @pytest.mark.parametrize("types", [(torch.bfloat16, torch.float32), (torch.float32, torch.bfloat16)], ids=["bf16-f32", "f32-bf16"])
 @pytest.mark.parametrize("act", [0, 1])
-@pytest.mark.parametrize("n,E,C,groups", [(16, 128, 4, 5), (16, 256, 4, 3), (4, 64, 4, 7), (8, 32, 32, 3)])
+@pytest.mark.parametrize("n,E,C,groups", [(16, 128, 4, 5), (16, 256, 4, 3), (4, 64, 4, 7), (8, 32, 32, 3),
+                                          (16, 128, 4, 257), (16, 256, 4, 129), (4, 64, 4, 513)])   # register tiles with tanh too
 def test_bfloat16_weights_with_mixed_types(M, n, E, C, groups, act, types):
     """The builds for every element type: results of another type than the inputs, with and without a table."""
     first, second = types
@@ -70,7 +75,7 @@ def test_bfloat16_weights_with_mixed_types(M, n, E, C, groups, act, types):
                                          grad_dtype=first, **kw))
 
 
-@pytest.mark.parametrize("case", [CASES[0], CASES[6], CASES[7]], ids=lambda c: "n%d_E%d_C%d_g%d_L%d_a%g" % c)
+@pytest.mark.parametrize("case", [CASES[0], CASES[10], CASES[11]], ids=lambda c: "n%d_E%d_C%d_g%d_L%d_a%g" % c)
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_one_array_per_stage(M, case, dtype):
     """NCN_W_ARRAYS: the weights of every stage where they are."""
