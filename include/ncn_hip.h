@@ -260,8 +260,8 @@ int ncn_inverse_indexed(const void* y, const void* ya, int in_dtype,
  * Replaces: the grouping of ncn_triton/group_tensors.py:8-18 (extract_group_index), which the reference only has as a
  *           helper that writes index tensors; level 0 is stage 0 of the stride permutation.  The same levels can be
  *           run through ncn_*_indexed with tables; these entry points need no table and, for n_cache 2 or 4 with a
- *           head width of 16 or 32, keep windows of n_cache^k rows in LDS over k levels per pass (such windows are
- *           closed: no halo, every pass in place), so a stack of log_n(N) levels costs two or three passes over HBM.
+ *           head width of 8 to 128 (powers of two), keep windows of n_cache^k rows on the chip over k levels per pass (such
+ *           windows are closed: no halo, every pass in place), so a stack of log_n(N) levels costs two or three passes over HBM.
  * n_cache^(first_level+n_levels) must divide N (NCN_ERR_SHAPE otherwise).  W, dW: [n_levels, 2E].
  * Arguments as in ncn_forward / ncn_backward.  Levels after the first pass run in place on y, ya (forward) and on
  * x_rec, xa_rec, dx, dxa (backward): use float32 outputs when more than one pass is needed, or the values between
@@ -294,8 +294,9 @@ int ncn_inverse_radix(const void* y, const void* ya, int in_dtype,
 
 /* How the calls above cut the levels into passes (the inverse uses the forward's cut); returns the number of passes or a negative error code and
  * writes up to max_passes records of 6 int32 into `out` (may be NULL):
- *   [0] first level of the pass relative to first_level   [1] levels in the pass   [2] 0 one-stage launch, 1 LDS windows
- *   [3] n_cache^(first level): distance in rows between the rows of a window   [4] rows of a window   [5] rows per workgroup
+ *   [0] first level of the pass relative to first_level   [1] levels in the pass   [2] 0 one-stage launch, 1 windows of several levels
+ *   [3] n_cache^(first level): distance in rows between the rows of a window   [4] rows of a window   [5] rows of a
+ *   batch entry that a workgroup takes (where they leave it partly empty, windows of the next entries may join them)
  * No reference counterpart. */
 int ncn_plan_radix(const ncn_shape* shape, int first_level, int n_levels, int activation, int backward, int32_t* out,
                    int max_passes);

@@ -6,14 +6,15 @@
 // LR = 2^lr_log2 row lanes, so that R * LR covers n_cache rows and F * LF the head's features with little padding
 // (any_tile() in ncn_launch.h; 5 rows of 40 features: R = 3, F = 5, LF = 8, LR = 2, one row of six padded).  Padded
 // features have zero weights and zero gradients, which stay zero; padded rows have zero gradients, which stay zero, and
-// never are a pivot.  The feature of a lane's register f is f * LF + (lane % LF): a load instruction reads LF consecutive
-// elements of a row, at any alignment, where F consecutive ones per lane would touch every line F times over.
+// never are a pivot.  Where a head is a whole number of lanes, a lane holds F adjacent features, which one instruction of up
+// to four words moves (AnyFrag); elsewhere the feature of register f is f * LF + (lane % LF), one word at a time, because a
+// lane's F adjacent features would reach past the head.
 //
 // What bounds it: vector issue, as for the shapes of powers of two; the levels of the cross-lane sums are taken under
 // wave-uniform branches because LF and LR are not known at compile time.  One lane per row with the state in LDS (the
 // generic kernels, which still take what fits no tile, scalars outside the scaled state and m < 0.85) leaves three quarters of
 // the time to LDS traffic and its barriers.
-// 16 x 1005 x 160 float32, groups of 5 rows, heads of 40: forward 113 -> 17.6 us, backward 519 -> 31.7 us per stage.
+// 16 x 1005 x 160 float32, groups of 5 rows, heads of 40: forward 113 -> 15.5 us, backward 519 -> 26.3 us per stage.
 #pragma once
 #include <type_traits>
 

@@ -488,7 +488,7 @@ def inverse_stages(y, ya, W, alpha, activation, cache_dim, nhead, first_stage, n
 def forward_radix(x, xa, W, alpha, activation, cache_dim, nhead, first_level, n_levels, *, m=M_DEFAULT,
                   out_dtype=None):
     """Levels first_level .. first_level+n_levels-1 of the radix-n digit grouping (ncn_triton/group_tensors.py:8-18)
-    without index tensors; W: [n_levels, 2E].  Several levels per pass stay in LDS for n_cache 2 and 4.  Outputs are
+    without index tensors; W: [n_levels, 2E].  Several levels run per pass over memory for n_cache 2 and 4.  Outputs are
     float32 unless out_dtype says otherwise (values between passes live in the outputs)."""
     shape = validate(x, xa, W, cache_dim, nhead, activation, 0, n_levels, alpha=alpha, m=m)
     dev = _require_gpu(x, xa, W)
