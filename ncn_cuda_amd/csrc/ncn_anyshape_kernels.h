@@ -319,12 +319,17 @@ __global__ void __launch_bounds__(kBlockThreads, R * F <= 16 ? 4 : R * F <= 20 ?
         float x[R][F], a[R][F];
         any_issue(A.in0, A.in_dtype, L, x);
         any_issue(A.in1, A.in_dtype, L, a);
-        any_weights(A, L, head, wi, wj);   // behind the tile's own loads: one latency, not two
+        if constexpr (!LENGTHS) any_weights(A, L, head, wi, wj);   // behind the tile's own loads: one latency, not two
         any_finish(A.in_dtype, x);
         any_finish(A.in_dtype, a);
-        if (LENGTHS) {   // rows past a context length pass through
-            any_store<true>(A, L, A.out0, A.out1, A.out_dtype, x, a);
-            if (!INVERSE && A.aux0) any_store<true>(A, L, A.aux0, A.aux1, NCN_F32, x, a);
+        if constexpr (LENGTHS) {
+            if (__any(L.live >= 0 && L.live < (int)A.n_cache)) {   // rows past a context length pass through
+                any_store<true>(A, L, A.out0, A.out1, A.out_dtype, x, a);
+                if (!INVERSE && A.aux0) any_store<true>(A, L, A.aux0, A.aux1, NCN_F32, x, a);
+            }
+            // after those stores, beside which the weights would take 10 to 20 registers: launches with lengths, 3 x 4 and 2 x 5
+            // tiles, were up to 1.17 times as long, by the waves that a SIMD then holds (four or five instead of six or seven)
+            any_weights(A, L, head, wi, wj);
         }
         any_fill_padding(L, x, INVERSE ? any_missing_undone(S) : 1.f);
         any_fill_padding(L, a);
