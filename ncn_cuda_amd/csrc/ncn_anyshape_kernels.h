@@ -327,8 +327,8 @@ __global__ void __launch_bounds__(kBlockThreads, R * F <= 16 ? 4 : R * F <= 20 ?
                 any_store<true>(A, L, A.out0, A.out1, A.out_dtype, x, a);
                 if (!INVERSE && A.aux0) any_store<true>(A, L, A.aux0, A.aux1, NCN_F32, x, a);
             }
-            // after those stores, beside which the weights would take 10 to 20 registers: launches with lengths, 3 x 4 and 2 x 5
-            // tiles, were up to 1.17 times as long, by the waves that a SIMD then holds (four or five instead of six or seven)
+            // after those stores, beside which the weights would take 10 to 20 registers and a SIMD hold four or five waves instead
+            // of six or seven: x[1559, 48, 40] bfloat16 with lengths, groups of 16, heads of 20, sigmoid, forward 44.7 us, here 37.8
             any_weights(A, L, head, wi, wj);
         }
         any_fill_padding(L, x, INVERSE ? any_missing_undone(S) : 1.f);

@@ -1,6 +1,7 @@
 // Planning and launching of multi-stage passes over levels of the radix-n digit grouping
 // (ncn_triton/group_tensors.py:8-18); the kernels are those of ncn_radix_kernels.h, built in ncn_radix_build.hip, and in
 // launches with few workgroups the RADIX builds of ncn_fused_kernels.h (ncn_radix_lds.hip).
+#include <algorithm>
 #include <climits>
 #include <cmath>
 #include <vector>
@@ -42,40 +43,46 @@ struct RadixLoads {
     bool lds;          // for the kernels that keep rows in LDS
 };
 
-// Whether a launch of so many workgroups, of `rows` rows each, runs on the kernels that keep rows in LDS.  A lane of the register
-// kernels holds 16 elements and more, and a workgroup takes the same time however few of its rows exist; the LDS kernels spread the
-// rows there are over 8 waves, 8 elements to a lane, which is the shorter chain as long as every workgroup starts at once and has
-// at most half the rows that fit.  tanh, us, LDS : registers, forward | backward, N = rows, by workgroups:
-//   groups of two, heads of  8,  8 rows, 3 levels  64:  6.0 : 11.0 | 11.0 : 12.6   256:  6.1 : 11.4 | 11.3 : 12.9   512:  8.1 : 11.8 | 12.8 : 12.9
-//   groups of two, heads of 32,  8 rows, 3 levels  64:  5.9 :  9.4 | 10.7 : 10.9   256:  6.0 :  9.5 | 10.9 : 11.2   512:  7.4 :  9.6 | 12.1 : 11.3
-//   groups of two, heads of 32, 128 rows, 7 levels 64: 11.9 : 15.8 | 22.1 : 18.1   256: 13.1 : 16.8 | 24.0 : 19.6   512: 20.2 : 19.4 | 36.7 : 32.3
-//   groups of two, heads of 64,  8 rows, 3 levels  64:  7.1 :  9.4 | 13.9 : 11.4   256:  7.3 :  9.5 | 14.3 : 11.6   512: 12.6 :  9.7 | 24.3 : 12.0
-//   groups of four, heads of 32, 64 rows, 3 levels 64:  8.2 : 12.9 | 14.3 : 16.4   256:  8.8 : 13.4 | 15.2 : 17.3   512: 11.9 : 14.0 | 19.8 : 18.3
-// With all the rows that fit (groups of two, heads of 16, 8 levels of 512 rows forward and 256 backward) registers win from the
-// first workgroup on, by 10 and 11 %.
-//   The other activations spend more instructions on an element, which 8 waves of few elements overlap better: the time on registers
-// over that in LDS, relu, groups of two, by workgroups (512, 2048, 6000 unless named), forward heads of 16: 128 rows of 512 2.12, 0.78,
-// 0.59, 256 rows 1.97, 1.23, 0.99, all 512 rows 1.27, 1.12, 1.07 (sigmoid 1.14, 1.03, 0.95); heads of 64: 64: 1.38, 256: 1.36, 512:
-// 0.86; groups of four, heads of 8: 512 of 1024 rows 1.23, 0.82, 0.82, all of them 0.80.  Backward, heads of 32, all 128 rows: 64:
-// 1.28, 256: 1.24, 512: 0.77; heads of 64 0.87 at 64.
-bool rows_in_lds(int nc, int ec, bool backward, bool tanh, uint32_t rows, uint32_t cap, int64_t workgroups) {
-    const bool half = 2 * rows <= cap, quarter = 4 * rows <= cap;
+// Whether a pass runs on the kernels that keep rows in LDS, in `lds` workgroups of `rows` rows each, or in `registers` workgroups on
+// those that hold `cap` rows in registers.  A lane of the latter holds 16 elements and more, and a workgroup takes the same time
+// however few of its rows exist; the former spread the rows there are over 8 waves, 8 elements to a lane, which is the shorter chain as
+// long as the workgroups start at once: two to a CU (one on heads of 64 and more) against three.
+//   Forward and inverse of tanh, us in LDS : in registers by workgroups (lds, registers).  Groups of two, heads of 8, 6 levels, 64 of
+// 1024 rows: (256, 16) 7.5 : 15.9, (512, 32) 9.0 : 15.9, (1024, 64) 16.3 : 16.3; 576 rows: (256, 144) 13.6 : 17.8, (512, 288) 20.5 : 27.3;
+// heads of 32, 5 levels, 96 of 256 rows: (512, 192) 14.3 : 13.2, (576, 216) 19.5 : 13.5; 8 levels, all rows: (256, 256) 22.6 : 18.5; heads
+// of 64, 5 levels, 32 of 128 rows: (256, 64) 10.0 : 12.5, (512, 128) 18.0 : 13.2.  So a pair on a CU takes 1.2 times as long as one workgroup,
+// more the fuller it is of rows, a workgroup longer with more rows, and one more in registers 0.6 of the first; their ratio is that of
+// the chains.
+//   The other activations spend more instructions on an element, and either kind takes whole rounds of what starts at once: relu,
+// groups of two, heads of 8, 5 levels, 32 rows: (512, 16) 14 : 36, (1024, 32) 25 : 36, (2048, 64) 48 : 36; heads of 32, 8 levels, all 256
+// rows: (512, 512) 49 : 60, (1024, 1024) 88 : 115; groups of four, heads of 8, 256 of 1024 rows: (512, 128) 22 : 30, (1024, 256) 40 : 33.
+//   Over 8684 passes of 16 to 16384 workgroups the choice takes 0.1 % longer than the better of the two, at
+// most 15 %.
+//   Backward, tanh, groups of two, heads of 8, 8 rows, 3 levels (256, 4) 11.2 : 12.8, (1024, 16) 21.1 : 13.0; heads of 32: 10.8 : 11.3,
+// 128 rows, 7 levels (256, 256) 23.3 : 19.3; groups of four, heads of 32, 64 rows, 3 levels (256, 128) 15.3 : 17.4, (512, 256)
+// 19.3 : 18.2.  Others, heads of 32, all 128 rows, registers over LDS: 64 workgroups 1.28, 256 1.24, 512 0.77; heads of 64 0.87 at 64.
+bool rows_in_lds(int nc, int ec, bool backward, bool tanh, uint32_t rows, uint32_t cap, int64_t lds, int64_t registers) {
+    const bool half = 2 * rows <= cap, wide = ec > 32;
+    if (backward) return lds <= 256 && (tanh ? half && (ec <= 16 || (ec <= 32 && nc == 4)) : !wide);
+    if (lds > 4096) return false;
+    auto rounds = [](int64_t workgroups, int64_t at_once) { return (double)((workgroups + at_once - 1) / at_once); };
+    if (tanh && wide) return lds <= 256 && half;
     if (tanh) {
-        if (!half) return false;
-        if (backward) return workgroups <= 256 && (ec <= 16 || (ec <= 32 && nc == 4));
-        return workgroups <= (ec <= 16 || (ec <= 32 && quarter) ? 512 : 256);
+        if (5 * rows > 4 * cap) return false;
+        const double full = (double)rows / cap, per_cu = rounds(lds, 256), pairs = std::floor(per_cu / 2);
+        const double in_lds = (pairs * (1.2 + 1.1 * full) + (per_cu - 2 * pairs)) * (1 + 1.2 * full * full);
+        return in_lds < (ec <= 16 ? 2.4 : 2.05) * (1 + 0.6 * (rounds(registers, 256) - 1));
     }
-    if (backward) return workgroups <= 256 && ec <= 32;
-    if (ec > 32) return workgroups <= 256;
-    if (nc == 4 && ec == 8 && !quarter) return half && workgroups <= 512;
-    return workgroups <= (quarter ? 512 : half ? 2048 : 4096);
+    // time of a round in LDS over one in registers
+    const double round = wide ? 0.7 : nc == 4 && ec == 8 ? (half ? 0.75 : 1.1) : half ? 0.42 : 0.66;
+    return round * rounds(lds, wide ? 256 : 512) < rounds(registers, 768);
 }
 
 RadixLoads radix_loads(const ncn_shape* sh, const RadixPass& p, bool backward, bool tanh) {
     const uint32_t cap = capacity_rows((int)(sh->E / sh->n_head), backward);
     const int64_t whole = sh->batch * (int64_t)p.loads, per = cap / p.span;
     const int64_t across = (sh->batch * (sh->N / p.span) + per - 1) / per;
-    if (rows_in_lds(sh->n_cache, (int)(sh->E / sh->n_head), backward, tanh, p.rows, cap, whole * sh->n_head))
+    if (rows_in_lds(sh->n_cache, (int)(sh->E / sh->n_head), backward, tanh, p.rows, cap, whole * sh->n_head, std::min(whole, across) * sh->n_head))
         return RadixLoads{p.rows, whole, false, true};
     if (across < whole) return RadixLoads{cap, across, true, false};
     return RadixLoads{p.rows, whole, false, false};

@@ -73,7 +73,7 @@ def test_other_activations(M, n, ec, L, act):
 
 # the same on launches that are large enough for the registers
 @pytest.mark.parametrize("act", [1, 2, 3, -1])
-@pytest.mark.parametrize("n,ec,L,batch,N", [(2, 32, 6, 300, 64), (4, 16, 3, 300, 64), (2, 128, 4, 150, 48), (4, 64, 3, 150, 64), (2, 8, 3, 300, 24)])
+@pytest.mark.parametrize("n,ec,L,batch,N", [(2, 32, 6, 600, 64), (4, 16, 3, 600, 64), (2, 128, 4, 150, 48), (4, 64, 3, 150, 64), (2, 8, 3, 600, 24)])
 def test_other_activations_on_many_workgroups(M, n, ec, L, batch, N, act):
     check(M, batch, N, ec, 2, n, 0, L, act, forward="radix", backward="radix")
 
@@ -84,6 +84,22 @@ def test_other_activations_on_many_workgroups(M, n, ec, L, batch, N, act):
                                                          (4, 16, 2, 192, 3, 1, "fused"), (2, 64, 2, 128, 5, -1, "radix"), (2, 1, 3, 48, 4, 0, "fused")])
 def test_few_workgroups(M, n, ec, batch, N, L, act, backward):
     check(M, batch, N, ec, 16 if ec == 1 else 2, n, 0, L, act, forward="fused", backward=backward)
+
+
+@pytest.mark.parametrize("n,ec,N,L,act,below,above", [
+    (2, 8, 24, 3, 0, 768, 769), (2, 32, 32, 5, 0, 512, 513), (2, 32, 192, 6, 0, 256, 384), (2, 8, 576, 6, 0, 512, 513), (2, 16, 448, 6, 0, None, 1),
+    (2, 32, 256, 7, 0, None, 1), (2, 64, 32, 4, 0, 256, 257), (4, 128, 16, 2, 0, 256, 257), (2, 16, 24, 3, 1, 1024, 1025), (2, 32, 192, 6, 1, 512, 513),
+    (4, 8, 64, 3, 2, 512, 513), (2, 64, 64, 5, -1, 256, 257)])
+def test_which_kernels_take_a_forward_pass(M, n, ec, N, L, act, below, above):
+    """By workgroups (one to a batch entry here): up to as many in LDS, from as many on in registers."""
+    W = torch.randn(L, 2 * ec, device="cuda") / n ** 0.5
+    for batch, kind in ((below, "fused"), (above, "radix")):
+        if batch:
+            x = torch.randn(batch, N, ec, device="cuda")
+            (y, ya), ran = kernels_of(lambda: M.forward_radix(x, x, W, 0.9, act, n, 1, 0, L))
+            assert {k.split("_")[0] for k in ran} == {kind}
+            _, ran = kernels_of(lambda: M.inverse_radix(y, ya, W, 0.9, act, n, 1, 0, L))
+            assert {k.split("_")[0] for k in ran} == {kind}
 
 
 @pytest.mark.parametrize("n,E,L,act", [(2, 32, 8, 0), (4, 64, 4, 0), (2, 8, 9, 2), (4, 16, 3, -1)])
@@ -99,11 +115,11 @@ def test_bfloat16_inputs_and_gradients(M, n, ec, L):
 # windows counted through batch entries: several entries to a workgroup, an entry that begins inside one and ends in the next, a
 # last workgroup that is not full; levels that do not start at the first; more and fewer windows to an entry than to a workgroup
 @pytest.mark.parametrize("batch,N,ec,n,first,L,act,dtype", [
-    (181, 4, 8, 2, 0, 2, 0, torch.float32), (190, 8, 32, 2, 0, 3, 0, torch.float32), (175, 80, 32, 2, 0, 4, 0, torch.float32),
-    (18, 640, 32, 2, 0, 7, 0, torch.float32), (91, 96, 64, 2, 0, 5, 0, torch.float32), (89, 48, 128, 2, 0, 4, 0, torch.float32),
-    (175, 96, 16, 2, 2, 3, 0, torch.float32), (173, 48, 32, 4, 0, 2, 0, torch.float32), (175, 192, 16, 4, 1, 2, 0, torch.bfloat16),
-    (181, 64, 8, 4, 0, 3, 2, torch.float32), (177, 48, 32, 2, 0, 4, -1, torch.bfloat16), (519, 56, 1, 2, 0, 3, 0, torch.float32),
-    (523, 16, 1, 4, 0, 2, 2, torch.float32)])
+    (259, 4, 8, 2, 0, 2, 0, torch.float32), (213, 8, 32, 2, 0, 3, 0, torch.float32), (215, 80, 32, 2, 0, 4, 0, torch.float32),
+    (41, 640, 32, 2, 0, 7, 0, torch.float32), (91, 96, 64, 2, 0, 5, 0, torch.float32), (89, 48, 128, 2, 0, 4, 0, torch.float32),
+    (215, 96, 16, 2, 2, 3, 0, torch.float32), (213, 48, 32, 4, 0, 2, 0, torch.float32), (215, 192, 16, 4, 1, 2, 0, torch.bfloat16),
+    (239, 64, 8, 4, 0, 3, 2, torch.float32), (379, 48, 32, 2, 0, 4, -1, torch.bfloat16), (819, 56, 1, 2, 0, 3, 0, torch.float32),
+    (1123, 16, 1, 4, 0, 2, 2, torch.float32)])
 def test_windows_of_several_batch_entries(M, batch, N, ec, n, first, L, act, dtype):
     # (heads of one feature are laid out as one of 16)
     check(M, batch, N, ec, 16 if ec == 1 else 3, n, first, L, act, dtype, forward="radix", backward="radix")
