@@ -355,6 +355,8 @@ size_t ncn_workspace_bytes_stages(const ncn_shape* shape, int first_stage, int n
  *   [2] kind: 0 one-stage launch, 1 halo window, 2 closed rings
  *   [3] class stride S0 in blocks   [4] window   [5] halo   [6] owned sub-blocks per window
  *   [7] windows per batch entry and ring tile (classes, or groups of classes for closed rings)
+ * The halo is what windows of plain blocks need; the launch loads the rows of the groups that the owned ones depend on,
+ * which are fewer (ncn_fused_kernels.h).  Stacks that are trained (ncn_stack_forward) and ncn_inverse_ws are cut by that smaller need.
  * No reference counterpart. */
 int ncn_plan_passes(const ncn_shape* shape, int first_stage, int n_stages, int activation, int backward, int32_t* out,
                     int max_passes);

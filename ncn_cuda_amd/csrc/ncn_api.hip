@@ -357,10 +357,10 @@ size_t base_workspace_bytes(const ncn_shape* sh) { return partial_buffer_bytes(s
 
 // the multi-stage plan of a stage range, or an empty vector when the one-stage loop should be used
 std::vector<FusedPass> multi_stage_plan(const ncn_shape* sh, int first_stage, int n_stages, int activation, bool backward,
-                                        int path = 2) {
+                                        int path = 2, bool sheared = false) {
     std::vector<FusedPass> none;
     if (n_stages < 2 || path != 2 || kernel_path(sh, activation) != 2 || !fused_supported(sh, activation)) return none;
-    std::vector<FusedPass> passes = plan_fused(sh, first_stage, n_stages, backward);
+    std::vector<FusedPass> passes = plan_fused(sh, first_stage, n_stages, backward, sheared);
     bool any = false;
     for (const FusedPass& p : passes) any = any || !p.single;
     return any ? passes : none;
@@ -699,9 +699,11 @@ static int inverse_impl(const void* y, const void* ya, int in_dtype, void* x, vo
     // several stages: LDS-resident passes, last pass of the range first.  Without scratch to ping-pong with, the
     // first pass to run goes from y, ya to x, xa and the others work in place on x, xa, which a halo pass must not,
     // so the stages of such a pass are undone by one-stage launches (closed passes and one-stage launches may).
+    // Where no pass has to work in place the cut is the one with the most stages to a halo pass.
     std::vector<FusedPass> passes;
+    const bool never_in_place = x != y && xa != ya && workspace && workspace_bytes >= temp_bytes(shape, false);
     if (grouping.permutation() && (out_dtype == NCN_F32 || n_stages == 1))
-        passes = multi_stage_plan(shape, first_stage, n_stages, activation, false, path);
+        passes = multi_stage_plan(shape, first_stage, n_stages, activation, false, path, never_in_place);
     auto run_stage = [&](int k, const void* i0, const void* i1, int i_dtype, void* o0, void* o1, int o_dtype) -> hipError_t {
         StageArgs a{};
         fill_common(a, shape, p, first_stage + k, alpha, m, activation, grouping, k);

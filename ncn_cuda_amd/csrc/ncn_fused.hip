@@ -66,13 +66,19 @@ bool fused_supported(const ncn_shape* sh, int activation) {
 
 namespace {
 
+// What a halo pass is planned with.  kBothSides: (n_cache - 1) sum(strides) groups on either side of the owned ones, what windows
+// of plain sub-blocks would need.  The cuts that ncn_plan_passes reports, and the workspaces that follow from them, are made
+// that way; the launch loads the groups that sheared windows need beside the owned ones, which are never more.
+// kSheared: those alone, so that halo passes hold more stages.
+enum class Halo { kBothSides, kSheared };
+
 // Prices and shapes the passes over stages [a, b) of a range (counted from `first`).  Window capacity in sub-blocks is a
 // power of two.
 class PassPlanner {
   public:
-    PassPlanner(const ncn_shape* sh, int first, int count, bool backward)
+    PassPlanner(const ncn_shape* sh, int first, int count, bool backward, Halo halo)
         : nc_(sh->n_cache), ec_((int)(sh->E / sh->n_head)), groups_((uint32_t)(sh->N / sh->n_cache)), backward_(backward),
-          s_(count) {
+          halo_(halo), s_(count) {
         const size_t state = nc_ == 2 ? pair_state_bytes(backward) : fused_state_bytes(backward);
         cap_rows_ = (uint32_t)(state / ((backward ? 4 : 2) * ec_ * sizeof(float)));
         cap_ = floor_pow2(cap_rows_ / nc_);
@@ -132,17 +138,42 @@ class PassPlanner {
             p.own = p.window;
             p.tiles_per_ring = 1;
             p.class_groups = s0 / rings;
-            return priced(writes_state, 1.0, b - a, true);
+            return priced(writes_state, 1.0, 1.0, b - a, true);
         }
         p.closed = 0;
-        p.window = cap_;
-        p.halo = (uint32_t)(nc_ - 1) * sum;
-        if (2 * p.halo >= cap_) return -1.0;
-        p.own = cap_ - 2 * p.halo;
-        if (p.own * 4 < cap_ * 3) return -1.0;  // more than a third of the window would be redundant work
-        p.tiles_per_ring = (p.ring + p.own - 1) / p.own;
         p.class_groups = s0;
-        return priced(writes_state, (double)cap_ / p.own, b - a, false);
+        // Stage k + 1 of the pass needs slot o of the groups o * step further on than stage k left them (steps around the
+        // ring the shorter way): what the window holds beside the owned groups in the stage that runs first, and what all
+        // stages do in beside them (`extra`, summed over the stages).
+        const uint32_t reach = (uint32_t)nc_ - 1;
+        uint64_t extra = 0;
+        p.before = p.after = 0;
+        p.shear[0] = 0;
+        for (int k = 1; k < b - a; ++k) {
+            const uint32_t up = (p.sub_stride[k] + p.ring - p.sub_stride[k - 1] % p.ring) % p.ring, down = p.ring - up;
+            const bool forth = up <= down;
+            p.shear[k] = p.shear[k - 1] + (forth ? (int32_t)up : -(int32_t)down);
+            (forth ? p.after : p.before) += reach * (forth ? up : down);
+            extra += (uint64_t)reach * (forth ? up : down) * k;   // the k stages before the step
+            if (p.before + p.after >= cap_) return -1.0;
+        }
+        if (halo_ == Halo::kBothSides) {
+            p.window = cap_;
+            p.halo = reach * sum;
+            if (2 * p.halo >= cap_) return -1.0;
+            p.own = cap_ - 2 * p.halo;
+            if (p.own * 4 < cap_ * 3) return -1.0;  // more than a third of the window would be redundant work
+            p.tiles_per_ring = (p.ring + p.own - 1) / p.own;
+            const double redundancy = (double)cap_ / p.own;
+            return priced(writes_state, redundancy, redundancy, b - a, false);
+        }
+        p.halo = p.before + p.after;
+        p.tiles_per_ring = (p.ring + cap_ - p.halo - 1) / (cap_ - p.halo);
+        p.own = (p.ring + p.tiles_per_ring - 1) / p.tiles_per_ring;   // windows of one size
+        p.window = p.own + p.halo;
+        if (p.own * 3 < p.window) return -1.0;
+        const double per_ring = (double)p.tiles_per_ring / p.ring;
+        return priced(writes_state, 1.0 + per_ring * p.halo, 1.0 + per_ring * (double)extra / (b - a), b - a, false);
     }
 
   private:
@@ -155,17 +186,19 @@ class PassPlanner {
     // the four-row kernels in proportion to their instruction counts).  The two overlap, better the more they differ:
     // the cube root of the sum of cubes follows the measured pass times to 5 % (a closed backward pass, whose windows
     // are the most scattered in memory, takes 1.1 times that).
-    double priced(bool writes_state, double redundancy, int stages, bool closed) const {
+    // loaded, computed: windows' share of the groups loaded, and done in a stage on average, over the owned ones
+    double priced(bool writes_state, double loaded, double computed, int stages, bool closed) const {
         const double arrays_in = backward_ ? 4.0 : 2.0, arrays_out = backward_ && writes_state ? 4.0 : 2.0;
         const double per_stage = nc_ == 2 ? (backward_ ? 1.4 : 0.76) : (backward_ ? 3.6 : 2.0);
-        const double traffic = arrays_in * redundancy + arrays_out;
-        const double issue = per_stage * stages * redundancy;
+        const double traffic = arrays_in * loaded + arrays_out;
+        const double issue = per_stage * stages * computed;
         return std::cbrt(traffic * traffic * traffic + issue * issue * issue) * (closed && backward_ ? 1.1 : 1.0);
     }
 
     int nc_, ec_;
     uint32_t groups_, cap_rows_, cap_, groups_pow2_;
     bool backward_;
+    Halo halo_;
     int max_stages_;
     std::vector<uint32_t> s_;
 };
@@ -213,8 +246,8 @@ std::vector<FusedPass> passes_of(const PassPlanner& planner, const CheapestCut& 
 }  // namespace
 
 // Cuts stages [first, first + count) into passes, ascending.
-std::vector<FusedPass> plan_fused(const ncn_shape* sh, int first, int count, bool backward) {
-    const PassPlanner planner(sh, first, count, backward);
+std::vector<FusedPass> plan_fused(const ncn_shape* sh, int first, int count, bool backward, bool sheared) {
+    const PassPlanner planner(sh, first, count, backward, sheared ? Halo::kSheared : Halo::kBothSides);
     FusedPass p{};
     const CheapestCut cut(0, count, planner.max_stages(), [&](int a, int b, bool writes_state) {
         return b - a == 1 ? planner.single(writes_state) : planner.make(a, b, writes_state, p);
@@ -225,12 +258,14 @@ std::vector<FusedPass> plan_fused(const ncn_shape* sh, int first, int count, boo
 // Where a stack that is trained keeps its activations.  The forward hands the values between two passes through memory
 // anyway: kept, they spare the backward the two arrays that a pass which starts there would otherwise write (and
 // the next one read back all the same).  Where both directions' passes begin and end is chosen together, by the prices
-// above: of x[64, 2048, 128], groups of 4, 6 stages, the forward runs {0,1} {2} {3} {4,5} either way, and the backward's
-// one-stage launches write 2 instead of 4 arrays: a training step of it in bfloat16 870 -> 772 us, with the conversions of
-// the results and weights that the passes now do themselves; x[32, 1024, 128] float32, 5 stages, 253 -> 227.  kKeep is what a kept range must gain to be worth its memory.
+// above.  kKeep is what a kept range must gain to be worth its memory.
+// With sheared windows, a training step against the cuts of two-sided halos: x[128, 8192, 128] float32, groups of 2, 13 stages, two
+// passes in either direction, {0-5} {6-12}, where the forward ran {0-4} {5-12} and the backward {0-2} {3-5} {6-12}: 4255 -> 3672 us;
+// x[64, 2048, 128] bfloat16, groups of 4, 6 stages, {0-2} {3-5} in place of {0,1} {2} {3} {4,5} and {0,1} {2} {3} {4} {5}:
+// 769 -> 634; x[32, 1024, 128] float32, groups of 4, 5 stages, {0-2} {3,4}: 179 to 189 -> 167.
 std::vector<StackRange> plan_stack(const ncn_shape* sh, int first, int count, bool multi_stage, int max_range, int max_saves) {
     constexpr double kKeep = 0.25;
-    const PassPlanner fwd(sh, first, count, false), bwd(sh, first, count, true);
+    const PassPlanner fwd(sh, first, count, false, Halo::kSheared), bwd(sh, first, count, true, Halo::kSheared);
     const int F = multi_stage ? fwd.max_stages() : 1, B = multi_stage ? bwd.max_stages() : 1;
     // prices of every pass, made once: [a][length], backward with and without handing the state on
     std::vector<double> fc((size_t)count * (kFusedMaxStages + 1), -1.0), bc(2 * fc.size(), -1.0);
@@ -304,18 +339,26 @@ hipError_t launch_fused(Pass pass, FusedArgs& a, const ncn_shape* sh, const Fuse
     a.class_stride = p.class_stride;
     a.ring = p.ring;
     a.ring_magic = (p.ring & (p.ring - 1)) == 0 ? 0u : (uint32_t)(((1ull << 32) + p.ring - 1) / p.ring);
-    a.window = p.window;
-    a.halo = p.halo;
     a.own = p.own;
     a.tiles_per_ring = p.tiles_per_ring;
     a.closed = p.closed;
     a.class_groups = p.class_groups;
     a.total_items = (uint32_t)fused_items(sh, p);
-    for (int k = 0; k < kFusedMaxStages; ++k) a.sub_stride[k] = k < p.count ? p.sub_stride[k] : 0;
+    if (p.closed) {
+        a.window = p.window;
+        for (int k = 0; k < p.count; ++k) a.sub_stride[k] = (int32_t)p.sub_stride[k];
+    } else {   // the window as the stage that runs first needs it
+        const int first = pass == kForward ? 0 : p.count - 1, last = p.count - 1 - first;
+        a.window = p.before + p.own + p.after;
+        a.halo = pass == kForward ? p.before : p.after;
+        a.shift = p.sub_stride[first] % p.ring;
+        for (int k = 0; k < p.count; ++k) a.sub_stride[k] = p.shear[k] - p.shear[first];
+        a.end_shear = a.sub_stride[last];
+    }
     a.scale_dn = (float)std::pow((double)a.tab.m, (double)(nc * p.count));
     a.scale_up = (float)std::pow((double)a.tab.m, -(double)(nc * p.count));
     const int grid = fused_grid(sh, p, backward, row_cap);
-    const size_t lds = fused_lds_bytes(nc, ec, backward, p.window, p.count);
+    const size_t lds = fused_lds_bytes(nc, ec, backward, a.window, p.count);
     if (headwise) return launch_fused_headwise(pass, a, nc, ec, grid, lds, s);
     if (a.ctx_len) return launch_fused_lengths(pass, a, nc, ec, grid, lds, s);
     return launch_fused_shape<false, false, false>(pass, a, nc, ec, grid, lds, s);

@@ -11,10 +11,15 @@
 // of consecutive sub-blocks of one (batch, head, class):
 //   * closed pass: the window is one whole ring, or several whole rings of adjacent classes when a ring is
 //     smaller than the window (indices wrap inside each ring): nothing outside is ever needed;
-//   * halo pass:   the window is `own` sub-blocks plus `halo` = (n_cache-1) * sum(s_l/S0) on each side.  Every
-//     stage updates the groups that lie completely inside the window; rows near the window edge go stale, but
-//     by construction never reach an owned row.  Only owned rows are written back and only groups whose slot-0
-//     sub-block is owned count towards dW, so the redundant halo work is invisible outside.
+//   * halo pass:   the window is a stretch of groups, sheared: slot o of it is not the sub-blocks of slot 0 but those
+//     that the groups read in the first stage to run (position q of slot o is sub-block sub0 + q + o*shift), which are
+//     loaded straight from where they are.  From one stage to the next a group's slot o moves by o times the difference of
+//     the two strides, so a stage needs (n_cache-1) * |difference| groups more than the one that follows it, on one
+//     side: a window of `own` groups carries (n_cache-1) * (largest - smallest stride) beside them (a window of plain
+//     sub-blocks loses (n_cache-1) * s_l/S0 on both sides at every stage: 90 groups on a side instead of 24 for strides 0, 1, 2, 4, 8
+//     and groups of four).  Groups that do not lie completely inside the window sit a stage out; their rows go stale,
+//     but never reach an owned group.  Only the rows of groups owned in the last stage to run are written back and only
+//     owned groups count towards dW, so the redundant halo work is invisible outside.
 // A halo pass must not run in place (another workgroup still needs the old value of an owned row as its halo),
 // a closed pass may.  The host (ncn_fused.hip) cuts a stage range into passes and ping-pongs buffers.
 //
@@ -85,13 +90,16 @@ struct FusedArgs {
     uint32_t class_stride;    // S0, in blocks
     uint32_t ring;            // sub-blocks per class = groups / S0 (a power of two, or an odd number times one)
     uint32_t window;          // sub-blocks held in LDS
-    uint32_t halo;            // sub-blocks of halo on each side (0 for a closed pass)
-    uint32_t own;             // owned sub-blocks per window (= ring for a closed pass)
+    uint32_t halo;            // groups of halo in front of the owned ones (0 for a closed pass)
+    uint32_t own;             // owned groups per window (= window for a closed pass)
+    uint32_t shift;           // halo pass: stride of the first stage to run, mod ring (0 for a closed pass)
+    int32_t end_shear;        // halo pass: sub_stride of the last stage to run (0 for a closed pass)
     uint32_t tiles_per_ring;  // ceil(ring / own)
     uint32_t closed;          // 1: the window holds window/ring whole rings (adjacent classes) and indices wrap
     uint32_t class_groups;    // closed: S0 / (window / ring) windows per batch entry; halo: S0
     uint32_t total_items;     // batch * class_groups * tiles_per_ring * n_head
-    uint32_t sub_stride[kFusedMaxStages];  // s_l / S0 per stage of the pass
+    // s_l / S0 per stage of the pass; halo pass: less that of the first stage to run
+    int32_t sub_stride[kFusedMaxStages];
     float scale_dn, scale_up;              // m^(n_cache * n_stages) and its reciprocal (backward: gradients leave as G m^T)
     // radix kernels whose workgroups hold windows of several batch entries: windows of an entry, 0 or ceil(2^31 / entry_windows),
     // and windows of all entries
@@ -189,7 +197,18 @@ __device__ __forceinline__ uint32_t fused_deal(const FusedArgs& A, uint32_t blk)
     return (first + r - head * n) * heads + head;
 }
 
-// element offset (without the feature) of local row `lr` = (window sub-block qi) * NC + slot
+// The groups that lie completely inside the window in a stage: `first` and up, `count` of them.
+struct StageGroups {
+    uint32_t first, count;
+};
+template <int NC>
+__device__ __forceinline__ StageGroups stage_groups(const FusedArgs& A, int ss) {
+    if (A.closed) return {0u, A.window};
+    const uint32_t out = (NC - 1) * (uint32_t)(ss < 0 ? -ss : ss);   // less than the window: it holds the owned groups too
+    return {ss < 0 ? out : 0u, A.window - out};
+}
+
+// element offset (without the feature) of local row `lr` = (window position qi) * NC + slot
 template <int NC, bool RADIX>
 __device__ __forceinline__ int64_t fused_row_offset(const FusedArgs& A, const FusedItem& it, uint32_t lr) {
     if (RADIX) {
@@ -200,8 +219,12 @@ __device__ __forceinline__ int64_t fused_row_offset(const FusedArgs& A, const Fu
         return it.base + pos * A.E;
     }
     const uint32_t qi = lr / NC, o = lr - qi * NC;
+    uint32_t sub0 = it.sub0 + o * A.shift;   // < NC * ring
+    if (NC > 2 && sub0 >= 2u * A.ring) sub0 -= 2u * A.ring;
+    if (sub0 >= A.ring) sub0 -= A.ring;
+    static_assert(RADIX || NC <= 4, "the wrap above");
     uint32_t sub, cls;
-    ring_place(A, it.sub0, it.cls, qi, sub, cls);
+    ring_place(A, sub0, it.cls, qi, sub, cls);
     const uint32_t blk = sub * A.class_stride + cls;
     return it.base + ((int64_t)blk * NC + o) * A.E;
 }
@@ -218,7 +241,8 @@ __device__ __forceinline__ uint32_t fused_lds_place(uint32_t lr) {
 // LDS row of slot i of the group whose slot-0 sub-block is window position qg
 // (RADIX: row of digit i at level log_n(sstride) of group qg; groups are numbered window by window)
 template <int NC, bool RADIX>
-__device__ __forceinline__ uint32_t fused_lds_row(const FusedArgs& A, uint32_t qg, uint32_t i, uint32_t sstride) {
+__device__ __forceinline__ uint32_t fused_lds_row(const FusedArgs& A, uint32_t qg, uint32_t i, int ss) {
+    const uint32_t sstride = (uint32_t)ss;   // (negative ones wrap back)
     if (RADIX) {
         constexpr uint32_t lg_nc = NC == 2 ? 1u : 2u;
         static_assert(NC == 2 || NC == 4, "digit arithmetic by shifts");
@@ -316,14 +340,20 @@ __device__ __forceinline__ void fused_commit_rows(const uint4 (&raw)[K], int dty
     }
 }
 
+// local row of the k-th row of the owned groups, as the last stage to run left it
+template <int NC>
+__device__ __forceinline__ uint32_t fused_owned_row(const FusedArgs& A, const FusedItem& it, uint32_t k) {
+    return (it.own_lo * NC + k) + (k % NC) * NC * (uint32_t)A.end_shear;
+}
+
 // LDS -> global for the owned rows, each value times `scale`
 template <int NC, int EC, int NW, bool RADIX>
 __device__ __forceinline__ void fused_store_rows_scaled(const FusedArgs& A, const FusedItem& it, const float* src,
                                                         float scale, void* dst, int dtype, float* copy32) {
     constexpr uint32_t CPR = EC / 4;
-    const uint32_t r0 = it.own_lo * NC, rows = it.own_cnt * NC;
+    const uint32_t rows = it.own_cnt * NC;
     for (uint32_t c = threadIdx.x; c < rows * CPR; c += 64 * NW) {
-        const uint32_t lr = r0 + c / CPR, c4 = c % CPR;
+        const uint32_t lr = fused_owned_row<NC>(A, it, c / CPR), c4 = c % CPR;
         float v[4];
         lds_load_frag<4>(src + fused_lds_place<NC>(lr) * EC + c4 * 4, v);
 #pragma unroll
@@ -395,19 +425,19 @@ __global__ void __launch_bounds__(64 * kFusedWavesFwd) fused_forward_kernel(cons
         }
         for (int sq = 0; sq < A.n_stages; ++sq) {
             const int st = INVERSE ? A.n_stages - 1 - sq : sq;
-            const uint32_t ss = A.sub_stride[st];
-            const uint32_t ngroups = A.closed ? A.window : A.window - (NC - 1) * ss;
+            const int ss = A.sub_stride[st];
+            const StageGroups here = stage_groups<NC>(A, ss);
             float wi[F], wj[F];
             lds_load_frag<F>(w_lds + st * 2 * EC + fl * F, wi);
             lds_load_frag<F>(w_lds + st * 2 * EC + EC + fl * F, wj);
-            for (uint32_t wt = wave; wt * T::GPW < ngroups; wt += NW) {
-                const uint32_t qg = wt * T::GPW + gw;
-                const bool valid = qg < ngroups;
+            for (uint32_t wt = wave; wt * T::GPW < here.count; wt += NW) {
+                const uint32_t qg = here.first + wt * T::GPW + gw;
+                const bool valid = qg - here.first < here.count;
                 float x[R][F], a[R][F];
                 uint32_t row[R];
 #pragma unroll
                 for (int rr = 0; rr < R; ++rr) {
-                    row[rr] = fused_lds_row<NC, RADIX>(A, valid ? qg : 0u, rl * R + rr, ss) * EC + fl * F;
+                    row[rr] = fused_lds_row<NC, RADIX>(A, valid ? qg : here.first, rl * R + rr, ss) * EC + fl * F;
                     lds_load_frag<F>(xs + row[rr], x[rr]);
                     lds_load_frag<F>(as + row[rr], a[rr]);
                 }
@@ -507,22 +537,22 @@ __global__ void __launch_bounds__(64 * kFusedWavesBwd, TANH_ONLY ? (R * F <= 8 ?
         const FusedItem it = fused_item<NC, EC, RADIX>(A, item);
         const int32_t len = LENGTHS ? max(0, min(A.ctx_len[it.batch], (int32_t)A.N)) : 0;
         for (int st = A.n_stages - 1; st >= 0; --st) {
-            const uint32_t ss = A.sub_stride[st];
-            const uint32_t ngroups = A.closed ? A.window : A.window - (NC - 1) * ss;
+            const int ss = A.sub_stride[st];
+            const StageGroups here = stage_groups<NC>(A, ss);
             float wi[F], wj[F], dwi[F], dwj[F];
             lds_load_frag<F>(w_lds + st * 2 * EC + fl * F, wi);
             lds_load_frag<F>(w_lds + st * 2 * EC + EC + fl * F, wj);
 #pragma unroll
             for (int f = 0; f < F; ++f) dwi[f] = dwj[f] = 0.f;
-            for (uint32_t wt = wave; wt * T::GPW < ngroups; wt += NW) {
-                const uint32_t qg = wt * T::GPW + gw;
-                const bool valid = qg < ngroups;
+            for (uint32_t wt = wave; wt * T::GPW < here.count; wt += NW) {
+                const uint32_t qg = here.first + wt * T::GPW + gw;
+                const bool valid = qg - here.first < here.count;
                 const float own = (valid && qg - it.own_lo < it.own_cnt) ? 1.0f : 0.0f;  // unsigned: lo <= qg < lo+cnt
                 float Y[R][F], B[R][F], G[R][F], P[R][F];
                 uint32_t row[R];
 #pragma unroll
                 for (int rr = 0; rr < R; ++rr) {
-                    row[rr] = fused_lds_row<NC, RADIX>(A, valid ? qg : 0u, rl * R + rr, ss) * EC + fl * F;
+                    row[rr] = fused_lds_row<NC, RADIX>(A, valid ? qg : here.first, rl * R + rr, ss) * EC + fl * F;
                     lds_load_frag<F>(ys + row[rr], Y[rr]);
                     lds_load_frag<F>(bs + row[rr], B[rr]);
                     lds_load_frag<F>(gs + row[rr], G[rr]);
@@ -593,9 +623,9 @@ __global__ void __launch_bounds__(64 * kFusedWavesBwd, TANH_ONLY ? (R * F <= 8 ?
         }
         auto write_out = [&]() {   // owned rows back to true values: g = G m^T, h = P m^T - (1-m) g, x = xs / kappa, xa = bh / b_scale
             constexpr uint32_t CPR = EC / 4;
-            const uint32_t r0 = it.own_lo * NC, nrows = it.own_cnt * NC;
+            const uint32_t nrows = it.own_cnt * NC;
             for (uint32_t c = threadIdx.x; c < nrows * CPR; c += 64 * NW) {
-                const uint32_t lr = r0 + c / CPR, c4 = c % CPR;
+                const uint32_t lr = fused_owned_row<NC>(A, it, c / CPR), c4 = c % CPR;
                 const int64_t off = fused_row_offset<NC, RADIX>(A, it, lr) + c4 * 4;
                 float g[4], h[4];
                 lds_load_frag<4>(gs + fused_lds_place<NC>(lr) * EC + c4 * 4, g);

@@ -100,8 +100,8 @@ __device__ __forceinline__ void pair_commit_slot1(const uint4 (&raw)[K], int dty
 }
 
 // window position of the sub-block that holds slot 1 of the group whose slot 0 is sub-block q
-__device__ __forceinline__ uint32_t pair_partner(const FusedArgs& A, uint32_t q, uint32_t ss) {
-    return A.closed ? ring_wrap(A, q, ss) : q + ss;   // closed: inside the group's own ring
+__device__ __forceinline__ uint32_t pair_partner(const FusedArgs& A, uint32_t q, int ss) {
+    return A.closed ? ring_wrap(A, q, (uint32_t)ss) : q + ss;   // closed: inside the group's own ring
 }
 
 // a lane's F features of an LDS row (or of a weight vector): its H chunks of 4
@@ -179,18 +179,18 @@ __global__ void __launch_bounds__(64 * kFusedWavesFwd, NCN_PAIR_FWD_WAVES) pair_
         __syncthreads();
         for (int sq = 0; sq < A.n_stages; ++sq) {
             const int st = INVERSE ? A.n_stages - 1 - sq : sq;
-            const uint32_t ss = A.sub_stride[st];
-            const uint32_t ngroups = A.closed ? window : window - ss;
+            const int ss = A.sub_stride[st];
+            const StageGroups here = stage_groups<NC>(A, ss);
             float wi[F], wj[F];
             pair_lds_load<EC>(w_lds + st * 2 * EC, fl, wi);
             pair_lds_load<EC>(w_lds + st * 2 * EC + EC, fl, wj);
 #pragma unroll
             for (int k = 0; k < KT; ++k) {
                 const uint32_t q = (uint32_t)(wave + k * NW) * T::GPW + gw;
-                // Lanes whose group does not exist in this stage (past the last group that lies inside the window)
+                // Lanes whose group does not exist in this stage (not completely inside the window)
                 // sit the tile out: every cross-lane sum of a step stays inside one group, so no lane a live group
                 // needs is off, and the rows of the lanes that are off keep their values.
-                if (q < ngroups) {
+                if (q - here.first < here.count) {   // unsigned: first <= q < first + count
                     const uint32_t row1 = pair_partner(A, q, ss) * EC;
                     pair_lds_load<EC>(xs1 + row1, fl, x[k][1]);
                     pair_lds_load<EC>(as1 + row1, fl, a[k][1]);
@@ -212,7 +212,7 @@ __global__ void __launch_bounds__(64 * kFusedWavesFwd, NCN_PAIR_FWD_WAVES) pair_
         }
         // owned rows out of the scaled form: slot 1 from LDS, slot 0 from the registers
         for (uint32_t c = threadIdx.x; c < it.own_cnt * CPR; c += 64 * NW) {
-            const uint32_t qi = it.own_lo + c / CPR, c4 = c % CPR;
+            const uint32_t qi = it.own_lo + c / CPR + A.end_shear, c4 = c % CPR;
             const int64_t off = fused_row_offset<NC, false>(A, it, 2u * qi + 1u) + c4 * 4;
             float v[4], u[4];
             lds_load_frag<4>(xs1 + qi * EC + c4 * 4, v);
@@ -414,8 +414,8 @@ __global__ void __launch_bounds__(64 * kPairWavesBwd, TANH_ONLY ? NCN_PAIR_BWD_W
         const FusedItem it = fused_item<NC, EC, false>(A, item);
         const int32_t len = LENGTHS ? max(0, min(A.ctx_len[it.batch], (int32_t)A.N)) : 0;
         for (int st = A.n_stages - 1; st >= 0; --st) {
-            const uint32_t ss = A.sub_stride[st];
-            const uint32_t ngroups = A.closed ? window : window - ss;
+            const int ss = A.sub_stride[st];
+            const StageGroups here = stage_groups<NC>(A, ss);
             float wi[F], wj[F], dw[2 * F];   // dw: this lane's share of dWi (first F) and dWj of the stage
             pair_lds_load<EC>(w_lds + st * 2 * EC, fl, wi);
             pair_lds_load<EC>(w_lds + st * 2 * EC + EC, fl, wj);
@@ -428,7 +428,7 @@ __global__ void __launch_bounds__(64 * kPairWavesBwd, TANH_ONLY ? NCN_PAIR_BWD_W
                 const uint32_t q = (uint32_t)(wave + k * NW) * T::GPW + gw;
                 // Lanes whose group does not exist in this stage sit the tile out (every cross-lane sum of a step
                 // stays inside one group); their rows keep their values.
-                if (q < ngroups) {
+                if (q - here.first < here.count) {   // unsigned: first <= q < first + count
                     const float own = (q - it.own_lo < it.own_cnt) ? 1.0f : 0.0f;  // unsigned: lo <= q < lo + cnt
                     const uint32_t row1 = pair_partner(A, q, ss) * EC;
                     pair_lds_load<EC>(ys1 + row1, fl, Y[k][1]);
@@ -484,7 +484,7 @@ __global__ void __launch_bounds__(64 * kPairWavesBwd, TANH_ONLY ? NCN_PAIR_BWD_W
         }
         auto write_out = [&]() {   // owned rows back to true values: g = G m^T, h = P m^T - (1-m) g, x = xs / kappa, xa = bh / b_scale
             for (uint32_t c = threadIdx.x; c < it.own_cnt * CPR; c += 64 * NW) {
-                const uint32_t qi = it.own_lo + c / CPR, c4 = c % CPR;
+                const uint32_t qi = it.own_lo + c / CPR + A.end_shear, c4 = c % CPR;
                 const int64_t off = fused_row_offset<NC, false>(A, it, 2u * qi + 1u) + c4 * 4;
                 float g[4], h[4];
                 lds_load_frag<4>(gs1 + qi * EC + c4 * 4, g);

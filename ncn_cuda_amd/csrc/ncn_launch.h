@@ -186,9 +186,14 @@ struct FusedPass {
     int single;        // 1: not worth fusing, run `first` with the one-stage kernel
     uint32_t class_stride, ring, window, halo, own, tiles_per_ring, closed, class_groups;
     uint32_t sub_stride[8];
+    // halo pass: what slot 1 has moved against its place at the pass's first stage, and the groups that the windows need in front
+    // of and behind the owned ones when the stages run in ascending order (the other way round in descending order)
+    int32_t shear[8];
+    uint32_t before, after;
 };
 bool fused_supported(const ncn_shape* sh, int activation);
-std::vector<FusedPass> plan_fused(const ncn_shape* sh, int first, int count, bool backward);
+// sheared = false: the cuts that ncn_plan_passes reports
+std::vector<FusedPass> plan_fused(const ncn_shape* sh, int first, int count, bool backward, bool sheared = false);
 // Consecutive stages of a trained stack whose last outputs are kept for the backward: the passes of both directions, in
 // ascending order, numbered relative to the planned stages.
 struct StackRange {

@@ -168,7 +168,7 @@ hipError_t launch_fused_radix(Pass pass, FusedArgs& a, const ncn_shape* sh, cons
         a.own = a.window;
         a.tiles_per_ring = 1;
         a.closed = 1;
-        for (int k = 0; k < p.count; ++k) a.sub_stride[k] = (uint32_t)ipow(nc, k);
+        for (int k = 0; k < p.count; ++k) a.sub_stride[k] = (int32_t)ipow(nc, k);
         a.scale_up = (float)std::pow((double)a.tab.m, -(double)(nc * p.count));
         return headwise ? launch_radix_lds<true>(pass, a, nc, ec, grid, s) : launch_radix_lds<false>(pass, a, nc, ec, grid, s);
     }
