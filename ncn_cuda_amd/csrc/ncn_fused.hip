@@ -17,7 +17,6 @@ namespace {
 // that loops over several windows keeps the phase it started in (measured on the 13-stage configuration: grids of
 // 4096 workgroups, 4.5 windows each, 5.35 ms per step; one window each 4.94).  The backward is further bounded by its
 // dW partial rows (one per n_head workgroups and stage), see fused_grid.
-constexpr int kFusedMaxGridFwd = 1 << 16;
 constexpr int kFusedMaxGridBwd = 1 << 16;
 
 size_t fused_lds_bytes(int nc, int ec, bool backward, uint32_t window, int n_stages) {
@@ -315,10 +314,10 @@ int64_t fused_items(const ncn_shape* sh, const FusedPass& p) {
 
 int fused_grid(const ncn_shape* sh, const FusedPass& p, bool backward, int row_cap) {
     const int64_t items = fused_items(sh, p);
-    // the forward kernels for groups of two rows take one window per workgroup and nothing else
-    if (!backward && sh->n_cache == 2) return items <= INT_MAX ? (int)items : 0;
-    int64_t cap = backward ? kFusedMaxGridBwd : kFusedMaxGridFwd;
-    if (backward) {  // partial rows (grid / n_head) * stages must fit the row_cap rows of the dW scratch
+    // the forward kernels take one window per workgroup and nothing else (the one for groups of four with lengths could loop)
+    if (!backward) return items <= INT_MAX ? (int)items : 0;
+    int64_t cap = kFusedMaxGridBwd;
+    {  // partial rows (grid / n_head) * stages must fit the row_cap rows of the dW scratch
         const int64_t by_rows = (int64_t)row_cap / p.count * sh->n_head;
         if (by_rows < cap) cap = by_rows;
     }

@@ -4,6 +4,7 @@
 #pragma once
 #include "ncn_fused_kernels.h"
 #include "ncn_fused_pair_kernels.h"
+#include "ncn_fused_quad_kernels.h"
 #include "ncn_launch.h"
 
 namespace ncn {
@@ -43,6 +44,27 @@ hipError_t launch_fused_build(Pass pass, const FusedArgs& a, int grid, size_t ld
             hipLaunchKernelGGL(k, dim3(grid), dim3(64 * kFusedWavesFwd), lds, s, a);
         }
         return hipGetLastError();
+    } else if constexpr (NC == 4 && !RADIX && !LENGTHS) {
+        auto launch = [&](auto k, int waves) {
+            if (a.window > (uint32_t)quad_groups(EC, waves)) return hipErrorInvalidConfiguration;
+            const size_t bytes = quad_lds_bytes(EC, waves, backward);
+            const hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(k), bytes);
+            if (e != hipSuccess) return e;
+            hipLaunchKernelGGL(k, dim3(grid), dim3(64 * waves), bytes, s, a);
+            return hipGetLastError();
+        };
+        const bool loop = (uint32_t)grid < a.total_items;
+        if (backward)
+            return tanh_only ? (loop ? launch(quad_backward_kernel<EC, true, true, HEADWISE>, kQuadWavesBwd)
+                                     : launch(quad_backward_kernel<EC, true, false, HEADWISE>, kQuadWavesBwd))
+                             : (loop ? launch(quad_backward_kernel<EC, false, true, HEADWISE>, kQuadWavesBwd)
+                                     : launch(quad_backward_kernel<EC, false, false, HEADWISE>, kQuadWavesBwd));
+        if (loop) return hipErrorInvalidConfiguration;   // one window each
+        if (pass == kInverse)
+            return tanh_only ? launch(quad_forward_kernel<EC, true, true, HEADWISE>, kQuadWavesFwd)
+                             : launch(quad_forward_kernel<EC, false, true, HEADWISE>, kQuadWavesFwd);
+        return tanh_only ? launch(quad_forward_kernel<EC, true, false, HEADWISE>, kQuadWavesFwd)
+                         : launch(quad_forward_kernel<EC, false, false, HEADWISE>, kQuadWavesFwd);
     } else {
         if (backward) {
             auto k = tanh_only ? fused_backward_kernel<NC, EC, t.r, t.f, true, RADIX, LENGTHS, HEADWISE>

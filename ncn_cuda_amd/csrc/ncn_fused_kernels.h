@@ -16,8 +16,8 @@
 //     loaded straight from where they are.  From one stage to the next a group's slot o moves by o times the difference of
 //     the two strides, so a stage needs (n_cache-1) * |difference| groups more than the one that follows it, on one
 //     side: a window of `own` groups carries (n_cache-1) * (largest - smallest stride) beside them (a window of plain
-//     sub-blocks loses (n_cache-1) * s_l/S0 on both sides at every stage: 90 groups on a side instead of 24 for strides 0, 1, 2, 4, 8
-//     and groups of four).  Groups that do not lie completely inside the window sit a stage out; their rows go stale,
+//     sub-blocks loses (n_cache-1) * s_l/S0 on both sides at every stage: 45 groups on either side instead of 24 on one for strides
+//     0, 1, 2, 4, 8 and groups of four).  Groups that do not lie completely inside the window sit a stage out; their rows go stale,
 //     but never reach an owned group.  Only the rows of groups owned in the last stage to run are written back and only
 //     owned groups count towards dW, so the redundant halo work is invisible outside.
 // A halo pass must not run in place (another workgroup still needs the old value of an owned row as its halo),
