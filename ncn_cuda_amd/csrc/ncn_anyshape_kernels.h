@@ -283,6 +283,7 @@ __device__ __forceinline__ void any_row_sums(const float (&x)[R][F], const float
 #pragma unroll
         for (int f = 0; f < F; ++f) c[rr] = fmaf(x[rr][f], wi[f], c[rr]);
     }
+    issue_first();   // (the wave stays at high priority)
     any_sum_rows<R>(c, lfl);
 }
 
@@ -334,6 +335,7 @@ __global__ void __launch_bounds__(kBlockThreads, R * F <= 16 ? 4 : R * F <= 20 ?
         any_fill_padding(L, x, INVERSE ? any_missing_undone(S) : 1.f);
         any_fill_padding(L, a);
         scale_tile<R, F>(x, a, S.kappa, INVERSE ? S.b_scale : S.a_scale);
+        const float keep = in_vector_register(INVERSE ? S.im : S.m);   // read twice per element and step
 #pragma unroll 1
         for (int k = 0; k < lr; ++k) {
             const int jo = INVERSE ? lr - 1 - k : k;
@@ -345,27 +347,34 @@ __global__ void __launch_bounds__(kBlockThreads, R * F <= 16 ? 4 : R * F <= 20 ?
 #pragma unroll
                     for (int rr = 0; rr < R; ++rr)
 #pragma unroll
-                        for (int f = 0; f < F; ++f) x[rr][f] = fmaf(S.im, x[rr][f], -a[rr][f]);
+                        for (int f = 0; f < F; ++f) x[rr][f] = fmaf(keep, x[rr][f], -a[rr][f]);
                 }
                 float xj[F], c[R];
                 any_broadcast<F>(x[jr], xj, lr > 1, src, lane, slots);
                 any_row_sums<R, F>(x, wi, dot_chain<F>(xj, wj), L.lfl, c);
+                if constexpr (TANH_ONLY) {
+                    float r[R][F];
+                    sigmoids(0, x, c, xj, r);
+                    issue_with_others();
 #pragma unroll
-                for (int rr = 0; rr < R; ++rr)
+                    for (int rr = 0; rr < R; ++rr)
 #pragma unroll
-                    for (int f = 0; f < F; ++f) {
-                        const float z = fmaf(c[rr], xj[f], x[rr][f]);
-                        const float keep = INVERSE ? S.im : S.m;
-                        if constexpr (TANH_ONLY) {
-                            const float r = __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(z) + 1.0f);
-                            a[rr][f] = fmaf(INVERSE ? S.bk1 : S.m2k2, r, fmaf(keep, a[rr][f], INVERSE ? S.bk0 : S.k2));
-                        } else {
-                            float Fv, w;
-                            act_Fw(z, S.activation, Fv, w);
-                            a[rr][f] = fmaf(INVERSE ? S.bk0 : S.k2, Fv, keep * a[rr][f]);
+                        for (int f = 0; f < F; ++f) {
+                            a[rr][f] = fmaf(INVERSE ? S.bk1 : S.m2k2, r[rr][f], fmaf(keep, a[rr][f], INVERSE ? S.bk0 : S.k2));
+                            if constexpr (!INVERSE) x[rr][f] = fmaf(keep, x[rr][f], a[rr][f]);
                         }
-                        if constexpr (!INVERSE) x[rr][f] = fmaf(S.m, x[rr][f], a[rr][f]);
-                    }
+                } else {
+                    issue_with_others();
+#pragma unroll
+                    for (int rr = 0; rr < R; ++rr)
+#pragma unroll
+                        for (int f = 0; f < F; ++f) {
+                            float Fv, w;
+                            act_Fw(fmaf(c[rr], xj[f], x[rr][f]), S.activation, Fv, w);
+                            a[rr][f] = fmaf(INVERSE ? S.bk0 : S.k2, Fv, keep * a[rr][f]);
+                            if constexpr (!INVERSE) x[rr][f] = fmaf(keep, x[rr][f], a[rr][f]);
+                        }
+                }
                 __builtin_amdgcn_sched_barrier(0);
             });
         }
@@ -451,20 +460,25 @@ __global__ void __launch_bounds__(kBlockThreads, R * F <= (LOOP ? 10 : 12) ? 4 :
                 any_row_sums<R, F>(Y, wi, dot_chain<F>(xj, wj), L.lfl, c);
 #pragma unroll
                 for (int f = 0; f < F; ++f) v[f] = 0.f;
+                if constexpr (!TANH_ONLY) issue_with_others();
 #pragma unroll
-                for (int rr = 0; rr < R; ++rr) {
+                for (int rr = 0; rr < R; ++rr) {   // exp2 and reciprocals of one row at a time: see backward_core
+                    float r[1][F];
+                    if constexpr (TANH_ONLY) {
+                        if (rr > 0) issue_first();
+                        sigmoids(rr, Y, c, xj, r);
+                        issue_with_others();
+                    }
                     rh[rr] = 0.f;
 #pragma unroll
                     for (int f = 0; f < F; ++f) {
-                        const float z = fmaf(c[rr], xj[f], Y[rr][f]);
                         float w;
                         if constexpr (TANH_ONLY) {
-                            const float r = __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(z) + 1.0f);
-                            B[rr][f] = fmaf(S.bk1, r, fmaf(S.im, B[rr][f], S.bk0));
-                            w = fmaf(-r, r, r);
+                            B[rr][f] = fmaf(S.bk1, r[0][f], fmaf(S.im, B[rr][f], S.bk0));
+                            w = fmaf(-r[0][f], r[0][f], r[0][f]);
                         } else {
                             float Fv;
-                            act_Fw(z, S.activation, Fv, w);
+                            act_Fw(fmaf(c[rr], xj[f], Y[rr][f]), S.activation, Fv, w);
                             B[rr][f] = fmaf(S.bk0, Fv, S.im * B[rr][f]);
                         }
                         const float U = P[rr][f] * w;
@@ -473,7 +487,9 @@ __global__ void __launch_bounds__(kBlockThreads, R * F <= (LOOP ? 10 : 12) ? 4 :
                         G[rr][f] = fmaf(S.ku, U, G[rr][f]);
                     }
                 }
+                issue_first();
                 any_sum_rows<R>(rh, L.lfl);
+                issue_with_others();
                 float rhosum = 0.f;
 #pragma unroll
                 for (int rr = 0; rr < R; ++rr) {
@@ -494,7 +510,9 @@ __global__ void __launch_bounds__(kBlockThreads, R * F <= (LOOP ? 10 : 12) ? 4 :
                     dwj[f] = fmaf(rhosum_w, xj[f], dwj[f]);
                     s[f] = fmaf(rhosum, wj[f], v[f]);
                 }
+                issue_first();
                 any_sum_span<F>(s, L.lfl, L.lfl + L.lrl);   // over the group's row lanes
+                issue_with_others();
 #pragma unroll
                 for (int f = 0; f < F; ++f) {
                     G[jr][f] = fmaf(selku, s[f], G[jr][f]);

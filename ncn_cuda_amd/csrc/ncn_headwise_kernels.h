@@ -17,6 +17,22 @@
 
 namespace ncn {
 
+// r = 1 / (1 + 2^z) of rows [r0, r0 + N) of a tile, z = x_i + c_i xs_j with c_i = x_i Wi' + xs_j Wj' (cj), at high priority.
+template <int N, int R, int F>
+__device__ __forceinline__ void headwise_sigmoids(int r0, const float (&x)[R][F], const float (&wi)[F], const float (&cj)[F],
+                                                  const float (&xj)[F], float (&r)[N][F]) {
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+#pragma unroll
+        for (int f = 0; f < F; ++f) r[k][f] = fmaf(fmaf(x[r0 + k][f], wi[f], cj[f]), xj[f], x[r0 + k][f]);
+    issue_first();
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+#pragma unroll
+        for (int f = 0; f < F; ++f) r[k][f] = __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(r[k][f]) + 1.0f);
+    issue_with_others();
+}
+
 // The three functions take the template and call arguments of forward_core, inverse_core and backward_core, so that a
 // kernel picks one or the other by name (ROWS only reaches the sum over a group's row lanes; KU_W has nothing to act
 // on here).
@@ -25,6 +41,7 @@ __device__ __forceinline__ void headwise_forward_core(float (&x)[R][F], float (&
                                                       const float (&wj)[F], const StepTable& S, int lane, float4* slots,
                                                       int live = NC) {
     using T = Tile<NC, EC, R, F>;
+    const float m = in_vector_register(S.m);
 #pragma unroll 1
     for (int jo = 0; jo < T::LR; ++jo) {
 #pragma unroll
@@ -34,21 +51,26 @@ __device__ __forceinline__ void headwise_forward_core(float (&x)[R][F], float (&
             row_lane_broadcast<T::LF, T::LR, F>(x[jr], xj, jo, lane, slots);
 #pragma unroll
             for (int f = 0; f < F; ++f) cj[f] = xj[f] * wj[f];
+            if constexpr (TANH_ONLY) {
+                float r[R][F];
+                headwise_sigmoids(0, x, wi, cj, xj, r);
 #pragma unroll
-            for (int rr = 0; rr < R; ++rr) {
+                for (int rr = 0; rr < R; ++rr)
 #pragma unroll
-                for (int f = 0; f < F; ++f) {
-                    const float c = fmaf(x[rr][f], wi[f], cj[f]);
-                    const float z = fmaf(c, xj[f], x[rr][f]);
-                    if constexpr (TANH_ONLY) {
-                        const float r = __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(z) + 1.0f);
-                        a[rr][f] = fmaf(S.m2k2, r, fmaf(S.m, a[rr][f], S.k2));
-                    } else {
-                        float Fv, w;
-                        act_Fw(z, S.activation, Fv, w);
-                        a[rr][f] = fmaf(S.k2, Fv, S.m * a[rr][f]);
+                    for (int f = 0; f < F; ++f) {
+                        a[rr][f] = fmaf(S.m2k2, r[rr][f], fmaf(m, a[rr][f], S.k2));
+                        x[rr][f] = fmaf(m, x[rr][f], a[rr][f]);
                     }
-                    x[rr][f] = fmaf(S.m, x[rr][f], a[rr][f]);
+            } else {
+#pragma unroll
+                for (int rr = 0; rr < R; ++rr) {
+#pragma unroll
+                    for (int f = 0; f < F; ++f) {
+                        float Fv, w;
+                        act_Fw(fmaf(fmaf(x[rr][f], wi[f], cj[f]), xj[f], x[rr][f]), S.activation, Fv, w);
+                        a[rr][f] = fmaf(S.k2, Fv, S.m * a[rr][f]);
+                        x[rr][f] = fmaf(S.m, x[rr][f], a[rr][f]);
+                    }
                 }
             }
         }
@@ -60,6 +82,7 @@ __device__ __forceinline__ void headwise_inverse_core(float (&y)[R][F], float (&
                                                       const float (&wj)[F], const StepTable& S, int lane, float4* slots,
                                                       int live = NC) {
     using T = Tile<NC, EC, R, F>;
+    const float im = in_vector_register(S.im);
 #pragma unroll 1
     for (int jo = T::LR - 1; jo >= 0; --jo) {
 #pragma unroll
@@ -68,23 +91,25 @@ __device__ __forceinline__ void headwise_inverse_core(float (&y)[R][F], float (&
 #pragma unroll
             for (int rr = 0; rr < R; ++rr)
 #pragma unroll
-                for (int f = 0; f < F; ++f) y[rr][f] = fmaf(S.im, y[rr][f], -b[rr][f]);
+                for (int f = 0; f < F; ++f) y[rr][f] = fmaf(im, y[rr][f], -b[rr][f]);
             float xj[F], cj[F];
             row_lane_broadcast<T::LF, T::LR, F>(y[jr], xj, jo, lane, slots);
 #pragma unroll
             for (int f = 0; f < F; ++f) cj[f] = xj[f] * wj[f];
+            if constexpr (TANH_ONLY) {
+                float r[R][F];
+                headwise_sigmoids(0, y, wi, cj, xj, r);
 #pragma unroll
-            for (int rr = 0; rr < R; ++rr) {
+                for (int rr = 0; rr < R; ++rr)
 #pragma unroll
-                for (int f = 0; f < F; ++f) {
-                    const float c = fmaf(y[rr][f], wi[f], cj[f]);
-                    const float z = fmaf(c, xj[f], y[rr][f]);
-                    if constexpr (TANH_ONLY) {
-                        const float r = __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(z) + 1.0f);
-                        b[rr][f] = fmaf(S.bk1, r, fmaf(S.im, b[rr][f], S.bk0));
-                    } else {
+                    for (int f = 0; f < F; ++f) b[rr][f] = fmaf(S.bk1, r[rr][f], fmaf(im, b[rr][f], S.bk0));
+            } else {
+#pragma unroll
+                for (int rr = 0; rr < R; ++rr) {
+#pragma unroll
+                    for (int f = 0; f < F; ++f) {
                         float Fv, w;
-                        act_Fw(z, S.activation, Fv, w);
+                        act_Fw(fmaf(fmaf(y[rr][f], wi[f], cj[f]), xj[f], y[rr][f]), S.activation, Fv, w);
                         b[rr][f] = fmaf(S.bk0, Fv, S.im * b[rr][f]);
                     }
                 }
@@ -122,34 +147,39 @@ __device__ __forceinline__ void headwise_backward_core(float (&Y)[R][F], float (
             row_lane_broadcast<T::LF, T::LR, F>(Y[jr], xj, jo, lane, slots);
 #pragma unroll
             for (int f = 0; f < F; ++f) cj[f] = xj[f] * wj[f];
+            constexpr int RC = 1;   // rows at a time (see backward_core; two would spill)
             if constexpr (T::LR == 1) {
                 // The whole group is in this lane: every row's share of the pivot row's gradient,
                 // ku (rh_if Wj'_f + c_if U_if) = ku U_if (xs_jf Wj'_f + c_if), goes straight into it, and dWj takes the
                 // row's rh_if as dWi does (no sums to carry through the step: fewer registers).
 #pragma unroll
-                for (int rr = 0; rr < R; ++rr) {
+                for (int r0 = 0; r0 < R; r0 += RC) {
+                    float r[RC][F];
+                    if constexpr (TANH_ONLY) headwise_sigmoids(r0, Y, wi, cj, xj, r);
 #pragma unroll
-                    for (int f = 0; f < F; ++f) {
-                        const float c = fmaf(Y[rr][f], wi[f], cj[f]);
-                        const float z = fmaf(c, xj[f], Y[rr][f]);
-                        float w;
-                        if constexpr (TANH_ONLY) {
-                            const float r = __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(z) + 1.0f);
-                            B[rr][f] = fmaf(S.bk1, r, fmaf(S.im, B[rr][f], S.bk0));   // bh before this step
-                            w = fmaf(-r, r, r);
-                        } else {
-                            float Fv;
-                            act_Fw(z, S.activation, Fv, w);
-                            B[rr][f] = fmaf(S.bk0, Fv, S.im * B[rr][f]);
+                    for (int k = 0; k < RC; ++k) {
+                        const int rr = r0 + k;
+#pragma unroll
+                        for (int f = 0; f < F; ++f) {
+                            const float c = fmaf(Y[rr][f], wi[f], cj[f]);
+                            float w;
+                            if constexpr (TANH_ONLY) {
+                                B[rr][f] = fmaf(S.bk1, r[k][f], fmaf(S.im, B[rr][f], S.bk0));   // bh before this step
+                                w = fmaf(-r[k][f], r[k][f], r[k][f]);
+                            } else {
+                                float Fv;
+                                act_Fw(fmaf(c, xj[f], Y[rr][f]), S.activation, Fv, w);
+                                B[rr][f] = fmaf(S.bk0, Fv, S.im * B[rr][f]);
+                            }
+                            const float U = P[rr][f] * w;
+                            const float rh = U * xj[f];
+                            const float krh = krho * rh;
+                            dwi[f] = fmaf(krh, Y[rr][f], dwi[f]);
+                            dwj[f] = fmaf(krh, xj[f], dwj[f]);
+                            G[rr][f] = fmaf(S.ku, fmaf(rh, wi[f], U), G[rr][f]);
+                            G[jr][f] = fmaf(S.ku * U, cj[f] + c, G[jr][f]);
+                            if (rr != jr) P[rr][f] = fmaf(S.om, G[rr][f], P[rr][f]);
                         }
-                        const float U = P[rr][f] * w;
-                        const float rh = U * xj[f];
-                        const float krh = krho * rh;
-                        dwi[f] = fmaf(krh, Y[rr][f], dwi[f]);
-                        dwj[f] = fmaf(krh, xj[f], dwj[f]);
-                        G[rr][f] = fmaf(S.ku, fmaf(rh, wi[f], U), G[rr][f]);
-                        G[jr][f] = fmaf(S.ku * U, cj[f] + c, G[jr][f]);
-                        if (rr != jr) P[rr][f] = fmaf(S.om, G[rr][f], P[rr][f]);
                     }
                 }
 #pragma unroll
@@ -159,28 +189,32 @@ __device__ __forceinline__ void headwise_backward_core(float (&Y)[R][F], float (
 #pragma unroll
             for (int f = 0; f < F; ++f) v[f] = rhs[f] = 0.f;
 #pragma unroll
-            for (int rr = 0; rr < R; ++rr) {
+            for (int r0 = 0; r0 < R; r0 += RC) {
+                float r[RC][F];
+                if constexpr (TANH_ONLY) headwise_sigmoids(r0, Y, wi, cj, xj, r);
 #pragma unroll
-                for (int f = 0; f < F; ++f) {
-                    const float c = fmaf(Y[rr][f], wi[f], cj[f]);
-                    const float z = fmaf(c, xj[f], Y[rr][f]);
-                    float w;
-                    if constexpr (TANH_ONLY) {
-                        const float r = __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(z) + 1.0f);
-                        B[rr][f] = fmaf(S.bk1, r, fmaf(S.im, B[rr][f], S.bk0));   // bh before this step
-                        w = fmaf(-r, r, r);
-                    } else {
-                        float Fv;
-                        act_Fw(z, S.activation, Fv, w);
-                        B[rr][f] = fmaf(S.bk0, Fv, S.im * B[rr][f]);
+                for (int k = 0; k < RC; ++k) {
+                    const int rr = r0 + k;
+#pragma unroll
+                    for (int f = 0; f < F; ++f) {
+                        const float c = fmaf(Y[rr][f], wi[f], cj[f]);
+                        float w;
+                        if constexpr (TANH_ONLY) {
+                            B[rr][f] = fmaf(S.bk1, r[k][f], fmaf(S.im, B[rr][f], S.bk0));   // bh before this step
+                            w = fmaf(-r[k][f], r[k][f], r[k][f]);
+                        } else {
+                            float Fv;
+                            act_Fw(fmaf(c, xj[f], Y[rr][f]), S.activation, Fv, w);
+                            B[rr][f] = fmaf(S.bk0, Fv, S.im * B[rr][f]);
+                        }
+                        const float U = P[rr][f] * w;
+                        const float rh = U * xj[f];
+                        v[f] = fmaf(c, U, v[f]);
+                        rhs[f] += rh;
+                        dwi[f] = fmaf(krho * rh, Y[rr][f], dwi[f]);
+                        G[rr][f] = fmaf(S.ku, fmaf(rh, wi[f], U), G[rr][f]);
+                        if (rr != jr) P[rr][f] = fmaf(S.om, G[rr][f], P[rr][f]);
                     }
-                    const float U = P[rr][f] * w;
-                    const float rh = U * xj[f];
-                    v[f] = fmaf(c, U, v[f]);
-                    rhs[f] += rh;
-                    dwi[f] = fmaf(krho * rh, Y[rr][f], dwi[f]);
-                    G[rr][f] = fmaf(S.ku, fmaf(rh, wi[f], U), G[rr][f]);
-                    if (rr != jr) P[rr][f] = fmaf(S.om, G[rr][f], P[rr][f]);
                 }
             }
             float t[F];
@@ -190,7 +224,9 @@ __device__ __forceinline__ void headwise_backward_core(float (&Y)[R][F], float (
                 // every row lane of the group adds its share of sum_i rh_if: the sum over lanes at the end completes it
                 dwj[f] = fmaf(krho * rhs[f], xj[f], dwj[f]);
             }
+            issue_first();
             lane_sum_n<T::LF, T::LPG, ROWS, F>(t);   // over the group's row lanes
+            issue_with_others();
 #pragma unroll
             for (int f = 0; f < F; ++f) {
                 G[jr][f] = fmaf(selku, t[f], G[jr][f]);

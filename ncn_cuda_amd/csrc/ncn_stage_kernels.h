@@ -143,7 +143,7 @@ __device__ __forceinline__ void act_Fw(float z, int code, float& Fv, float& w) {
 }
 
 // The row sums c_i = <xs_i, Wi'> + <xs_j, Wj'> of a lane's R rows: a chain of FMAs per row that starts from the lane's
-// share e of <xs_j, Wj'>, then all R sums cross the LF lanes of a row together.
+// share e of <xs_j, Wj'>, then all R sums cross the LF lanes of a row together.  Leaves the wave at high priority.
 template <int LF, int R, int F, bool ROWS>
 __device__ __forceinline__ void row_sums(const float (&x)[R][F], const float (&wi)[F], float e, float (&c)[R]) {
 #pragma unroll
@@ -152,7 +152,18 @@ __device__ __forceinline__ void row_sums(const float (&x)[R][F], const float (&w
 #pragma unroll
         for (int f = 0; f < F; ++f) c[rr] = fmaf(x[rr][f], wi[f], c[rr]);
     }
+    issue_first();
     lane_sum_n<1, LF, ROWS, R>(c);
+}
+
+// r = 1 / (1 + 2^z) of rows [r0, r0 + N) of a tile, z = x_i + c_i xs_j.
+template <int N, int R, int F>
+__device__ __forceinline__ void sigmoids(int r0, const float (&x)[R][F], const float (&c)[R], const float (&xj)[F], float (&r)[N][F]) {
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+#pragma unroll
+        for (int f = 0; f < F; ++f)
+            r[k][f] = __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(fmaf(c[r0 + k], xj[f], x[r0 + k][f])) + 1.0f);
 }
 
 template <int F>
@@ -178,6 +189,7 @@ __device__ __forceinline__ void forward_core(float (&x)[R][F], float (&a)[R][F],
                                              const float (&wj)[F], const StepTable& S, int lane, float4* slots,
                                              int live = NC) {
     using T = Tile<NC, EC, R, F>;
+    const float m = in_vector_register(S.m);   // read twice per element and step
 #pragma unroll 1
     for (int jo = 0; jo < T::LR; ++jo) {
 #pragma unroll
@@ -186,20 +198,29 @@ __device__ __forceinline__ void forward_core(float (&x)[R][F], float (&a)[R][F],
             float xj[F], c[R];
             row_lane_broadcast<T::LF, T::LR, F>(x[jr], xj, jo, lane, slots);
             row_sums<T::LF, R, F, ROWS>(x, wi, dot_chain<F>(xj, wj), c);
+            if constexpr (TANH_ONLY) {
+                float r[R][F];
+                sigmoids(0, x, c, xj, r);
+                issue_with_others();
 #pragma unroll
-            for (int rr = 0; rr < R; ++rr) {
+                for (int rr = 0; rr < R; ++rr)
 #pragma unroll
-                for (int f = 0; f < F; ++f) {
-                    const float z = fmaf(c[rr], xj[f], x[rr][f]);
-                    if constexpr (TANH_ONLY) {
-                        const float r = __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(z) + 1.0f);
-                        a[rr][f] = fmaf(S.m2k2, r, fmaf(S.m, a[rr][f], S.k2));
-                    } else {
+                    for (int f = 0; f < F; ++f) {
+                        a[rr][f] = fmaf(S.m2k2, r[rr][f], fmaf(m, a[rr][f], S.k2));
+                        x[rr][f] = fmaf(m, x[rr][f], a[rr][f]);
+                    }
+            } else {
+                issue_with_others();
+#pragma unroll
+                for (int rr = 0; rr < R; ++rr) {
+#pragma unroll
+                    for (int f = 0; f < F; ++f) {
+                        const float z = fmaf(c[rr], xj[f], x[rr][f]);
                         float Fv, w;
                         act_Fw(z, S.activation, Fv, w);
                         a[rr][f] = fmaf(S.k2, Fv, S.m * a[rr][f]);
+                        x[rr][f] = fmaf(S.m, x[rr][f], a[rr][f]);
                     }
-                    x[rr][f] = fmaf(S.m, x[rr][f], a[rr][f]);
                 }
             }
         }
@@ -217,6 +238,7 @@ __device__ __forceinline__ void inverse_core(float (&y)[R][F], float (&b)[R][F],
                                              const float (&wj)[F], const StepTable& S, int lane, float4* slots,
                                              int live = NC) {
     using T = Tile<NC, EC, R, F>;
+    const float im = in_vector_register(S.im);   // read twice per element and step
 #pragma unroll 1
     for (int jo = T::LR - 1; jo >= 0; --jo) {
 #pragma unroll
@@ -225,19 +247,25 @@ __device__ __forceinline__ void inverse_core(float (&y)[R][F], float (&b)[R][F],
 #pragma unroll
             for (int rr = 0; rr < R; ++rr)
 #pragma unroll
-                for (int f = 0; f < F; ++f) y[rr][f] = fmaf(S.im, y[rr][f], -b[rr][f]);
+                for (int f = 0; f < F; ++f) y[rr][f] = fmaf(im, y[rr][f], -b[rr][f]);
             float xj[F], c[R];
             row_lane_broadcast<T::LF, T::LR, F>(y[jr], xj, jo, lane, slots);
             row_sums<T::LF, R, F, ROWS>(y, wi, dot_chain<F>(xj, wj), c);
+            if constexpr (TANH_ONLY) {
+                float r[R][F];
+                sigmoids(0, y, c, xj, r);
+                issue_with_others();
 #pragma unroll
-            for (int rr = 0; rr < R; ++rr) {
+                for (int rr = 0; rr < R; ++rr)
 #pragma unroll
-                for (int f = 0; f < F; ++f) {
-                    const float z = fmaf(c[rr], xj[f], y[rr][f]);
-                    if constexpr (TANH_ONLY) {
-                        const float r = __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(z) + 1.0f);
-                        b[rr][f] = fmaf(S.bk1, r, fmaf(S.im, b[rr][f], S.bk0));
-                    } else {
+                    for (int f = 0; f < F; ++f) b[rr][f] = fmaf(S.bk1, r[rr][f], fmaf(im, b[rr][f], S.bk0));
+            } else {
+                issue_with_others();
+#pragma unroll
+                for (int rr = 0; rr < R; ++rr) {
+#pragma unroll
+                    for (int f = 0; f < F; ++f) {
+                        const float z = fmaf(c[rr], xj[f], y[rr][f]);
                         float Fv, w;
                         act_Fw(z, S.activation, Fv, w);
                         b[rr][f] = fmaf(S.bk0, Fv, S.im * b[rr][f]);
@@ -303,35 +331,47 @@ __device__ __forceinline__ void backward_core(float (&Y)[R][F], float (&B)[R][F]
             float xj[F], c[R], rh[R];
             row_lane_broadcast<T::LF, T::LR, F>(Y[jr], xj, jo, lane, slots);
             row_sums<T::LF, R, F, ROWS>(Y, wi, dot_chain<F>(xj, wj), c);
+            // exp2 and reciprocals a few rows at a time (all rows' r at once would not fit the registers), each time at high
+            // priority, and what is made of them at low: see issue_first
+            constexpr int RC = F <= 4 && R % 2 == 0 ? 2 : 1;
+            if constexpr (!TANH_ONLY) issue_with_others();
             if constexpr (T::LR == 1) {
                 // The whole group is in this lane: the pivot row's share sum_i c_i U_i goes straight into its gradient
                 // (no sum across lanes to wait for), with the pivot's own two terms merged into one coefficient.
-                float kc[R];
 #pragma unroll
-                for (int rr = 0; rr < R; ++rr) kc[rr] = (rr == jr) ? fmaf(S.ku, c[rr], S.ku) : S.ku * c[rr];
+                for (int r0 = 0; r0 < R; r0 += RC) {
+                    float r[RC][F];
+                    if constexpr (TANH_ONLY) {
+                        if (r0 > 0) issue_first();
+                        sigmoids(r0, Y, c, xj, r);
+                        issue_with_others();
+                    }
 #pragma unroll
-                for (int rr = 0; rr < R; ++rr) {
-                    rh[rr] = 0.f;
+                    for (int k = 0; k < RC; ++k) {
+                        const int rr = r0 + k;
+                        const float kc = (rr == jr) ? fmaf(S.ku, c[rr], S.ku) : S.ku * c[rr];
+                        rh[rr] = 0.f;
 #pragma unroll
-                    for (int f = 0; f < F; ++f) {
-                        const float z = fmaf(c[rr], xj[f], Y[rr][f]);
-                        float w;
-                        if constexpr (TANH_ONLY) {
-                            const float r = __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(z) + 1.0f);
-                            B[rr][f] = fmaf(S.bk1, r, fmaf(S.im, B[rr][f], S.bk0));   // bh before this step
-                            w = fmaf(-r, r, r);
-                        } else {
-                            float Fv;
-                            act_Fw(z, S.activation, Fv, w);
-                            B[rr][f] = fmaf(S.bk0, Fv, S.im * B[rr][f]);
+                        for (int f = 0; f < F; ++f) {
+                            float w;
+                            if constexpr (TANH_ONLY) {
+                                B[rr][f] = fmaf(S.bk1, r[k][f], fmaf(S.im, B[rr][f], S.bk0));   // bh before this step
+                                w = fmaf(-r[k][f], r[k][f], r[k][f]);
+                            } else {
+                                float Fv;
+                                act_Fw(fmaf(c[rr], xj[f], Y[rr][f]), S.activation, Fv, w);
+                                B[rr][f] = fmaf(S.bk0, Fv, S.im * B[rr][f]);
+                            }
+                            const float U = P[rr][f] * w;
+                            rh[rr] = fmaf(U, xj[f], rh[rr]);
+                            if (rr != jr) G[rr][f] = fmaf(S.ku, U, G[rr][f]);
+                            G[jr][f] = fmaf(kc, U, G[jr][f]);
                         }
-                        const float U = P[rr][f] * w;
-                        rh[rr] = fmaf(U, xj[f], rh[rr]);
-                        if (rr != jr) G[rr][f] = fmaf(S.ku, U, G[rr][f]);
-                        G[jr][f] = fmaf(kc[rr], U, G[jr][f]);
                     }
                 }
+                issue_first();
                 lane_sum_n<1, T::LF, ROWS, R>(rh);
+                issue_with_others();
                 float rhosum = 0.f;
 #pragma unroll
                 for (int rr = 0; rr < R; ++rr) {
@@ -359,28 +399,38 @@ __device__ __forceinline__ void backward_core(float (&Y)[R][F], float (&B)[R][F]
 #pragma unroll
             for (int f = 0; f < F; ++f) v[f] = 0.f;
 #pragma unroll
-            for (int rr = 0; rr < R; ++rr) {
-                rh[rr] = 0.f;
+            for (int r0 = 0; r0 < R; r0 += RC) {
+                float r[RC][F];
+                if constexpr (TANH_ONLY) {
+                    if (r0 > 0) issue_first();
+                    sigmoids(r0, Y, c, xj, r);
+                    issue_with_others();
+                }
 #pragma unroll
-                for (int f = 0; f < F; ++f) {
-                    const float z = fmaf(c[rr], xj[f], Y[rr][f]);
-                    float w;
-                    if constexpr (TANH_ONLY) {
-                        const float r = __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(z) + 1.0f);
-                        B[rr][f] = fmaf(S.bk1, r, fmaf(S.im, B[rr][f], S.bk0));   // bh before this step
-                        w = fmaf(-r, r, r);
-                    } else {
-                        float Fv;
-                        act_Fw(z, S.activation, Fv, w);
-                        B[rr][f] = fmaf(S.bk0, Fv, S.im * B[rr][f]);
+                for (int k = 0; k < RC; ++k) {
+                    const int rr = r0 + k;
+                    rh[rr] = 0.f;
+#pragma unroll
+                    for (int f = 0; f < F; ++f) {
+                        float w;
+                        if constexpr (TANH_ONLY) {
+                            B[rr][f] = fmaf(S.bk1, r[k][f], fmaf(S.im, B[rr][f], S.bk0));   // bh before this step
+                            w = fmaf(-r[k][f], r[k][f], r[k][f]);
+                        } else {
+                            float Fv;
+                            act_Fw(fmaf(c[rr], xj[f], Y[rr][f]), S.activation, Fv, w);
+                            B[rr][f] = fmaf(S.bk0, Fv, S.im * B[rr][f]);
+                        }
+                        const float U = P[rr][f] * w;
+                        rh[rr] = fmaf(U, xj[f], rh[rr]);
+                        v[f] = fmaf(c[rr], U, v[f]);
+                        G[rr][f] = fmaf(S.ku, U, G[rr][f]);
                     }
-                    const float U = P[rr][f] * w;
-                    rh[rr] = fmaf(U, xj[f], rh[rr]);
-                    v[f] = fmaf(c[rr], U, v[f]);
-                    G[rr][f] = fmaf(S.ku, U, G[rr][f]);
                 }
             }
+            issue_first();
             lane_sum_n<1, T::LF, ROWS, R>(rh);
+            issue_with_others();
             float rhosum = 0.f;
 #pragma unroll
             for (int rr = 0; rr < R; ++rr) {
@@ -401,7 +451,9 @@ __device__ __forceinline__ void backward_core(float (&Y)[R][F], float (&B)[R][F]
                 dwj[f] = fmaf(rhosum_w, xj[f], dwj[f]);
                 t[f] = fmaf(rhosum, wj[f], v[f]);
             }
+            issue_first();
             lane_sum_n<T::LF, T::LPG, ROWS, F>(t);   // over the group's row lanes
+            issue_with_others();
 #pragma unroll
             for (int f = 0; f < F; ++f) {
                 G[jr][f] = fmaf(selku, t[f], G[jr][f]);
@@ -453,7 +505,7 @@ __device__ __forceinline__ void backward_steps(float (&Y)[R][F], float (&B)[R][F
                 P[rr][f] *= isc;
             }
         }
-    backward_core<NC, EC, R, F, MASKED, TANH_ONLY, STEP_MASK>(Y, B, G, P, wi, wj, dwi, dwj, own, S, 0, lane, slots,
+    backward_core<NC, EC, R, F, MASKED, TANH_ONLY, STEP_MASK, true>(Y, B, G, P, wi, wj, dwi, dwj, own, S, 0, lane, slots,
                                                              live);
     const float dn = S.m_pow_n;       // NC steps done: undo the scaling of the gradients
 #pragma unroll
@@ -582,7 +634,7 @@ __global__ void __launch_bounds__(kBlockThreads, (R == 4 && F == 4) ? 5 : 1) sta
         if (A.aux0) { NCN_STORE_DEAD_ROWS(A.aux0, A.aux1, NCN_F32, x, a) }
         NCN_ZERO_DEAD_ROWS(x, a, true)
         scale_tile<R, F>(x, a, A.tab.kappa, A.tab.a_scale);
-        forward_core<NC, EC, R, F, TANH_ONLY, INDEXED>(x, a, wi, wj, A.tab, lane, slots, live);
+        forward_core<NC, EC, R, F, TANH_ONLY, INDEXED, true>(x, a, wi, wj, A.tab, lane, slots, live);
         scale_tile<R, F>(x, a, A.tab.inv_kappa, A.tab.inv_a_scale);
 #pragma unroll
         for (int rr = 0; rr < R; ++rr) {
@@ -616,7 +668,7 @@ __global__ void __launch_bounds__(kBlockThreads, (R == 4 && F == 4) ? 5 : 1) sta
         NCN_STORE_DEAD_ROWS(A.out0, A.out1, out_dtype, y, b)
         NCN_ZERO_DEAD_ROWS(y, b, true)
         scale_tile<R, F>(y, b, A.tab.kappa, A.tab.b_scale);
-        inverse_core<NC, EC, R, F, TANH_ONLY, INDEXED>(y, b, wi, wj, A.tab, lane, slots, live);
+        inverse_core<NC, EC, R, F, TANH_ONLY, INDEXED, true>(y, b, wi, wj, A.tab, lane, slots, live);
         scale_tile<R, F>(y, b, A.tab.inv_kappa, A.tab.inv_b_scale);
 #pragma unroll
         for (int rr = 0; rr < R; ++rr) {
