@@ -165,8 +165,8 @@ __device__ __forceinline__ void store_frag(void* base, int dtype, int64_t off, b
 // a kernel issues the loads of all its input tiles before it finishes the first, so that their latencies overlap
 // instead of following one another (converting each fragment as it is loaded waits for every load in turn).
 // The offsets must be valid addresses for every lane (lanes without work read some row of their own batch entry and
-// are zeroed afterwards where that matters).
-template <int R, int FPL>
+// are zeroed afterwards where that matters).  STREAM: float32 with the non-temporal hint.
+template <int R, int FPL, bool STREAM = false>
 __device__ __forceinline__ void issue_tile(const void* base, int dtype, const int64_t (&off)[R], float (&v)[R][FPL],
                                            int64_t plane = 0) {
     static_assert(FPL % 4 == 0, "fragment must be a multiple of 4 features");
@@ -177,7 +177,9 @@ __device__ __forceinline__ void issue_tile(const void* base, int dtype, const in
         for (int rr = 0; rr < R; ++rr)
 #pragma unroll
             for (int k = 0; k < FPL / 4; ++k) {
-                const float4 t = reinterpret_cast<const float4*>(static_cast<const float*>(base) + off[rr])[k];
+                typedef float Chunk __attribute__((ext_vector_type(4)));
+                const Chunk* const at = reinterpret_cast<const Chunk*>(static_cast<const float*>(base) + off[rr]) + k;
+                const Chunk t = STREAM ? __builtin_nontemporal_load(at) : *at;
                 v[rr][4 * k] = t.x; v[rr][4 * k + 1] = t.y; v[rr][4 * k + 2] = t.z; v[rr][4 * k + 3] = t.w;
             }
     } else if (dtype == NCN_BF16) {

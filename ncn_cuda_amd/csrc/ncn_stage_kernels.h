@@ -567,6 +567,26 @@ __device__ __forceinline__ int dtype_of(int from_args, int when_bf16) {
     return TYPES == kF32Types ? NCN_F32 : TYPES == kBf16Types ? when_bf16 : from_args;
 }
 
+// float32 launches on arrays of that many elements ask for their rows with the non-temporal hint, in tiles of 16 elements and more and
+// rows of whole cache lines (others share theirs with the next head's wave): what they read is not read again before it has
+// left the 256 MB memory-side cache, and without the hint it takes the place of what the launch before wrote.  On arrays of an eighth of
+// that cache and less the inputs still lie in it.  Launches, us, without : with, groups of 8 rows, heads of 32, x[b, 2048, 128]: b = 12
+// (12 MB an array) forward 14.3 : 14.5, backward 22.6 : 22.8; 20 (21 MB) 18.8 : 19.5, 32.1 : 33.1; 28 (29 MB) 26.8 : 26.7, 46.2 : 45.7; 40
+// (42 MB) 37.5 : 36.2, 60.1 : 58.8.  Training steps: 4 stages, b = 32 333 : 327, 64 606 : 568, 128 1128 : 1077; groups of 16, 3
+// stages, x[64, 4096, 128] 1280 : 1243; groups of 2, whose tiles are 2 x 4, 186 : 202.  bfloat16, whose rows of 64 bytes share lines:
+// x[128, 4096, 128], groups of 16, 3 stages 2453 : 2520.  Stores with the hint: b = 64 594 : 604.
+constexpr int64_t kStreamElements = 1 << 23;
+#define NCN_REQUEST(STREAM, ...)                                                                \
+    if (TYPES == kF32Types && EC % 32 == 0 && R * F >= 16 && A.plane >= kStreamElements) {      \
+        constexpr bool STREAM = true;                                                           \
+        asm volatile("");   /* the two sides are not alike, or the compiler makes one of them and drops the hint */ \
+        __VA_ARGS__                                                                             \
+        asm volatile("");                                                                       \
+    } else {                                                                                    \
+        constexpr bool STREAM = false;                                                          \
+        __VA_ARGS__                                                                             \
+    }
+
 // Rows past a context length take no part in the stage: they pass through.  (A launch of its own for them, one element per
 // lane, cost 38 us per stage and direction on 32 x 4096 x 128 bfloat16 with a quarter of the rows past their lengths, 0.22 of
 // the 0.89 ms of a three-stage training step.)  The builds for one type store them as they were loaded.  In the builds for
@@ -625,8 +645,7 @@ __global__ void __launch_bounds__(kBlockThreads, (R == 4 && F == 4) ? 5 : 1) sta
         int64_t off[R];
         const int live = tile_offsets<NC, EC, R, F, INDEXED>(A, t, lane, head, off);
         float x[R][F], a[R][F];
-        issue_tile<R, F>(A.in0, in_dtype, off, x);
-        issue_tile<R, F>(A.in1, in_dtype, off, a);
+        NCN_REQUEST(STREAM, issue_tile<R, F, STREAM>(A.in0, in_dtype, off, x); issue_tile<R, F, STREAM>(A.in1, in_dtype, off, a);)
         NCN_FINISH_W_ONCE
         finish_tile<R, F>(in_dtype, x);
         finish_tile<R, F>(in_dtype, a);
@@ -660,8 +679,7 @@ __global__ void __launch_bounds__(kBlockThreads, (R == 4 && F == 4) ? 5 : 1) sta
         int64_t off[R];
         const int live = tile_offsets<NC, EC, R, F, INDEXED>(A, t, lane, head, off);
         float y[R][F], b[R][F];
-        issue_tile<R, F>(A.in0, in_dtype, off, y, A.plane);
-        issue_tile<R, F>(A.in1, in_dtype, off, b, A.plane);
+        NCN_REQUEST(STREAM, issue_tile<R, F, STREAM>(A.in0, in_dtype, off, y, A.plane); issue_tile<R, F, STREAM>(A.in1, in_dtype, off, b, A.plane);)
         NCN_FINISH_W_ONCE
         finish_tile<R, F>(in_dtype, y);
         finish_tile<R, F>(in_dtype, b);
@@ -704,12 +722,9 @@ __global__ void __launch_bounds__(kBlockThreads, (TANH_ONLY && R * F <= 16 && F 
         int64_t off[R];
         const int live = tile_offsets<NC, EC, R, F, INDEXED>(A, t, lane, head, off);
         float Y[R][F], B[R][F], G[R][F], H[R][F];
-        issue_tile<R, F>(A.in0, in_dtype, off, Y, A.plane);
-        issue_tile<R, F>(A.in1, in_dtype, off, B, A.plane);
-        issue_tile<R, F>(A.g0, g_dtype, off, G);
-        if (A.g1) {
-            issue_tile<R, F>(A.g1, g_dtype, off, H);
-        } else {
+        NCN_REQUEST(STREAM, issue_tile<R, F, STREAM>(A.in0, in_dtype, off, Y, A.plane); issue_tile<R, F, STREAM>(A.in1, in_dtype, off, B, A.plane);
+                    issue_tile<R, F, STREAM>(A.g0, g_dtype, off, G); if (A.g1) issue_tile<R, F, STREAM>(A.g1, g_dtype, off, H);)
+        if (!A.g1) {
 #pragma unroll
             for (int rr = 0; rr < R; ++rr)
 #pragma unroll
@@ -768,6 +783,7 @@ __global__ void __launch_bounds__(kBlockThreads, (TANH_ONLY && R * F <= 16 && F 
 #undef NCN_ZERO_DEAD_ROWS
 #undef NCN_STORE_DEAD_ROWS
 #undef NCN_PASS_DEAD_ROWS
+#undef NCN_REQUEST
 #undef NCN_FINISH_W_ONCE
 #undef NCN_WAVE_PROLOGUE
 
