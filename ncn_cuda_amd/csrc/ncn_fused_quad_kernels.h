@@ -9,8 +9,8 @@
 // lengths, keep every row in LDS, spread a group over two lanes per feature and pass the pivot row between them.)
 //
 // x[64, 2048, 128] bfloat16, groups of 4, 6 stages in two passes: forward passes 109 + 128 -> 94 + 115 us, backward 268 + 239 ->
-// 227 + 202; x[32, 1024, 128] float32, 5 stages: 37 + 23 -> 35 + 21 and 62 + 51 -> 55 + 44.  Without loads and stores the larger
-// ones take 77 + 88 and 181 + 159, without steps 44 + 69 and 85 + 99, without the exchanges' barriers 4 % less.
+// 227 + 202; x[32, 1024, 128] float32, 5 stages: 37 + 23 -> 35 + 21 and 62 + 51 -> 55 + 44.  With issue_first (ncn_device.h) the larger
+// ones take 80 + 102 and 168 + 153: without loads and stores 67 + 78 and 155 + 136, without steps 43 + 69 and 86 + 98.
 #pragma once
 #include "ncn_fused_kernels.h"
 
@@ -18,7 +18,8 @@ namespace ncn {
 
 constexpr int kQuadF = 4;              // features per lane
 // Waves per workgroup: windows of 2048 / EC groups forward, 1024 / EC backward.  (Backward windows of 8 waves, with
-// half the halo: x[64, 2048, 128], groups of 4, 6 stages 539 us a training step against 527; 5 stages of x[32, 1024, 128] 151 both.)
+// half the halo, have all waves of a workgroup wait for each other: 207 + 185 us the passes of x[64, 2048, 128] above against 157 + 145, 46 + 56 those
+// of x[32, 1024, 128] against 39 + 48.)
 constexpr int kQuadWavesFwd = 8, kQuadWavesBwd = 4;
 constexpr int quad_groups(int ec, int waves) { return waves * (64 * kQuadF / ec); }   // groups of the largest window
 constexpr size_t quad_lds_bytes(int ec, int waves, bool backward) {
