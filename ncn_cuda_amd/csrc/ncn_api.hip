@@ -872,7 +872,7 @@ static int backward_impl(const void* y, const void* ya, int y_dtype, const void*
             void* ddxa = to_out ? dxa : static_cast<void*>(t[3]);
             const int d_dtype = to_out ? dx_dtype : NCN_F32;
             // a partial row of a multi-stage pass holds its stages side by side, as dW does
-            const int rows = ps.single ? p.partial_rows : fused_grid(shape, ps, true, fused_cap) / shape->n_head;
+            const int rows = ps.single ? p.partial_rows : fused_backward_grid(shape, ps, fused_cap) / shape->n_head;
             float* region;
             hipError_t err = reducer.reserve(rows, ps.count, &region);
             if (err != hipSuccess) return (int)err;
@@ -1381,7 +1381,7 @@ int ncn_stack_backward(const float* y, const float* ya, const float* saves, cons
             // the first pass of a range hands no reconstructed inputs on: the range before it has kept its outputs
             float* rec = k == 0 ? nullptr : static_cast<float*>(pair(gp + (int)(k - 1) % 2, 0));
             float* reca = k == 0 ? nullptr : static_cast<float*>(pair(gp + (int)(k - 1) % 2, 1));
-            const int rows = ps.single ? p.partial_rows : fused_grid(shape, ps, true, c.row_cap) / shape->n_head;
+            const int rows = ps.single ? p.partial_rows : fused_backward_grid(shape, ps, c.row_cap) / shape->n_head;
             float* region;
             hipError_t err = reducer.reserve(rows, ps.count, &region);
             if (err != hipSuccess) return (int)err;

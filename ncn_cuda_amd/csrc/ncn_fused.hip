@@ -1,5 +1,5 @@
 // Planning and launching of the multi-stage (LDS-resident) passes; kernels in ncn_fused_kernels.h.
-#include <climits>
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
@@ -16,8 +16,12 @@ namespace {
 // with their neighbours on the CU, so that the loads and stores of one run under the stages of the other; a workgroup
 // that loops over several windows keeps the phase it started in (measured on the 13-stage configuration: grids of
 // 4096 workgroups, 4.5 windows each, 5.35 ms per step; one window each 4.94).  The backward is further bounded by its
-// dW partial rows (one per n_head workgroups and stage), see fused_grid.
+// dW partial rows (one per n_head workgroups and stage), see fused_backward_grid.
 constexpr int kFusedMaxGridBwd = 1 << 16;
+// Windows of a forward launch: a launch holds less than 2^32 work-items.  More windows are given to several launches, by batch entries
+// (each of 4 groups of four rows, heads of 8: from 1.07e9 elements on).
+constexpr int64_t kFusedMaxGridFwd = ((int64_t(1) << 32) - 1) / (64 * kFusedWavesFwd);
+static_assert(kQuadWavesFwd <= kFusedWavesFwd, "threads of a forward workgroup");
 
 size_t fused_lds_bytes(int nc, int ec, bool backward, uint32_t window, int n_stages) {
     const TileShape t = fast_tile(nc, ec);
@@ -76,7 +80,7 @@ enum class Halo { kBothSides, kSheared };
 class PassPlanner {
   public:
     PassPlanner(const ncn_shape* sh, int first, int count, bool backward, Halo halo)
-        : nc_(sh->n_cache), ec_((int)(sh->E / sh->n_head)), groups_((uint32_t)(sh->N / sh->n_cache)), backward_(backward),
+        : nc_(sh->n_cache), ec_((int)(sh->E / sh->n_head)), heads_(sh->n_head), groups_((uint32_t)(sh->N / sh->n_cache)), backward_(backward),
           halo_(halo), s_(count) {
         const size_t state = nc_ == 2 ? pair_state_bytes(backward) : fused_state_bytes(backward);
         cap_rows_ = (uint32_t)(state / ((backward ? 4 : 2) * ec_ * sizeof(float)));
@@ -137,6 +141,7 @@ class PassPlanner {
             p.own = p.window;
             p.tiles_per_ring = 1;
             p.class_groups = s0 / rings;
+            if (!fits_launch(p)) return -1.0;
             return priced(writes_state, 1.0, 1.0, b - a, true);
         }
         p.closed = 0;
@@ -163,6 +168,7 @@ class PassPlanner {
             p.own = cap_ - 2 * p.halo;
             if (p.own * 4 < cap_ * 3) return -1.0;  // more than a third of the window would be redundant work
             p.tiles_per_ring = (p.ring + p.own - 1) / p.own;
+            if (!fits_launch(p)) return -1.0;
             const double redundancy = (double)cap_ / p.own;
             return priced(writes_state, redundancy, redundancy, b - a, false);
         }
@@ -170,12 +176,16 @@ class PassPlanner {
         p.tiles_per_ring = (p.ring + cap_ - p.halo - 1) / (cap_ - p.halo);
         p.own = (p.ring + p.tiles_per_ring - 1) / p.tiles_per_ring;   // windows of one size
         p.window = p.own + p.halo;
-        if (p.own * 3 < p.window) return -1.0;
+        if (p.own * 3 < p.window || !fits_launch(p)) return -1.0;
         const double per_ring = (double)p.tiles_per_ring / p.ring;
         return priced(writes_state, 1.0 + per_ring * p.halo, 1.0 + per_ring * (double)extra / (b - a), b - a, false);
     }
 
   private:
+    // the windows of one batch entry in a launch (backward workgroups walk over windows)
+    bool fits_launch(const FusedPass& p) const {
+        return backward_ || (int64_t)p.class_groups * p.tiles_per_ring * heads_ <= kFusedMaxGridFwd;
+    }
     // What a pass costs, in the time one array of the activations' size takes to cross HBM at copy speed.  Traffic: the
     // pass reads 4 (forward 2) arrays of its windows (window / own times the data) and writes as many of its
     // owned rows; a backward pass that hands no reconstructed inputs on writes the two gradients
@@ -194,7 +204,7 @@ class PassPlanner {
         return std::cbrt(traffic * traffic * traffic + issue * issue * issue) * (closed && backward_ ? 1.1 : 1.0);
     }
 
-    int nc_, ec_;
+    int nc_, ec_, heads_;
     uint32_t groups_, cap_rows_, cap_, groups_pow2_;
     bool backward_;
     Halo halo_;
@@ -312,20 +322,19 @@ int64_t fused_items(const ncn_shape* sh, const FusedPass& p) {
     return sh->batch * (int64_t)p.class_groups * p.tiles_per_ring * sh->n_head;
 }
 
-int fused_grid(const ncn_shape* sh, const FusedPass& p, bool backward, int row_cap) {
-    const int64_t items = fused_items(sh, p);
-    // the forward kernels take one window per workgroup and nothing else (the one for groups of four with lengths could loop)
-    if (!backward) return items <= INT_MAX ? (int)items : 0;
-    int64_t cap = kFusedMaxGridBwd;
-    {  // partial rows (grid / n_head) * stages must fit the row_cap rows of the dW scratch
-        const int64_t by_rows = (int64_t)row_cap / p.count * sh->n_head;
-        if (by_rows < cap) cap = by_rows;
-    }
-    int64_t g = items < cap ? items : cap;
-    g = g / sh->n_head * sh->n_head;
-    if (g < sh->n_head) g = sh->n_head;
-    return (int)g;
+int fused_backward_grid(const ncn_shape* sh, const FusedPass& p, int row_cap) {
+    const int64_t cap = std::min<int64_t>(kFusedMaxGridBwd, (int64_t)row_cap / p.count * sh->n_head);
+    const int64_t g = std::min(fused_items(sh, p), cap) / sh->n_head * sh->n_head;
+    return (int)std::max<int64_t>(g, sh->n_head);
 }
+
+namespace {
+
+const void* elements_at(const void* base, int dtype, int64_t at) {
+    return base ? static_cast<const char*>(base) + at * (dtype == NCN_F32 ? 4 : 2) : nullptr;
+}
+
+}  // namespace
 
 hipError_t launch_fused(Pass pass, FusedArgs& a, const ncn_shape* sh, const FusedPass& p, hipStream_t s, int row_cap,
                         bool headwise) {
@@ -342,7 +351,6 @@ hipError_t launch_fused(Pass pass, FusedArgs& a, const ncn_shape* sh, const Fuse
     a.tiles_per_ring = p.tiles_per_ring;
     a.closed = p.closed;
     a.class_groups = p.class_groups;
-    a.total_items = (uint32_t)fused_items(sh, p);
     if (p.closed) {
         a.window = p.window;
         for (int k = 0; k < p.count; ++k) a.sub_stride[k] = (int32_t)p.sub_stride[k];
@@ -356,11 +364,33 @@ hipError_t launch_fused(Pass pass, FusedArgs& a, const ncn_shape* sh, const Fuse
     }
     a.scale_dn = (float)std::pow((double)a.tab.m, (double)(nc * p.count));
     a.scale_up = (float)std::pow((double)a.tab.m, -(double)(nc * p.count));
-    const int grid = fused_grid(sh, p, backward, row_cap);
     const size_t lds = fused_lds_bytes(nc, ec, backward, a.window, p.count);
-    if (headwise) return launch_fused_headwise(pass, a, nc, ec, grid, lds, s);
-    if (a.ctx_len) return launch_fused_lengths(pass, a, nc, ec, grid, lds, s);
-    return launch_fused_shape<false, false, false>(pass, a, nc, ec, grid, lds, s);
+    auto launch = [&](const FusedArgs& args, int grid) {
+        if (headwise) return launch_fused_headwise(pass, args, nc, ec, grid, lds, s);
+        if (args.ctx_len) return launch_fused_lengths(pass, args, nc, ec, grid, lds, s);
+        return launch_fused_shape<false, false, false>(pass, args, nc, ec, grid, lds, s);
+    };
+    const int64_t items = fused_items(sh, p);
+    a.total_items = (uint32_t)items;
+    if (backward) return launch(a, fused_backward_grid(sh, p, row_cap));
+    // a workgroup for every window
+    if (items <= kFusedMaxGridFwd) return launch(a, (int)items);
+    const int64_t per_entry = items / sh->batch, entries = kFusedMaxGridFwd / per_entry;   // at least one: fits_launch
+    for (int64_t b = 0; b < sh->batch; b += entries) {
+        const int64_t at = b * sh->N * sh->E, n = std::min(entries, sh->batch - b) * per_entry;
+        FusedArgs part = a;
+        part.in0 = elements_at(a.in0, a.in_dtype, at);
+        part.in1 = elements_at(a.in1, a.in_dtype, at);
+        part.out0 = const_cast<void*>(elements_at(a.out0, a.out_dtype, at));
+        part.out1 = const_cast<void*>(elements_at(a.out1, a.out_dtype, at));
+        part.aux0 = a.aux0 ? a.aux0 + at : nullptr;
+        part.aux1 = a.aux1 ? a.aux1 + at : nullptr;
+        part.ctx_len = a.ctx_len ? a.ctx_len + b : nullptr;
+        part.total_items = (uint32_t)n;
+        const hipError_t err = launch(part, (int)n);
+        if (err != hipSuccess) return err;
+    }
+    return hipSuccess;
 }
 
 }  // namespace ncn

@@ -204,8 +204,9 @@ struct StackRange {
 std::vector<StackRange> plan_stack(const ncn_shape* sh, int first, int count, bool multi_stage, int max_range, int max_saves);
 // windows of a pass (== workgroups, when every workgroup takes one)
 int64_t fused_items(const ncn_shape* sh, const FusedPass& p);
-// row_cap: rows of the dW partial buffer a backward pass may fill (grid / n_head rows per stage)
-int fused_grid(const ncn_shape* sh, const FusedPass& p, bool backward, int row_cap = kMaxGridX);
+// workgroups of a backward pass.  row_cap: rows of the dW partial buffer it may fill (grid / n_head rows per stage)
+int fused_backward_grid(const ncn_shape* sh, const FusedPass& p, int row_cap);
+// row_cap: as above
 // headwise: `sh` is the layout of a call on heads of one feature (headwise_width(E) adjacent heads to a "head")
 hipError_t launch_fused(Pass pass, FusedArgs& a, const ncn_shape* sh, const FusedPass& p, hipStream_t s,
                         int row_cap = kMaxGridX, bool headwise = false);

@@ -291,6 +291,26 @@ def test_backward_with_the_smaller_workspace_loops_over_windows(M):
     assert O.rel_err(dW, ref[4]) < 1e-6
 
 
+@pytest.mark.parametrize("n", [2, 4])
+def test_more_windows_than_a_launch_holds(M, n):
+    """2^23 windows of 512 threads are more work-items than a launch takes: the call runs in several launches, with the bits of the
+    same call on parts of the batch."""
+    batch, N, E, L = (1 << 23) + 5, 4 * n, 8, 2
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x, xa = (torch.randn(batch, N, E, device="cuda", generator=g) for _ in range(2))
+    W = torch.randn(L, 2 * E, device="cuda", generator=g) * 0.3
+    lens = (torch.arange(batch, device="cuda") % (N + 1)).to(torch.int32)
+    for kw in ({}, {"ctx_len": lens}):
+        y, ya = M.forward_stages(x, xa, W, 0.9, 0, n, 1, 0, L, **kw)
+        r, ra = M.inverse_stages(y, ya, W, 0.9, 0, n, 1, 0, L, **kw)
+        for part in (slice(0, batch // 2), slice(batch // 2, None)):
+            pkw = {k: v[part] for k, v in kw.items()}
+            py, pya = M.forward_stages(x[part], xa[part], W, 0.9, 0, n, 1, 0, L, **pkw)
+            pr, pra = M.inverse_stages(py, pya, W, 0.9, 0, n, 1, 0, L, **pkw)
+            assert torch.equal(y[part], py) and torch.equal(ya[part], pya)
+            assert torch.equal(r[part], pr) and torch.equal(ra[part], pra)
+
+
 @pytest.mark.parametrize("case", [
     (3, 1024, 64, 2, 2, 0, 11),    # several multi-stage passes (halo and closed)
     (1, 256, 32, 1, 2, 0, 8),      # one pass covers the range

@@ -399,6 +399,17 @@ def test_multi_stage_plan_declines_ineligible_shapes(lib):
     assert [p[2] for p in fwd][-1] == 2 and len(fwd) <= 4
 
 
+@pytest.mark.parametrize("n", [2, 4])
+def test_forward_passes_have_windows_that_a_launch_holds(lib, n):
+    """A launch holds less than 2^32 work-items, 512 to a window: a batch entry with more windows has one launch per stage in the
+    forward (the backward's workgroups walk over windows).  More windows in all are no reason: launches split the batch."""
+    most = (2 ** 32 - 1) // 512
+    for heads, passes in ((most, 1), (most + 1, 0)):
+        shape = _shape(lib, 1, 4 * n, 8 * heads, heads, n)
+        assert len(_passes(lib, shape, 0, 2, False)) == passes and len(_passes(lib, shape, 0, 2, True)) == 1
+    assert len(_passes(lib, _shape(lib, most + 1, 4 * n, 8, 1, n), 0, 2, False)) == 1
+
+
 @pytest.mark.parametrize("dims", [(2, 1024, 128, 4, 4, 5), (1, 256, 32, 4, 2, 8), (2, 1020, 64, 2, 4, 3)])
 def test_stack_plan_takes_bounds_of_any_size(lib, dims):
     """max_range and max_saves up to the largest int bound no more than the number of stages does."""
