@@ -177,10 +177,15 @@ __device__ __forceinline__ void issue_tile(const void* base, int dtype, const in
         for (int rr = 0; rr < R; ++rr)
 #pragma unroll
             for (int k = 0; k < FPL / 4; ++k) {
-                typedef float Chunk __attribute__((ext_vector_type(4)));
-                const Chunk* const at = reinterpret_cast<const Chunk*>(static_cast<const float*>(base) + off[rr]) + k;
-                const Chunk t = STREAM ? __builtin_nontemporal_load(at) : *at;
-                v[rr][4 * k] = t.x; v[rr][4 * k + 1] = t.y; v[rr][4 * k + 2] = t.z; v[rr][4 * k + 3] = t.w;
+                const float* const at = static_cast<const float*>(base) + off[rr] + 4 * k;
+                if constexpr (STREAM) {
+                    typedef float Chunk __attribute__((ext_vector_type(4)));   // what the builtin takes
+                    const Chunk t = __builtin_nontemporal_load(reinterpret_cast<const Chunk*>(at));
+                    v[rr][4 * k] = t.x; v[rr][4 * k + 1] = t.y; v[rr][4 * k + 2] = t.z; v[rr][4 * k + 3] = t.w;
+                } else {   // a float4: as that vector type, the general builds on tiles of 4 x 8 take up to 64 registers more
+                    const float4 t = *reinterpret_cast<const float4*>(at);
+                    v[rr][4 * k] = t.x; v[rr][4 * k + 1] = t.y; v[rr][4 * k + 2] = t.z; v[rr][4 * k + 3] = t.w;
+                }
             }
     } else if (dtype == NCN_BF16) {
 #pragma unroll
