@@ -567,17 +567,21 @@ __device__ __forceinline__ int dtype_of(int from_args, int when_bf16) {
     return TYPES == kF32Types ? NCN_F32 : TYPES == kBf16Types ? when_bf16 : from_args;
 }
 
-// float32 launches on arrays of that many elements ask for their rows with the non-temporal hint, in tiles of 16 elements and more and
-// rows of whole cache lines (others share theirs with the next head's wave): what they read is not read again before it has
-// left the 256 MB memory-side cache, and without the hint it takes the place of what the launch before wrote.  On arrays of an eighth of
+// float32 launches on arrays of that many elements ask for their rows with the non-temporal hint, on tiles of 4 x 4 and heads of
+// 32, where every load instruction takes whole cache lines: what they read is not read again before it has left the 256 MB
+// memory-side cache, and without the hint it takes the place of what the launch before wrote.  On arrays of an eighth of
 // that cache and less the inputs still lie in it.  Launches, us, without : with, groups of 8 rows, heads of 32, x[b, 2048, 128]: b = 12
 // (12 MB an array) forward 14.3 : 14.5, backward 22.6 : 22.8; 20 (21 MB) 18.8 : 19.5, 32.1 : 33.1; 28 (29 MB) 26.8 : 26.7, 46.2 : 45.7; 40
 // (42 MB) 37.5 : 36.2, 60.1 : 58.8.  Training steps: 4 stages, b = 32 333 : 327, 64 606 : 568, 128 1128 : 1077; groups of 16, 3
-// stages, x[64, 4096, 128] 1280 : 1243; groups of 2, whose tiles are 2 x 4, 186 : 202.  bfloat16, whose rows of 64 bytes share lines:
-// x[128, 4096, 128], groups of 16, 3 stages 2453 : 2520.  Stores with the hint: b = 64 594 : 604.
+// stages, x[64, 4096, 128] 1280 : 1243.  bfloat16, whose rows of 64 bytes share lines: x[128, 4096, 128], groups of 16, 3 stages 2453 : 2520.
+// Stores with the hint: b = 64 594 : 604.
+//   Lanes with eight features come back to every line with their second load, and narrower heads share theirs with the next head's wave.
+// Heads of 64, x[b, 2048, 256], 3 stages without gradients and trained, b = 16, 32, 64: groups of two 71 : 85, 132 : 147, 294 : 332 and 209 : 223,
+// 400 : 390, 760 : 802; of four 71 : 83, 137 : 145, 304 : 347 and 219 : 227, -, 772 : 833; of eight 97 : 100, 165 : 172, 328 : 315 and 282 :
+// 276, 497 : 484, 916 : 890, behind tables 272 : 280, -, 880 : 902, inverse 95 : 101, 160 : 173, 298 : 309.  Tiles of 2 x 4: 186 : 202.
 constexpr int64_t kStreamElements = 1 << 23;
 #define NCN_REQUEST(STREAM, ...)                                                                \
-    if (TYPES == kF32Types && EC % 32 == 0 && R * F >= 16 && A.plane >= kStreamElements) {      \
+    if (TYPES == kF32Types && EC == 32 && R == 4 && F == 4 && A.plane >= kStreamElements) {         \
         constexpr bool STREAM = true;                                                           \
         asm volatile("");   /* the two sides are not alike, or the compiler makes one of them and drops the hint */ \
         __VA_ARGS__                                                                             \

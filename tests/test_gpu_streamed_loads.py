@@ -1,4 +1,4 @@
-"""float32 one-stage launches on arrays of 2^23 elements and more load their rows with a cache hint: the same bits as the halves of
+"""float32 one-stage launches of heads of 32 on arrays of 2^23 elements and more load their rows with a cache hint: the same bits as the halves of
 the batch, which are below that size, in every direction, with plain and gathered groups and with rows past a length."""
 import pytest
 import torch
@@ -22,8 +22,8 @@ def inputs(b, N, E, n):
     return x, xa, dy, dya, torch.randn(1, 2 * E, device="cuda", generator=gen) * (0.3 / n ** 0.5)
 
 
-# at the size itself and beyond; tiles of 4 x 4 and 4 x 8, groups of 8 to 32 rows
-@pytest.mark.parametrize("b,N,E,C,n", [(32, 2048, 128, 4, 8), (34, 2048, 128, 4, 16), (16, 2080, 256, 2, 16), (16, 2080, 256, 4, 32), (16, 2056, 256, 4, 8)])
+# at the size itself and beyond, groups of 8 to 32 rows with the hint; tiles of 4 x 8 without
+@pytest.mark.parametrize("b,N,E,C,n", [(32, 2048, 128, 4, 8), (34, 2048, 128, 4, 16), (32, 2080, 128, 4, 32), (16, 2080, 256, 2, 16), (16, 2080, 256, 4, 32), (16, 2056, 256, 4, 8)])
 def test_halves_of_the_batch(M, b, N, E, C, n):
     x, xa, dy, dya, W = inputs(b, N, E, n)
     assert x.numel() >= 1 << 23 > x.numel() // 2
