@@ -331,9 +331,12 @@ __device__ __forceinline__ void backward_core(float (&Y)[R][F], float (&B)[R][F]
             float xj[F], c[R], rh[R];
             row_lane_broadcast<T::LF, T::LR, F>(Y[jr], xj, jo, lane, slots);
             row_sums<T::LF, R, F, ROWS>(Y, wi, dot_chain<F>(xj, wj), c);
-            // exp2 and reciprocals a few rows at a time (all rows' r at once would not fit the registers), each time at high
-            // priority, and what is made of them at low: see issue_first
-            constexpr int RC = F <= 4 && R % 2 == 0 ? 2 : 1;
+            // exp2 and reciprocals a row at a time (all rows' r at once would not fit the registers), each time at high priority, and
+            // what is made of them at low: see issue_first.  Two rows where the whole group is in the lane; over several row lanes two
+            // make the one-stage builds spill up to 7 registers.  us, two rows : one, x[32, 4096, 128], groups of 8 float32 117 : 112,
+            // bfloat16 102 : 93, mixed 110 : 102, of 16 158 : 161, 150 : 146, 151 : 145; whole groups in a lane, x[64, 4096, 128],
+            // groups of two, 10 stages 563 : 579, x[64, 2048, 128] bfloat16, groups of four, 6 stages 478 : 482.
+            constexpr int RC = T::LR == 1 && F <= 4 && R % 2 == 0 ? 2 : 1;
             if constexpr (!TANH_ONLY) issue_with_others();
             if constexpr (T::LR == 1) {
                 // The whole group is in this lane: the pivot row's share sum_i c_i U_i goes straight into its gradient

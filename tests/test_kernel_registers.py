@@ -70,3 +70,9 @@ def test_forward_on_wide_tiles_runs_three_waves(kernels):
     three waves per SIMD (one build for heads of one feature has always had two more)."""
     _at_most(kernels, r"stage_(forward|inverse)_kernel<\d+,\d+,4,8,\w+,\w+,-?\d>", 168, 0, 96)
     _at_most(kernels, r"headwise_forward_kernel<64,32,4,8,\w+,\w+,\w+>", 170, 0, 8)
+
+
+def test_one_stage_backward_does_not_spill(kernels):
+    """The backward builds on tiles of 4 x 4 with a wave for every tile, all types."""
+    _at_most(kernels, r"stage_backward_kernel<\d+,\d+,4,4,true,false,false,(-1|0|1)>", 128, 0, 45)
+    _at_most(kernels, r"stage_backward_kernel<\d+,\d+,4,4,true,true,false,(-1|0|1)>", 128, 1, 45)
