@@ -17,9 +17,9 @@ hipError_t launch_fused_build(Pass pass, const FusedArgs& a, int grid, size_t ld
     const bool backward = pass == kBackward;
     const bool tanh_only = a.tab.activation == NCN_ACT_TANH;
     hipError_t err;
+    if (!backward && (uint32_t)grid != a.total_items) return hipErrorInvalidConfiguration;   // the forward kernels take one window each
     if constexpr (NC == 2 && !RADIX) {
         static_assert(t.r == 2, "the two-row kernels keep both rows of a group in one lane");
-        if (!backward && (uint32_t)grid != a.total_items) return hipErrorInvalidConfiguration;   // one window each
         if (backward) {
             // a workgroup per window when the dW scratch has the rows for it, else workgroups that loop over windows
             const bool loop = (uint32_t)grid < a.total_items;
@@ -59,7 +59,6 @@ hipError_t launch_fused_build(Pass pass, const FusedArgs& a, int grid, size_t ld
                                      : launch(quad_backward_kernel<EC, true, false, HEADWISE>, kQuadWavesBwd))
                              : (loop ? launch(quad_backward_kernel<EC, false, true, HEADWISE>, kQuadWavesBwd)
                                      : launch(quad_backward_kernel<EC, false, false, HEADWISE>, kQuadWavesBwd));
-        if (loop) return hipErrorInvalidConfiguration;   // one window each
         if (pass == kInverse)
             return tanh_only ? launch(quad_forward_kernel<EC, true, true, HEADWISE>, kQuadWavesFwd)
                              : launch(quad_forward_kernel<EC, false, true, HEADWISE>, kQuadWavesFwd);

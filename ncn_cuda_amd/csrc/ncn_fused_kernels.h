@@ -282,8 +282,7 @@ __device__ __forceinline__ void lds_store_frag(float* row, const float (&v)[F]) 
 }
 
 // Window rows on their way from global memory to LDS: 4 features per thread and trip, kept as raw bits so that
-// nothing waits for the loads until fused_commit_rows turns them into floats.  A workgroup fetches the window of
-// its next item while it computes the current one.
+// nothing waits for the loads until fused_commit_rows turns them into floats.
 template <int NC, int EC, int NW, int K, bool RADIX>
 __device__ __forceinline__ void fused_window_offsets(const FusedArgs& A, const FusedItem& it, uint32_t rows,
                                                      int64_t (&off)[K]) {
@@ -384,6 +383,8 @@ __device__ __forceinline__ void fused_load_weights(const FusedArgs& A, int head,
 // past the length stay in LDS as they came (a row may be live in one stage of the pass and past the length in another).
 // HEADWISE: heads of one feature laid out as heads of EC adjacent ones (ncn_headwise_kernels.h): the same windows, tiles
 // and weights, the step code without sums across a row's lanes.
+// One window per workgroup: a loop that fetches the next window ahead holds its rows in registers through all stages, 105 to 160 of
+// them where 49 to 98 do, and a CU then holds one workgroup of 8 waves in place of two.
 template <int NC, int EC, int R, int F, bool TANH_ONLY, bool RADIX = false, bool INVERSE = false, bool LENGTHS = false,
           bool HEADWISE = false>
 __global__ void __launch_bounds__(64 * kFusedWavesFwd) fused_forward_kernel(const FusedArgs A) {
@@ -399,73 +400,64 @@ __global__ void __launch_bounds__(64 * kFusedWavesFwd) fused_forward_kernel(cons
     float* as = lds + rows * EC;
     float* w_lds = as + rows * EC;                              // [kFusedMaxStages][2][EC]
     float4* slots = reinterpret_cast<float4*>(w_lds + kFusedMaxStages * 2 * EC) + wave * (F / 4) * 64;
-    const uint32_t item0 = gridDim.x == A.total_items ? fused_deal<EC>(A, blockIdx.x) : blockIdx.x;
-    fused_load_weights<EC, NW>(A, item0 % A.n_head, w_lds);   // every item of this workgroup has this head
-
-    // trips of 64 * NW threads over the float4 chunks of the largest window the LDS budget allows
-    constexpr int K = (int)((kFusedStateBytesFwd / 2 / sizeof(float4) + 64 * NW - 1) / (64 * NW));
-    uint4 rx[K], ra[K];
-    if (item0 < A.total_items) {
+    const uint32_t item = fused_deal<EC>(A, blockIdx.x);   // the launch has a workgroup for every window
+    if (item >= A.total_items) return;
+    const FusedItem it = fused_item<NC, EC, RADIX>(A, item);
+    fused_load_weights<EC, NW>(A, it.head, w_lds);
+    {
+        // trips of 64 * NW threads over the float4 chunks of the largest window the LDS budget allows
+        constexpr int K = (int)((kFusedStateBytesFwd / 2 / sizeof(float4) + 64 * NW - 1) / (64 * NW));
+        uint4 rx[K], ra[K];
         int64_t off[K];
-        fused_window_offsets<NC, EC, NW, K, RADIX>(A, fused_item<NC, EC, RADIX>(A, item0), rows, off);
+        fused_window_offsets<NC, EC, NW, K, RADIX>(A, it, rows, off);
         fused_fetch_rows<K>(A.in0, A.in_dtype, off, rx);
         fused_fetch_rows<K>(A.in1, A.in_dtype, off, ra);
-    }
-    for (uint32_t item = item0; item < A.total_items; item += gridDim.x) {
-        const FusedItem it = fused_item<NC, EC, RADIX>(A, item);
-        const int32_t len = LENGTHS ? max(0, min(A.ctx_len[it.batch], (int32_t)A.N)) : 0;
         fused_commit_rows<NC, EC, NW, K>(rx, A.in_dtype, xs, rows, A.tab.kappa);
         fused_commit_rows<NC, EC, NW, K>(ra, A.in_dtype, as, rows, INVERSE ? A.tab.b_scale : A.tab.a_scale);
-        __syncthreads();
-        if (item + gridDim.x < A.total_items) {   // the next window travels while this one is computed
-            int64_t off[K];
-            fused_window_offsets<NC, EC, NW, K, RADIX>(A, fused_item<NC, EC, RADIX>(A, item + gridDim.x), rows, off);
-            fused_fetch_rows<K>(A.in0, A.in_dtype, off, rx);
-            fused_fetch_rows<K>(A.in1, A.in_dtype, off, ra);
-        }
-        for (int sq = 0; sq < A.n_stages; ++sq) {
-            const int st = INVERSE ? A.n_stages - 1 - sq : sq;
-            const int ss = A.sub_stride[st];
-            const StageGroups here = stage_groups<NC>(A, ss);
-            float wi[F], wj[F];
-            lds_load_frag<F>(w_lds + st * 2 * EC + fl * F, wi);
-            lds_load_frag<F>(w_lds + st * 2 * EC + EC + fl * F, wj);
-            for (uint32_t wt = wave; wt * T::GPW < here.count; wt += NW) {
-                const uint32_t qg = here.first + wt * T::GPW + gw;
-                const bool valid = qg - here.first < here.count;
-                float x[R][F], a[R][F];
-                uint32_t row[R];
+    }
+    const int32_t len = LENGTHS ? max(0, min(A.ctx_len[it.batch], (int32_t)A.N)) : 0;
+    __syncthreads();
+    for (int sq = 0; sq < A.n_stages; ++sq) {
+        const int st = INVERSE ? A.n_stages - 1 - sq : sq;
+        const int ss = A.sub_stride[st];
+        const StageGroups here = stage_groups<NC>(A, ss);
+        float wi[F], wj[F];
+        lds_load_frag<F>(w_lds + st * 2 * EC + fl * F, wi);
+        lds_load_frag<F>(w_lds + st * 2 * EC + EC + fl * F, wj);
+        for (uint32_t wt = wave; wt * T::GPW < here.count; wt += NW) {
+            const uint32_t qg = here.first + wt * T::GPW + gw;
+            const bool valid = qg - here.first < here.count;
+            float x[R][F], a[R][F];
+            uint32_t row[R];
+#pragma unroll
+            for (int rr = 0; rr < R; ++rr) {
+                row[rr] = fused_lds_row<NC, RADIX>(A, valid ? qg : here.first, rl * R + rr, ss) * EC + fl * F;
+                lds_load_frag<F>(xs + row[rr], x[rr]);
+                lds_load_frag<F>(as + row[rr], a[rr]);
+            }
+            const int live = !LENGTHS ? NC : valid ? fused_live_rows<NC>(A, it, qg, len) : 0;
+            if constexpr (HEADWISE) {
+                if (INVERSE) headwise_inverse_core<NC, EC, R, F, TANH_ONLY, LENGTHS, true>(x, a, wi, wj, A.tab, lane, slots, live);
+                else headwise_forward_core<NC, EC, R, F, TANH_ONLY, LENGTHS, true>(x, a, wi, wj, A.tab, lane, slots, live);
+            } else {
+                if (INVERSE) inverse_core<NC, EC, R, F, TANH_ONLY, LENGTHS, true>(x, a, wi, wj, A.tab, lane, slots, live);
+                else forward_core<NC, EC, R, F, TANH_ONLY, LENGTHS, true>(x, a, wi, wj, A.tab, lane, slots, live);
+            }
+            if (valid) {
 #pragma unroll
                 for (int rr = 0; rr < R; ++rr) {
-                    row[rr] = fused_lds_row<NC, RADIX>(A, valid ? qg : here.first, rl * R + rr, ss) * EC + fl * F;
-                    lds_load_frag<F>(xs + row[rr], x[rr]);
-                    lds_load_frag<F>(as + row[rr], a[rr]);
-                }
-                const int live = !LENGTHS ? NC : valid ? fused_live_rows<NC>(A, it, qg, len) : 0;
-                if constexpr (HEADWISE) {
-                    if (INVERSE) headwise_inverse_core<NC, EC, R, F, TANH_ONLY, LENGTHS, true>(x, a, wi, wj, A.tab, lane, slots, live);
-                    else headwise_forward_core<NC, EC, R, F, TANH_ONLY, LENGTHS, true>(x, a, wi, wj, A.tab, lane, slots, live);
-                } else {
-                    if (INVERSE) inverse_core<NC, EC, R, F, TANH_ONLY, LENGTHS, true>(x, a, wi, wj, A.tab, lane, slots, live);
-                    else forward_core<NC, EC, R, F, TANH_ONLY, LENGTHS, true>(x, a, wi, wj, A.tab, lane, slots, live);
-                }
-                if (valid) {
-#pragma unroll
-                    for (int rr = 0; rr < R; ++rr) {
-                        if (LENGTHS && rl * R + rr >= live) continue;
-                        lds_store_frag<F>(xs + row[rr], x[rr]);
-                        lds_store_frag<F>(as + row[rr], a[rr]);
-                    }
+                    if (LENGTHS && rl * R + rr >= live) continue;
+                    lds_store_frag<F>(xs + row[rr], x[rr]);
+                    lds_store_frag<F>(as + row[rr], a[rr]);
                 }
             }
-            __syncthreads();
         }
-        // out of the scaled form
-        fused_store_rows_scaled<NC, EC, NW, RADIX>(A, it, xs, A.tab.inv_kappa, A.out0, A.out_dtype, A.aux0);
-        fused_store_rows_scaled<NC, EC, NW, RADIX>(A, it, as, INVERSE ? A.tab.inv_b_scale : A.tab.inv_a_scale, A.out1,
-                                                   A.out_dtype, A.aux1);
         __syncthreads();
     }
+    // out of the scaled form
+    fused_store_rows_scaled<NC, EC, NW, RADIX>(A, it, xs, A.tab.inv_kappa, A.out0, A.out_dtype, A.aux0);
+    fused_store_rows_scaled<NC, EC, NW, RADIX>(A, it, as, INVERSE ? A.tab.inv_b_scale : A.tab.inv_a_scale, A.out1,
+                                               A.out_dtype, A.aux1);
 }
 
 template <int NC, int EC, int R, int F, bool TANH_ONLY, bool RADIX = false, bool LENGTHS = false, bool HEADWISE = false>

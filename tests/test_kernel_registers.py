@@ -76,3 +76,8 @@ def test_one_stage_backward_does_not_spill(kernels):
     """The backward builds on tiles of 4 x 4 with a wave for every tile, all types."""
     _at_most(kernels, r"stage_backward_kernel<\d+,\d+,4,4,true,false,false,(-1|0|1)>", 128, 0, 45)
     _at_most(kernels, r"stage_backward_kernel<\d+,\d+,4,4,true,true,false,(-1|0|1)>", 128, 1, 45)
+
+
+def test_forward_windows_in_lds_run_two_workgroups(kernels):
+    """Workgroups of 8 waves: 128 VGPRs are two to a CU."""
+    _at_most(kernels, r"fused_forward_kernel<.*>", 128, 0, 96)
