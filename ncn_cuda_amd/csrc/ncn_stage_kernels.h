@@ -729,8 +729,12 @@ __global__ void __launch_bounds__(kBlockThreads, (TANH_ONLY && R * F <= 16 && F 
         int64_t off[R];
         const int live = tile_offsets<NC, EC, R, F, INDEXED>(A, t, lane, head, off);
         float Y[R][F], B[R][F], G[R][F], H[R][F];
-        NCN_REQUEST(STREAM, issue_tile<R, F, STREAM>(A.in0, in_dtype, off, Y, A.plane); issue_tile<R, F, STREAM>(A.in1, in_dtype, off, B, A.plane);
-                    issue_tile<R, F, STREAM>(A.g0, g_dtype, off, G); if (A.g1) issue_tile<R, F, STREAM>(A.g1, g_dtype, off, H);)
+        constexpr bool VECTOR = F > 4;
+        NCN_REQUEST(STREAM,
+                    issue_tile<R, F, STREAM, STREAM || VECTOR>(A.in0, in_dtype, off, Y, A.plane);
+                    issue_tile<R, F, STREAM, STREAM || VECTOR>(A.in1, in_dtype, off, B, A.plane);
+                    issue_tile<R, F, STREAM, STREAM || VECTOR>(A.g0, g_dtype, off, G);
+                    if (A.g1) issue_tile<R, F, STREAM, STREAM || VECTOR>(A.g1, g_dtype, off, H);)
         if (!A.g1) {
 #pragma unroll
             for (int rr = 0; rr < R; ++rr)
