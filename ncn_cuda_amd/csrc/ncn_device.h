@@ -266,17 +266,24 @@ __device__ __forceinline__ void store_elem(void* base, int dtype, int64_t off, f
 // (with the sums across lanes all on DPP operands; with ds_swizzle for strides of 4 and more, which paid before, 64.6).
 // Launches overlap that with their memory traffic in part: training steps, us, of x[128, 4096, 128] bfloat16, groups of 16, 3 stages
 // 2632 -> 2433; of x[128, 8192, 128], groups of 2, 13 stages 3670 -> 3445; of x[64, 2048, 128] bfloat16, groups of 4, 6 stages 537 -> 470;
-// inference of x[16, 4096, 128] bfloat16, groups of 16, 3 stages 128 -> 113.
+// inference of x[16, 4096, 128] bfloat16, groups of 16, 3 stages 128 -> 113.  Forward and inverse with other activations (no batch of
+// exp2, and the compiler does not schedule across the two functions) leave both out, which call sites say with ON.
 // ---------------------------------------------------------------------------------------------
+template <bool ON = true>
 __device__ __forceinline__ void issue_first() {
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_setprio(3);
-    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (ON) {
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_setprio(3);
+        __builtin_amdgcn_sched_barrier(0);
+    }
 }
+template <bool ON = true>
 __device__ __forceinline__ void issue_with_others() {
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_setprio(0);
-    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (ON) {
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_setprio(0);
+        __builtin_amdgcn_sched_barrier(0);
+    }
 }
 
 // A constant of the launch that most instructions of a stretch would read from a scalar register: only every other instruction of

@@ -41,7 +41,7 @@ __device__ __forceinline__ void headwise_forward_core(float (&x)[R][F], float (&
                                                       const float (&wj)[F], const StepTable& S, int lane, float4* slots,
                                                       int live = NC) {
     using T = Tile<NC, EC, R, F>;
-    const float m = in_vector_register(S.m);
+    const float m = TANH_ONLY ? in_vector_register(S.m) : S.m;
 #pragma unroll 1
     for (int jo = 0; jo < T::LR; ++jo) {
 #pragma unroll
@@ -82,7 +82,7 @@ __device__ __forceinline__ void headwise_inverse_core(float (&y)[R][F], float (&
                                                       const float (&wj)[F], const StepTable& S, int lane, float4* slots,
                                                       int live = NC) {
     using T = Tile<NC, EC, R, F>;
-    const float im = in_vector_register(S.im);
+    const float im = TANH_ONLY ? in_vector_register(S.im) : S.im;
 #pragma unroll 1
     for (int jo = T::LR - 1; jo >= 0; --jo) {
 #pragma unroll

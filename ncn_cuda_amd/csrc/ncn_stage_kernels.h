@@ -143,8 +143,8 @@ __device__ __forceinline__ void act_Fw(float z, int code, float& Fv, float& w) {
 }
 
 // The row sums c_i = <xs_i, Wi'> + <xs_j, Wj'> of a lane's R rows: a chain of FMAs per row that starts from the lane's
-// share e of <xs_j, Wj'>, then all R sums cross the LF lanes of a row together.  Leaves the wave at high priority.
-template <int LF, int R, int F, bool ROWS>
+// share e of <xs_j, Wj'>, then all R sums cross the LF lanes of a row together.  PRIORITY: leaves the wave at high priority.
+template <int LF, int R, int F, bool ROWS, bool PRIORITY>
 __device__ __forceinline__ void row_sums(const float (&x)[R][F], const float (&wi)[F], float e, float (&c)[R]) {
 #pragma unroll
     for (int rr = 0; rr < R; ++rr) {
@@ -152,7 +152,7 @@ __device__ __forceinline__ void row_sums(const float (&x)[R][F], const float (&w
 #pragma unroll
         for (int f = 0; f < F; ++f) c[rr] = fmaf(x[rr][f], wi[f], c[rr]);
     }
-    issue_first();
+    issue_first<PRIORITY>();
     lane_sum_n<1, LF, ROWS, R>(c);
 }
 
@@ -189,7 +189,9 @@ __device__ __forceinline__ void forward_core(float (&x)[R][F], float (&a)[R][F],
                                              const float (&wj)[F], const StepTable& S, int lane, float4* slots,
                                              int live = NC) {
     using T = Tile<NC, EC, R, F>;
-    const float m = in_vector_register(S.m);   // read twice per element and step
+    // read twice per element and step; with other activations the register is dearer (headwise inverse, relu, behind a table, x[24, 4096, 256],
+    // groups of 16: five waves per SIMD instead of four, 183 us : 207)
+    const float m = TANH_ONLY ? in_vector_register(S.m) : S.m;
 #pragma unroll 1
     for (int jo = 0; jo < T::LR; ++jo) {
 #pragma unroll
@@ -197,7 +199,7 @@ __device__ __forceinline__ void forward_core(float (&x)[R][F], float (&a)[R][F],
             if (STEP_MASK && jo * R + jr >= live) continue;  // the lanes of a group agree: no lane it needs is off
             float xj[F], c[R];
             row_lane_broadcast<T::LF, T::LR, F>(x[jr], xj, jo, lane, slots);
-            row_sums<T::LF, R, F, ROWS>(x, wi, dot_chain<F>(xj, wj), c);
+            row_sums<T::LF, R, F, ROWS, TANH_ONLY>(x, wi, dot_chain<F>(xj, wj), c);
             if constexpr (TANH_ONLY) {
                 float r[R][F];
                 sigmoids(0, x, c, xj, r);
@@ -210,7 +212,6 @@ __device__ __forceinline__ void forward_core(float (&x)[R][F], float (&a)[R][F],
                         x[rr][f] = fmaf(m, x[rr][f], a[rr][f]);
                     }
             } else {
-                issue_with_others();
 #pragma unroll
                 for (int rr = 0; rr < R; ++rr) {
 #pragma unroll
@@ -238,7 +239,7 @@ __device__ __forceinline__ void inverse_core(float (&y)[R][F], float (&b)[R][F],
                                              const float (&wj)[F], const StepTable& S, int lane, float4* slots,
                                              int live = NC) {
     using T = Tile<NC, EC, R, F>;
-    const float im = in_vector_register(S.im);   // read twice per element and step
+    const float im = TANH_ONLY ? in_vector_register(S.im) : S.im;   // read twice per element and step
 #pragma unroll 1
     for (int jo = T::LR - 1; jo >= 0; --jo) {
 #pragma unroll
@@ -250,7 +251,7 @@ __device__ __forceinline__ void inverse_core(float (&y)[R][F], float (&b)[R][F],
                 for (int f = 0; f < F; ++f) y[rr][f] = fmaf(im, y[rr][f], -b[rr][f]);
             float xj[F], c[R];
             row_lane_broadcast<T::LF, T::LR, F>(y[jr], xj, jo, lane, slots);
-            row_sums<T::LF, R, F, ROWS>(y, wi, dot_chain<F>(xj, wj), c);
+            row_sums<T::LF, R, F, ROWS, TANH_ONLY>(y, wi, dot_chain<F>(xj, wj), c);
             if constexpr (TANH_ONLY) {
                 float r[R][F];
                 sigmoids(0, y, c, xj, r);
@@ -260,7 +261,6 @@ __device__ __forceinline__ void inverse_core(float (&y)[R][F], float (&b)[R][F],
 #pragma unroll
                     for (int f = 0; f < F; ++f) b[rr][f] = fmaf(S.bk1, r[rr][f], fmaf(im, b[rr][f], S.bk0));
             } else {
-                issue_with_others();
 #pragma unroll
                 for (int rr = 0; rr < R; ++rr) {
 #pragma unroll
@@ -330,7 +330,7 @@ __device__ __forceinline__ void backward_core(float (&Y)[R][F], float (&B)[R][F]
                 for (int f = 0; f < F; ++f) Y[rr][f] = fmaf(S.im, Y[rr][f], -B[rr][f]);  // xs before this step
             float xj[F], c[R], rh[R];
             row_lane_broadcast<T::LF, T::LR, F>(Y[jr], xj, jo, lane, slots);
-            row_sums<T::LF, R, F, ROWS>(Y, wi, dot_chain<F>(xj, wj), c);
+            row_sums<T::LF, R, F, ROWS, true>(Y, wi, dot_chain<F>(xj, wj), c);
             // exp2 and reciprocals a row at a time (all rows' r at once would not fit the registers), each time at high priority, and
             // what is made of them at low: see issue_first.  Two rows where the whole group is in the lane; over several row lanes two
             // make the one-stage builds spill up to 7 registers.  us, two rows : one, x[32, 4096, 128], groups of 8 float32 117 : 112,

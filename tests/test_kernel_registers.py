@@ -81,3 +81,10 @@ def test_one_stage_backward_does_not_spill(kernels):
 def test_forward_windows_in_lds_run_two_workgroups(kernels):
     """Workgroups of 8 waves: 128 VGPRs are two to a CU."""
     _at_most(kernels, r"fused_forward_kernel<.*>", 128, 0, 96)
+
+
+def test_other_activations_keep_their_waves(kernels):
+    """Inverse builds for activations other than tanh on heads of one feature and tiles of 4 x 4, plain and gathered: five
+    waves per SIMD (one build has always had one register more)."""
+    _at_most(kernels, r"headwise_forward_kernel<\d+,\d+,4,4,false,true,\w+>", 97, 0, 20)
+    _at_most(kernels, r"headwise_forward_kernel<\d+,\d+,4,4,false,true,true>", 96, 0, 10)
