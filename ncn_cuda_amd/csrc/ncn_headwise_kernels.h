@@ -152,10 +152,14 @@ __device__ __forceinline__ void headwise_backward_core(float (&Y)[R][F], float (
                 // The whole group is in this lane: every row's share of the pivot row's gradient,
                 // ku (rh_if Wj'_f + c_if U_if) = ku U_if (xs_jf Wj'_f + c_if), goes straight into it, and dWj takes the
                 // row's rh_if as dWi does (no sums to carry through the step: fewer registers).
+                // exp2 at high priority, of a row at a time, not on groups of two rows: there it spills 6 to 8 registers, 66 in the looping
+                // build with lengths.  us, with : without, heads of one feature, groups of two, x[80, 8192, 128] looping over windows 2212 : 2096,
+                // with lengths 2481 : 1946, x[32, 4096, 128], 10 stages 367 : 361; groups of four, x[64, 2048, 128], 6 stages 548 : 572.
+                constexpr bool kBatch = R > 2;
 #pragma unroll
                 for (int r0 = 0; r0 < R; r0 += RC) {
                     float r[RC][F];
-                    if constexpr (TANH_ONLY) headwise_sigmoids(r0, Y, wi, cj, xj, r);
+                    if constexpr (TANH_ONLY && kBatch) headwise_sigmoids(r0, Y, wi, cj, xj, r);
 #pragma unroll
                     for (int k = 0; k < RC; ++k) {
                         const int rr = r0 + k;
@@ -164,6 +168,7 @@ __device__ __forceinline__ void headwise_backward_core(float (&Y)[R][F], float (
                             const float c = fmaf(Y[rr][f], wi[f], cj[f]);
                             float w;
                             if constexpr (TANH_ONLY) {
+                                if constexpr (!kBatch) r[k][f] = __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(fmaf(c, xj[f], Y[rr][f])) + 1.0f);
                                 B[rr][f] = fmaf(S.bk1, r[k][f], fmaf(S.im, B[rr][f], S.bk0));   // bh before this step
                                 w = fmaf(-r[k][f], r[k][f], r[k][f]);
                             } else {

@@ -88,3 +88,8 @@ def test_other_activations_keep_their_waves(kernels):
     waves per SIMD (one build has always had one register more)."""
     _at_most(kernels, r"headwise_forward_kernel<\d+,\d+,4,4,false,true,\w+>", 97, 0, 20)
     _at_most(kernels, r"headwise_forward_kernel<\d+,\d+,4,4,false,true,true>", 96, 0, 10)
+
+def test_backward_on_groups_of_two_heads_of_one_feature(kernels):
+    """With a window for every workgroup (four registers have always spilled at heads laid out in eights), and looping over windows."""
+    _at_most(kernels, r"pair_backward_kernel<\d+,true,\w+,false,true>", 128, 4, 6)
+    _at_most(kernels, r"pair_backward_kernel<\d+,true,\w+,true,true>", 128, 18, 6)
