@@ -310,6 +310,9 @@ __device__ __forceinline__ void backward_core(float (&Y)[R][F], float (&B)[R][F]
                                               float (&dwj)[F], float own, const StepTable& S, int step_base, int lane,
                                               float4* slots, int live = NC) {
     using T = Tile<NC, EC, R, F>;
+    // Rows of 16 features over two lanes (a radix pass on groups of two) have one instruction across lanes in a sum and no register to
+    // spare: with priorities 25 spill in place of 5 (x[64, 4096, 128], 12 levels backward 692 us : 664).
+    constexpr bool kPriority = !(T::LR == 1 && T::LF == 2 && F == 8);
     const int rl = (lane / T::LF) % T::LR;
     float wiku[KU_W ? F : 1];   // ku Wi': G += rh (ku Wi') spares the product ku rh of every row and step
     if constexpr (KU_W) {
@@ -330,14 +333,14 @@ __device__ __forceinline__ void backward_core(float (&Y)[R][F], float (&B)[R][F]
                 for (int f = 0; f < F; ++f) Y[rr][f] = fmaf(S.im, Y[rr][f], -B[rr][f]);  // xs before this step
             float xj[F], c[R], rh[R];
             row_lane_broadcast<T::LF, T::LR, F>(Y[jr], xj, jo, lane, slots);
-            row_sums<T::LF, R, F, ROWS, true>(Y, wi, dot_chain<F>(xj, wj), c);
+            row_sums<T::LF, R, F, ROWS, kPriority>(Y, wi, dot_chain<F>(xj, wj), c);
             // exp2 and reciprocals a row at a time (all rows' r at once would not fit the registers), each time at high priority, and
             // what is made of them at low: see issue_first.  Two rows where the whole group is in the lane; over several row lanes two
             // make the one-stage builds spill up to 7 registers.  us, two rows : one, x[32, 4096, 128], groups of 8 float32 117 : 112,
             // bfloat16 102 : 93, mixed 110 : 102, of 16 158 : 161, 150 : 146, 151 : 145; whole groups in a lane, x[64, 4096, 128],
             // groups of two, 10 stages 563 : 579, x[64, 2048, 128] bfloat16, groups of four, 6 stages 478 : 482.
             constexpr int RC = T::LR == 1 && F <= 4 && R % 2 == 0 ? 2 : 1;
-            if constexpr (!TANH_ONLY) issue_with_others();
+            if constexpr (!TANH_ONLY) issue_with_others<kPriority>();
             if constexpr (T::LR == 1) {
                 // The whole group is in this lane: the pivot row's share sum_i c_i U_i goes straight into its gradient
                 // (no sum across lanes to wait for), with the pivot's own two terms merged into one coefficient.
@@ -345,9 +348,9 @@ __device__ __forceinline__ void backward_core(float (&Y)[R][F], float (&B)[R][F]
                 for (int r0 = 0; r0 < R; r0 += RC) {
                     float r[RC][F];
                     if constexpr (TANH_ONLY) {
-                        if (r0 > 0) issue_first();
+                        if (r0 > 0) issue_first<kPriority>();
                         sigmoids(r0, Y, c, xj, r);
-                        issue_with_others();
+                        issue_with_others<kPriority>();
                     }
 #pragma unroll
                     for (int k = 0; k < RC; ++k) {
@@ -372,9 +375,9 @@ __device__ __forceinline__ void backward_core(float (&Y)[R][F], float (&B)[R][F]
                         }
                     }
                 }
-                issue_first();
+                issue_first<kPriority>();
                 lane_sum_n<1, T::LF, ROWS, R>(rh);
-                issue_with_others();
+                issue_with_others<kPriority>();
                 float rhosum = 0.f;
 #pragma unroll
                 for (int rr = 0; rr < R; ++rr) {

@@ -93,3 +93,6 @@ def test_backward_on_groups_of_two_heads_of_one_feature(kernels):
     """With a window for every workgroup (four registers have always spilled at heads laid out in eights), and looping over windows."""
     _at_most(kernels, r"pair_backward_kernel<\d+,true,\w+,false,true>", 128, 4, 6)
     _at_most(kernels, r"pair_backward_kernel<\d+,true,\w+,true,true>", 128, 18, 6)
+
+def test_radix_backward_spills_little(kernels):
+    _at_most(kernels, r"radix_backward_kernel<\d,\d+,true,false,false>", 128, 5, 10)
