@@ -48,14 +48,17 @@ hipError_t launch_any_forward(Pass pass, const StageArgs& a, int grid_x, hipStre
         return hipGetLastError();                                                       \
     }
 #else
+    const bool priority = tanh_only && !kLengths && a.n_cache >= kAnyPriorityRows;
 #define NCN_CASE(R, F)                                                                  \
     if (r == R && f == F) {                                                             \
         if (pass == kInverse) {                                                         \
-            if (tanh_only) NCN_LAUNCH((any_forward_kernel<R, F, true, true, kLengths>));          \
-            else NCN_LAUNCH((any_forward_kernel<R, F, false, true, kLengths>));                   \
+            if (priority) NCN_LAUNCH((any_forward_kernel<R, F, true, true, kLengths, !kLengths>)); \
+            else if (tanh_only) NCN_LAUNCH((any_forward_kernel<R, F, true, true, kLengths, false>)); \
+            else NCN_LAUNCH((any_forward_kernel<R, F, false, true, kLengths, false>));            \
         } else {                                                                        \
-            if (tanh_only) NCN_LAUNCH((any_forward_kernel<R, F, true, false, kLengths>));         \
-            else NCN_LAUNCH((any_forward_kernel<R, F, false, false, kLengths>));                  \
+            if (priority) NCN_LAUNCH((any_forward_kernel<R, F, true, false, kLengths, !kLengths>)); \
+            else if (tanh_only) NCN_LAUNCH((any_forward_kernel<R, F, true, false, kLengths, false>)); \
+            else NCN_LAUNCH((any_forward_kernel<R, F, false, false, kLengths, false>));           \
         }                                                                               \
         return hipGetLastError();                                                       \
     }

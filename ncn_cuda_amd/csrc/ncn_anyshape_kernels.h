@@ -275,7 +275,7 @@ __device__ __forceinline__ void any_broadcast(const float (&v)[F], float (&out)[
     for (int f = 0; f < F; ++f) out[f] = slots[f * 64 + src];
 }
 
-template <int R, int F>
+template <bool PRIORITY, int R, int F>
 __device__ __forceinline__ void any_row_sums(const float (&x)[R][F], const float (&wi)[F], float e, int lfl, float (&c)[R]) {
 #pragma unroll
     for (int rr = 0; rr < R; ++rr) {
@@ -283,7 +283,7 @@ __device__ __forceinline__ void any_row_sums(const float (&x)[R][F], const float
 #pragma unroll
         for (int f = 0; f < F; ++f) c[rr] = fmaf(x[rr][f], wi[f], c[rr]);
     }
-    issue_first();   // (the wave stays at high priority)
+    issue_first<PRIORITY>();   // (the wave stays at high priority)
     any_sum_rows<R>(c, lfl);
 }
 
@@ -311,8 +311,15 @@ __device__ __forceinline__ void for_each_row(const Fn& f) {
     const StepTable& S = A.tab;                                                                 \
     float wi[F], wj[F];
 
+constexpr int kAnyPriorityRows = 12;
+
 // INVERSE = false: x, xa -> y, ya (optional float32 copies);  true: y, ya -> x, xa
-template <int R, int F, bool TANH_ONLY, bool INVERSE, bool LENGTHS>
+// PRIORITY: exp2 at high priority, one constant in a vector register (issue_first, in_vector_register), for launches with
+// kAnyPriorityRows and more to a group and no lengths.  us, without : with (x[24, 8192, ~256] float32, forward / inverse): groups of 48,
+// heads of 20 602 : 525 / 597 : 526, of 24, 12 386 : 357 / 366 : 347, of 20, 40 345 : 326 / 338 : 321, of 12, 48 208 : 201 / 206 : 192; of 10,
+// 40 218 : 235 / 212 : 228, of 5, 5 430 : 430 / 452 : 470, of 3, 7 the same.  With lengths 381 : 366 / 376 : 358, 265 : 272 / 275 : 273, 244 : 242 /
+// 242 : 233, 168 : 177 / 176 : 176, of 5, 5 601 : 597 / 584 : 625, of 3, 7 467 : 497 / 487 : 486; so not there, nor with other activations.
+template <int R, int F, bool TANH_ONLY, bool INVERSE, bool LENGTHS, bool PRIORITY>
 __global__ void __launch_bounds__(kBlockThreads, R * F <= 16 ? 4 : R * F <= 20 ? 3 : 2) any_forward_kernel(const StageArgs A) {
     NCN_ANY_PROLOGUE
     for (uint32_t t = gwave / A.n_head; t < A.total_tiles; t += tile_step) {
@@ -335,7 +342,7 @@ __global__ void __launch_bounds__(kBlockThreads, R * F <= 16 ? 4 : R * F <= 20 ?
         any_fill_padding(L, x, INVERSE ? any_missing_undone(S) : 1.f);
         any_fill_padding(L, a);
         scale_tile<R, F>(x, a, S.kappa, INVERSE ? S.b_scale : S.a_scale);
-        const float keep = in_vector_register(INVERSE ? S.im : S.m);   // read twice per element and step
+        const float keep = PRIORITY ? in_vector_register(INVERSE ? S.im : S.m) : INVERSE ? S.im : S.m;   // read twice per element and step
 #pragma unroll 1
         for (int k = 0; k < lr; ++k) {
             const int jo = INVERSE ? lr - 1 - k : k;
@@ -351,11 +358,11 @@ __global__ void __launch_bounds__(kBlockThreads, R * F <= 16 ? 4 : R * F <= 20 ?
                 }
                 float xj[F], c[R];
                 any_broadcast<F>(x[jr], xj, lr > 1, src, lane, slots);
-                any_row_sums<R, F>(x, wi, dot_chain<F>(xj, wj), L.lfl, c);
+                any_row_sums<PRIORITY, R, F>(x, wi, dot_chain<F>(xj, wj), L.lfl, c);
                 if constexpr (TANH_ONLY) {
                     float r[R][F];
                     sigmoids(0, x, c, xj, r);
-                    issue_with_others();
+                    issue_with_others<PRIORITY>();
 #pragma unroll
                     for (int rr = 0; rr < R; ++rr)
 #pragma unroll
@@ -364,7 +371,6 @@ __global__ void __launch_bounds__(kBlockThreads, R * F <= 16 ? 4 : R * F <= 20 ?
                             if constexpr (!INVERSE) x[rr][f] = fmaf(keep, x[rr][f], a[rr][f]);
                         }
                 } else {
-                    issue_with_others();
 #pragma unroll
                     for (int rr = 0; rr < R; ++rr)
 #pragma unroll
@@ -457,10 +463,9 @@ __global__ void __launch_bounds__(kBlockThreads, R * F <= (LOOP ? 10 : 12) ? 4 :
                     for (int f = 0; f < F; ++f) Y[rr][f] = fmaf(S.im, Y[rr][f], -B[rr][f]);
                 float xj[F], c[R], rh[R], v[F];
                 any_broadcast<F>(Y[jr], xj, lr > 1, src, lane, slots);
-                any_row_sums<R, F>(Y, wi, dot_chain<F>(xj, wj), L.lfl, c);
+                any_row_sums<TANH_ONLY, R, F>(Y, wi, dot_chain<F>(xj, wj), L.lfl, c);
 #pragma unroll
                 for (int f = 0; f < F; ++f) v[f] = 0.f;
-                if constexpr (!TANH_ONLY) issue_with_others();
 #pragma unroll
                 for (int rr = 0; rr < R; ++rr) {   // exp2 and reciprocals of one row at a time: see backward_core
                     float r[1][F];
@@ -487,9 +492,9 @@ __global__ void __launch_bounds__(kBlockThreads, R * F <= (LOOP ? 10 : 12) ? 4 :
                         G[rr][f] = fmaf(S.ku, U, G[rr][f]);
                     }
                 }
-                issue_first();
+                issue_first<TANH_ONLY>();
                 any_sum_rows<R>(rh, L.lfl);
-                issue_with_others();
+                issue_with_others<TANH_ONLY>();
                 float rhosum = 0.f;
 #pragma unroll
                 for (int rr = 0; rr < R; ++rr) {
@@ -510,9 +515,9 @@ __global__ void __launch_bounds__(kBlockThreads, R * F <= (LOOP ? 10 : 12) ? 4 :
                     dwj[f] = fmaf(rhosum_w, xj[f], dwj[f]);
                     s[f] = fmaf(rhosum, wj[f], v[f]);
                 }
-                issue_first();
+                issue_first<TANH_ONLY>();
                 any_sum_span<F>(s, L.lfl, L.lfl + L.lrl);   // over the group's row lanes
-                issue_with_others();
+                issue_with_others<TANH_ONLY>();
 #pragma unroll
                 for (int f = 0; f < F; ++f) {
                     G[jr][f] = fmaf(selku, s[f], G[jr][f]);

@@ -96,3 +96,8 @@ def test_backward_on_groups_of_two_heads_of_one_feature(kernels):
 
 def test_radix_backward_spills_little(kernels):
     _at_most(kernels, r"radix_backward_kernel<\d,\d+,true,false,false>", 128, 5, 10)
+
+def test_odd_shapes_keep_their_waves(kernels):
+    """Builds without priorities on tiles of 4 x 4 run five waves per SIMD, of 5 x 5 four."""
+    _at_most(kernels, r"any_forward_kernel<4,4,\w+,\w+,\w+,false>", 96, 0, 8)
+    _at_most(kernels, r"any_forward_kernel<5,5,\w+,\w+,\w+,false>", 128, 0, 8)
