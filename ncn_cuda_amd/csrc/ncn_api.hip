@@ -227,6 +227,14 @@ void fill_step_table(StepTable& t, int n_cache, float alpha, float m, int activa
     t.inv_m_pow_n = (float)std::pow(md, -(double)n_cache);
     t.reserved2 = 0.f;
     for (int k = 0; k < 64; ++k) t.krho[k] = (float)((1.0 - al) * 4.0 * om * std::pow(md, (double)k) / (kappa * kappa));
+    const float near = (float)im, other = std::nextafterf(near, (double)near < im ? INFINITY : 0.f);
+    double off = 0.0;   // of the product so far, relative
+    for (float& v : t.im_at) {
+        const double with_near = off + ((double)near * md - 1.0), with_other = off + ((double)other * md - 1.0);
+        const bool take_near = std::fabs(with_near) <= std::fabs(with_other);
+        v = take_near ? near : other;
+        off = take_near ? with_near : with_other;
+    }
     cached = t;
     cached_n = n_cache;
 }

@@ -455,10 +455,10 @@ __global__ void __launch_bounds__(64 * kPairWavesBwd, TANH_ONLY ? NCN_PAIR_BWD_W
                         for (int f = 0; f < F; ++f) Y[k][1][f] = B[k][1][f] = G[k][1][f] = P[k][1][f] = 0.f;
                     }
                     if constexpr (HEADWISE)
-                        headwise_backward_core<NC, EC, R, F, true, TANH_ONLY, LENGTHS, true, false>(
+                        headwise_backward_core<NC, EC, R, F, true, TANH_ONLY, LENGTHS, true, false, true>(
                             Y[k], B[k], G[k], P[k], wi, wj, dwi, dwj, own, A.tab, (A.n_stages - 1 - st) * NC, lane, nullptr, live);
                     else
-                        backward_core<NC, EC, R, F, true, TANH_ONLY, LENGTHS, true, false>(
+                        backward_core<NC, EC, R, F, true, TANH_ONLY, LENGTHS, true, false, true>(
                             Y[k], B[k], G[k], P[k], wi, wj, dwi, dwj, own, A.tab, (A.n_stages - 1 - st) * NC, lane, nullptr, live);
                     if (!LENGTHS || live > 1) {
                         pair_lds_store<EC>(ys1 + row1, fl, Y[k][1]);

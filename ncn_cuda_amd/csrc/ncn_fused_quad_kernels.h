@@ -263,9 +263,9 @@ __global__ void __launch_bounds__(64 * kQuadWavesBwd, TANH_ONLY ? 4 : 2) quad_ba
                 lds_load_frag<F>(w_lds + st * 2 * EC + EC + fl * F, wj);
                 const int done = (A.n_stages - 1 - st) * NC;
                 if constexpr (HEADWISE)
-                    headwise_backward_core<NC, EC, R, F, true, TANH_ONLY, false, true, false>(Y, B, G, P, wi, wj, dwi, dwj, own, A.tab, done, lane, nullptr);
+                    headwise_backward_core<NC, EC, R, F, true, TANH_ONLY, false, true, false, true>(Y, B, G, P, wi, wj, dwi, dwj, own, A.tab, done, lane, nullptr);
                 else
-                    backward_core<NC, EC, R, F, true, TANH_ONLY, false, true, false>(Y, B, G, P, wi, wj, dwi, dwj, own, A.tab, done, lane, nullptr);
+                    backward_core<NC, EC, R, F, true, TANH_ONLY, false, true, false, true>(Y, B, G, P, wi, wj, dwi, dwj, own, A.tab, done, lane, nullptr);
             }
             {   // the wave's dW of the stage into its place: every lane ends up with one or more complete sums
                 const int first = quad_scatter_sum<LF>(dw, lane);

@@ -124,7 +124,7 @@ __device__ __forceinline__ void headwise_inverse_core(float (&y)[R][F], float (&
 // step_base inversion steps were done before (several stages in a row keep counting); with MASKED the dW shares are
 // weighted by `own` (1, or 0 for a group whose dW another window accounts for).
 template <int NC, int EC, int R, int F, bool MASKED, bool TANH_ONLY = true, bool STEP_MASK = false, bool ROWS = false,
-          bool KU_W = true>
+          bool KU_W = true, bool IM_AT = false>
 __device__ __forceinline__ void headwise_backward_core(float (&Y)[R][F], float (&B)[R][F], float (&G)[R][F],
                                                        float (&P)[R][F], const float (&wi)[F], const float (&wj)[F],
                                                        float (&dwi)[F], float (&dwj)[F], float own, const StepTable& S,
@@ -139,10 +139,11 @@ __device__ __forceinline__ void headwise_backward_core(float (&Y)[R][F], float (
             if (STEP_MASK && jo * R + jr >= live) continue;
             const int ts = step_base + (T::LR - 1 - jo) * R + (R - 1 - jr);   // inversion steps done so far
             const float krho = MASKED ? S.krho[ts] * own : S.krho[ts];
+            const float im = IM_AT ? S.im_at[ts] : S.im;
 #pragma unroll
             for (int rr = 0; rr < R; ++rr)
 #pragma unroll
-                for (int f = 0; f < F; ++f) Y[rr][f] = fmaf(S.im, Y[rr][f], -B[rr][f]);  // xs before this step
+                for (int f = 0; f < F; ++f) Y[rr][f] = fmaf(im, Y[rr][f], -B[rr][f]);  // xs before this step
             float xj[F], cj[F];
             row_lane_broadcast<T::LF, T::LR, F>(Y[jr], xj, jo, lane, slots);
 #pragma unroll
@@ -169,12 +170,12 @@ __device__ __forceinline__ void headwise_backward_core(float (&Y)[R][F], float (
                             float w;
                             if constexpr (TANH_ONLY) {
                                 if constexpr (!kBatch) r[k][f] = __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(fmaf(c, xj[f], Y[rr][f])) + 1.0f);
-                                B[rr][f] = fmaf(S.bk1, r[k][f], fmaf(S.im, B[rr][f], S.bk0));   // bh before this step
+                                B[rr][f] = fmaf(S.bk1, r[k][f], fmaf(im, B[rr][f], S.bk0));   // bh before this step
                                 w = fmaf(-r[k][f], r[k][f], r[k][f]);
                             } else {
                                 float Fv;
                                 act_Fw(fmaf(c, xj[f], Y[rr][f]), S.activation, Fv, w);
-                                B[rr][f] = fmaf(S.bk0, Fv, S.im * B[rr][f]);
+                                B[rr][f] = fmaf(S.bk0, Fv, im * B[rr][f]);
                             }
                             const float U = P[rr][f] * w;
                             const float rh = U * xj[f];
@@ -205,12 +206,12 @@ __device__ __forceinline__ void headwise_backward_core(float (&Y)[R][F], float (
                         const float c = fmaf(Y[rr][f], wi[f], cj[f]);
                         float w;
                         if constexpr (TANH_ONLY) {
-                            B[rr][f] = fmaf(S.bk1, r[k][f], fmaf(S.im, B[rr][f], S.bk0));   // bh before this step
+                            B[rr][f] = fmaf(S.bk1, r[k][f], fmaf(im, B[rr][f], S.bk0));   // bh before this step
                             w = fmaf(-r[k][f], r[k][f], r[k][f]);
                         } else {
                             float Fv;
                             act_Fw(fmaf(c, xj[f], Y[rr][f]), S.activation, Fv, w);
-                            B[rr][f] = fmaf(S.bk0, Fv, S.im * B[rr][f]);
+                            B[rr][f] = fmaf(S.bk0, Fv, im * B[rr][f]);
                         }
                         const float U = P[rr][f] * w;
                         const float rh = U * xj[f];

@@ -303,8 +303,9 @@ __device__ __forceinline__ void inverse_core(float (&y)[R][F], float (&b)[R][F],
 // STEP_MASK: steps j >= live leave the registers as they are (the caller scales G, P as if they had been done).
 // ---------------------------------------------------------------------------------------------
 // KU_W: the products ku Wi' are kept beside the weights (F more registers, one multiplication less per row and step).
+// IM_AT: 1/m of each step from the table (im_at).
 template <int NC, int EC, int R, int F, bool MASKED, bool TANH_ONLY = true, bool STEP_MASK = false, bool ROWS = false,
-          bool KU_W = true>
+          bool KU_W = true, bool IM_AT = false>
 __device__ __forceinline__ void backward_core(float (&Y)[R][F], float (&B)[R][F], float (&G)[R][F], float (&P)[R][F],
                                               const float (&wi)[F], const float (&wj)[F], float (&dwi)[F],
                                               float (&dwj)[F], float own, const StepTable& S, int step_base, int lane,
@@ -327,10 +328,11 @@ __device__ __forceinline__ void backward_core(float (&Y)[R][F], float (&B)[R][F]
             if (STEP_MASK && jo * R + jr >= live) continue;  // lanes of a group agree: no lane it needs is off
             const int ts = step_base + (T::LR - 1 - jo) * R + (R - 1 - jr);   // inversion steps done so far
             const float krho = MASKED ? S.krho[ts] * own : S.krho[ts];
+            const float im = IM_AT ? S.im_at[ts] : S.im;
 #pragma unroll
             for (int rr = 0; rr < R; ++rr)
 #pragma unroll
-                for (int f = 0; f < F; ++f) Y[rr][f] = fmaf(S.im, Y[rr][f], -B[rr][f]);  // xs before this step
+                for (int f = 0; f < F; ++f) Y[rr][f] = fmaf(im, Y[rr][f], -B[rr][f]);  // xs before this step
             float xj[F], c[R], rh[R];
             row_lane_broadcast<T::LF, T::LR, F>(Y[jr], xj, jo, lane, slots);
             row_sums<T::LF, R, F, ROWS, kPriority>(Y, wi, dot_chain<F>(xj, wj), c);
@@ -361,12 +363,12 @@ __device__ __forceinline__ void backward_core(float (&Y)[R][F], float (&B)[R][F]
                         for (int f = 0; f < F; ++f) {
                             float w;
                             if constexpr (TANH_ONLY) {
-                                B[rr][f] = fmaf(S.bk1, r[k][f], fmaf(S.im, B[rr][f], S.bk0));   // bh before this step
+                                B[rr][f] = fmaf(S.bk1, r[k][f], fmaf(im, B[rr][f], S.bk0));   // bh before this step
                                 w = fmaf(-r[k][f], r[k][f], r[k][f]);
                             } else {
                                 float Fv;
                                 act_Fw(fmaf(c[rr], xj[f], Y[rr][f]), S.activation, Fv, w);
-                                B[rr][f] = fmaf(S.bk0, Fv, S.im * B[rr][f]);
+                                B[rr][f] = fmaf(S.bk0, Fv, im * B[rr][f]);
                             }
                             const float U = P[rr][f] * w;
                             rh[rr] = fmaf(U, xj[f], rh[rr]);
@@ -420,12 +422,12 @@ __device__ __forceinline__ void backward_core(float (&Y)[R][F], float (&B)[R][F]
                     for (int f = 0; f < F; ++f) {
                         float w;
                         if constexpr (TANH_ONLY) {
-                            B[rr][f] = fmaf(S.bk1, r[k][f], fmaf(S.im, B[rr][f], S.bk0));   // bh before this step
+                            B[rr][f] = fmaf(S.bk1, r[k][f], fmaf(im, B[rr][f], S.bk0));   // bh before this step
                             w = fmaf(-r[k][f], r[k][f], r[k][f]);
                         } else {
                             float Fv;
                             act_Fw(fmaf(c[rr], xj[f], Y[rr][f]), S.activation, Fv, w);
-                            B[rr][f] = fmaf(S.bk0, Fv, S.im * B[rr][f]);
+                            B[rr][f] = fmaf(S.bk0, Fv, im * B[rr][f]);
                         }
                         const float U = P[rr][f] * w;
                         rh[rr] = fmaf(U, xj[f], rh[rr]);

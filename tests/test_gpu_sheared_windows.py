@@ -25,6 +25,25 @@ CASES = [
 ]
 
 
+@pytest.mark.parametrize("case", [(64, 32, 64, 2, 4, 0, 6), (64, 32, 32, 32, 4, 1, 6), (64, 64, 64, 2, 2, 0, 7), (64, 64, 32, 32, 2, 2, 7)],
+                         ids=lambda c: "_".join(map(str, c)))
+def test_many_steps_are_undone_without_drift(case):
+    """What the passes reconstruct is off by rounding errors of either sign, not by that of 1/m once for every step.  m is one whose 1/m
+    is 5.9e-8 off in float32: 24 or 14 steps would drift by 1.4e-6 or 8e-7 (less what xa makes up for; 3.7e-7 to 9.8e-7 measured).  The
+    other constants are off once, by half a unit each (6e-8), four of them in a step: 2.4e-7."""
+    from ncn_cuda_amd import ncn_cuda_module as M
+    batch, groups, E, C, n, first, L = case
+    x, xa, Ws, dy, dya = O.make_inputs(batch, n * groups, E, L, n, seed=sum(case), xa_zero=False)
+    m = 0.900225818157196   # a float32
+    d = torch.float64
+    y, ya = O.net_forward(x.to(d).cuda(), xa.to(d).cuda(), [w.to(d).cuda() for w in Ws], 0.9, n, C, m=m, first_stage=first)
+    W = torch.stack([w.reshape(-1) for w in Ws]).cuda()
+    back = M.backward_stages(y.float(), ya.float(), dy.cuda(), dya.cuda(), W, 0.9, 0, n, C, first, L, m=m)
+    for got, want in ((back[0].cpu().to(d), x.to(d)), (back[1].cpu().to(d), xa.to(d))):
+        drift = abs(float(((got - want) * want).sum() / (want * want).sum()))
+        assert drift < 2.4e-7
+
+
 @pytest.mark.parametrize("case", CASES, ids=lambda c: "_".join(map(str, c)))
 def test_stack_and_inverse(case):
     from ncn_cuda_amd import ncn_cuda_module as M
