@@ -291,6 +291,41 @@ def test_backward_with_the_smaller_workspace_loops_over_windows(M):
     assert O.rel_err(dW, ref[4]) < 1e-6
 
 
+@pytest.mark.parametrize("act", [0, 2], ids=["tanh", "sigmoid"])
+@pytest.mark.parametrize("heads", [1, 32], ids=["heads_of_32", "one_feature_heads"])
+def test_groups_of_four_loop_over_windows(M, heads, act):
+    """The same for the kernels of groups of four rows: bits of dx, dxa, x_rec, xa_rec as with a workgroup for every window, dW up to
+    the order of its sums."""
+    import ctypes
+    from ncn_cuda_amd import _lib
+    batch, N, E, n, L = 400, 4096, 32, 4, 3
+    g = torch.Generator(device="cuda").manual_seed(heads)
+    x, xa, dy, dya = (torch.randn(batch, N, E, device="cuda", generator=g) for _ in range(4))
+    W = torch.randn(L, 2 * E, device="cuda", generator=g) * 0.2
+    y, ya = M.forward_stages(x, xa, W, 0.9, act, n, heads, 0, L)
+    ref = M.backward_stages(y, ya, dy, dya, W, 0.9, act, n, heads, 0, L)
+    lib = _lib.load()
+    shape, passes = _lib.NcnShape(batch, N, E, heads, n), (ctypes.c_int32 * 64)()
+    small = lib.ncn_workspace_bytes(ctypes.byref(shape)) + 4 * x.numel() * 4
+    k = lib.ncn_plan_passes(ctypes.byref(shape), 0, L, act, 1, passes, 8)
+    # a partial row of 2 E floats for every window and stage of a pass is more than that workspace holds
+    looping = [batch * passes[8 * j + 7] * -(-(N // n // passes[8 * j + 3]) // passes[8 * j + 6]) * passes[8 * j + 1] * 2 * E * 4 >
+               lib.ncn_workspace_bytes(ctypes.byref(shape)) for j in range(k) if passes[8 * j + 2] == 1]
+    assert any(looping)
+    ws = torch.empty(small, dtype=torch.uint8, device="cuda")
+    out = [torch.empty_like(x) for _ in range(4)]       # dx, dxa, x_rec, xa_rec
+    dW = torch.empty(L, 2 * E, device="cuda")
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    rc = lib.ncn_backward(p(y), p(ya), 0, p(dy), p(dya), 0, p(out[0]), p(out[1]), 0, p(out[2]), p(out[3]), p(W), p(dW),
+                          p(ws), ctypes.c_size_t(small), ctypes.byref(shape), 0, L, 0.9, 0.9, act,
+                          ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0
+    torch.cuda.synchronize()
+    assert torch.equal(out[2], ref[0]) and torch.equal(out[3], ref[1])
+    assert torch.equal(out[0], ref[2]) and torch.equal(out[1], ref[3])
+    assert O.rel_err(dW, ref[4]) < 1e-5   # sums of 4e5 groups in another order
+
+
 @pytest.mark.parametrize("n", [2, 4])
 def test_more_windows_than_a_launch_holds(M, n):
     """2^23 windows of 512 threads are more work-items than a launch takes: the call runs in several launches, with the bits of the
