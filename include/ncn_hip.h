@@ -355,11 +355,23 @@ size_t ncn_workspace_bytes_stages(const ncn_shape* shape, int first_stage, int n
  *   [2] kind: 0 one-stage launch, 1 halo window, 2 closed rings
  *   [3] class stride S0 in blocks   [4] window   [5] halo   [6] owned sub-blocks per window
  *   [7] windows per batch entry and ring tile (classes, or groups of classes for closed rings)
- * The halo is what windows of plain blocks need; the launch loads the rows of the groups that the owned ones depend on,
- * which are fewer (ncn_fused_kernels.h).  Stacks that are trained (ncn_stack_forward) and ncn_inverse_ws are cut by that smaller need.
+ * The window and the halo are those of the plan, what windows of plain blocks need; the launch loads the rows of the groups that the
+ * owned ones depend on, which are fewer (ncn_fused_kernels.h).  Stacks that are trained (ncn_stack_forward) and ncn_inverse_ws are cut by
+ * that smaller need: ncn_plan_sheared_passes.
  * No reference counterpart. */
 int ncn_plan_passes(const ncn_shape* shape, int first_stage, int n_stages, int activation, int backward, int32_t* out,
                     int max_passes);
+
+/* The cuts by sheared windows, for inspection and tests: with max_range = 0 what ncn_inverse_ws runs (backward = 0) when it has
+ * scratch for two arrays and no pass works in place; with max_range, max_saves >= 1 what ncn_stack_forward (backward = 0) or
+ * ncn_stack_backward (1) runs, range by range.  Returns the number of passes (0: one launch per stage) or a negative error code;
+ * writes up to max_passes records of 10 int32 into `out` (may be NULL):
+ *   [0] to [3] as above   [4] groups that a window loads   [5], [6], [7] those in front of the owned ones, owned, and behind them (a
+ *   direction that runs the stages in descending order has the first and the last the other way round)
+ *   [8] classes, or groups of classes for closed rings   [9] windows per ring (a multiple of [6] that covers the ring)
+ * No reference counterpart. */
+int ncn_plan_sheared_passes(const ncn_shape* shape, int first_stage, int n_stages, int activation, int backward, int max_range,
+                            int max_saves, int32_t* out, int max_passes);
 
 /* 2: hand-tuned register kernel, 1: generic LDS kernel, 0: not supported (n_cache > 64, or the
  * head width does not fit the generic kernel's LDS).  Register kernels exist for n_cache 2, 4, 8, 16, 32, 64 with

@@ -15,7 +15,7 @@ ACT_TANH, ACT_RELU, ACT_SIGMOID, ACT_LEAKY_RELU, ACT_LINEAR = 0, 1, 2, 3, -1
 
 EXPORTS = ("ncn_forward", "ncn_backward", "ncn_inverse", "ncn_forward_indexed", "ncn_backward_indexed",
            "ncn_inverse_indexed", "ncn_inverse_ws", "ncn_forward_radix", "ncn_backward_radix", "ncn_inverse_radix", "ncn_plan_radix", "ncn_workspace_bytes", "ncn_workspace_bytes_stages",
-           "ncn_plan_passes", "ncn_kernel_path",
+           "ncn_plan_passes", "ncn_plan_sheared_passes", "ncn_kernel_path",
            "ncn_check_shape", "ncn_error_string", "ncn_version", "ncn_backward_static", "ncn_static_scratch_bytes", "ncn_kernel_path_scalars",
            "ncn_stack_plan", "ncn_stack_forward", "ncn_stack_backward", "ncn_build_id", "ncn_probe_issue", "ncn_probe_issue_info")
 
@@ -109,6 +109,8 @@ def load():
     lib.ncn_workspace_bytes_stages.argtypes = [shp, i, i, i, i]
     lib.ncn_plan_passes.restype = i
     lib.ncn_plan_passes.argtypes = [shp, i, i, i, i, ctypes.POINTER(ctypes.c_int32), i]
+    lib.ncn_plan_sheared_passes.restype = i
+    lib.ncn_plan_sheared_passes.argtypes = [shp, i, i, i, i, i, i, ctypes.POINTER(ctypes.c_int32), i]
     lib.ncn_kernel_path.restype = i
     lib.ncn_kernel_path.argtypes = [shp]
     lib.ncn_kernel_path_scalars.restype = i

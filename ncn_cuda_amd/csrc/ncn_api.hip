@@ -1266,6 +1266,29 @@ struct StackCall {
     }
 };
 
+int ncn_plan_sheared_passes(const ncn_shape* shape, int first_stage, int n_stages, int activation, int backward, int max_range,
+                            int max_saves, int32_t* out, int max_passes) {
+    const int rc = check_shape(shape, first_stage, n_stages, activation);
+    if (rc != NCN_OK) return rc;
+    std::vector<FusedPass> passes;
+    if (max_range == 0) {
+        ncn_shape as_wide;
+        passes = multi_stage_plan(planning_shape(shape, &as_wide), first_stage, n_stages, activation, backward != 0, 2, true);
+    } else {
+        StackCall c;   // (any scalars of the register kernels)
+        if (!c.plan(shape, first_stage, n_stages, activation, 0.5f, 0.5f, max_range, max_saves)) return 0;
+        for (const StackRange& r : *c.ranges) passes.insert(passes.end(), backward ? r.bwd.begin() : r.fwd.begin(), backward ? r.bwd.end() : r.fwd.end());
+    }
+    for (int k = 0; out && k < (int)passes.size() && k < max_passes; ++k) {
+        const FusedPass& p = passes[k];
+        const bool halo = !p.single && !p.closed;
+        const int32_t record[10] = {p.first, p.count, p.single ? 0 : p.closed ? 2 : 1, (int32_t)p.class_stride, (int32_t)p.window, halo ? (int32_t)p.before : 0,
+                                    (int32_t)p.own, halo ? (int32_t)p.after : 0, (int32_t)p.class_groups, (int32_t)p.tiles_per_ring};
+        std::copy(record, record + 10, out + 10 * k);
+    }
+    return (int)passes.size();
+}
+
 int ncn_stack_plan(const ncn_shape* shape, int first_stage, int n_stages, float alpha, float m, int activation,
                    int max_range, int max_saves, int grad_dtype, int64_t* out) {
     const int rc = check_shape(shape, first_stage, n_stages, activation);

@@ -389,6 +389,59 @@ def test_multi_stage_plan_invariants(lib, dims, backward):
     assert nxt == count
 
 
+# batch, groups, E, heads, n_cache, first stage, stages
+SHEARED = [(128, 4096, 128, 4, 2, 0, 13), (2, 514, 64, 2, 2, 0, 9), (2, 514, 64, 2, 2, 10, 5), (1, 4096, 32, 1, 2, 3, 8), (2, 260, 64, 2, 2, 0, 7),
+           (1, 1030, 16, 2, 2, 0, 8), (1, 300, 256, 2, 2, 1, 6), (1, 514, 32, 32, 2, 9, 6), (2, 514, 128, 2, 2, 0, 9), (64, 512, 128, 4, 4, 0, 6), (2, 130, 64, 2, 4, 0, 6),
+           (2, 130, 64, 2, 4, 8, 4), (2, 130, 128, 2, 4, 0, 6), (1, 320, 64, 4, 4, 2, 5), (1, 320, 64, 1, 4, 1, 5), (1, 600, 16, 2, 4, 0, 6), (1, 70, 128, 1, 4, 0, 5),
+           (1, 130, 64, 64, 4, 8, 4)]
+
+
+@pytest.mark.parametrize("dims", SHEARED, ids=lambda d: "_".join(map(str, d)))
+def test_sheared_windows_hold_what_their_owned_groups_need(lib, dims):
+    """Every cut by sheared windows (the inverse, both directions of a trained stack): passes tile the stages, windows tile the ring and
+    fit the LDS, and, stage by stage, every row of an owned group has been through all the stages before it."""
+    batch, groups, E, C, n, first, L = dims
+    shape = _shape(lib, batch, n * groups, E, C, n)
+    wide = next(w for w in (32, 16, 8, 4, 1) if E % w == 0) if C == E else E // C
+    halos = falling = 0
+    for backward, descending, max_range, max_saves in ((0, True, 0, 0), (0, False, min(L, 26 // n), L), (1, True, min(L, 26 // n), L), (1, True, L, 1)):
+        buf = (ctypes.c_int32 * 640)()
+        k = lib.load().ncn_plan_sheared_passes(ctypes.byref(shape), first, L, 0, backward, max_range, max_saves, buf, 64)
+        passes = [tuple(buf[10 * j:10 * j + 10]) for j in range(k)]
+        assert 1 <= k <= L and [p[0] for p in passes] == [sum(p[1] for p in passes[:j]) for j in range(k)] and sum(p[1] for p in passes) == L
+        for p_first, count, kind, s0, window, before, own, after, classes, tiles in passes:
+            if kind == 0:
+                assert count == 1
+                continue
+            ring = groups // s0
+            assert 2 <= count <= 8 and groups % s0 == 0
+            assert window * (1 if n == 2 else n) * wide * 4 * (4 if backward else 2) <= 64 * 1024
+            if kind == 2:
+                assert window == own and window % ring == 0 and classes * (window // ring) == s0 and before == after == 0
+                continue
+            halos += 1
+            assert window == before + own + after and classes == s0 and (tiles - 1) * own < ring <= tiles * own
+            strides = [0 if first + p_first + j == 0 else pow(2, first + p_first + j - 1, groups) for j in range(count)]
+            assert all(s % s0 == 0 for s in strides)
+            steps = [(b - a) // s0 % ring for a, b in zip(strides, strides[1:])]
+            steps = [s if s <= ring - s else s - ring for s in steps]   # the shorter way around the ring
+            falling += any(s < 0 for s in steps)
+            if descending:
+                steps = [-s for s in reversed(steps)]
+            front = after if descending else before
+            sound = {(o, p) for o in range(n) for p in range(window)}   # slot o at window position p
+            at = 0
+            for j in range(count):
+                at += steps[j - 1] if j else 0
+                whole = [q for q in range(window) if all(0 <= q + o * at < window for o in range(n))]
+                kept = [q for q in whole if all((o, q + o * at) in sound for o in range(n))]
+                sound = {(o, q + o * at) for q in kept for o in range(n)}
+            assert set(range(front, front + own)) <= set(kept)
+    if dims in ((2, 514, 64, 2, 2, 10, 5), (1, 514, 32, 32, 2, 9, 6), (2, 130, 64, 2, 4, 8, 4), (1, 130, 64, 64, 4, 8, 4)):
+        assert falling
+    assert halos
+
+
 def test_multi_stage_plan_declines_ineligible_shapes(lib):
     assert _passes(lib, _shape(lib, 128, 4096, 128, 4, 16), 0, 3, False) == []   # n_cache = 16: arithmetic-bound
     assert _passes(lib, _shape(lib, 2, 60, 32, 4, 4), 0, 3, False) == []         # 15 groups: no power of two divides them
