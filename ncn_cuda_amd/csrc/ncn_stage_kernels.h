@@ -189,7 +189,7 @@ __device__ __forceinline__ void forward_core(float (&x)[R][F], float (&a)[R][F],
                                              const float (&wj)[F], const StepTable& S, int lane, float4* slots,
                                              int live = NC) {
     using T = Tile<NC, EC, R, F>;
-    // read twice per element and step; with other activations the register is dearer (headwise inverse, relu, behind a table, x[24, 4096, 256],
+    // read twice per element and step; with other activations the register is dearer (headwise inverse, sigmoid, behind a table, x[24, 4096, 256],
     // groups of 16: five waves per SIMD instead of four, 183 us : 207)
     const float m = TANH_ONLY ? in_vector_register(S.m) : S.m;
 #pragma unroll 1

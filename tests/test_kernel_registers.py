@@ -89,13 +89,16 @@ def test_other_activations_keep_their_waves(kernels):
     _at_most(kernels, r"headwise_forward_kernel<\d+,\d+,4,4,false,true,\w+>", 97, 0, 20)
     _at_most(kernels, r"headwise_forward_kernel<\d+,\d+,4,4,false,true,true>", 96, 0, 10)
 
+
 def test_backward_on_groups_of_two_heads_of_one_feature(kernels):
     """With a window for every workgroup (four registers have always spilled at heads laid out in eights), and looping over windows."""
     _at_most(kernels, r"pair_backward_kernel<\d+,true,\w+,false,true>", 128, 4, 6)
     _at_most(kernels, r"pair_backward_kernel<\d+,true,\w+,true,true>", 128, 18, 6)
 
+
 def test_radix_backward_spills_little(kernels):
     _at_most(kernels, r"radix_backward_kernel<\d,\d+,true,false,false>", 128, 5, 10)
+
 
 def test_odd_shapes_keep_their_waves(kernels):
     """Builds without priorities on tiles of 4 x 4 run five waves per SIMD, of 5 x 5 four."""
