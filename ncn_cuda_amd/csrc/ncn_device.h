@@ -300,9 +300,10 @@ __device__ __forceinline__ float in_vector_register(float v) {
 // ---------------------------------------------------------------------------------------------
 // cross-lane moves inside one 64-wide wavefront
 // ---------------------------------------------------------------------------------------------
-// value of lane (lane ^ S).  ROWS: stride 8 as a DPP row rotation instead of a trip through the LDS crossbar
-// (costs the same issue slots, and on kernels that are bound by issue a little more through its wait states; pays
-// on kernels that wait on latency).
+// value of lane (lane ^ S).  ROWS: stride 8 as a DPP row rotation instead of a trip through the LDS crossbar: sooner back, and with
+// issue_first around the sums cheaper on kernels that are bound by issue too (there it cost more before: see the figures above;
+// the one-stage kernels for heads of one feature, whose only sum across lanes is the pivot row's, keep the crossbar).  Strides 16 and 32,
+// and 4 in a sum that does not start at stride 1, have no such form.
 template <int S, bool ROWS = false>
 __device__ __forceinline__ float lane_xor(float v) {
     static_assert(S == 1 || S == 2 || S == 4 || S == 8 || S == 16 || S == 32, "power of two below 64");

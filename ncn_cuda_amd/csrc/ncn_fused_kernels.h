@@ -42,8 +42,8 @@
 
 namespace ncn {
 
-// The step code is instantiated with ROWS = true here: these kernels wait on latency rather than on issue slots, and
-// reductions through DPP row operations come back sooner than through the LDS crossbar (measured 2.5 % on 13 stages).
+// The step code is instantiated with ROWS = true, as in the one-stage kernels: sums through DPP row operations come back sooner than
+// through the LDS crossbar (2.5 % on 13 stages, where latency is waited for).
 constexpr int kFusedMaxStages = 8;
 // LDS for the row arrays of one workgroup (2 forward and inverse, 4 backward)
 #ifndef NCN_FUSED_STATE_FWD

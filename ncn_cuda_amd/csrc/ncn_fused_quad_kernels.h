@@ -196,7 +196,9 @@ __device__ __forceinline__ int quad_scatter_sum(float (&v)[8], int lane) {
     return first;
 }
 
-// LOOP: workgroups walk over several windows (more windows than dW partial rows).
+// LOOP: workgroups walk over several windows (more windows than dW partial rows).  It spills 22 to 26 registers at four waves per SIMD, as
+// builds for other activations on heads of one feature do at two (28 to 49); a wave less spills nothing and is slower: x[256, 8192, 128], 6 stages,
+// heads of 8 16.2 ms : 20.9, of 32 9.0 : 8.9; sigmoid, heads of one feature, x[256, 4096, 128] 6.1 : 7.2.
 template <int EC, bool TANH_ONLY, bool LOOP, bool HEADWISE>
 __global__ void __launch_bounds__(64 * kQuadWavesBwd, TANH_ONLY ? 4 : 2) quad_backward_kernel(const FusedArgs A) {
     constexpr int NC = 4, R = 4, F = kQuadF, NW = kQuadWavesBwd, LF = EC / F, GPW = 64 / LF, W = NW * GPW;
