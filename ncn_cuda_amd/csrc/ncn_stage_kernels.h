@@ -184,14 +184,14 @@ __device__ __forceinline__ float dot_chain(const float (&a)[F], const float (&b)
 // group switched off (a group that a context length cuts runs one step per live row,
 // ncn_triton/ncn_triton_old.py:93-96).  Every cross-lane exchange of a step stays inside one group.
 // ---------------------------------------------------------------------------------------------
-template <int NC, int EC, int R, int F, bool TANH_ONLY = true, bool STEP_MASK = false, bool ROWS = false>
+template <int NC, int EC, int R, int F, bool TANH_ONLY = true, bool STEP_MASK = false, bool ROWS = false, bool PRIORITY = true>
 __device__ __forceinline__ void forward_core(float (&x)[R][F], float (&a)[R][F], const float (&wi)[F],
                                              const float (&wj)[F], const StepTable& S, int lane, float4* slots,
                                              int live = NC) {
     using T = Tile<NC, EC, R, F>;
     // read twice per element and step; with other activations the register is dearer (headwise inverse, sigmoid, behind a table, x[24, 4096, 256],
     // groups of 16: five waves per SIMD instead of four, 183 us : 207)
-    const float m = TANH_ONLY ? in_vector_register(S.m) : S.m;
+    const float m = TANH_ONLY && PRIORITY ? in_vector_register(S.m) : S.m;
 #pragma unroll 1
     for (int jo = 0; jo < T::LR; ++jo) {
 #pragma unroll
@@ -199,11 +199,11 @@ __device__ __forceinline__ void forward_core(float (&x)[R][F], float (&a)[R][F],
             if (STEP_MASK && jo * R + jr >= live) continue;  // the lanes of a group agree: no lane it needs is off
             float xj[F], c[R];
             row_lane_broadcast<T::LF, T::LR, F>(x[jr], xj, jo, lane, slots);
-            row_sums<T::LF, R, F, ROWS, TANH_ONLY>(x, wi, dot_chain<F>(xj, wj), c);
+            row_sums<T::LF, R, F, ROWS, TANH_ONLY && PRIORITY>(x, wi, dot_chain<F>(xj, wj), c);
             if constexpr (TANH_ONLY) {
                 float r[R][F];
                 sigmoids(0, x, c, xj, r);
-                issue_with_others();
+                issue_with_others<PRIORITY>();
 #pragma unroll
                 for (int rr = 0; rr < R; ++rr)
 #pragma unroll
@@ -234,12 +234,12 @@ __device__ __forceinline__ void forward_core(float (&x)[R][F], float (&a)[R][F],
 // on the scaled state: y holds xs, b holds bh (see StepTable).
 // STEP_MASK: a group with `live` < NC live rows only undoes its steps live-1 .. 0.
 // ---------------------------------------------------------------------------------------------
-template <int NC, int EC, int R, int F, bool TANH_ONLY, bool STEP_MASK = false, bool ROWS = false>
+template <int NC, int EC, int R, int F, bool TANH_ONLY, bool STEP_MASK = false, bool ROWS = false, bool PRIORITY = true>
 __device__ __forceinline__ void inverse_core(float (&y)[R][F], float (&b)[R][F], const float (&wi)[F],
                                              const float (&wj)[F], const StepTable& S, int lane, float4* slots,
                                              int live = NC) {
     using T = Tile<NC, EC, R, F>;
-    const float im = TANH_ONLY ? in_vector_register(S.im) : S.im;   // read twice per element and step
+    const float im = TANH_ONLY && PRIORITY ? in_vector_register(S.im) : S.im;   // read twice per element and step
 #pragma unroll 1
     for (int jo = T::LR - 1; jo >= 0; --jo) {
 #pragma unroll
@@ -251,11 +251,11 @@ __device__ __forceinline__ void inverse_core(float (&y)[R][F], float (&b)[R][F],
                 for (int f = 0; f < F; ++f) y[rr][f] = fmaf(im, y[rr][f], -b[rr][f]);
             float xj[F], c[R];
             row_lane_broadcast<T::LF, T::LR, F>(y[jr], xj, jo, lane, slots);
-            row_sums<T::LF, R, F, ROWS, TANH_ONLY>(y, wi, dot_chain<F>(xj, wj), c);
+            row_sums<T::LF, R, F, ROWS, TANH_ONLY && PRIORITY>(y, wi, dot_chain<F>(xj, wj), c);
             if constexpr (TANH_ONLY) {
                 float r[R][F];
                 sigmoids(0, y, c, xj, r);
-                issue_with_others();
+                issue_with_others<PRIORITY>();
 #pragma unroll
                 for (int rr = 0; rr < R; ++rr)
 #pragma unroll
@@ -305,7 +305,7 @@ __device__ __forceinline__ void inverse_core(float (&y)[R][F], float (&b)[R][F],
 // KU_W: the products ku Wi' are kept beside the weights (F more registers, one multiplication less per row and step).
 // IM_AT: 1/m of each step from the table (im_at).
 template <int NC, int EC, int R, int F, bool MASKED, bool TANH_ONLY = true, bool STEP_MASK = false, bool ROWS = false,
-          bool KU_W = true, bool IM_AT = false>
+          bool KU_W = true, bool IM_AT = false, bool PRIORITY = true>
 __device__ __forceinline__ void backward_core(float (&Y)[R][F], float (&B)[R][F], float (&G)[R][F], float (&P)[R][F],
                                               const float (&wi)[F], const float (&wj)[F], float (&dwi)[F],
                                               float (&dwj)[F], float own, const StepTable& S, int step_base, int lane,
@@ -313,7 +313,7 @@ __device__ __forceinline__ void backward_core(float (&Y)[R][F], float (&B)[R][F]
     using T = Tile<NC, EC, R, F>;
     // Rows of 16 features over two lanes (a radix pass on groups of two) have one instruction across lanes in a sum and no register to
     // spare: with priorities 25 spill in place of 5 (x[64, 4096, 128], 12 levels backward 692 us : 664).
-    constexpr bool kPriority = !(T::LR == 1 && T::LF == 2 && F == 8);
+    constexpr bool kPriority = PRIORITY && !(T::LR == 1 && T::LF == 2 && F == 8);
     const int rl = (lane / T::LF) % T::LR;
     float wiku[KU_W ? F : 1];   // ku Wi': G += rh (ku Wi') spares the product ku rh of every row and step
     if constexpr (KU_W) {
@@ -409,7 +409,7 @@ __device__ __forceinline__ void backward_core(float (&Y)[R][F], float (&B)[R][F]
 #pragma unroll
             for (int r0 = 0; r0 < R; r0 += RC) {
                 float r[RC][F];
-                if constexpr (TANH_ONLY) {
+                if constexpr (TANH_ONLY && kPriority) {
                     if (r0 > 0) issue_first();
                     sigmoids(r0, Y, c, xj, r);
                     issue_with_others();
@@ -422,6 +422,7 @@ __device__ __forceinline__ void backward_core(float (&Y)[R][F], float (&B)[R][F]
                     for (int f = 0; f < F; ++f) {
                         float w;
                         if constexpr (TANH_ONLY) {
+                            if constexpr (!kPriority) r[k][f] = __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(fmaf(c[rr], xj[f], Y[rr][f])) + 1.0f);
                             B[rr][f] = fmaf(S.bk1, r[k][f], fmaf(im, B[rr][f], S.bk0));   // bh before this step
                             w = fmaf(-r[k][f], r[k][f], r[k][f]);
                         } else {
@@ -436,9 +437,9 @@ __device__ __forceinline__ void backward_core(float (&Y)[R][F], float (&B)[R][F]
                     }
                 }
             }
-            issue_first();
+            issue_first<kPriority>();
             lane_sum_n<1, T::LF, ROWS, R>(rh);
-            issue_with_others();
+            issue_with_others<kPriority>();
             float rhosum = 0.f;
 #pragma unroll
             for (int rr = 0; rr < R; ++rr) {
@@ -459,9 +460,9 @@ __device__ __forceinline__ void backward_core(float (&Y)[R][F], float (&B)[R][F]
                 dwj[f] = fmaf(rhosum_w, xj[f], dwj[f]);
                 t[f] = fmaf(rhosum, wj[f], v[f]);
             }
-            issue_first();
+            issue_first<kPriority>();
             lane_sum_n<T::LF, T::LPG, ROWS, F>(t);   // over the group's row lanes
-            issue_with_others();
+            issue_with_others<kPriority>();
 #pragma unroll
             for (int f = 0; f < F; ++f) {
                 G[jr][f] = fmaf(selku, t[f], G[jr][f]);
@@ -494,7 +495,7 @@ __device__ __forceinline__ void scale_tile(float (&x)[R][F], float (&a)[R][F], f
 
 // one stage of the backward from true values to true values: G, H true gradients in and out; Y, B true outputs in,
 // true inputs out
-template <int NC, int EC, int R, int F, bool MASKED, bool TANH_ONLY, bool STEP_MASK = false>
+template <int NC, int EC, int R, int F, bool MASKED, bool TANH_ONLY, bool STEP_MASK = false, bool PRIORITY = true>
 __device__ __forceinline__ void backward_steps(float (&Y)[R][F], float (&B)[R][F], float (&G)[R][F], float (&P)[R][F],
                                                const float (&wi)[F], const float (&wj)[F], float (&dwi)[F],
                                                float (&dwj)[F], float own, const StepTable& S, int lane,
@@ -513,7 +514,7 @@ __device__ __forceinline__ void backward_steps(float (&Y)[R][F], float (&B)[R][F
                 P[rr][f] *= isc;
             }
         }
-    backward_core<NC, EC, R, F, MASKED, TANH_ONLY, STEP_MASK, true>(Y, B, G, P, wi, wj, dwi, dwj, own, S, 0, lane, slots,
+    backward_core<NC, EC, R, F, MASKED, TANH_ONLY, STEP_MASK, true, true, false, PRIORITY>(Y, B, G, P, wi, wj, dwi, dwj, own, S, 0, lane, slots,
                                                              live);
     const float dn = S.m_pow_n;       // NC steps done: undo the scaling of the gradients
 #pragma unroll
@@ -573,6 +574,17 @@ __device__ __forceinline__ void backward_steps(float (&Y)[R][F], float (&B)[R][F
 template <int TYPES>
 __device__ __forceinline__ int dtype_of(int from_args, int when_bf16) {
     return TYPES == kF32Types ? NCN_F32 : TYPES == kBf16Types ? when_bf16 : from_args;
+}
+
+// Where a stage's launches raise the priority of waves (issue_first).  Not for float32 on heads of less than a cache line and small groups: they wait for
+// lines that the next heads' waves ask for at about the same time, and waves that go first drift apart.  us, x[b, 4096, E], one stage, with : without
+// (0.18).  Forward, groups of 16, heads of 4, x[24, ., 64] 41.9 : 38.8 (39.5); of 8, heads of 8, x[24, ., 128] 46.6 : 43.2 (43.7); of 4, heads of 8,
+// x[64, ., 128] 168 : 161 (161).  Backward, groups of 8, heads of 16, x[64, ., 256] 386 : 361 (362); of 16, heads of 4, x[64, ., 64] 186 : 178 (177), where
+// exp2 of a row at a time without priorities take 203; of 4 and 2 as fast with them or faster (heads of 8, x[64, ., 256] 402 : 415).  Larger groups
+// gain 5 to 15 % at any width.
+constexpr bool stage_priority(int nc, int ec, int types, bool backward) {
+    const bool narrow = ec == 4 ? nc <= 16 : ec <= 16 && nc <= 8;
+    return !(types == kF32Types && narrow && (!backward || nc >= 8));
 }
 
 // float32 launches on arrays of that many elements ask for their rows with the non-temporal hint, on tiles of 4 x 4 and heads of
@@ -665,7 +677,7 @@ __global__ void __launch_bounds__(kBlockThreads, (R == 4 && F == 4) ? 5 : 1) sta
         if (A.aux0) { NCN_STORE_DEAD_ROWS(A.aux0, A.aux1, NCN_F32, x, a) }
         NCN_ZERO_DEAD_ROWS(x, a, true)
         scale_tile<R, F>(x, a, A.tab.kappa, A.tab.a_scale);
-        forward_core<NC, EC, R, F, TANH_ONLY, INDEXED, true>(x, a, wi, wj, A.tab, lane, slots, live);
+        forward_core<NC, EC, R, F, TANH_ONLY, INDEXED, true, stage_priority(NC, EC, TYPES, false)>(x, a, wi, wj, A.tab, lane, slots, live);
         scale_tile<R, F>(x, a, A.tab.inv_kappa, A.tab.inv_a_scale);
 #pragma unroll
         for (int rr = 0; rr < R; ++rr) {
@@ -698,7 +710,7 @@ __global__ void __launch_bounds__(kBlockThreads, (R == 4 && F == 4) ? 5 : 1) sta
         NCN_STORE_DEAD_ROWS(A.out0, A.out1, out_dtype, y, b)
         NCN_ZERO_DEAD_ROWS(y, b, true)
         scale_tile<R, F>(y, b, A.tab.kappa, A.tab.b_scale);
-        inverse_core<NC, EC, R, F, TANH_ONLY, INDEXED, true>(y, b, wi, wj, A.tab, lane, slots, live);
+        inverse_core<NC, EC, R, F, TANH_ONLY, INDEXED, true, stage_priority(NC, EC, TYPES, false)>(y, b, wi, wj, A.tab, lane, slots, live);
         scale_tile<R, F>(y, b, A.tab.inv_kappa, A.tab.inv_b_scale);
 #pragma unroll
         for (int rr = 0; rr < R; ++rr) {
@@ -759,7 +771,7 @@ __global__ void __launch_bounds__(kBlockThreads, (TANH_ONLY && R * F <= 16 && F 
         if (A.aux0) { NCN_STORE_DEAD_ROWS(A.aux0, A.aux1, NCN_F32, Y, B) }
         NCN_ZERO_DEAD_ROWS(Y, B, false)
         NCN_ZERO_DEAD_ROWS(G, H, false)
-        backward_steps<NC, EC, R, F, false, TANH_ONLY, INDEXED>(Y, B, G, H, wi, wj, dwi, dwj, 1.0f, A.tab, lane, slots,
+        backward_steps<NC, EC, R, F, false, TANH_ONLY, INDEXED, stage_priority(NC, EC, TYPES, true)>(Y, B, G, H, wi, wj, dwi, dwj, 1.0f, A.tab, lane, slots,
                                                                live);
 #pragma unroll
         for (int rr = 0; rr < R; ++rr) {
