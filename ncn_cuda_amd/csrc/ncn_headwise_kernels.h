@@ -230,9 +230,9 @@ __device__ __forceinline__ void headwise_backward_core(float (&Y)[R][F], float (
                 // every row lane of the group adds its share of sum_i rh_if: the sum over lanes at the end completes it
                 dwj[f] = fmaf(krho * rhs[f], xj[f], dwj[f]);
             }
-            issue_first();
+            issue_first<TANH_ONLY>();
             lane_sum_n<T::LF, T::LPG, ROWS, F>(t);   // over the group's row lanes
-            issue_with_others();
+            issue_with_others<TANH_ONLY>();
 #pragma unroll
             for (int f = 0; f < F; ++f) {
                 G[jr][f] = fmaf(selku, t[f], G[jr][f]);
